@@ -401,13 +401,15 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.blk_cp_a, (void *)m.blk_cp_b, (void *)m.blk_jd, (void *)m.blk_pcol, (void *)m.blk_prp,
                     (void *)m.blk_pdg, (void *)m.fs_col, (void *)m.fs_meta, (void *)m.blk_fdesc, (void *)m.blk_fpair,
                     (void *)m.blk_elp, (void *)m.blk_elr, (void *)m.blk_enlev, (void *)m.ell_col, (void *)m.ell_len, (void *)m.csr_ell,
+                    (void *)m.z_lcol, (void *)m.z_hcol, (void *)m.z_hslot, (void *)m.z_hcnt, (void *)m.z_send,
+                    (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_nchf, (void *)m.z_nchb,
                     (void *)m.fwd_rows, (void *)m.fwd_lptr, (void *)m.fwd_nlev, (void *)m.bwd_rows,
                     (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_el, (void *)m.tvd_kn, m.tvd_w,
                     (void *)m.tvd_lev, (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem})
         dfree(q);
     Solver &v = M.sv;
     for (void *q : {v.lu, v.ell_a, v.fs_val, v.r0, v.r, v.p0, v.p1, v.v0, v.v1, v.s, v.t, v.dx, v.b, v.x0, (void *)v.part,
-                    (void *)v.scal, (void *)v.ctrl, v.a32, (void *)v.r64, v.zprev})
+                    (void *)v.scal, (void *)v.ctrl, v.a32, (void *)v.r64, v.zprev, v.xch, (void *)v.pslot})
         dfree(q);
     for (hipStream_t st : M.tr_stream) (void)hipStreamSynchronize(st);
     for (hipStream_t st : M.tr_stream) (void)hipStreamDestroy(st);
@@ -836,6 +838,29 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
                 rc |= dalloc(M, &m.fs_col, fcol.size()) || upload(M, m.fs_col, fcol.data(), fcol.size());
                 rc |= dalloc(M, &m.fs_meta, fmeta.size()) || upload(M, m.fs_meta, fmeta.data(), fmeta.size());
                 rc |= dalloc_s(M, &M.sv.fs_val, (size_t)kEllWidth * nkn);
+            }
+            // tables and slots of the one-launch solve
+            ZetaTables zt;
+            host_zeta_tables(nkn, M.h_rowptr, M.h_cols, bs, (int)M.esize(), zt);
+            M.sv.zeta_t = zt.threads;
+            M.sv.zeta_nwg = zt.nwg;
+            M.sv.zeta_group = zt.group;
+            M.sv.zeta_hmax = zt.hmax;
+            M.sv.zeta_chmax = zt.chmax;
+            M.sv.zeta_nsend = zt.nsend;
+            M.sv.zeta_occ[0] = M.sv.zeta_occ[1] = 0;
+            if (zt.threads > 0) {
+                rc |= dalloc(M, &m.z_lcol, zt.lcol.size()) || upload(M, m.z_lcol, zt.lcol.data(), zt.lcol.size());
+                rc |= dalloc(M, &m.z_hcol, zt.hcol.size()) || upload(M, m.z_hcol, zt.hcol.data(), zt.hcol.size());
+                rc |= dalloc(M, &m.z_hslot, zt.hslot.size()) || upload(M, m.z_hslot, zt.hslot.data(), zt.hslot.size());
+                rc |= dalloc(M, &m.z_hcnt, zt.hcnt.size()) || upload(M, m.z_hcnt, zt.hcnt.data(), zt.hcnt.size());
+                rc |= dalloc(M, &m.z_send, zt.send.size()) || upload(M, m.z_send, zt.send.data(), zt.send.size());
+                rc |= dalloc(M, &m.z_chf, zt.chf.size()) || upload(M, m.z_chf, zt.chf.data(), zt.chf.size());
+                rc |= dalloc(M, &m.z_chb, zt.chb.size()) || upload(M, m.z_chb, zt.chb.data(), zt.chb.size());
+                rc |= dalloc(M, &m.z_nchf, zt.nchf.size()) || upload(M, m.z_nchf, zt.nchf.data(), zt.nchf.size());
+                rc |= dalloc(M, &m.z_nchb, zt.nchb.size()) || upload(M, m.z_nchb, zt.nchb.data(), zt.nchb.size());
+                rc |= dalloc_s(M, &M.sv.xch, (size_t)4 * zt.nsend);
+                rc |= dalloc(M, &M.sv.pslot, kZetaSlotWords);
             }
             rc |= dalloc(M, &m.ell_col, ecol.size()) || upload(M, m.ell_col, ecol.data(), ecol.size());
             rc |= dalloc(M, &m.ell_len, elen.size()) || upload(M, m.ell_len, elen.data(), elen.size());

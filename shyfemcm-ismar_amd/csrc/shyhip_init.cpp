@@ -628,4 +628,122 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
     });
 }
 
+// Tables of the one-launch zeta solve.  It needs: one row per work-item,
+// every row within the ELL slots, one work-item per workgroup to collect the
+// partial sums (at most 256 workgroups), and halos of at most 2 entries (256
+// work-items) or 1 (more) per work-item.  Workgroups of 256 work-items up to
+// kZetaSmall of them, else of 512: the product and sweeps take longer there,
+// the exchange among half as many is faster.  Measured steps, 256 against
+// 512 (hydro only, FP64 / FP32): 20k nodes 0.277 / 0.319 against 0.296 /
+// 0.333 ms, 50k nodes 0.391 / 0.448 against 0.371 / 0.403 ms; the line lies
+// between.  Blocks longer than 512 rows take 1024.
+constexpr int kZetaSmall = 128;
+
+static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
+                        int esize, int T, ZetaTables &zt) {
+    const int nblk = bs.nblk, group = T / bs.brows, brows = group * bs.brows, nwg = (nblk + group - 1) / group;
+    if (nwg > 256) return false;
+    // halos: the columns outside the workgroup's rows, ascending
+    std::vector<std::vector<int>> halo(nwg);
+    parallel_for(nwg, 16, [&](int b_begin, int b_end) {
+        for (int b = b_begin; b < b_end; b++) {
+            const int b0 = b * brows, b1 = std::min(n, b0 + brows);
+            std::vector<int> &h = halo[b];
+            for (int q = rowptr[b0]; q < rowptr[b1]; q++)
+                if (cols[q] < b0 || cols[q] >= b1) h.push_back(cols[q]);
+            std::sort(h.begin(), h.end());
+            h.erase(std::unique(h.begin(), h.end()), h.end());
+        }
+    });
+    int hmax = 1;
+    for (const auto &h : halo) hmax = std::max(hmax, (int)h.size());
+    if (hmax > (T == 256 ? 512 : T)) return false;
+    zt.hmax = hmax;
+    zt.hcol.assign((size_t)nwg * hmax, 0);
+    zt.hcnt.assign(nwg, 0);
+    zt.hslot.assign((size_t)nwg * hmax, 0);
+    zt.send.assign(n, -1);
+    zt.lcol.assign((size_t)(kEllWidth / 2) * n, 0u);
+    // value slots in row order, each workgroup's first slot on a line of its own
+    for (const auto &h : halo)
+        for (int j : h) zt.send[j] = 0;
+    zt.nsend = 0;
+    for (int b = 0; b < nwg; b++) {
+        for (int i = b * brows; i < std::min(n, (b + 1) * brows); i++)
+            if (zt.send[i] == 0) zt.send[i] = zt.nsend++;
+        zt.nsend = (zt.nsend + 15) / 16 * 16;
+    }
+    for (int b = 0; b < nwg; b++) {
+        zt.hcnt[b] = (int)halo[b].size();
+        for (size_t h = 0; h < halo[b].size(); h++) {
+            zt.hcol[(size_t)b * hmax + h] = halo[b][h];
+            zt.hslot[(size_t)b * hmax + h] = zt.send[halo[b][h]];
+        }
+    }
+    parallel_for(nwg, 16, [&](int b_begin, int b_end) {
+        for (int b = b_begin; b < b_end; b++) {
+            const int b0 = b * brows, b1 = std::min(n, b0 + brows);
+            for (int i = b0; i < b1; i++) {
+                const int q0 = rowptr[i], len = rowptr[i + 1] - q0;
+                for (int k = 0; k < kEllWidth; k++) {
+                    int idx = i - b0;                       // padding: the row itself
+                    if (k < len) {
+                        const int j = cols[q0 + k];
+                        idx = (j >= b0 && j < b1)
+                                  ? j - b0
+                                  : brows + (int)(std::lower_bound(halo[b].begin(), halo[b].end(), j) - halo[b].begin());
+                    }
+                    zt.lcol[(size_t)(k / 2) * n + i] |= (unsigned)(idx * esize) << (16 * (k & 1));
+                }
+            }
+        }
+    });
+    // exact substitution: the rows of each level in chunks of 64; the chunk
+    // list ends with three empty chunks (the substitution reads ahead)
+    const int stride = bs.brows + 1;
+    std::vector<std::vector<unsigned>> ch[2];
+    for (int dir = 0; dir < 2; dir++) {
+        const std::vector<int> &lptr = dir == 0 ? bs.fwd_lptr : bs.bwd_lptr;
+        const std::vector<int> &nlev = dir == 0 ? bs.fwd_nlev : bs.bwd_nlev;
+        std::vector<int> &nch = dir == 0 ? zt.nchf : zt.nchb;
+        ch[dir].resize(nblk);
+        nch.assign(nblk, 0);
+        for (int b = 0; b < nblk; b++) {
+            for (int l = 0; l < nlev[b]; l++) {
+                const int t1 = lptr[(size_t)b * stride + l + 1];
+                for (int t = lptr[(size_t)b * stride + l]; t < t1; t += 64)
+                    ch[dir][b].push_back((unsigned)t | (unsigned)std::min(64, t1 - t) << 16);
+            }
+            nch[b] = (int)ch[dir][b].size();
+        }
+    }
+    int chmax = 0;
+    for (int b = 0; b < nblk; b++) chmax = std::max({chmax, zt.nchf[b] + 3, zt.nchb[b] + 3});
+    zt.chmax = chmax;
+    for (int dir = 0; dir < 2; dir++) {
+        std::vector<unsigned> &out = dir == 0 ? zt.chf : zt.chb;
+        out.assign((size_t)nblk * chmax, 0u);
+        for (int b = 0; b < nblk; b++) std::copy(ch[dir][b].begin(), ch[dir][b].end(), out.begin() + (size_t)b * chmax);
+    }
+    zt.threads = T;
+    zt.nwg = nwg;
+    zt.group = group;
+    return true;
+}
+
+void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
+                      int esize, ZetaTables &zt) {
+    zt = ZetaTables();
+    if (bs.brows > 1024) return;
+    for (int i = 0; i < n; i++)
+        if (rowptr[i + 1] - rowptr[i] > kEllWidth) return;
+    if (bs.brows > 512) {
+        zeta_tables(n, rowptr, cols, bs, esize, 1024, zt);
+        return;
+    }
+    const int n256 = bs.brows <= 256 ? (bs.nblk + 256 / bs.brows - 1) / (256 / bs.brows) : 1 << 30;
+    if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, zt)) return;
+    if (bs.brows <= 256) zeta_tables(n, rowptr, cols, bs, esize, 256, zt);
+}
+
 }  // namespace shy

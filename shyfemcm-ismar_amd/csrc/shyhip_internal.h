@@ -86,6 +86,16 @@ struct Mesh {                 // device copies of init-time data
     // row itself) and nL | cnt << 8 per row (absent if a block row is longer
     // than kEllWidth)
     int *fs_col = nullptr, *fs_meta = nullptr;
+    // one-launch solve (host_zeta_tables): byte offsets of each row's ELL
+    // columns in its workgroup's operand (rows, then halo), two per word
+    // [k/2][nkn]; each workgroup's halo rows, their value slots and number;
+    // the value slot of a row that is in another one's halo (or -1): a
+    // workgroup's slots lie together; the exact substitutions' chunks (at most 64 rows of one
+    // level: first position | rows << 16, positions in fwd_rows / bwd_rows
+    // relative to the block) and chunks per block
+    unsigned *z_lcol = nullptr, *z_chf = nullptr, *z_chb = nullptr;
+    int *z_hcol = nullptr, *z_hslot = nullptr, *z_hcnt = nullptr, *z_send = nullptr, *z_nchf = nullptr,
+        *z_nchb = nullptr;
     int *fwd_rows = nullptr, *fwd_lptr = nullptr, *fwd_nlev = nullptr;
     int *bwd_rows = nullptr, *bwd_lptr = nullptr, *bwd_nlev = nullptr;
     // TVD upwind tables: per element 6 ordered pairs (ic,id); [p*nel + ie]
@@ -157,9 +167,10 @@ struct State {
 // iteration-limit flags, its matvec count, iterations of all inner solves of
 // this zeta solve, FP64 refinement converged, factorisation failure,
 // refinements done; words CT_ITS..CT_NREF are cleared at the start of a solve
-// CT_RITS.. hold the iterations of each refinement round (FP32 path)
+// CT_RITS.. hold the iterations of each refinement round (FP32 path);
+// CT_WAIT: a workgroup of the one-launch solve waited too long for another
 enum { CT_STOPIT = 0, CT_CONV = 1, CT_FAIL = 2, CT_NMV = 3, CT_ITS = 4, CT_REFCONV = 5, CT_FACTOR = 6,
-       CT_NREF = 7, CT_MAXIT = 8, CT_RITS = 9, CT_NRITS = 6, CT_WORDS = 16 };
+       CT_NREF = 7, CT_MAXIT = 8, CT_RITS = 9, CT_NRITS = 6, CT_WAIT = 15, CT_WORDS = 16 };
 
 struct Solver {               // Krylov work space (value type V = S of the model)
     int nblk = 0, brows = 0, max_blk_nnz = 0, max_blk_pairs = 0, nparts = 0, max_elev = 0;
@@ -183,7 +194,17 @@ struct Solver {               // Krylov work space (value type V = S of the mode
     bool fed = false;         // the assembly already wrote the solve's inputs (ELL
                               // slots, FP32 copy, initial guess, cleared words)
     double *r64 = nullptr;    // FP64 residual (refinement)
+    // one-launch solve: its workgroup size (0: not possible for this basin),
+    // workgroups and diagonal blocks of each, halo and chunk strides, exchange slots (4 buffers: values, partials);
+    // workgroups per compute unit of each kind of triangular solve (0: not
+    // asked yet, -1: cannot run), device and its compute units
+    int zeta_t = 0, zeta_nwg = 0, zeta_group = 1, zeta_hmax = 0, zeta_chmax = 0, zeta_nsend = 0;
+    void *xch = nullptr;
+    unsigned long long *pslot = nullptr;
+    int zeta_occ[2] = {0, 0}, zeta_dev = 0, zeta_cus = 0;
 };
+
+constexpr size_t kZetaSlotWords = (size_t)4 * 16 * 512 * 5;   // partial-sum slots of the one-launch solve
 
 // kernel groups timed with HIP events when timing is enabled
 enum TimerId { T_SETDRY = 0, T_COPY, T_INTERN, T_SETNOD, T_ZETA, T_SOLVE, T_WETDRY, T_FINAL, T_SETUVD, T_DEPTH,
@@ -402,6 +423,15 @@ struct BlockSchedule {
 };
 void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, int brows,
                          BlockSchedule &bs);
+// tables of the one-launch solve (Mesh::z_*) for values of esize bytes;
+// threads: its workgroup size, 0 when the basin's blocks do not fit it
+struct ZetaTables {
+    int threads = 0, nwg = 0, group = 1, hmax = 0, chmax = 0, nsend = 0;
+    std::vector<unsigned> lcol, chf, chb;
+    std::vector<int> hcol, hslot, hcnt, send, nchf, nchb;
+};
+void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
+                      int esize, ZetaTables &zt);
 
 // kernel launchers (shyhip_hydro.hip, shyhip_solver.hip, shyhip_conz.hip)
 int launch_set_dry(Model &M, int iweich, int bnewtime, int *changed);

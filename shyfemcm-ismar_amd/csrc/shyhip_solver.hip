@@ -13,18 +13,21 @@
 // Krylov method: BiCGStab in the arrangement the reference uses -- runrc with
 // ipar(2)=1, which bisinit maps to LEFT preconditioning (spk_iters.f90:
 // 1061-1334, 3433-3500) -- with stopping test ||M^-1 r|| <= rtol*||M^-1 r0||
-// + atol and at most itermax matvecs.  One iteration is two kernels: every
-// vector update is fused into the SpMV/preconditioner kernel that consumes
-// it (the update of x and r closing an iteration is done by the first kernel
-// of the next, from five dot products of the second), and every dot product
-// is written as per-workgroup partials that every workgroup of the next
-// kernel reduces itself in the same fixed order -- no atomics or
-// device-scope fences, visibility comes from the kernel boundary, and all
-// workgroups (and all runs) see bitwise identical scalars.
+// + atol and at most itermax matvecs.  Basins whose blocks can all be
+// resident at once are solved in one launch (k_zeta, see there).  The others
+// take two kernels per iteration: every vector update is fused into the
+// SpMV/preconditioner kernel that consumes it (the update of x and r closing
+// an iteration is done by the first kernel of the next, from five dot
+// products of the second), and every dot product is written as per-workgroup
+// partials that every workgroup of the next kernel reduces itself in the
+// same fixed order -- no atomics or device-scope fences, visibility comes
+// from the kernel boundary, and all workgroups (and all runs) see bitwise
+// identical scalars.
 // The FP32 path runs this in FP32 inside an FP64 iterative refinement whose
-// control also lives on the device: every kernel of a refinement round
-// returns at once when the FP64 residual test has passed, so the host
-// enqueues the expected number of rounds and reads the flags once.
+// control also lives on the device: inside the one launch, or every kernel
+// of a refinement round returns at once when the FP64 residual test has
+// passed, so the host enqueues the expected number of rounds and reads the
+// flags once.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -32,7 +35,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <functional>
+#include <mutex>
 
 #include "shyhip_internal.h"
 
@@ -71,6 +76,12 @@ struct SolvArgs {
     double *part, *scal;
     int *ctrl;
     int nparts;      // stride of one partial-sum array
+    // exchange slots of the one-launch solve, emptied by the factorisation
+    // (null: not used)
+    void *xch;
+    unsigned long long *pslot;
+    const int *send;
+    int nsend, zgroup;
 };
 
 template <typename V>
@@ -100,6 +111,13 @@ static SolvArgs<V> solv_args(Model &M, const V *A, V *b, V *x0) {
     a.v0 = (V *)M.sv.v0; a.v1 = (V *)M.sv.v1; a.s = (V *)M.sv.s; a.t = (V *)M.sv.t; a.dx = (V *)M.sv.dx;
     a.part = M.sv.part; a.scal = M.sv.scal; a.ctrl = M.sv.ctrl;
     a.nparts = M.sv.nparts;
+    if (M.sv.zeta_t > 0) {
+        a.xch = M.sv.xch;
+        a.pslot = M.sv.pslot;
+        a.send = M.m.z_send;
+        a.nsend = M.sv.zeta_nsend;
+        a.zgroup = M.sv.zeta_group;
+    }
     return a;
 }
 
@@ -448,11 +466,16 @@ constexpr int kFactorThreads = 256;
 constexpr int kWarmEntries = 8;
 
 template <typename V>
+__device__ inline void zeta_empty_slots(const SolvArgs<V> &a, int blk, int b0, int nb);
+
+template <typename V>
 __global__ __launch_bounds__(kFactorThreads) void k_bilu_factor(SolvArgs<V> a, int stage, int sweeps) {
     extern __shared__ double smem[];
     V *val = reinterpret_cast<V *>(smem);
     const int blk = blockIdx.x, b0 = blk * a.brows;
     const int nb = min(a.n, b0 + a.brows) - b0;
+    // the one-launch solve that follows: no slot filled, no flag set
+    if (a.pslot) zeta_empty_slots(a, blk, b0, nb);
     const int q0 = a.brp[b0], q1 = a.brp[b0 + nb], ne = q1 - q0;
     const int p0 = a.cp_ptr[q0], np = a.cp_ptr[q1] - p0;
     const int nl = a.enlev[blk];
@@ -995,6 +1018,764 @@ __global__ __launch_bounds__(kThreads) void k_resid_check(const double *part, in
     }
 }
 
+// ---------------------------------------------------------------- one-launch solve
+// The whole Krylov solve (and on the FP32 path the refinement around it) in
+// one launch, one workgroup per diagonal block, one row per work-item: the
+// row's matrix and factor entries and its vector elements stay in registers
+// for the solve, and the workgroups exchange what the next half iteration
+// needs through memory instead of ending the kernel.
+//
+// What bounds it: the chain of a half iteration -- product, triangular
+// sweeps, one exchange -- not bytes (8 MB per product on 50k rows).  As two
+// kernels per iteration the same chain also paid a kernel boundary and two
+// rounds of loads of the matrix, factors and vectors every time: 16.4 us per
+// FP64 iteration on the 50k-node lagoon (196 blocks), 9.7 us as one launch;
+// a hydro step there 0.60 -> 0.37 ms, on 3k nodes 0.35 -> 0.21 ms, FP32 on
+// 60k nodes 0.61 -> 0.40 ms.  A load that sees another XCD's store takes
+// 0.9 us (12 workgroups) to 1.5 us (98), the two sums 0.4 us, the product
+// and 3 sweeps 1.6 us (256 work-items) or 2.0 us (512).
+//
+// Exchange.  Each half iteration has an epoch.  A workgroup puts its partial
+// sums into its own slots, and the elements of v (or t) that rows of other
+// blocks multiply into theirs; the readers wait until a slot holds a value.
+// Every slot is one machine word, written and read by relaxed agent-scope
+// atomics (they go through to memory that all XCDs see), and an empty slot
+// holds a NaN pattern that no put ever writes, so a word is its own flag and
+// an exchange is one store and one load latency long.  Slots rotate over
+// four buffers: at epoch e a workgroup has every partial of epoch e-1, so
+// every workgroup has finished reading epoch e-2, and it empties its own
+// slots of that buffer (next used at e+2), with the stores complete before
+// it puts its partials of epoch e.  The factorisation kernel of each solve
+// empties all slots.
+//
+// A block's neighbour rows in other blocks (its halo) are kept as well: the
+// recurrences of p, r, s (and the correction) are run on them redundantly,
+// with the same operations, so only v and t are exchanged and the halo
+// values have the owner's bits.  Every workgroup adds the partial sums in the
+// same fixed order, so all of them (and all runs) take the same decisions.
+//
+// The waits are bounded: the launch is made only when all its workgroups
+// can be resident together (zeta_slots), and a wait that still runs out sets
+// CT_WAIT and ends the workgroup.  Every other workgroup then runs out of
+// its own wait, and the host makes the solve with the two-kernel iteration.
+// The result counts only once every workgroup has written its part of it:
+// each puts one more partial after its stores, and the workgroup that sets
+// the convergence flags collects them first.
+constexpr int kWaitExpired = -9;
+constexpr int kSpinLimit = 1 << 17;      // polls of one wait (about 0.1 s)
+constexpr int kZetaBufs = 4;
+// Partial sums per workgroup and buffer, and their copies: every workgroup
+// reads everyone's, so one copy makes all workgroups wait for the same few
+// memory lines (196 workgroups: a half iteration of 5.8 us with one copy,
+// 5.3 us with 16); each workgroup puts its sums into every copy and reads
+// one.  Copies lie apart.
+constexpr int kPartSlots = 5;
+constexpr int kPartCopies = 16;
+constexpr int kPartStride = 512 * 5;     // words per copy: [kPartSlots][512], at most 256 of each used
+
+template <typename V>
+struct Slot;
+template <>
+struct Slot<double> {
+    using U = unsigned long long;
+    static constexpr U empty = 0x7ff8a5a55a5a0001ull, nan = 0x7ff8000000000000ull;
+};
+template <>
+struct Slot<float> {
+    using U = unsigned;
+    static constexpr U empty = 0x7fc0a5a5u, nan = 0x7fc00000u;
+};
+template <typename V>
+__device__ inline void slot_put(typename Slot<V>::U *p, V v) {
+    using U = typename Slot<V>::U;
+    __hip_atomic_store(p, v == v ? __builtin_bit_cast(U, v) : Slot<V>::nan, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+__device__ inline void slot_clear(U *p, U empty) {
+    __hip_atomic_store(p, empty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+__device__ inline U slot_get(const U *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ inline unsigned long long *part_slot(unsigned long long *pslot, int buf, int copy, int k, int wg) {
+    return pslot + ((size_t)buf * kPartCopies + copy) * kPartStride + k * 512 + wg;
+}
+
+// the slots of block blk empty in every buffer, and the solve's flags clear
+template <typename V>
+__device__ inline void zeta_empty_slots(const SolvArgs<V> &a, int blk, int b0, int nb) {
+    auto *xch = (typename Slot<V>::U *)a.xch;
+    for (int b = 0; b < kZetaBufs; b++) {
+        for (int li = threadIdx.x; li < nb; li += blockDim.x)
+            if (const int q = a.send[b0 + li]; q >= 0) slot_clear(xch + (size_t)b * a.nsend + q, Slot<V>::empty);
+        if (blk % a.zgroup == 0 && threadIdx.x < kPartSlots * kPartCopies)
+            slot_clear(part_slot(a.pslot, b, threadIdx.x % kPartCopies, threadIdx.x / kPartCopies, blk / a.zgroup),
+                       Slot<double>::empty);
+    }
+    if (blk == 0 && threadIdx.x == 0) {
+        a.ctrl[CT_CONV] = 0; a.ctrl[CT_FAIL] = 0; a.ctrl[CT_MAXIT] = 0; a.ctrl[CT_WAIT] = 0;
+    }
+}
+
+// every store this work-item has issued is complete
+__device__ __attribute__((always_inline)) inline void wait_stores() {
+    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+}
+
+struct ZetaArgs {
+    int nwg, group;                      // workgroups, diagonal blocks of each
+    int hmax;                            // halo stride per workgroup
+    const unsigned *lcol;                // byte offsets of the row's columns, two per word [k/2][n]
+    const int *hcol, *hslot, *hcnt;      // halo rows and their slots [wg*hmax + h], their number
+    const int *send;                     // slot of a row in other workgroups' halos, or -1
+    int nsend;                           // value slots per buffer
+    // exact substitution: rows in its order, their chunks (stride per block)
+    const int *rows_f, *rows_b;
+    const unsigned *chunk_f, *chunk_b;
+    const int *nch_f, *nch_b;
+    int chmax;
+    void *xch;                           // value slots [buf][nsend]
+    unsigned long long *pslot;           // partial-sum slots [buf][kPartCopies][kPartStride]
+    // FP32 path: the FP64 system and its refinement
+    const double *rhs;
+    double *x;
+    double tol;
+    int maxref;
+};
+
+// sums over a workgroup of T work-items, like block_sum; TAG keeps the LDS
+// of consecutive sums apart, so one barrier per sum is enough (a sum's LDS
+// is written again only after other barriers)
+template <int T, int NQ, int TAG>
+__device__ __attribute__((always_inline)) inline void wg_sum(double (&v)[NQ]) {
+    __shared__ double red[NQ][T / 64];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) v[q] = wave_sum(v[q]);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) red[q][threadIdx.x >> 6] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+        if constexpr (T / 64 >= 8) {
+            // 8 or 16 wavefronts: their sums one per lane of half a row or a row
+            double t = red[q][threadIdx.x & (T / 64 - 1)];
+            t = t + dpp_f64<0xB1>(t);
+            t = t + dpp_f64<0x4E>(t);
+            t = t + dpp_f64<0x141>(t);
+            v[q] = T / 64 == 8 ? t : t + dpp_f64<0x140>(t);
+        } else {
+            double t = red[q][0];
+#pragma unroll
+            for (int w = 1; w < T / 64; w++) t += red[q][w];
+            v[q] = t;
+        }
+    }
+}
+
+// Exact substitution with one triangular factor of a block by one wavefront
+// (wavefront g of the workgroup takes its block g): rows level by level (a level's rows depend only on earlier
+// levels), up to 64 rows of a level at a time, one lane per row.  One
+// wavefront needs no barrier between levels (its LDS accesses run in
+// order).  The rows lie in LDS in the order of the substitution, their first
+// kSubFirst entries slot-major with zero padding, so the next chunk's
+// entries are read, at fixed offsets from one address, while the current
+// chunk waits for its operands: a chunk costs one LDS gather and its chain of
+// subtractions.  What bounds it is that chain times the number of levels
+// (62 levels each way on the 41x21 basin: with a barrier of the workgroup
+// per level and the factors in global memory a solve of 20 iterations took
+// 3.7 ms, with the factors read in the list order by one wavefront 1.26 ms,
+// in this layout 0.95 ms).
+// A row's word: byte offset of its value | further entries << 16 (these few
+// rows take them from the block's entry list).
+constexpr int kSubFirst = 4;
+
+template <typename V, int ROWS>
+struct SubExact {
+    const V *val, *piv;                  // [kSubFirst][ROWS], inverted pivots [ROWS]
+    const unsigned *col;                 // byte offsets [kSubFirst / 2][ROWS], two per word
+    const unsigned *row, *tail;          // the rows' words and first further entries [ROWS]
+    const unsigned *chunk;               // first row | rows << 16 of each chunk of the block
+    const V *lu;                         // the block's entries and local columns (global memory)
+    const int *pcol;
+    int nch, r0;                         // chunks and first row of the block
+
+    template <bool BACK>
+    __device__ __attribute__((always_inline)) inline void run(V *y) const {
+        const int lane = threadIdx.x & 63;
+        char *yb = reinterpret_cast<char *>(y);
+        auto at = [&](unsigned o) __attribute__((always_inline)) -> V & { return *reinterpret_cast<V *>(yb + o); };
+        V v[kSubFirst], p = 0, rhs;
+        unsigned c[kSubFirst / 2], r, r1;
+        unsigned w = chunk[0], w1 = chunk[1], w2 = chunk[2];      // (padded)
+        // (lanes beyond a chunk's rows read some row and write nothing)
+        auto pos = [&](unsigned c0) __attribute__((always_inline)) { return min(r0 + (int)(c0 & 0xffffu) + lane, ROWS - 1); };
+        int t = pos(w), t1 = pos(w1);
+        r = row[t];
+        r1 = row[t1];
+        auto entries = [&](int tt) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < kSubFirst; k++) v[k] = val[k * ROWS + tt];
+#pragma unroll
+            for (int k = 0; k < kSubFirst / 2; k++) c[k] = col[k * ROWS + tt];
+            if (BACK) p = piv[tt];
+        };
+        entries(t);
+        rhs = at(r & 0xffffu);
+        for (int ch = 0; ch < nch; ch++) {
+            V g[kSubFirst], vc[kSubFirst];
+#pragma unroll
+            for (int k = 0; k < kSubFirst; k++) {
+                g[k] = at((k & 1) ? c[k / 2] >> 16 : c[k / 2] & 0xffffu);
+                vc[k] = v[k];
+            }
+            V acc = rhs;
+            const V pc = p;
+            const unsigned rc = r;
+            const int tc = t;
+            const bool on = lane < (int)(w >> 16);
+            // ahead: the next chunk's entries, the one after's row word
+            w = w1; w1 = w2; w2 = chunk[ch + 3];
+            t = t1; r = r1;
+            entries(t);
+            rhs = at(r & 0xffffu);
+            t1 = pos(w1);
+            r1 = row[t1];
+#pragma unroll
+            for (int k = 0; k < kSubFirst; k++) acc = acc - vc[k] * g[k];
+            const int more = on ? (int)(rc >> 16) : 0;
+            if (__any(more)) {
+                const int q = (int)tail[tc];
+                for (int k = 0; k < more; k++) acc = acc - lu[q + k] * y[r0 + pcol[q + k]];
+            }
+            if (on) at(rc & 0xffffu) = BACK ? pc * acc : acc;
+        }
+    }
+};
+
+// One row of the solve and its block's halo entries, in registers (1024
+// work-items have half the registers of 256 each: they read the matrix row
+// from cache in every product instead of spilling).  The entries of a row
+// are padded with zeros at the row's own column, so that all operands are
+// read at once and the terms added without a test per entry (a test each
+// made every entry wait for its own LDS read: 2.8 us of product and sweeps
+// per half iteration on 256 rows, 1.6 us without); the last slots, which few rows
+// fill, are taken only by the wavefronts that hold such a row.
+constexpr int kRowFirst = 8;             // matrix entries always taken
+constexpr int kTriWidth = kFacWidth - 1; // entries of a row on one side of the diagonal
+constexpr int kTriFirst = 6;             // of these always taken
+
+template <typename V, int T, int KH, bool EXACT>
+struct ZetaRow {
+    using U = typename Slot<V>::U;
+    static constexpr bool kHold = T <= 512;
+    static constexpr int kTri = EXACT ? 1 : kTriWidth, kTriWords = (kTri + 1) / 2;
+    // matrix row; (sweeps) factor row: L and U entries, inverted pivot
+    V a[kHold ? kEllWidth : 1], l[kTri], u[kTri], dinv = 0;
+    unsigned lc[kHold ? kEllWidth / 2 : 1], llc[kTriWords], uc[kTriWords];
+    const V *ga;
+    const unsigned *glc;
+    bool more_a = false, more_l = false, more_u = false;   // some row of the wavefront fills the last slots
+    int i, wg, nh, nwg, n, sweeps, send, nsend;
+    bool mine;
+    int hslot[KH];
+    // LDS: operand (rows, then halo), two row buffers; exact: block factors
+    V *X, *y, *w;
+    SubExact<V, T> sf, sb;
+    int rows, group;
+    U *xch;
+    unsigned long long *pslot;
+    int epoch = 0;
+    int *dead;
+
+    // byte offset k of the offsets packed two per word
+    __device__ static __attribute__((always_inline)) inline unsigned off(const unsigned *words, int k) {
+        return (k & 1) ? words[k / 2] >> 16 : words[k / 2] & 0xffffu;
+    }
+    __device__ static __attribute__((always_inline)) inline V at(const V *base, unsigned o) {
+        return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + o);
+    }
+    // t + SIGN * (terms K0 .. K1-1 of the row v, c), in order
+    template <int K0, int K1, int SIGN>
+    __device__ static __attribute__((always_inline)) inline V terms(V t, const V *v, const unsigned *c, const V *x) {
+        V g[K1 - K0];
+#pragma unroll
+        for (int k = K0; k < K1; k++) g[k - K0] = at(x, off(c, k));
+#pragma unroll
+        for (int k = K0; k < K1; k++) t = SIGN > 0 ? t + v[k] * g[k - K0] : t - v[k] * g[k - K0];
+        return t;
+    }
+    // operand of the product: this row's element and its halo entries
+    __device__ __attribute__((always_inline)) inline void operand(V own, const V (&h)[KH]) {
+        if (mine) X[threadIdx.x] = own;
+#pragma unroll
+        for (int k = 0; k < KH; k++)
+            if ((int)threadIdx.x + k * T < nh) X[rows + threadIdx.x + k * T] = h[k];
+    }
+    // A X of this row, terms in column order
+    __device__ __attribute__((always_inline)) inline V product() {
+        V t = 0;
+        if constexpr (kHold) {
+            __syncthreads();
+            t = terms<0, kRowFirst, 1>(t, a, lc, X);
+            if (more_a) t = terms<kRowFirst, kEllWidth, 1>(t, a, lc, X);
+        } else {
+            V av[kEllWidth];
+            unsigned cv[kEllWidth / 2];
+#pragma unroll
+            for (int k = 0; k < kEllWidth; k++) av[k] = mine ? ga[(size_t)k * n + i] : (V)0;
+            columns(cv);
+            __syncthreads();
+            t = terms<0, kRowFirst, 1>(t, av, cv, X);
+            if (more_a) t = terms<kRowFirst, kEllWidth, 1>(t, av, cv, X);
+        }
+        return t;
+    }
+    __device__ __attribute__((always_inline)) inline void columns(unsigned (&cv)[kEllWidth / 2]) const {
+#pragma unroll
+        for (int k = 0; k < kEllWidth / 2; k++) {
+            if constexpr (kHold) cv[k] = lc[k];
+            else cv[k] = mine ? glc[(size_t)k * n + i] : 0u;
+        }
+    }
+    // (LU)^-1 of the block applied to the rows' values t: this row's result
+    // (the operations of FacRow::lusol and block_lusol)
+    __device__ __attribute__((always_inline)) inline V precond(V t) {
+        if (mine) y[threadIdx.x] = t;
+        __syncthreads();
+        if constexpr (EXACT) {
+            if ((int)threadIdx.x < 64 * group) {
+                sf.template run<false>(y);
+                sb.template run<true>(y);
+            }
+            __syncthreads();
+            return mine ? y[threadIdx.x] : (V)0;
+        } else {
+            V *src = y, *dst = w, bl = t, cur = t;
+            for (int s = 1; s < sweeps; s++) {
+                cur = terms<0, kTriFirst, -1>(bl, l, llc, src);
+                if (more_l) cur = terms<kTriFirst, kTri, -1>(cur, l, llc, src);
+                if (mine) dst[threadIdx.x] = cur;
+                __syncthreads();
+                V *sw = src; src = dst; dst = sw;
+            }
+            bl = cur;
+            cur = dinv * bl;
+            for (int s = 1; s < sweeps; s++) {
+                if (mine) dst[threadIdx.x] = cur;
+                __syncthreads();
+                V *sw = src; src = dst; dst = sw;
+                cur = terms<0, kTriFirst, -1>(bl, u, uc, src);
+                if (more_u) cur = terms<kTriFirst, kTri, -1>(cur, u, uc, src);
+                cur = dinv * cur;
+            }
+            return cur;
+        }
+    }
+    // Exchange of one epoch: the workgroups' partial sums of q (totals
+    // returned to everyone) and, with HALO, the rows' values own (the halo
+    // entries returned in h).  False when a wait ran out.
+    template <int NQ, bool HALO>
+    __device__ __attribute__((always_inline)) inline bool exchange(double (&q)[NQ], V own, V (&h)[KH]) {
+        if (nwg == 1) {
+            wg_sum<T, NQ, 0>(q);
+            return true;
+        }
+        const int buf = epoch & (kZetaBufs - 1);
+        U *vs = xch + (size_t)buf * nsend;
+        wait_stores();          // the slots emptied after the last exchange
+        if (HALO && send >= 0) slot_put<V>(vs + send, own);
+        wg_sum<T, NQ, 0>(q);
+        const int tk = threadIdx.x / kPartCopies, tcopy = threadIdx.x % kPartCopies;
+        if (tk < NQ) {
+            double mine_q = q[0];
+#pragma unroll
+            for (int k = 1; k < NQ; k++)
+                if (tk == k) mine_q = q[k];
+            slot_put<double>(part_slot(pslot, buf, tcopy, tk, wg), mine_q);
+        }
+        const unsigned long long *ps = part_slot(pslot, buf, wg % kPartCopies, 0, threadIdx.x);
+        unsigned long long pv[NQ];
+        U hv[KH];
+        const bool hasp = (int)threadIdx.x < nwg;
+        int spin = 0;
+        for (;;) {
+            bool ok = true;
+            if (hasp)
+#pragma unroll
+                for (int k = 0; k < NQ; k++) pv[k] = slot_get(ps + k * 512);
+            if (HALO)
+#pragma unroll
+                for (int k = 0; k < KH; k++)
+                    if ((int)threadIdx.x + k * T < nh) hv[k] = slot_get(vs + hslot[k]);
+            if (hasp)
+#pragma unroll
+                for (int k = 0; k < NQ; k++) ok = ok && pv[k] != Slot<double>::empty;
+            if (HALO)
+#pragma unroll
+                for (int k = 0; k < KH; k++)
+                    if ((int)threadIdx.x + k * T < nh) ok = ok && hv[k] != Slot<V>::empty;
+            if (ok) break;
+            if (++spin > kSpinLimit) {
+                *dead = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+#pragma unroll
+        for (int k = 0; k < NQ; k++) q[k] = hasp ? 0. + __builtin_bit_cast(double, pv[k]) : 0.;
+        wg_sum<T, NQ, 1>(q);
+        if (HALO)
+#pragma unroll
+            for (int k = 0; k < KH; k++)
+                h[k] = (int)threadIdx.x + k * T < nh ? __builtin_bit_cast(V, hv[k]) : (V)0;
+        if (*dead) return false;
+        // every workgroup has put its partials of this epoch, so the slots
+        // of the epoch before are read out: empty them for epoch + 3, and
+        // have that done before the next epoch's partials (one barrier later)
+        if (epoch >= 1) {
+            const int b1 = (epoch - 1) & (kZetaBufs - 1);
+            if (send >= 0) slot_clear(xch + (size_t)b1 * nsend + send, Slot<V>::empty);
+            if ((int)threadIdx.x < kPartSlots * kPartCopies)
+                slot_clear(part_slot(pslot, b1, tcopy, tk, wg), Slot<double>::empty);
+        }
+        epoch++;
+        return true;
+    }
+};
+
+// dynamic LDS of k_zeta
+struct ZetaLds {
+    size_t x, y, w, sub[2], total;
+};
+template <typename V>
+__host__ __device__ inline ZetaLds zeta_lds(int rows, int group, int hmax, int chmax, int threads, bool exact) {
+    const size_t sub = (size_t)threads * ((kSubFirst + 1) * sizeof(V) + (kSubFirst / 2 + 2) * sizeof(unsigned)) +
+                       (size_t)group * chmax * sizeof(unsigned);
+    auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
+    ZetaLds l;
+    size_t o = 0;
+    // the operand also holds the FP64 residual's (rows and halo)
+    l.x = o; o += up((size_t)(rows + hmax) * sizeof(double));
+    l.y = o; o += up((size_t)rows * sizeof(V));
+    l.w = o; o += exact ? 0 : up((size_t)rows * sizeof(V));
+    for (int d = 0; d < 2; d++) { l.sub[d] = o; o += exact ? up(sub) : 0; }
+    l.total = o;
+    return l;
+}
+
+// the rows of the workgroup's blocks into LDS, in the order of one substitution
+template <typename V, int T, bool BACK>
+__device__ __attribute__((always_inline)) inline SubExact<V, T> stage_sub(const SolvArgs<V> &a, const ZetaArgs &z,
+                                                                          int wg, unsigned char *lds) {
+    SubExact<V, T> s;
+    V *val = reinterpret_cast<V *>(lds), *piv = val + kSubFirst * T;
+    unsigned *col = reinterpret_cast<unsigned *>(piv + T), *row = col + (kSubFirst / 2) * T, *tail = row + T,
+             *chunk = tail + T;
+    const int *nch = BACK ? z.nch_b : z.nch_f;
+    const unsigned *chunks = BACK ? z.chunk_b : z.chunk_f;
+    // position t: row rows[..] of the block t / brows
+    const int t = threadIdx.x, g = t / a.brows, r0 = g * a.brows, blk = wg * z.group + g;
+    const bool on = g < z.group && blk < a.nblk && blk * a.brows + t - r0 < a.n;
+    const V *lu = a.lu + (on ? (size_t)blk * a.mx : 0);
+    const int *pcol = a.pcol + (on ? (size_t)blk * a.mx : 0);
+    int li = 0, d = 0, e0 = 0, cnt = 0;
+    if (on) {
+        const int *rp = a.prp + (size_t)blk * (a.brows + 1);
+        li = (BACK ? z.rows_b : z.rows_f)[blk * a.brows + t - r0];
+        d = a.pdg[(size_t)blk * a.brows + li];
+        e0 = BACK ? d + 1 : rp[li];
+        cnt = BACK ? rp[li + 1] - e0 : d - e0;
+    }
+    unsigned c[kSubFirst];
+#pragma unroll
+    for (int k = 0; k < kSubFirst; k++) {
+        val[k * T + t] = k < cnt ? lu[e0 + k] : (V)0;
+        c[k] = on ? (unsigned)((r0 + (k < cnt ? pcol[e0 + k] : li)) * (int)sizeof(V)) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kSubFirst / 2; k++) col[k * T + t] = c[2 * k] | c[2 * k + 1] << 16;
+    piv[t] = BACK && on ? lu[d] : (V)0;
+    row[t] = on ? (unsigned)((r0 + li) * (int)sizeof(V)) | (unsigned)max(0, cnt - kSubFirst) << 16 : 0u;
+    tail[t] = (unsigned)(e0 + kSubFirst);
+    for (int e = t; e < z.group * z.chmax; e += T) {
+        const int b = wg * z.group + e / z.chmax;
+        chunk[e] = b < a.nblk ? chunks[(size_t)b * z.chmax + e % z.chmax] : 0u;
+    }
+    s.val = val; s.piv = piv; s.col = col; s.row = row; s.tail = tail;
+    // this wavefront's block
+    const int w = min((int)threadIdx.x >> 6, z.group - 1), wb = wg * z.group + w;
+    s.chunk = chunk + w * z.chmax;
+    s.r0 = w * a.brows;
+    s.nch = wb < a.nblk ? nch[wb] : 0;
+    s.lu = a.lu + (wb < a.nblk ? (size_t)wb * a.mx : 0);
+    s.pcol = a.pcol + (wb < a.nblk ? (size_t)wb * a.mx : 0);
+    return s;
+}
+
+template <typename V, int T, int KH, bool EXACT>
+__global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
+    constexpr bool REFINE = sizeof(V) == 4;
+    extern __shared__ double smem[];
+    __shared__ int dead;
+    unsigned char *lds = reinterpret_cast<unsigned char *>(smem);
+    const ZetaLds L = zeta_lds<V>(z.group * a.brows, z.group, z.hmax, z.chmax, T, EXACT);
+    const int tid = threadIdx.x;
+    if (tid == 0) dead = 0;
+    ZetaRow<V, T, KH, EXACT> R;
+    R.wg = xcd_block(blockIdx.x, gridDim.x);
+    R.nwg = z.nwg; R.n = a.n; R.sweeps = a.sweeps; R.rows = z.group * a.brows; R.group = z.group;
+    const int b0 = R.wg * R.rows, nb = min(a.n, b0 + R.rows) - b0;
+    R.i = b0 + tid;
+    R.mine = tid < nb;
+    R.nh = z.hcnt[R.wg];
+    R.X = reinterpret_cast<V *>(lds + L.x);
+    R.y = reinterpret_cast<V *>(lds + L.y);
+    R.w = reinterpret_cast<V *>(lds + L.w);
+    R.xch = (typename Slot<V>::U *)z.xch;
+    R.pslot = z.pslot;
+    R.dead = &dead;
+    R.send = -1;
+    R.nsend = z.nsend;
+    int hcol[KH];
+    double *X64 = reinterpret_cast<double *>(lds + L.x);
+    const size_t n = a.n;
+    const int i = R.i;
+#pragma unroll
+    for (int k = 0; k < KH; k++) {
+        const bool on = tid + k * T < R.nh;
+        const size_t h = (size_t)R.wg * z.hmax + tid + k * T;
+        hcol[k] = on ? z.hcol[h] : 0;
+        R.hslot[k] = on ? z.hslot[h] : 0;
+    }
+    constexpr bool HOLD = ZetaRow<V, T, KH, EXACT>::kHold;
+    R.ga = a.ell_a;
+    R.glc = z.lcol;
+#pragma unroll
+    for (int k = 0; k < (HOLD ? kEllWidth : 1); k++) R.a[k] = 0;
+#pragma unroll
+    for (int k = 0; k < (HOLD ? kEllWidth / 2 : 1); k++) R.lc[k] = 0;
+    double a64[REFINE && HOLD ? kEllWidth : 1] = {};
+    int q64 = 0;
+    double b64 = 0., x64 = 0., xh64[KH] = {};
+    V bown = 0;
+    int len = 0;
+    if (R.mine) {
+        R.send = z.send[i];
+        len = a.ell_len[i];
+        if constexpr (HOLD) {
+#pragma unroll
+            for (int k = 0; k < kEllWidth; k++) R.a[k] = a.ell_a[(size_t)k * n + i];
+#pragma unroll
+            for (int k = 0; k < kEllWidth / 2; k++) R.lc[k] = z.lcol[(size_t)k * n + i];
+        }
+        if (REFINE) {
+            q64 = a.rowptr[i];
+            if constexpr (HOLD) {
+#pragma unroll
+                for (int k = 0; k < kEllWidth; k++)
+                    if (k < len) a64[k] = a.aval[q64 + k];
+            }
+            b64 = z.rhs[i];
+            x64 = z.x[i];
+        } else {
+            bown = a.b[i];
+            x64 = (double)a.x0[i];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < KH; k++)
+        if (tid + k * T < R.nh) xh64[k] = REFINE ? z.x[hcol[k]] : (double)a.x0[hcol[k]];
+    R.more_a = __any(len > kRowFirst);
+#pragma unroll
+    for (int k = 0; k < R.kTri; k++) R.l[k] = R.u[k] = 0;
+#pragma unroll
+    for (int k = 0; k < R.kTriWords; k++) R.llc[k] = R.uc[k] = 0;
+    if constexpr (EXACT) {
+        R.sf = stage_sub<V, T, false>(a, z, R.wg, lds + L.sub[0]);
+        R.sb = stage_sub<V, T, true>(a, z, R.wg, lds + L.sub[1]);
+    } else {
+        int nl = 0, nu = 0;
+        if (R.mine) {
+            const int meta = a.fs_meta[i], self = tid, r0 = tid / a.brows * a.brows;
+            nl = meta & 255;
+            nu = (meta >> 8) - nl - 1;
+            R.dinv = a.fs_val[i];
+#pragma unroll
+            for (int k = 0; k < kTriWidth; k++) {
+                const bool hl = k < nl, hu = k < nu;
+                const size_t sl = (size_t)(k + 1) * n + i, su = (size_t)(nl + 1 + k) * n + i;
+                const unsigned cl = (unsigned)((hl ? r0 + a.fs_col[sl] : self) * (int)sizeof(V));
+                const unsigned cu = (unsigned)((hu ? r0 + a.fs_col[su] : self) * (int)sizeof(V));
+                R.l[k] = hl ? a.fs_val[sl] : (V)0;
+                R.u[k] = hu ? a.fs_val[su] : (V)0;
+                R.llc[k / 2] |= cl << (16 * (k & 1));
+                R.uc[k / 2] |= cu << (16 * (k & 1));
+            }
+        }
+        R.more_l = __any(nl > kTriFirst);
+        R.more_u = __any(nu > kTriFirst);
+    }
+    int conv = 0, fail = 0, maxit = 0, nmv = 1, its = 0, nref = 0, refconv = 0;
+    double rn = 0.;
+    V dx = 0;
+    for (;;) {
+        V rhs, hdx[KH];
+        if (REFINE) {
+            // FP64 residual of the current x and its test (k_resid64, k_resid_check)
+            __syncthreads();
+            if (R.mine) X64[tid] = x64;
+#pragma unroll
+            for (int k = 0; k < KH; k++)
+                if (tid + k * T < R.nh) X64[R.rows + tid + k * T] = xh64[k];
+            __syncthreads();
+            double t = 0.;
+            unsigned cv[kEllWidth / 2];
+            R.columns(cv);
+#pragma unroll
+            for (int k = 0; k < kEllWidth; k++)
+                if (k < len) t = t + (HOLD ? a64[HOLD ? k : 0] : a.aval[q64 + k]) * X64[R.off(cv, k) / sizeof(V)];
+            const double r = b64 - t;
+            double rs[2] = {R.mine ? r * r : 0., R.mine ? b64 * b64 : 0.};
+            V none[KH];
+            if (!R.template exchange<2, false>(rs, (V)0, none)) { fail = kWaitExpired; break; }
+            rn = sqrt(rs[0]);
+            if (rn <= z.tol * sqrt(rs[1])) { refconv = 1; break; }
+            if (nref >= z.maxref) break;
+            nref++;
+            rhs = (V)r;
+        } else {
+            // b - A x0
+            V h[KH];
+#pragma unroll
+            for (int k = 0; k < KH; k++) h[k] = (V)xh64[k];
+            R.operand((V)x64, h);
+            const V t = R.product();
+            rhs = bown - t;
+        }
+        // r0 = M^-1 rhs
+        V r = R.precond(rhs), p = 0, v = 0, s = 0, t = 0;
+        V hr[KH], hp[KH], hv[KH], hs[KH], ht[KH];
+#pragma unroll
+        for (int k = 0; k < KH; k++) { hp[k] = hv[k] = hs[k] = ht[k] = 0; hdx[k] = 0; }
+        if (!R.mine) r = 0;
+        const V r0 = r;
+        dx = 0;
+        conv = fail = maxit = 0;
+        double q5[5] = {0., 0., 0., 0., 0.}, q1[1] = {(double)r * (double)r};
+        if (!R.template exchange<1, true>(q1, r, hr)) { fail = kWaitExpired; break; }
+        double target = 0., alpha = 0., rho = q1[0], rho_prev = 0., omega = 0.;
+        for (int it = 0;; it++) {
+            if (it == 0) {
+                rn = sqrt(q1[0]);
+                target = a.rtol * rn + a.atol;
+            } else {
+                // q5: (t,t) (t,s) (s,s) (r0,s) (r0,t)
+                if (breakdown(q5[0])) { fail = -3; break; }
+                omega = q5[1] / q5[0];
+                if (breakdown(omega)) { fail = -3; break; }
+                rn = sqrt(fmax(0., q5[2] - 2. * omega * q5[1] + omega * omega * q5[0]));
+                rho = q5[3] - omega * q5[4];
+                const V va = (V)alpha, vo = (V)omega;
+                dx = dx + (va * p + vo * s);
+                r = s - vo * t;
+#pragma unroll
+                for (int k = 0; k < KH; k++) {
+                    if (REFINE) hdx[k] = hdx[k] + (va * hp[k] + vo * hs[k]);
+                    hr[k] = hs[k] - vo * ht[k];
+                }
+                its++;
+            }
+            nmv = 1 + 2 * it;
+            if (!(rn > target)) { conv = 1; break; }
+            if (it > 0 && a.itermax > 0 && 1 + 2 * it >= a.itermax) { maxit = 1; break; }
+            if (it == 0) {
+                p = r;
+#pragma unroll
+                for (int k = 0; k < KH; k++) hp[k] = hr[k];
+            } else {
+                if (breakdown(rho)) { fail = -3; break; }
+                const V vb = (V)(rho * alpha / (omega * rho_prev)), vo = (V)omega;
+                p = r + vb * (p - vo * v);
+#pragma unroll
+                for (int k = 0; k < KH; k++) hp[k] = hr[k] + vb * (hp[k] - vo * hv[k]);
+            }
+            rho_prev = rho;
+            R.operand(p, hp);
+            v = R.precond(R.product());
+            q1[0] = R.mine ? (double)r0 * (double)v : 0.;
+            if (!R.template exchange<1, true>(q1, v, hv)) { fail = kWaitExpired; break; }
+            if (breakdown(q1[0])) { fail = -3; break; }
+            alpha = rho / q1[0];
+            const V va = (V)alpha;
+            s = r - va * v;
+#pragma unroll
+            for (int k = 0; k < KH; k++) hs[k] = hr[k] - va * hv[k];
+            R.operand(s, hs);
+            t = R.precond(R.product());
+            const double tv = R.mine ? (double)t : 0., sv = R.mine ? (double)s : 0., r0v = (double)r0;
+            q5[0] = tv * tv;
+            q5[1] = tv * sv;
+            q5[2] = sv * sv;
+            q5[3] = r0v * sv;
+            q5[4] = r0v * tv;
+            if (!R.template exchange<5, true>(q5, t, ht)) { fail = kWaitExpired; break; }
+        }
+        if (!REFINE || fail == kWaitExpired) break;
+        if (tid == 0 && R.wg == 0 && nref <= CT_NRITS) a.ctrl[CT_RITS + nref - 1] = (nmv - 1) / 2;
+        // x += correction
+        x64 = x64 + (double)dx;
+#pragma unroll
+        for (int k = 0; k < KH; k++) xh64[k] = xh64[k] + (double)hdx[k];
+    }
+    if (fail == kWaitExpired) {
+        if (tid == 0) a.ctrl[CT_WAIT] = 1;
+        return;
+    }
+    if (R.mine) {
+        if (REFINE) z.x[i] = x64;
+        else a.dx[i] = dx;
+    }
+    // commit: workgroup 0 sets the flags after everyone's stores
+    if (z.nwg > 1) {
+        const int buf = R.epoch & (kZetaBufs - 1);
+        unsigned long long *ps = part_slot(z.pslot, buf, 0, 0, 0);
+        wait_stores();
+        __syncthreads();
+        if (tid == 0) slot_put<double>(ps + R.wg, 1.);
+        if (R.wg != 0) return;
+        if (tid < z.nwg) {
+            int spin = 0;
+            while (slot_get(ps + tid) == Slot<double>::empty) {
+                if (++spin > kSpinLimit) {
+                    dead = 1;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        __syncthreads();
+        if (dead) {
+            if (tid == 0) a.ctrl[CT_WAIT] = 1;
+            return;
+        }
+    }
+    if (tid == 0 && R.wg == 0) {
+        a.ctrl[CT_STOPIT] = 1;
+        a.ctrl[CT_CONV] = conv;
+        a.ctrl[CT_FAIL] = fail;
+        a.ctrl[CT_MAXIT] = maxit;
+        a.ctrl[CT_NMV] = nmv;
+        a.ctrl[CT_ITS] = its;
+        a.ctrl[CT_NREF] = nref;
+        a.ctrl[CT_REFCONV] = refconv;
+        a.scal[REFINE ? SC_RES64 : SC_RNORM] = rn;
+    }
+}
+
 // ---------------------------------------------------------------- host driver
 // one read-back: the solver's control words (into h_pinned[16..]) and the
 // device error word and counter d_err[0..1] (into h_pinned[0..1])
@@ -1031,6 +1812,7 @@ static size_t apply_lds(const Model &M) {
 // sweeps of a warm start (four reach the iteration counts of exact factors
 // on the 50k-node lagoon, two do not), and exact factorisations at least
 // every kWarmRefresh solves
+constexpr int kMaxRefine = 40;          // FP64 refinement rounds of a solve
 constexpr int kWarmSweeps = 4;
 constexpr int kWarmRefresh = 16;
 
@@ -1048,6 +1830,25 @@ static int factor(Model &M, SolvArgs<V> &a) {
                  M.stream, a, stage, sweeps);
     HIPCHK(M, hipGetLastError());
     M.sv.have_lu = true;
+    return 0;
+}
+
+// iterations and errors of a finished BiCGStab solve from its control words
+static int krylov_outcome(Model &M, const int *c, int *iters, int slot) {
+    if (iters) *iters = (c[CT_NMV] - 1) / 2;
+    M.sv.last_its[slot] = (c[CT_NMV] - 1) / 2;
+    if (c[CT_FACTOR] != 0) {
+        M.err = "zeta solver: zero pivot in the block factorisation (row " + std::to_string(c[CT_FACTOR]) + ")";
+        return 2;
+    }
+    if (c[CT_FAIL] != 0 || c[CT_MAXIT] != 0) {
+        M.err = "zeta solver: BiCGStab failed (code " + std::to_string(c[CT_FAIL] ? c[CT_FAIL] : -1) + ")";
+        return 2;
+    }
+    if (!c[CT_CONV]) {
+        M.err = "zeta solver: no convergence";
+        return 2;
+    }
     return 0;
 }
 
@@ -1096,21 +1897,7 @@ static int bicgstab_t(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x
         if (c[CT_CONV] || c[CT_FAIL] || c[CT_MAXIT] || it >= maxit) break;
         chunk = 2;
     }
-    if (iters) *iters = (c[CT_NMV] - 1) / 2;
-    M.sv.last_its[slot] = (c[CT_NMV] - 1) / 2;
-    if (c[CT_FACTOR] != 0) {
-        M.err = "zeta solver: zero pivot in the block factorisation (row " + std::to_string(c[CT_FACTOR]) + ")";
-        return 2;
-    }
-    if (c[CT_FAIL] != 0 || c[CT_MAXIT] != 0) {
-        M.err = "zeta solver: BiCGStab failed (code " + std::to_string(c[CT_FAIL] ? c[CT_FAIL] : -1) + ")";
-        return 2;
-    }
-    if (!c[CT_CONV]) {
-        M.err = "zeta solver: no convergence";
-        return 2;
-    }
-    return 0;
+    return krylov_outcome(M, c, iters, slot);
 }
 
 template <typename V>
@@ -1162,6 +1949,125 @@ static int enqueue_inner(Model &M, SolvArgs<V> &a, int chunk) {
     }
 }
 
+
+// The one-launch solve: kernel of the workgroup size, the halo entries per
+// work-item and the kind of triangular solve.
+template <typename V>
+using ZetaKernel = void (*)(SolvArgs<V>, ZetaArgs);
+template <typename V>
+static ZetaKernel<V> zeta_kernel(const Model &M) {
+    const bool exact = M.p.tri_sweeps == 0;
+    if (M.sv.zeta_t == 1024) return k_zeta<V, 1024, 1, true>;
+    if (M.sv.zeta_t == 512) return exact ? k_zeta<V, 512, 1, true> : k_zeta<V, 512, 1, false>;
+    if (M.sv.zeta_hmax <= 256) return exact ? k_zeta<V, 256, 1, true> : k_zeta<V, 256, 1, false>;
+    return exact ? k_zeta<V, 256, 2, true> : k_zeta<V, 256, 2, false>;
+}
+
+// Workgroups of the one-launch solve wait for each other, so a launch is
+// made only when all of them can be resident together with those of every
+// other such launch of this process: each takes its share of the device's
+// compute units (workgroups / workgroups that fit one unit) out of the
+// units that are not taken, and waits for them otherwise (a solve holds
+// them for some hundred microseconds).  Launches that need no other
+// workgroup to proceed (everything else) end by themselves and only delay it.
+namespace {
+struct ZetaUnits {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::unordered_map<int, double> used;     // per device
+};
+ZetaUnits &zeta_units() {
+    static ZetaUnits u;
+    return u;
+}
+struct ZetaHold {
+    int dev;
+    double cost;
+    ZetaHold(int d, double c, double cap) : dev(d), cost(c) {
+        ZetaUnits &u = zeta_units();
+        std::unique_lock<std::mutex> lk(u.mu);
+        u.cv.wait(lk, [&] { return u.used[dev] + cost <= cap; });
+        u.used[dev] += cost;
+    }
+    ~ZetaHold() {
+        ZetaUnits &u = zeta_units();
+        {
+            std::lock_guard<std::mutex> lk(u.mu);
+            u.used[dev] -= cost;
+        }
+        u.cv.notify_all();
+    }
+    ZetaHold(const ZetaHold &) = delete;
+    ZetaHold &operator=(const ZetaHold &) = delete;
+};
+}  // namespace
+
+// LDS, device share and capacity of this model's one-launch solve under its
+// current parameters; cost < 0: it cannot run (the two-kernel iteration does)
+struct ZetaPlan {
+    size_t lds = 0;
+    int dev = 0;
+    double cost = -1., cap = 0.;
+};
+template <typename V>
+static ZetaPlan zeta_plan(Model &M) {
+    ZetaPlan p;
+    Solver &v = M.sv;
+    if (v.zeta_t == 0) return p;
+    const bool exact = M.p.tri_sweeps == 0;
+    // sweeps keep the factor row in registers (and need its slot-major copy)
+    if (!exact && (!v.fs_val || v.brows > kThreads)) return p;
+    p.lds = zeta_lds<V>(v.zeta_group * v.brows, v.zeta_group, v.zeta_hmax, v.zeta_chmax, v.zeta_t, exact).total;
+    if (v.zeta_occ[exact] == 0) {
+        // asked once per model and kind
+        int dev = 0, cus = 0, occ = 0, lds_max = 0;
+        v.zeta_occ[exact] = -1;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+            p.lds + 8192 > (size_t)lds_max)
+            return p;
+        const void *fn = (const void *)zeta_kernel<V>(M);
+        if (p.lds > kLdsLimit &&
+            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
+            return p;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, v.zeta_t, p.lds) != hipSuccess || occ < 1) return p;
+        v.zeta_occ[exact] = occ;
+        v.zeta_dev = dev;
+        v.zeta_cus = cus;
+    }
+    if (v.zeta_occ[exact] < 1) return p;
+    p.dev = v.zeta_dev;
+    p.cap = 0.875 * v.zeta_cus;      // some units left to the rest of the step
+    const double cost = (double)v.zeta_nwg / v.zeta_occ[exact];
+    if (cost <= p.cap) p.cost = cost;
+    return p;
+}
+
+// the launch, `tail` and the read-back of the control words; *done false
+// when a wait expired
+template <typename V>
+static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::function<int()> &tail, int *c, bool *done) {
+    ZetaArgs z;
+    std::memset(&z, 0, sizeof z);
+    z.nwg = M.sv.zeta_nwg; z.group = M.sv.zeta_group;
+    z.hmax = M.sv.zeta_hmax; z.chmax = M.sv.zeta_chmax;
+    z.lcol = M.m.z_lcol; z.hcol = M.m.z_hcol; z.hslot = M.m.z_hslot; z.hcnt = M.m.z_hcnt;
+    z.send = M.m.z_send; z.nsend = M.sv.zeta_nsend;
+    z.rows_f = M.m.fwd_rows; z.rows_b = M.m.bwd_rows;
+    z.chunk_f = M.m.z_chf; z.chunk_b = M.m.z_chb; z.nch_f = M.m.z_nchf; z.nch_b = M.m.z_nchb;
+    z.xch = M.sv.xch; z.pslot = M.sv.pslot;
+    z.rhs = M.s.rhs; z.x = M.s.x; z.tol = M.p.refine_rtol; z.maxref = kMaxRefine;
+    ZetaHold hold(p.dev, p.cost, p.cap);
+    static_assert(kZetaSlotWords == (size_t)kZetaBufs * kPartCopies * kPartStride, "partial slots");
+    hipLaunchKernelGGL(zeta_kernel<V>(M), dim3(M.sv.zeta_nwg), dim3(M.sv.zeta_t), p.lds, M.stream, a, z);
+    HIPCHK(M, hipGetLastError());
+    if (tail && tail()) return 1;
+    if (read_ctrl(M, c, CT_WORDS)) return 1;
+    *done = c[CT_CONV] || c[CT_REFCONV] || !c[CT_WAIT];
+    return 0;
+}
+
 int solver_setup(Model &M) { (void)M; return 0; }
 
 // the words of one zeta solve, for a second attempt at it
@@ -1206,7 +2112,16 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
             HIPCHK(M, hipGetLastError());
             return 0;
         };
-        const int rc = bicgstab<double>(M, a, &its, 0, 0, tail);
+        int rc = 0;
+        bool done = false;
+        const ZetaPlan plan = zeta_plan<double>(M);
+        if (plan.cost >= 0.) {
+            int c[CT_WORDS] = {};
+            if (zeta_run<double>(M, plan, a, tail, c, &done)) return 1;
+            if (done) rc = krylov_outcome(M, c, &its, 0);
+            else M.solver_retries++;
+        }
+        if (!done) rc = bicgstab<double>(M, a, &its, 0, 0, tail);
         it_total = its;
         if (rc) return rc;
     } else {
@@ -1230,7 +2145,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         if (factor<float>(M, a)) return 1;
         a.rtol = M.p.inner_rtol;
         a.atol = 0.0;
-        const int maxref = 40;
+        const int maxref = kMaxRefine;
         const int itmax_inner = M.p.itermax > 0 ? (M.p.itermax + 1) / 2 : 500;
         // iterations enqueued for round r: that round's count in the previous
         // solve plus one (kernels beyond convergence return at once but
@@ -1254,17 +2169,27 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         // chunks, sized from the previous solve, cut them short or the system
         // changed), so each later round gets twice the iterations of the last
         int plan = std::min((int)CT_NRITS, std::max(1, M.sv.last_nref)), enq = 0, c[CT_WORDS] = {}, boost = 1;
+        const ZetaPlan zp = zeta_plan<float>(M);
+        bool done = false;
+        if (zp.cost >= 0.) {
+            auto tail = [&]() -> int { return wetdry(M.sv.ctrl + CT_REFCONV, nullptr); };
+            if (zeta_run<float>(M, zp, a, tail, c, &done)) return 1;
+            if (done) enq = maxref;       // all its rounds are behind it
+            else M.solver_retries++;
+        }
         for (;;) {
-            for (int r = 0; r < plan && enq < maxref; r++, enq++) {
-                if (resid() || enqueue_inner<float>(M, a, std::min(itmax_inner, chunk_of(enq) * boost))) return 1;
-                hipLaunchKernelGGL(k_bicg_finish<float>, dim3(g1), dim3(kThreads), 0, M.stream, (const float *)x0,
-                                   (const float *)a.dx, M.s.x, n, 1, (const int *)M.sv.ctrl);
+            if (!done) {
+                for (int r = 0; r < plan && enq < maxref; r++, enq++) {
+                    if (resid() || enqueue_inner<float>(M, a, std::min(itmax_inner, chunk_of(enq) * boost))) return 1;
+                    hipLaunchKernelGGL(k_bicg_finish<float>, dim3(g1), dim3(kThreads), 0, M.stream, (const float *)x0,
+                                       (const float *)a.dx, M.s.x, n, 1, (const int *)M.sv.ctrl);
+                }
+                if (resid()) return 1;
+                if (wetdry(M.sv.ctrl + CT_REFCONV, nullptr)) return 1;
+                if (read_ctrl(M, c, CT_WORDS)) return 1;
             }
-            if (resid()) return 1;
-            if (wetdry(M.sv.ctrl + CT_REFCONV, nullptr)) return 1;
-            if (read_ctrl(M, c, CT_WORDS)) return 1;
             if (c[CT_FACTOR] != 0) {
-                        M.err = "zeta solver: zero pivot in the block factorisation (row " + std::to_string(c[CT_FACTOR]) + ")";
+                M.err = "zeta solver: zero pivot in the block factorisation (row " + std::to_string(c[CT_FACTOR]) + ")";
                 return 2;
             }
             if (c[CT_REFCONV]) break;
