@@ -629,8 +629,8 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
 }
 
 // Tables of the one-launch zeta solve.  It needs: one row per work-item,
-// every row within the ELL slots, one work-item per workgroup to collect the
-// partial sums (at most 256 workgroups), and halos of at most 2 entries (256
+// every row within the ELL slots, one work-item per diagonal block to collect
+// the partial sums (at most 512 blocks), and halos of at most 2 entries (256
 // work-items) or 1 (more) per work-item.  Workgroups of 256 work-items up to
 // kZetaSmall of them, else of 512: the product and sweeps take longer there,
 // the exchange among half as many is faster.  Measured steps, 256 against
@@ -641,8 +641,10 @@ constexpr int kZetaSmall = 128;
 
 static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
                         int esize, int T, ZetaTables &zt) {
-    const int nblk = bs.nblk, group = T / bs.brows, brows = group * bs.brows, nwg = (nblk + group - 1) / group;
-    if (nwg > 256) return false;
+    // several blocks only of whole wavefronts (their sums are kept apart)
+    const int nblk = bs.nblk, group = bs.brows % 64 == 0 ? T / bs.brows : 1, brows = group * bs.brows;
+    const int nwg = (nblk + group - 1) / group;
+    if (nblk > T || nblk > 512) return false;
     // halos: the columns outside the workgroup's rows, ascending
     std::vector<std::vector<int>> halo(nwg);
     parallel_for(nwg, 16, [&](int b_begin, int b_end) {
@@ -741,7 +743,7 @@ void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<i
         zeta_tables(n, rowptr, cols, bs, esize, 1024, zt);
         return;
     }
-    const int n256 = bs.brows <= 256 ? (bs.nblk + 256 / bs.brows - 1) / (256 / bs.brows) : 1 << 30;
+    const int n256 = bs.brows <= 256 ? (bs.brows % 64 == 0 ? (n + 255) / 256 : bs.nblk) : 1 << 30;
     if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, zt)) return;
     if (bs.brows <= 256) zeta_tables(n, rowptr, cols, bs, esize, 256, zt);
 }

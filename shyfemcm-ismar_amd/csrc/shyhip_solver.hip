@@ -81,7 +81,7 @@ struct SolvArgs {
     void *xch;
     unsigned long long *pslot;
     const int *send;
-    int nsend, zgroup;
+    int nsend;
 };
 
 template <typename V>
@@ -116,7 +116,6 @@ static SolvArgs<V> solv_args(Model &M, const V *A, V *b, V *x0) {
         a.pslot = M.sv.pslot;
         a.send = M.m.z_send;
         a.nsend = M.sv.zeta_nsend;
-        a.zgroup = M.sv.zeta_group;
     }
     return a;
 }
@@ -1051,8 +1050,10 @@ __global__ __launch_bounds__(kThreads) void k_resid_check(const double *part, in
 // A block's neighbour rows in other blocks (its halo) are kept as well: the
 // recurrences of p, r, s (and the correction) are run on them redundantly,
 // with the same operations, so only v and t are exchanged and the halo
-// values have the owner's bits.  Every workgroup adds the partial sums in the
-// same fixed order, so all of them (and all runs) take the same decisions.
+// values have the owner's bits.  The partial sums are those of the diagonal blocks
+// and every workgroup adds them in the order of the two-kernel iteration, so
+// all of them (and all runs) take the same decisions and the FP64 solve of
+// blocks of 256 rows has that iteration's bits.
 //
 // The waits are bounded: the launch is made only when all its workgroups
 // can be resident together (zeta_slots), and a wait that still runs out sets
@@ -1064,14 +1065,14 @@ __global__ __launch_bounds__(kThreads) void k_resid_check(const double *part, in
 constexpr int kWaitExpired = -9;
 constexpr int kSpinLimit = 1 << 17;      // polls of one wait (about 0.1 s)
 constexpr int kZetaBufs = 4;
-// Partial sums per workgroup and buffer, and their copies: every workgroup
-// reads everyone's, so one copy makes all workgroups wait for the same few
-// memory lines (196 workgroups: a half iteration of 5.8 us with one copy,
-// 5.3 us with 16); each workgroup puts its sums into every copy and reads
-// one.  Copies lie apart.
+// Partial sums per diagonal block and buffer, and their copies: every
+// workgroup reads all of them, so one copy makes all workgroups wait for the
+// same few memory lines (196 workgroups: a half iteration of 5.8 us with one
+// copy, 5.3 us with 16); each workgroup puts its sums into every copy and
+// reads one.  Copies lie apart.
 constexpr int kPartSlots = 5;
 constexpr int kPartCopies = 16;
-constexpr int kPartStride = 512 * 5;     // words per copy: [kPartSlots][512], at most 256 of each used
+constexpr int kPartStride = 512 * 5;     // words per copy: [kPartSlots][512 blocks]
 
 template <typename V>
 struct Slot;
@@ -1100,8 +1101,8 @@ __device__ inline U slot_get(const U *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ inline unsigned long long *part_slot(unsigned long long *pslot, int buf, int copy, int k, int wg) {
-    return pslot + ((size_t)buf * kPartCopies + copy) * kPartStride + k * 512 + wg;
+__device__ inline unsigned long long *part_slot(unsigned long long *pslot, int buf, int copy, int k, int blk) {
+    return pslot + ((size_t)buf * kPartCopies + copy) * kPartStride + k * 512 + blk;
 }
 
 // the slots of block blk empty in every buffer, and the solve's flags clear
@@ -1111,8 +1112,8 @@ __device__ inline void zeta_empty_slots(const SolvArgs<V> &a, int blk, int b0, i
     for (int b = 0; b < kZetaBufs; b++) {
         for (int li = threadIdx.x; li < nb; li += blockDim.x)
             if (const int q = a.send[b0 + li]; q >= 0) slot_clear(xch + (size_t)b * a.nsend + q, Slot<V>::empty);
-        if (blk % a.zgroup == 0 && threadIdx.x < kPartSlots * kPartCopies)
-            slot_clear(part_slot(a.pslot, b, threadIdx.x % kPartCopies, threadIdx.x / kPartCopies, blk / a.zgroup),
+        if (threadIdx.x < kPartSlots * kPartCopies)
+            slot_clear(part_slot(a.pslot, b, threadIdx.x % kPartCopies, threadIdx.x / kPartCopies, blk),
                        Slot<double>::empty);
     }
     if (blk == 0 && threadIdx.x == 0) {
@@ -1145,36 +1146,6 @@ struct ZetaArgs {
     double tol;
     int maxref;
 };
-
-// sums over a workgroup of T work-items, like block_sum; TAG keeps the LDS
-// of consecutive sums apart, so one barrier per sum is enough (a sum's LDS
-// is written again only after other barriers)
-template <int T, int NQ, int TAG>
-__device__ __attribute__((always_inline)) inline void wg_sum(double (&v)[NQ]) {
-    __shared__ double red[NQ][T / 64];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) v[q] = wave_sum(v[q]);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int q = 0; q < NQ; q++) red[q][threadIdx.x >> 6] = v[q];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        if constexpr (T / 64 >= 8) {
-            // 8 or 16 wavefronts: their sums one per lane of half a row or a row
-            double t = red[q][threadIdx.x & (T / 64 - 1)];
-            t = t + dpp_f64<0xB1>(t);
-            t = t + dpp_f64<0x4E>(t);
-            t = t + dpp_f64<0x141>(t);
-            v[q] = T / 64 == 8 ? t : t + dpp_f64<0x140>(t);
-        } else {
-            double t = red[q][0];
-#pragma unroll
-            for (int w = 1; w < T / 64; w++) t += red[q][w];
-            v[q] = t;
-        }
-    }
-}
 
 // Exact substitution with one triangular factor of a block by one wavefront
 // (wavefront g of the workgroup takes its block g): rows level by level (a level's rows depend only on earlier
@@ -1279,7 +1250,7 @@ struct ZetaRow {
     const V *ga;
     const unsigned *glc;
     bool more_a = false, more_l = false, more_u = false;   // some row of the wavefront fills the last slots
-    int i, wg, nh, nwg, n, sweeps, send, nsend;
+    int i, wg, nh, nblk, n, sweeps, send, nsend;
     bool mine;
     int hslot[KH];
     // LDS: operand (rows, then halo), two row buffers; exact: block factors
@@ -1380,27 +1351,39 @@ struct ZetaRow {
     // entries returned in h).  False when a wait ran out.
     template <int NQ, bool HALO>
     __device__ __attribute__((always_inline)) inline bool exchange(double (&q)[NQ], V own, V (&h)[KH]) {
-        if (nwg == 1) {
-            wg_sum<T, NQ, 0>(q);
-            return true;
-        }
+        // the wavefronts' sums
+        __shared__ double red[NQ][T / 64], tot[NQ][kWaves], hi[NQ][T > kThreads ? kThreads : 1];
+#pragma unroll
+        for (int k = 0; k < NQ; k++) q[k] = wave_sum(q[k]);
         const int buf = epoch & (kZetaBufs - 1);
         U *vs = xch + (size_t)buf * nsend;
         wait_stores();          // the slots emptied after the last exchange
         if (HALO && send >= 0) slot_put<V>(vs + send, own);
-        wg_sum<T, NQ, 0>(q);
-        const int tk = threadIdx.x / kPartCopies, tcopy = threadIdx.x % kPartCopies;
-        if (tk < NQ) {
-            double mine_q = q[0];
+        if ((threadIdx.x & 63) == 0)
 #pragma unroll
-            for (int k = 1; k < NQ; k++)
-                if (tk == k) mine_q = q[k];
-            slot_put<double>(part_slot(pslot, buf, tcopy, tk, wg), mine_q);
+            for (int k = 0; k < NQ; k++) red[k][threadIdx.x >> 6] = q[k];
+        __syncthreads();
+        // Each block's sum: its wavefronts' in order (a workgroup with more
+        // than one block has blocks of whole wavefronts).
+        const int bw = group == 1 ? T / 64 : rows / (64 * group);
+        if (nblk == 1) {
+#pragma unroll
+            for (int k = 0; k < NQ; k++) {
+                q[k] = red[k][0];
+                for (int w = 1; w < bw; w++) q[k] += red[k][w];
+            }
+            return true;
+        }
+        for (int e = threadIdx.x; e < NQ * group * kPartCopies; e += T) {
+            const int copy = e % kPartCopies, g = e / kPartCopies % group, k = e / (kPartCopies * group);
+            double t = red[k][g * bw];
+            for (int w = 1; w < bw; w++) t += red[k][g * bw + w];
+            if (wg * group + g < nblk) slot_put<double>(part_slot(pslot, buf, copy, k, wg * group + g), t);
         }
         const unsigned long long *ps = part_slot(pslot, buf, wg % kPartCopies, 0, threadIdx.x);
         unsigned long long pv[NQ];
         U hv[KH];
-        const bool hasp = (int)threadIdx.x < nwg;
+        const bool hasp = (int)threadIdx.x < nblk;
         int spin = 0;
         for (;;) {
             bool ok = true;
@@ -1425,9 +1408,34 @@ struct ZetaRow {
             }
             __builtin_amdgcn_s_sleep(1);
         }
+        // the total, in the order of Partials: work-item i holds partials i
+        // and i + 256, then the wavefronts' sums, then these in order
 #pragma unroll
         for (int k = 0; k < NQ; k++) q[k] = hasp ? 0. + __builtin_bit_cast(double, pv[k]) : 0.;
-        wg_sum<T, NQ, 1>(q);
+        if (T > kThreads && nblk > kThreads) {
+            if (threadIdx.x >= kThreads && threadIdx.x < 2 * kThreads)
+#pragma unroll
+                for (int k = 0; k < NQ; k++) hi[k][threadIdx.x - kThreads] = q[k];
+            __syncthreads();
+            if (threadIdx.x < kThreads)
+#pragma unroll
+                for (int k = 0; k < NQ; k++) q[k] += hi[k][threadIdx.x];
+        }
+        if (threadIdx.x < kThreads) {
+#pragma unroll
+            for (int k = 0; k < NQ; k++) q[k] = wave_sum(q[k]);
+            if ((threadIdx.x & 63) == 0)
+#pragma unroll
+                for (int k = 0; k < NQ; k++) tot[k][threadIdx.x >> 6] = q[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NQ; k++) {
+            double t = tot[k][0];
+#pragma unroll
+            for (int w = 1; w < kWaves; w++) t += tot[k][w];
+            q[k] = t;
+        }
         if (HALO)
 #pragma unroll
             for (int k = 0; k < KH; k++)
@@ -1439,8 +1447,12 @@ struct ZetaRow {
         if (epoch >= 1) {
             const int b1 = (epoch - 1) & (kZetaBufs - 1);
             if (send >= 0) slot_clear(xch + (size_t)b1 * nsend + send, Slot<V>::empty);
-            if ((int)threadIdx.x < kPartSlots * kPartCopies)
-                slot_clear(part_slot(pslot, b1, tcopy, tk, wg), Slot<double>::empty);
+            for (int e = threadIdx.x; e < kPartSlots * group * kPartCopies; e += T) {
+                const int g = e / kPartCopies % group;
+                if (wg * group + g < nblk)
+                    slot_clear(part_slot(pslot, b1, e % kPartCopies, e / (kPartCopies * group), wg * group + g),
+                               Slot<double>::empty);
+            }
         }
         epoch++;
         return true;
@@ -1527,7 +1539,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
     if (tid == 0) dead = 0;
     ZetaRow<V, T, KH, EXACT> R;
     R.wg = xcd_block(blockIdx.x, gridDim.x);
-    R.nwg = z.nwg; R.n = a.n; R.sweeps = a.sweeps; R.rows = z.group * a.brows; R.group = z.group;
+    R.nblk = a.nblk; R.n = a.n; R.sweeps = a.sweeps; R.rows = z.group * a.brows; R.group = z.group;
     const int b0 = R.wg * R.rows, nb = min(a.n, b0 + R.rows) - b0;
     R.i = b0 + tid;
     R.mine = tid < nb;
@@ -2025,7 +2037,7 @@ static ZetaPlan zeta_plan(Model &M) {
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-            p.lds + 8192 > (size_t)lds_max)
+            p.lds + 20480 > (size_t)lds_max)
             return p;
         const void *fn = (const void *)zeta_kernel<V>(M);
         if (p.lds > kLdsLimit &&
