@@ -405,7 +405,8 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_nchf, (void *)m.z_nchb,
                     (void *)m.fwd_rows, (void *)m.fwd_lptr, (void *)m.fwd_nlev, (void *)m.bwd_rows,
                     (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_el, (void *)m.tvd_kn, m.tvd_w,
-                    (void *)m.tvd_lev, (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem})
+                    (void *)m.tvd_lev, (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem,
+                    (void *)m.conz_nent, (void *)m.conz_nplace})
         dfree(q);
     Solver &v = M.sv;
     for (void *q : {v.lu, v.ell_a, v.fs_val, v.r0, v.r, v.p0, v.p1, v.v0, v.v1, v.s, v.t, v.dx, v.b, v.x0, (void *)v.part,
@@ -617,6 +618,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         rc |= dalloc_s(M, &m.areakv, area.size()) || upload_s(M, m.areakv, area.data(), area.size());
     }
     // node -> element incidence: element order and colour order
+    std::vector<int> inc_ptr, inc_lev;      // list starts, bottom layers by colour-order position
     {
         std::vector<int> ptr(nkn + 1, 0), el(3 * (size_t)nel), elc(3 * (size_t)nel);
         for (int ie = 0; ie < nel; ie++)
@@ -660,6 +662,8 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         rc |= dalloc(M, &m.inc_cnt, icnt.size()) || upload(M, m.inc_cnt, icnt.data(), icnt.size());
         rc |= dalloc(M, &m.inc_el, iel.size()) || upload(M, m.inc_el, iel.data(), iel.size());
         rc |= dalloc(M, &m.inc_elc, ielc.size()) || upload(M, m.inc_elc, ielc.data(), ielc.size());
+        inc_ptr.swap(ptr);
+        inc_lev.swap(slev);
     }
     // conz3d work division: the element-layer list (chunks of kConzChunk
     // elements, layer by layer) and the node tiles (at most node_tile nodes
@@ -707,6 +711,36 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         m.ntile_tn = tn;
         rc |= dalloc(M, &m.conz_eitem, items.size()) || upload(M, m.conz_eitem, items.data(), items.size());
         rc |= dalloc(M, &m.conz_ntile, tiles.size()) || upload(M, m.conz_ntile, tiles.data(), tiles.size());
+        static_assert(3 * kIncWidth <= 31, "one word of reach bits");
+        std::vector<int> ent((size_t)m.n_ntile * kNodeItems * 4, -1), place(nkn);
+        parallel_for(m.n_ntile, 64, [&](int t_begin, int t_end) {
+            for (int t = t_begin; t < t_end; t++) {
+                int next = 0, lmax = 0;
+                for (int k = tiles[t]; k < tiles[t + 1]; k++) {
+                    place[k] = next;
+                    next += ilhkv[k];
+                    lmax = std::max(lmax, ilhkv[k]);
+                }
+                int *e = &ent[(size_t)t * kNodeItems * 4];
+                for (int l = 1; l <= lmax; l++)
+                    for (int k = tiles[t]; k < tiles[t + 1]; k++) {
+                        if (ilhkv[k] < l) continue;
+                        const int q0 = inc_ptr[k], cnt = inc_ptr[k + 1] - q0;
+                        int reach = 0;
+                        for (int s = 0; s < std::min(cnt, kIncWidth); s++)
+                            for (int d = 0; d < 3; d++)
+                                if (inc_lev[q0 + s] >= l + d) reach |= 1 << (d * kIncWidth + s);
+                        e[0] = (l - 1) | (ilhkv[k] - 1) << 5 | (place[k] + l - 1) << 10 |
+                               std::min(cnt, kNodeCntMax) << 18;
+                        e[1] = q0;
+                        e[2] = reach;
+                        e[3] = k;
+                        e += 4;
+                    }
+            }
+        });
+        rc |= dalloc(M, &m.conz_nent, ent.size()) || upload(M, m.conz_nent, ent.data(), ent.size());
+        rc |= dalloc(M, &m.conz_nplace, place.size()) || upload(M, m.conz_nplace, place.data(), place.size());
     }
     // CSR pattern
     rc |= dalloc(M, &m.rowptr, nkn + 1) || upload(M, m.rowptr, M.h_rowptr.data(), nkn + 1);

@@ -8,7 +8,7 @@
 //                scheme with node gradients) -> 3*fl per vertex, stored by
 //                the vertex's position in its node's colour-order incidence
 //                list.
-//   k_conz_node  one workgroup per node tile (at most 64 nodes and 256
+//   k_conz_node  one workgroup per node tile (at most 256 nodes and 256
 //                node-layers).  Phase 1, one work-item per node-layer: the
 //                vertical diffusion/advection terms of the node column (they
 //                depend on an element only through its bottom layer, so
@@ -66,6 +66,9 @@ struct ConzArgs {
     // element-layer work list and node tiles (see Mesh)
     const int *eitem, *ntile;
     int n_eitem;
+    const int4 *nent;                // node tiles' entries, and the nodes' first places in their tiles
+    const int *nplace;
+    int clear_below;                 // also write the zeros below the bottom
     // the step's element-layer records (k_conz_prep): int and double columns
     int *rec_i;
     double *rec_d;
@@ -530,66 +533,40 @@ __device__ inline double tvd_face(double conc, double cond, double conu, double 
 // EXT: the tracer's own terms (one tracer per launch): sinking in the
 // vertical velocity, nudging in the explicit term (concentration_omp.f90:
 // 479,697-701,727-735) and loads after the boundary flux (:816-834)
-template <typename S, int NL, int NT, bool EXT>
+//
+// What bounds it: the chain of a work-item -- its loads, about 20 FP64
+// divisions, the column solve -- in one pass of 2,400 wavefronts, then the
+// tracers' traffic on large basins.  Everything of a node-layer that only the
+// mesh decides (its node and place in the tile, its list's start and length,
+// which incident elements reach the layer, the next one and the one after)
+// is one 16-byte table entry (Mesh::conz_nent), so the loads form two rounds:
+// the entry, then all the rest.  Listing the tile's node-layers in the kernel
+// instead (a ballot per layer, one work-item adding up 48 counts, three
+// barriers), reading the list start and the elements' layers as data, and
+// evaluating a limited face per sign of the vertical velocity took 26.5 us a
+// launch on the 50k-node lagoon and 159 us on 300k nodes of 20 layers (T and
+// S, FP64), against 21.5 and 115 us.
+template <typename S, int NT, bool EXT>
 __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
     using R = S;
-    // phase-1 results by list position: right-hand sides of NT tracers and
-    // the three diagonals of the column matrix
+    // phase-1 results by place in the tile (node after node, top down):
+    // right-hand sides of NT tracers and the three diagonals of the column
+    // matrix
     __shared__ double cnP[NT][kNodeItems], cdP[kNodeItems], cloP[kNodeItems], chiP[kNodeItems];
-    __shared__ int items[kNodeItems];                 // kk | l << 16
-    constexpr int kWaves = kThreads / 64;
-    // per wavefront and layer: its nodes that have the layer (bit per lane)
-    // and the list position of the first of them
-    __shared__ unsigned long long lmask[kWaves][NL + 1];
-    __shared__ int lbase[kWaves][NL + 1];
-    __shared__ int nitems_s;
     const int nkn = a.nkn;
     const int tile = xcd_block();
+    const int4 ent = a.nent[(size_t)tile * kNodeItems + threadIdx.x];
     const int k0 = a.ntile[tile], tn = a.ntile[tile + 1] - k0;
     const double ad = a.ad, aa = a.aa, adt = 1. - a.ad, aat = 1. - a.aa;
     const bool btvdv = a.itvdv > 0;
-    const int nlv = min(a.nlv, NL);
 
-    // The tile's node-layers that exist (l <= ilhkv of the node, members
-    // still substepping), layer by layer with the nodes ascending in each:
-    // phase 1 takes exactly these, and a layer's loads stay in node order.
-    // Work-item kk owns node kk; each wavefront counts its nodes per layer
-    // with a ballot, one work-item turns the counts into list positions.
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    int lmk = 0;
-    if ((int)threadIdx.x < tn) {
-        const int k = k0 + threadIdx.x;
-        lmk = min(a.ilhkv[k], nlv);
-        if (a.mem_istot && a.isact > a.mem_istot[a.node_mem[k]]) lmk = 0;
-    }
-    for (int l = 1; l <= nlv; l++) {
-        const unsigned long long m = __ballot(lmk >= l);
-        if (lane == 0) lmask[wv][l] = m;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int off = 0;
-        for (int l = 1; l <= nlv; l++)
-            for (int w = 0; w < kWaves; w++) {
-                lbase[w][l] = off;
-                off += __popcll(lmask[w][l]);
-            }
-        nitems_s = off;
-    }
-    __syncthreads();
-    const int nitems = nitems_s;
-    if (nitems > kNodeItems) {      // the tile table guarantees otherwise
-        if (threadIdx.x == 0) atomicCAS(a.err, 0, ERR_CONZ);
-        return;
-    }
-    for (int l = 1; l <= lmk; l++) items[lbase[wv][l] + __popcll(lmask[wv][l] & below)] = (int)threadIdx.x | (l << 16);
-    __syncthreads();
-
-    // phase 1: one work-item per node-layer
-    for (int it = threadIdx.x; it < nitems; it += blockDim.x) {
-        const int kk = items[it] & 0xffff, l = items[it] >> 16, k = k0 + kk;
-        const int lmaxk = a.ilhkv[k];
+    // phase 1: one work-item per node-layer; members past their last substep
+    // are left alone
+    bool on = ent.x >= 0;
+    const int k = on ? ent.w : 0;
+    if (a.mem_istot && on && a.isact > a.mem_istot[a.node_mem[k]]) on = false;
+    if (on) {
+        const int l = (ent.x & 31) + 1, lmaxk = ((ent.x >> 5) & 31) + 1, it = (ent.x >> 10) & 255;
         double dt = a.dt, rso = a.rso, rsn = a.rsn;
         if (a.mem_istot) {
             const int ist = a.mem_istot[a.node_mem[k]];
@@ -600,7 +577,25 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
         }
         const double rsot = 1. - rso, rsnt = 1. - rsn;
         // incident elements in colour order: list positions q0 .. q0+cnt-1
-        const int q0 = a.nkc_ptr[k], cnt = a.nkc_ptr[k + 1] - q0;
+        const int q0 = ent.y;
+        int cnt = ent.x >> 18;
+        if (cnt == kNodeCntMax) cnt = a.nkc_ptr[k + 1] - q0;
+        // The first kIncWidth positions are read unconditionally (clamped to
+        // the list), contiguous for the node; the last two pairs only by
+        // wavefronts that hold such a node; the rest one by one.
+        double saj[kIncWidth], shf0[kIncWidth], shf1[kIncWidth];
+        const size_t hl = (size_t)(l - 1) * NT * a.nslot;
+        const bool any6 = __any(cnt > 6), any8 = __any(cnt > 8);
+#pragma unroll
+        for (int s = 0; s < kIncWidth; s++) {
+            saj[s] = 0.; shf0[s] = 0.; shf1[s] = 0.;
+            if (s < 6 || (s < 8 ? any6 : any8)) {
+                const int q = min(q0 + s, a.nslot - 1);
+                saj[s] = a.slot_aj4[q];
+                shf0[s] = (double)a.hbuf[hl + q];
+                if (NT > 1) shf1[s] = (double)a.hbuf[hl + (size_t)a.nslot + q];
+            }
+        }
         // node column around l (zero outside 1..lmaxk)
         double ckw[NT][5], hokw[5], hnkw[5];
 #pragma unroll
@@ -646,14 +641,18 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
         // for v >= 1, and the upstream value beyond the next layer for v = 2.
         // Each distinct term is computed once, with the arithmetic of the
         // truncated column (vertical_flux_ie: zero at the column's ends).
+        // Without a layer below l its coefficients are zero; the explicit
+        // part of the diffusion (adt) is left out when there is none.
         const double hom = hokw[1], hoc = hokw[2], hop = hokw[3];
         const double hnm = hnkw[1], hnc = hnkw[2], hnp = hnkw[3];
         const double pm = (l - 1 >= 1) ? 1. : 0.;
-        const double hmotop = 2. * rvptop * pm / (hom + hoc);
         const double hmntop = 2. * rvptop * pm / (hnm + hnc);
-        // [0]: no layer below l (pp = 0, the lower neighbour zero), [1]: one
-        const double hmobot[2] = {2. * rvpbot * 0. / (hoc + 0.), 2. * rvpbot * 1. / (hoc + hop)};
-        const double hmnbot[2] = {2. * rvpbot * 0. / (hnc + 0.), 2. * rvpbot * 1. / (hnc + hnp)};
+        const double hmnbot[2] = {0., 2. * rvpbot * 1. / (hnc + hnp)};
+        double hmotop = 0., hmobot = 0.;
+        if (adt != 0.) {
+            hmotop = 2. * rvptop * pm / (hom + hoc);
+            hmobot = 2. * rvpbot * 1. / (hoc + hop);
+        }
         // matrix coefficients: [0] for v = 0, [1] for v >= 1 (the lower
         // diagonal does not depend on the truncation)
         double clcv[2], clpv[2], clm = 0.;
@@ -683,37 +682,31 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const double c0 = ckw[t][0], c1 = ckw[t][1], c2 = ckw[t][2], c3 = ckw[t][3], c4 = ckw[t][4];
-            fd0[t] = adt * ((c2 - 0.) * hmobot[0] - (c1 - c2) * hmotop);
-            fd1[t] = adt * ((c2 - c3) * hmobot[1] - (c1 - c2) * hmotop);
+            fd0[t] = adt * ((c2 - 0.) * 0. - (c1 - c2) * hmotop);
+            fd1[t] = adt * ((c2 - c3) * hmobot - (c1 - c2) * hmotop);
             // flux across the top interface (none at the surface): [0]
-            // without a layer below l, [1] with one (they differ only in
-            // the upstream value of a rising flow)
+            // without a layer below l, [1] with one.  They differ only for a
+            // rising flow, whose upstream value [0] is the downstream one: the
+            // limiter is zero there and the face takes the centre's value.
             double vt[2] = {0., 0.};
             if (l >= 2) {
                 const double w = wtop;
-                if (!btvdv) {
-                    vt[0] = vt[1] = w * ((w > 0.) ? c2 : c1);
-                } else if (w > 0.) {
-                    vt[0] = w * tvd_face(c2, c1, c1, alfa_t);
-                    vt[1] = w * tvd_face(c2, c1, c3, alfa_t);
-                } else {
-                    vt[0] = vt[1] = w * tvd_face(c1, c2, (l - 2 >= 1) ? c0 : c2, alfa_t);
-                }
+                const bool up = w > 0.;
+                double face = up ? c2 : c1;
+                if (btvdv) face = tvd_face(face, up ? c1 : c2, up ? c3 : (l - 2 >= 1 ? c0 : c2), alfa_t);
+                vt[1] = w * face;
+                vt[0] = up ? w * c2 : vt[1];
             }
             // flux across the bottom interface (none for v = 0): [0] for
-            // v = 1, [1] for v = 2 (they differ only in the upstream value
-            // of a rising flow)
+            // v = 1, [1] for v = 2, differing in the same way
             double vb[2];
             {
                 const double w = wbot;
-                if (!btvdv) {
-                    vb[0] = vb[1] = w * ((w > 0.) ? c3 : c2);
-                } else if (w > 0.) {
-                    vb[0] = w * tvd_face(c3, c2, c2, alfa_b);
-                    vb[1] = w * tvd_face(c3, c2, c4, alfa_b);
-                } else {
-                    vb[0] = vb[1] = w * tvd_face(c2, c3, (l - 1 >= 1) ? c1 : c3, alfa_b);
-                }
+                const bool up = w > 0.;
+                double face = up ? c3 : c2;
+                if (btvdv) face = tvd_face(face, up ? c2 : c3, up ? c4 : (l - 1 >= 1 ? c1 : c3), alfa_b);
+                vb[1] = w * face;
+                vb[0] = up ? w * c3 : vb[1];
             }
             fw0[t] = aat * (vt[0] - 0.);
             fw1[t] = aat * (vt[1] - vb[0]);
@@ -723,16 +716,16 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
         double cn[NT], cd = 0., clo = 0., chi = 0.;
 #pragma unroll
         for (int t = 0; t < NT; t++) cn[t] = 0.;
-        // One element's terms (bottom layer ilev, 4 * area aj4, horizontal
-        // terms hf0 and hf1 of tracers 0 and 1).  A macro rather than a
-        // lambda: the lambda's captures stayed in scratch memory.
+        // One element's terms (whether it has layer l, the next one, the one
+        // after; 4 * area aj4, horizontal terms hf0 and hf1 of tracers 0 and
+        // 1).  A macro rather than a lambda: the lambda's captures stayed in
+        // scratch memory.
         static_assert(NT <= 2, "two tracers per launch");
-#define CONZ_ADD(ilev_, aj4_, hf0_, hf1_)                                                            \
+#define CONZ_ADD(has_, deep_, deeper_, aj4_, hf0_, hf1_)                                             \
     do {                                                                                           \
-        const int ilev = (ilev_);                                                                  \
-        if (ilev >= l) {                                                                           \
+        if (has_) {                                                                                \
             const double aj4 = (aj4_), hfv[2] = {(hf0_), (hf1_)};                                  \
-            const bool deep = ilev > l, deeper = ilev > l + 1; /* v >= 1, v == 2 */                \
+            const bool deep = (deep_), deeper = (deeper_); /* v >= 1, v == 2 */                    \
             _Pragma("unroll") for (int t = 0; t < NT; t++) {                                       \
                 const double fw = deeper ? fw2[t] : (deep ? fw1[t] : fw0[t]);                      \
                 const double fd = deep ? fd1[t] : fd0[t];                                          \
@@ -744,25 +737,18 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
             cd += aj4 * dt * (deep ? clcv[1] : clcv[0]) + aj4 * (1. + dt * 0.) * hnc;              \
         }                                                                                          \
     } while (0)
-        // the first kIncWidth positions are read unconditionally (clamped
-        // to the list), contiguous for the node; the rest one by one
-        int slv[kIncWidth];
-        double saj[kIncWidth], shf0[kIncWidth], shf1[kIncWidth];
-        const size_t hl = (size_t)(l - 1) * NT * a.nslot;
-#pragma unroll
-        for (int s = 0; s < kIncWidth; s++) {
-            const int q = min(q0 + s, a.nslot - 1);
-            slv[s] = a.slot_lev[q];
-            saj[s] = a.slot_aj4[q];
-            shf0[s] = (double)a.hbuf[hl + q];
-            shf1[s] = NT > 1 ? (double)a.hbuf[hl + (size_t)a.nslot + q] : 0.;
-        }
+        // (a position beyond the list has no layer)
+        const unsigned reach = (unsigned)ent.z;
 #pragma unroll
         for (int s = 0; s < kIncWidth; s++)
-            if (s < cnt) CONZ_ADD(slv[s], saj[s], shf0[s], shf1[s]);
-        for (int q = q0 + kIncWidth; q < q0 + cnt; q++)
-            CONZ_ADD(a.slot_lev[q], a.slot_aj4[q], (double)a.hbuf[hl + q],
+            if (s < 6 || (s < 8 ? any6 : any8))
+                CONZ_ADD((reach >> s) & 1u, (reach >> (kIncWidth + s)) & 1u, (reach >> (2 * kIncWidth + s)) & 1u, saj[s],
+                         shf0[s], shf1[s]);
+        for (int q = q0 + kIncWidth; q < q0 + cnt; q++) {
+            const int ilev = a.slot_lev[q];
+            CONZ_ADD(ilev >= l, ilev > l, ilev > l + 1, a.slot_aj4[q], (double)a.hbuf[hl + q],
                      NT > 1 ? (double)a.hbuf[hl + (size_t)a.nslot + q] : 0.);
+        }
 #undef CONZ_ADD
         // conz3d_nodes: boundary mass flux
         if (a.mflux) {
@@ -802,18 +788,16 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
     __syncthreads();
 
     // phase 2: the column solve of conz3d_nodes, one work-item per node; the
-    // tracers share the column matrix and its elimination.  Layer l of node
-    // kk sits at list position lstart[l] + (tile nodes before kk that have
-    // a layer l).
-    const int kk = threadIdx.x, k = k0 + kk;
+    // tracers share the column matrix and its elimination.  Layer l of a
+    // node lies l - 1 places after its first one.
+    const int kk = threadIdx.x, kn = k0 + kk;
     if (kk >= tn) return;
-    if (a.mem_istot && a.isact > a.mem_istot[a.node_mem[k]]) return;
-    const int lmaxk = a.ilhkv[k];
-    auto pos = [&](int l0) -> int { return lbase[wv][l0 + 1] + __popcll(lmask[wv][l0 + 1] & below); };
-    auto cn = [&](int t, int l0) -> double & { return cnP[t][pos(l0)]; };
-    auto cd = [&](int l0) -> double & { return cdP[pos(l0)]; };
-    auto clo = [&](int l0) -> double & { return cloP[pos(l0)]; };
-    auto chi = [&](int l0) -> double & { return chiP[pos(l0)]; };
+    if (a.mem_istot && a.isact > a.mem_istot[a.node_mem[kn]]) return;
+    const int lmaxk = a.ilhkv[kn], p0 = a.nplace[kn];
+    auto cn = [&](int t, int l0) -> double & { return cnP[t][p0 + l0]; };
+    auto cd = [&](int l0) -> double & { return cdP[p0 + l0]; };
+    auto clo = [&](int l0) -> double & { return cloP[p0 + l0]; };
+    auto chi = [&](int l0) -> double & { return chiP[p0 + l0]; };
     bool bad = false;
     if ((aa == 0. && ad == 0.) || a.nlv == 1) {
         for (int l = 1; l <= lmaxk; l++)
@@ -858,19 +842,24 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
     }
     if (bad) { atomicCAS(a.err, 0, ERR_CONZ); return; }
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-        for (int l = 1; l <= a.nlvdi; l++) a.c[t][(size_t)(l - 1) * nkn + k] = (S)(l <= lmaxk ? cn(t, l - 1) : 0.);
+    for (int t = 0; t < NT; t++) {
+        for (int l = 1; l <= lmaxk; l++) a.c[t][(size_t)(l - 1) * nkn + kn] = (S)cn(t, l - 1);
+        // zero below the bottom: once per step (nothing else writes there)
+        if (a.clear_below)
+            for (int l = lmaxk + 1; l <= a.nlvdi; l++) a.c[t][(size_t)(l - 1) * nkn + kn] = (S)0;
+    }
 }
 
 template <typename S>
 static ConzArgs<S> conz_args(Model &M, const TracerSet &ts, int istot, int isact, void *hbuf, void *rec);
 
-template <typename S, int NL, int NT>
-static int conz_nl(Model &M, const TracerSet &ts, int istot, int isact, hipStream_t st, void *hbuf, void *rec,
-                   bool prep) {
+template <typename S, int NT>
+static int conz_t(Model &M, const TracerSet &ts, int istot, int isact, hipStream_t st, void *hbuf, void *rec,
+                  bool prep) {
     if (!M.m.conz_eitem || !M.m.conz_ntile) return hip_check(M, hipErrorNotInitialized, "conz3d: no basin");
     if (!rec) return hip_check(M, hipErrorInvalidValue, "conz3d: no element-layer record buffer");
-    const ConzArgs<S> a = conz_args<S>(M, ts, istot, isact, hbuf, rec);
+    ConzArgs<S> a = conz_args<S>(M, ts, istot, isact, hbuf, rec);
+    a.clear_below = prep;          // a step's first substep, and every substep called by itself
     const int ge = (M.m.n_eitem + kThreads - 1) / kThreads;
     if (prep) {
         launch_timed(M, T_CONZ_PREP, k_conz_prep<S>, dim3(ge), dim3(kThreads), 0, st, a);
@@ -893,9 +882,9 @@ static int conz_nl(Model &M, const TracerSet &ts, int istot, int isact, hipStrea
     HIPCHK(M, hipGetLastError());
     if (a.cobs || a.wsinkv || a.load) {
         if (NT != 1) return hip_check(M, hipErrorInvalidValue, "conz3d: tracer terms need one tracer per launch");
-        launch_timed(M, T_CONZ_NODE, k_conz_node<S, NL, 1, true>, dim3(M.m.n_ntile), dim3(kThreads), 0, st, a);
+        launch_timed(M, T_CONZ_NODE, k_conz_node<S, 1, true>, dim3(M.m.n_ntile), dim3(kThreads), 0, st, a);
     } else {
-        launch_timed(M, T_CONZ_NODE, k_conz_node<S, NL, NT, false>, dim3(M.m.n_ntile), dim3(kThreads), 0, st, a);
+        launch_timed(M, T_CONZ_NODE, k_conz_node<S, NT, false>, dim3(M.m.n_ntile), dim3(kThreads), 0, st, a);
     }
     HIPCHK(M, hipGetLastError());
     return 0;
@@ -938,6 +927,7 @@ static ConzArgs<S> conz_args(Model &M, const TracerSet &ts, int istot, int isact
     a.hbuf = (S *)hbuf;
     a.err = M.d_err;
     a.eitem = M.m.conz_eitem; a.n_eitem = M.m.n_eitem; a.ntile = M.m.conz_ntile;
+    a.nent = (const int4 *)M.m.conz_nent; a.nplace = M.m.conz_nplace;
     if (ts.n == 1 && tracer_has_terms(M, ts.itr[0])) {
         const int t = ts.itr[0];
         if (M.tr_robs[t] != 0.f && M.s.cobs[t] && M.s.rtauv[t]) {
@@ -975,22 +965,6 @@ size_t conz_record_bytes(const Model &M) { return conz_rec_bytes(M.m.n_eitem); }
 size_t conz_hbuf_terms(const Model &M, int ntr) { return (size_t)ntr * 3 * M.nlvdi * M.nel; }
 size_t conz_hbuf_elems(const Model &M, int ntr) {
     return conz_hbuf_terms(M, ntr) + (size_t)ntr * 2 * M.nlvdi * M.nkn;
-}
-
-template <typename S, int NT>
-static int conz_t(Model &M, const TracerSet &ts, int istot, int isact, hipStream_t st, void *hbuf, void *rec,
-                  bool prep) {
-    switch (M.nl_tmpl) {
-    case 1: return conz_nl<S, 1, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 2: return conz_nl<S, 2, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 4: return conz_nl<S, 4, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 8: return conz_nl<S, 8, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 12: return conz_nl<S, 12, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 16: return conz_nl<S, 16, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 20: return conz_nl<S, 20, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    case 24: return conz_nl<S, 24, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    default: return conz_nl<S, 32, NT>(M, ts, istot, isact, st, hbuf, rec, prep);
-    }
 }
 
 // uvtopr (transforms.f90:215-270) at the open-boundary nodes followed by

@@ -34,6 +34,7 @@ constexpr int kIncWidth = 10;                        // incident elements per no
 constexpr int kConzChunk = 64;
 constexpr int kNodeTileMax = kThreads;
 constexpr int kNodeItems = kThreads;
+constexpr int kNodeCntMax = 63;                      // list lengths from here on are read from the list
 
 // error codes written by kernels into Model::d_err[0]
 enum DevErr { ERR_NONE = 0, ERR_SETNOD = 1, ERR_SETUVD = 3, ERR_SETDEPTH = 4, ERR_VOLUME = 5,
@@ -109,6 +110,13 @@ struct Mesh {                 // device copies of init-time data
     // tiles as first nodes [n_ntile + 1], built for at most ntile_tn nodes
     int *conz_eitem = nullptr, *conz_ntile = nullptr;
     int n_eitem = 0, n_ntile = 0, ntile_tn = 0;
+    // the tiles' node-layers, layer by layer with the nodes ascending in each,
+    // [tile*kNodeItems + i] as int4: {(l-1) | (lmax-1) << 5 | place << 10 |
+    // list length << 18 (at most kNodeCntMax), list start, elements of the
+    // first kIncWidth list positions that have layer l / l+1 / l+2 (one bit
+    // each, kIncWidth apart), node}, -1 in the first word of unused entries;
+    // and each node's first place in its tile (its layers follow one another)
+    int *conz_nent = nullptr, *conz_nplace = nullptr;
     // the node-layer list, k << 5 | (l - 1), in chunks of kConzChunk nodes
     // taken layer by layer (scalar_stability)
     int *conz_nitem = nullptr;
