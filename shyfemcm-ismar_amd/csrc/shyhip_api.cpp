@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -24,6 +25,21 @@ int hip_check(Model &M, hipError_t e, const char *what) {
     if (e == hipSuccess) return 0;
     M.err = std::string("HIP error in ") + what + ": " + hipGetErrorString(e);
     return 1;
+}
+
+int wait_report(Model &M, int word, int seq) {
+    const auto there = [&] { return __atomic_load_n(M.h_pinned + word, __ATOMIC_ACQUIRE) == seq; };
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 1;; i++) {
+        if (there()) return 0;
+        if ((i & 255) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(4)) break;
+    }
+    HIPCHK(M, hipStreamSynchronize(M.stream));
+    if (!there()) {
+        M.err = "the device's report did not arrive";
+        return 1;
+    }
+    return 0;
 }
 
 std::recursive_mutex &device_lock() {
@@ -313,11 +329,12 @@ int shyhip_create(shyhip_model **out, int precision, int nkn, int nel, int nlvdi
             delete h;
             return fail(nullptr, "stream");
         }
-        if (hip_check(M, hipHostMalloc((void **)&M.h_pinned, 64 * sizeof(int)), "hipHostMalloc")) {
+        if (hip_check(M, hipHostMalloc((void **)&M.h_pinned, 64 * sizeof(int), hipHostMallocCoherent), "hipHostMalloc")) {
             delete h;
             return fail(nullptr, "pinned");
         }
     }
+    std::memset(M.h_pinned, 0, 64 * sizeof(int));
     // default parameters (def_para.f90)
     shyhip_params &p = M.p;
     p.dt = 300.; p.azpar = 0.5f; p.ampar = 0.5f; p.afpar = 0.5f; p.atpar = 1.f; p.adpar = 1.f; p.aapar = 1.f;
@@ -541,7 +558,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
                      dalloc(M, &M.d_mem_istot, 2 * (size_t)nmem) || dalloc(M, &M.d_mem_stab, 3 * (size_t)nmem);
             if (rc) return 1;
             std::lock_guard<std::recursive_mutex> lock(device_lock());
-            HIPCHK(M, hipHostMalloc((void **)&M.h_mem_stab, 2 * (size_t)nmem * sizeof(unsigned long long)));
+            HIPCHK(M, hipHostMalloc((void **)&M.h_mem_stab, 2 * (size_t)nmem * sizeof(unsigned long long), hipHostMallocCoherent));
             M.cur_mem_istot = M.d_mem_istot;
         }
     }

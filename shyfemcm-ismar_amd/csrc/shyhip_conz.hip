@@ -1389,20 +1389,31 @@ __global__ void __launch_bounds__(kThreads) k_conz_stab(int nkn, int nel, int nl
 // shympi_max of a real), rindex = dt * index / rstol in the model's real,
 // istot = 1 + rindex truncated.  w holds nmem maxima, then nmem istot and
 // nmem rindex bits (as double); istot also goes to mem_istot (may be null);
-// the maxima are cleared for the next call.  One work-item per member.
+// the maxima are cleared for the next call.  One work-item per member of one
+// workgroup; the results also go to the host's pinned memory (host: nmem
+// istot, nmem rindex), with the number of this report (hseq) behind them.
+constexpr int kStabFinal = 256;
+
 template <typename S>
-__global__ void k_conz_stab_final(unsigned long long *w, int nmem, S dt, float rstol, int *mem_istot) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= nmem) return;
-    double stabind = __longlong_as_double((long long)w[m]);
-    stabind = (double)(float)stabind;
-    const S sindex = (S)(stabind / (double)rstol);
-    const S ri = dt * sindex;
-    const int ist = (int)((S)1 + ri);
-    w[nmem + m] = (unsigned long long)(long long)ist;
-    w[2 * nmem + m] = (unsigned long long)__double_as_longlong((double)ri);
-    if (mem_istot) mem_istot[m] = ist;
-    w[m] = 0ull;
+__global__ __launch_bounds__(kStabFinal) void k_conz_stab_final(unsigned long long *w, int nmem, S dt, float rstol,
+                                                                int *mem_istot, unsigned long long *host, int *hseq,
+                                                                int seq) {
+    for (int m = threadIdx.x; m < nmem; m += kStabFinal) {
+        double stabind = __longlong_as_double((long long)w[m]);
+        stabind = (double)(float)stabind;
+        const S sindex = (S)(stabind / (double)rstol);
+        const S ri = dt * sindex;
+        const int ist = (int)((S)1 + ri);
+        w[nmem + m] = (unsigned long long)(long long)ist;
+        w[2 * nmem + m] = (unsigned long long)__double_as_longlong((double)ri);
+        host[m] = (unsigned long long)(long long)ist;
+        host[nmem + m] = (unsigned long long)__double_as_longlong((double)ri);
+        if (mem_istot) mem_istot[m] = ist;
+        w[m] = 0ull;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(hseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // per member (nmem = 1: the model): istot[m] and rindex[m] on the host
@@ -1429,13 +1440,12 @@ static int stab_t(Model &M, float rstol, int *istot, double *rindex) {
                        (const S *)M.s.difhv, M.p.rkpar > 0.f ? (const S *)M.m.wdif : (const S *)nullptr,
                        robs, (const S *)rtauv, wsink, (const S *)wsinkv, nmem > 1 ? M.d_node_mem : nullptr, w);
     HIPCHK(M, hipGetLastError());
-    hipLaunchKernelGGL(k_conz_stab_final<S>, dim3((nmem + 63) / 64), dim3(64), 0, M.stream, w, nmem, (S)M.p.dt,
-                       rstol, nmem > 1 ? M.cur_mem_istot : nullptr);
+    unsigned long long *hbuf = nmem > 1 ? M.h_mem_stab : (unsigned long long *)(M.h_pinned + HP_STAB);
+    const int seq = ++M.report_seq;
+    hipLaunchKernelGGL(k_conz_stab_final<S>, dim3(1), dim3(kStabFinal), 0, M.stream, w, nmem, (S)M.p.dt, rstol,
+                       nmem > 1 ? M.cur_mem_istot : nullptr, hbuf, M.h_pinned + HP_SEQ_STAB, seq);
     HIPCHK(M, hipGetLastError());
-    unsigned long long *hbuf = nmem > 1 ? M.h_mem_stab : (unsigned long long *)(M.h_pinned + 8);
-    HIPCHK(M, hipMemcpyAsync(hbuf, w + nmem, 2 * nmem * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             M.stream));
-    HIPCHK(M, hipStreamSynchronize(M.stream));
+    if (wait_report(M, HP_SEQ_STAB, seq)) return 1;
     for (int m = 0; m < nmem; m++) {
         istot[m] = (int)(long long)hbuf[m];
         std::memcpy(&rindex[m], &hbuf[nmem + m], sizeof(double));

@@ -180,6 +180,10 @@ struct State {
 enum { CT_STOPIT = 0, CT_CONV = 1, CT_FAIL = 2, CT_NMV = 3, CT_ITS = 4, CT_REFCONV = 5, CT_FACTOR = 6,
        CT_NREF = 7, CT_MAXIT = 8, CT_RITS = 9, CT_NRITS = 6, CT_WAIT = 15, CT_WORDS = 16 };
 
+// words of Model::h_pinned: device error words, scalar-stability results (one
+// model), solver control words, and the numbers of the last reports
+enum { HP_ERR = 0, HP_STAB = 8, HP_CTRL = 16, HP_SEQ = 40, HP_SEQ_STAB = 41 };
+
 struct Solver {               // Krylov work space (value type V = S of the model)
     int nblk = 0, brows = 0, max_blk_nnz = 0, max_blk_pairs = 0, nparts = 0, max_elev = 0;
     int last_its[8] = {};     // iteration count of the previous solve, per solve kind
@@ -271,7 +275,8 @@ struct Model {
     int nnz = 0, ncolor = 0, nbnd = 0;
     int *d_err = nullptr;     // [16] device error words + counters; [8..13] the
                               // scalar-stability maximum and result (64-bit words)
-    int *h_pinned = nullptr;  // pinned host mirror for small readbacks
+    int *h_pinned = nullptr;  // pinned host mirror for small readbacks (HP_*), written by kernels
+    int report_seq = 0;       // number of the last report a kernel was asked for
     double dtime = 0., dtime_old = -1.;
     bool has_coriolis = false, has_mflux = false, tvd_ready = false;
     // each tracer's nudging factor, sinking velocity and load factor
@@ -526,6 +531,11 @@ int launch_bndo(Model &M, const TracerSet &ts, hipStream_t st, int isact, void *
 int launch_scalar_stability(Model &M, float rstol, int *istot, double *rindex);
 
 // helpers
+// Waits until word `word` of h_pinned holds seq, which a kernel on the
+// model's stream writes after its results: polled for a few milliseconds (a
+// stream synchronisation returns 10 us later, and a copy before it is one
+// more kernel), then by synchronising.
+int wait_report(Model &M, int word, int seq);
 int hip_check(Model &M, hipError_t e, const char *what);
 // One lock for the operations that may synchronise the whole device --
 // allocating and freeing device or pinned memory -- and for stream capture,

@@ -1789,13 +1789,27 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
 }
 
 // ---------------------------------------------------------------- host driver
-// one read-back: the solver's control words (into h_pinned[16..]) and the
-// device error word and counter d_err[0..1] (into h_pinned[0..1])
+// The solver's control words and the device error words into the host's
+// pinned memory, then the number of this report: the host waits for it
+// (wait_report) instead of two copies and a stream synchronisation.
+__global__ __launch_bounds__(64) void k_report(const int *ctrl, const int *err, int *host, int seq) {
+    const int t = threadIdx.x;
+    if (t < CT_WORDS) host[HP_CTRL + t] = ctrl[t];
+    else if (t < CT_WORDS + 2) host[HP_ERR + t - CT_WORDS] = err[t - CT_WORDS];
+    __threadfence_system();
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(host + HP_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// one read-back: the solver's control words and the device error word and
+// counter d_err[0..1] (into h_pinned[HP_ERR..])
 static int read_ctrl(Model &M, int *out, int n) {
-    HIPCHK(M, hipMemcpyAsync(M.h_pinned + 16, M.sv.ctrl, sizeof(int) * n, hipMemcpyDeviceToHost, M.stream));
-    HIPCHK(M, hipMemcpyAsync(M.h_pinned, M.d_err, 2 * sizeof(int), hipMemcpyDeviceToHost, M.stream));
-    HIPCHK(M, hipStreamSynchronize(M.stream));
-    for (int i = 0; i < n; i++) out[i] = M.h_pinned[16 + i];
+    const int seq = ++M.report_seq;
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, M.stream, (const int *)M.sv.ctrl, (const int *)M.d_err,
+                       M.h_pinned, seq);
+    HIPCHK(M, hipGetLastError());
+    if (wait_report(M, HP_SEQ, seq)) return 1;
+    for (int i = 0; i < n; i++) out[i] = M.h_pinned[HP_CTRL + i];
     return 0;
 }
 
