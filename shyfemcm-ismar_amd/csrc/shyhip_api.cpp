@@ -419,7 +419,8 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.blk_pdg, (void *)m.fs_col, (void *)m.fs_meta, (void *)m.blk_fdesc, (void *)m.blk_fpair,
                     (void *)m.blk_elp, (void *)m.blk_elr, (void *)m.blk_enlev, (void *)m.ell_col, (void *)m.ell_len, (void *)m.csr_ell,
                     (void *)m.z_lcol, (void *)m.z_hcol, (void *)m.z_hslot, (void *)m.z_hcnt, (void *)m.z_send,
-                    (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_nchf, (void *)m.z_nchb,
+                    (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_dentf, (void *)m.z_dentb, (void *)m.z_dptrf,
+                    (void *)m.z_dptrb, (void *)m.z_nchf, (void *)m.z_nchb,
                     (void *)m.fwd_rows, (void *)m.fwd_lptr, (void *)m.fwd_nlev, (void *)m.bwd_rows,
                     (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_el, (void *)m.tvd_kn, m.tvd_w,
                     (void *)m.tvd_lev, (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem,
@@ -892,10 +893,12 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
             }
             // tables and slots of the one-launch solve
             ZetaTables zt;
-            host_zeta_tables(nkn, M.h_rowptr, M.h_cols, bs, (int)M.esize(), zt);
+            host_zeta_tables(nkn, M.h_rowptr, M.h_cols, bs, (int)M.esize(), M.p.tri_sweeps == 0, zt);
             M.sv.zeta_t = zt.threads;
             M.sv.zeta_nwg = zt.nwg;
             M.sv.zeta_group = zt.group;
+            M.sv.zeta_members = zt.members;
+            M.sv.zeta_dmax = zt.dmax;
             M.sv.zeta_hmax = zt.hmax;
             M.sv.zeta_chmax = zt.chmax;
             M.sv.zeta_nsend = zt.nsend;
@@ -910,6 +913,12 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
                 rc |= dalloc(M, &m.z_chb, zt.chb.size()) || upload(M, m.z_chb, zt.chb.data(), zt.chb.size());
                 rc |= dalloc(M, &m.z_nchf, zt.nchf.size()) || upload(M, m.z_nchf, zt.nchf.data(), zt.nchf.size());
                 rc |= dalloc(M, &m.z_nchb, zt.nchb.size()) || upload(M, m.z_nchb, zt.nchb.data(), zt.nchb.size());
+                if (zt.members > 0) {
+                    rc |= dalloc(M, &m.z_dentf, zt.dentf.size()) || upload(M, m.z_dentf, zt.dentf.data(), zt.dentf.size());
+                    rc |= dalloc(M, &m.z_dentb, zt.dentb.size()) || upload(M, m.z_dentb, zt.dentb.data(), zt.dentb.size());
+                    rc |= dalloc(M, &m.z_dptrf, zt.dptrf.size()) || upload(M, m.z_dptrf, zt.dptrf.data(), zt.dptrf.size());
+                    rc |= dalloc(M, &m.z_dptrb, zt.dptrb.size()) || upload(M, m.z_dptrb, zt.dptrb.data(), zt.dptrb.size());
+                }
                 rc |= dalloc_s(M, &M.sv.xch, (size_t)4 * zt.nsend);
                 rc |= dalloc(M, &M.sv.pslot, kZetaSlotWords);
             }

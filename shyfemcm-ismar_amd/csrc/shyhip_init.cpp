@@ -638,13 +638,14 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
 // 0.333 ms, 50k nodes 0.391 / 0.448 against 0.371 / 0.403 ms; the line lies
 // between.  Blocks longer than 512 rows take 1024.
 constexpr int kZetaSmall = 128;
+constexpr int kZetaDense = 220;          // workgroups of a solve with dense rows (each takes a compute unit)
 
 static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
-                        int esize, int T, ZetaTables &zt) {
+                        int esize, int T, int members, ZetaTables &zt) {
     // several blocks only of whole wavefronts (their sums are kept apart)
-    const int nblk = bs.nblk, group = bs.brows % 64 == 0 ? T / bs.brows : 1, brows = group * bs.brows;
+    const int nblk = bs.nblk, group = members == 0 && bs.brows % 64 == 0 ? T / bs.brows : 1, brows = group * bs.brows;
     const int nwg = (nblk + group - 1) / group;
-    if (nblk > T || nblk > 512) return false;
+    if (nblk > T || nblk > 512 || (members > 0 && nblk * members > kZetaDense)) return false;
     // halos: the columns outside the workgroup's rows, ascending
     std::vector<std::vector<int>> halo(nwg);
     parallel_for(nwg, 16, [&](int b_begin, int b_end) {
@@ -666,7 +667,9 @@ static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector
     zt.hslot.assign((size_t)nwg * hmax, 0);
     zt.send.assign(n, -1);
     zt.lcol.assign((size_t)(kEllWidth / 2) * n, 0u);
-    // value slots in row order, each workgroup's first slot on a line of its own
+    // value slots in row order, each workgroup's first slot on a line of its
+    // own (a block of several workgroups: every row)
+    if (members > 1) std::fill(zt.send.begin(), zt.send.end(), 0);
     for (const auto &h : halo)
         for (int j : h) zt.send[j] = 0;
     zt.nsend = 0;
@@ -727,25 +730,77 @@ static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector
         out.assign((size_t)nblk * chmax, 0u);
         for (int b = 0; b < nblk; b++) std::copy(ch[dir][b].begin(), ch[dir][b].end(), out.begin() + (size_t)b * chmax);
     }
+    if (members > 0) {
+        // the transposed factors: for the row j at a position of the forward
+        // order, the entries (k, j) with k < j, which lie in U; backward, the
+        // entries (k, j) with k > j, in L
+        int dmax = 1;
+        std::vector<std::vector<unsigned>> ent[2];
+        for (int dir = 0; dir < 2; dir++) {
+            const std::vector<int> &rows = dir == 0 ? bs.fwd_rows : bs.bwd_rows;
+            std::vector<int> &ptr = dir == 0 ? zt.dptrf : zt.dptrb;
+            ent[dir].resize(nblk);
+            ptr.assign((size_t)nblk * stride, 0);
+            for (int b = 0; b < nblk; b++) {
+                const int b0 = b * bs.brows, nb = std::min(n, b0 + bs.brows) - b0, e0 = bs.rowptr[b0];
+                int *p = &ptr[(size_t)b * stride];
+                for (int t = 0; t < nb; t++) {
+                    const int j = rows[b0 + t];
+                    for (int q = bs.rowptr[b0 + j]; q < bs.rowptr[b0 + j + 1]; q++) {
+                        const int k = bs.cols[q];
+                        if (dir == 0 ? k >= j : k <= j) continue;
+                        int tq = -1;
+                        for (int r = bs.rowptr[b0 + k]; r < bs.rowptr[b0 + k + 1]; r++)
+                            if (bs.cols[r] == j) tq = r - e0;
+                        if (tq < 0 || tq > 0xffff) return false;      // (the pattern is symmetric)
+                        ent[dir][b].push_back((unsigned)tq | (unsigned)k << 16);
+                    }
+                    p[t + 1] = (int)ent[dir][b].size();
+                }
+                for (int t = nb; t < bs.brows; t++) p[t + 1] = p[nb];
+                dmax = std::max(dmax, (int)ent[dir][b].size());
+            }
+        }
+        zt.dmax = dmax;
+        for (int dir = 0; dir < 2; dir++) {
+            std::vector<unsigned> &out = dir == 0 ? zt.dentf : zt.dentb;
+            out.assign((size_t)nblk * dmax, 0u);
+            for (int b = 0; b < nblk; b++)
+                std::copy(ent[dir][b].begin(), ent[dir][b].end(), out.begin() + (size_t)b * dmax);
+        }
+        // LDS while the rows are computed (the kernel's zeta_lds), a
+        // workgroup's share of 160 KB less what it needs besides
+        const size_t setup = (size_t)bs.brows * (T == 512 ? 64 : 12) * esize + (size_t)(dmax + bs.brows) * (esize + 2) +
+                             4 * (size_t)bs.brows + 64;
+        if (setup > 140 * 1024) return false;
+    }
     zt.threads = T;
-    zt.nwg = nwg;
+    zt.nwg = members > 0 ? nblk * members : nwg;
     zt.group = group;
+    zt.members = members;
     return true;
 }
 
 void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
-                      int esize, ZetaTables &zt) {
+                      int esize, bool exact, ZetaTables &zt) {
     zt = ZetaTables();
     if (bs.brows > 1024) return;
     for (int i = 0; i < n; i++)
         if (rowptr[i + 1] - rowptr[i] > kEllWidth) return;
+    if (exact) {
+        // dense rows of the blocks' inverses: 64 rows of a block of at most
+        // 256, or 12 of a larger one, per workgroup (DenseShape)
+        const int T = bs.brows <= 256 ? 512 : 1024, own = T == 512 ? 64 : 12;
+        if (zeta_tables(n, rowptr, cols, bs, esize, T, (bs.brows + own - 1) / own, zt)) return;
+        zt = ZetaTables();
+    }
     if (bs.brows > 512) {
-        zeta_tables(n, rowptr, cols, bs, esize, 1024, zt);
+        zeta_tables(n, rowptr, cols, bs, esize, 1024, 0, zt);
         return;
     }
     const int n256 = bs.brows <= 256 ? (bs.brows % 64 == 0 ? (n + 255) / 256 : bs.nblk) : 1 << 30;
-    if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, zt)) return;
-    if (bs.brows <= 256) zeta_tables(n, rowptr, cols, bs, esize, 256, zt);
+    if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, 0, zt)) return;
+    if (bs.brows <= 256) zeta_tables(n, rowptr, cols, bs, esize, 256, 0, zt);
 }
 
 }  // namespace shy

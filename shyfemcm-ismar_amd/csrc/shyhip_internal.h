@@ -95,6 +95,10 @@ struct Mesh {                 // device copies of init-time data
     // level: first position | rows << 16, positions in fwd_rows / bwd_rows
     // relative to the block) and chunks per block
     unsigned *z_lcol = nullptr, *z_chf = nullptr, *z_chb = nullptr;
+    // dense rows (exact solves of small basins): entries of the transposed
+    // factors in the order of the two substitutions and their starts
+    unsigned *z_dentf = nullptr, *z_dentb = nullptr;
+    int *z_dptrf = nullptr, *z_dptrb = nullptr;
     int *z_hcol = nullptr, *z_hslot = nullptr, *z_hcnt = nullptr, *z_send = nullptr, *z_nchf = nullptr,
         *z_nchb = nullptr;
     int *fwd_rows = nullptr, *fwd_lptr = nullptr, *fwd_nlev = nullptr;
@@ -207,10 +211,11 @@ struct Solver {               // Krylov work space (value type V = S of the mode
                               // slots, FP32 copy, initial guess, cleared words)
     double *r64 = nullptr;    // FP64 residual (refinement)
     // one-launch solve: its workgroup size (0: not possible for this basin),
-    // workgroups and diagonal blocks of each, halo and chunk strides, exchange slots (4 buffers: values, partials);
+    // workgroups and diagonal blocks of each (or workgroups per block, for
+    // dense rows, else 0, with their entry stride), halo and chunk strides, exchange slots (4 buffers: values, partials);
     // workgroups per compute unit of each kind of triangular solve (0: not
     // asked yet, -1: cannot run), device and its compute units
-    int zeta_t = 0, zeta_nwg = 0, zeta_group = 1, zeta_hmax = 0, zeta_chmax = 0, zeta_nsend = 0;
+    int zeta_t = 0, zeta_nwg = 0, zeta_group = 1, zeta_members = 0, zeta_dmax = 0, zeta_hmax = 0, zeta_chmax = 0, zeta_nsend = 0;
     void *xch = nullptr;
     unsigned long long *pslot = nullptr;
     int zeta_occ[2] = {0, 0}, zeta_dev = 0, zeta_cus = 0;
@@ -439,12 +444,12 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
 // tables of the one-launch solve (Mesh::z_*) for values of esize bytes;
 // threads: its workgroup size, 0 when the basin's blocks do not fit it
 struct ZetaTables {
-    int threads = 0, nwg = 0, group = 1, hmax = 0, chmax = 0, nsend = 0;
-    std::vector<unsigned> lcol, chf, chb;
-    std::vector<int> hcol, hslot, hcnt, send, nchf, nchb;
+    int threads = 0, nwg = 0, group = 1, members = 0, dmax = 0, hmax = 0, chmax = 0, nsend = 0;
+    std::vector<unsigned> lcol, chf, chb, dentf, dentb;
+    std::vector<int> hcol, hslot, hcnt, send, nchf, nchb, dptrf, dptrb;
 };
 void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
-                      int esize, ZetaTables &zt);
+                      int esize, bool exact, ZetaTables &zt);
 
 // kernel launchers (shyhip_hydro.hip, shyhip_solver.hip, shyhip_conz.hip)
 int launch_set_dry(Model &M, int iweich, int bnewtime, int *changed);

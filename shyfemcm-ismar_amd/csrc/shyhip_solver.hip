@@ -81,7 +81,7 @@ struct SolvArgs {
     void *xch;
     unsigned long long *pslot;
     const int *send;
-    int nsend;
+    int nsend, zmembers;              // (zmembers: partial sums per block)
 };
 
 template <typename V>
@@ -116,6 +116,7 @@ static SolvArgs<V> solv_args(Model &M, const V *A, V *b, V *x0) {
         a.pslot = M.sv.pslot;
         a.send = M.m.z_send;
         a.nsend = M.sv.zeta_nsend;
+        a.zmembers = std::max(1, M.sv.zeta_members);
     }
     return a;
 }
@@ -1112,8 +1113,9 @@ __device__ inline void zeta_empty_slots(const SolvArgs<V> &a, int blk, int b0, i
     for (int b = 0; b < kZetaBufs; b++) {
         for (int li = threadIdx.x; li < nb; li += blockDim.x)
             if (const int q = a.send[b0 + li]; q >= 0) slot_clear(xch + (size_t)b * a.nsend + q, Slot<V>::empty);
-        if (threadIdx.x < kPartSlots * kPartCopies)
-            slot_clear(part_slot(a.pslot, b, threadIdx.x % kPartCopies, threadIdx.x / kPartCopies, blk),
+        for (int e = threadIdx.x; e < kPartSlots * kPartCopies * a.zmembers; e += blockDim.x)
+            slot_clear(part_slot(a.pslot, b, e % kPartCopies, e / kPartCopies % kPartSlots,
+                                 blk * a.zmembers + e / (kPartCopies * kPartSlots)),
                        Slot<double>::empty);
     }
     if (blk == 0 && threadIdx.x == 0) {
@@ -1138,6 +1140,12 @@ struct ZetaArgs {
     const unsigned *chunk_f, *chunk_b;
     const int *nch_f, *nch_b;
     int chmax;
+    // dense rows of the block inverses: workgroups per block; the transposed
+    // factors' entries (value's place | row << 16) in the order of rows_f and
+    // rows_b [blk*dmax + e] and their starts by position [blk*(brows+1) + t]
+    int members, dmax;
+    const unsigned *dent_f, *dent_b;
+    const int *dptr_f, *dptr_b;
     void *xch;                           // value slots [buf][nsend]
     unsigned long long *pslot;           // partial-sum slots [buf][kPartCopies][kPartStride]
     // FP32 path: the FP64 system and its refinement
@@ -1227,6 +1235,28 @@ struct SubExact {
     }
 };
 
+// Triangular solves of the one-launch kernel: Jacobi sweeps with the factor
+// row in registers, exact substitution, or exact by dense rows of the blocks'
+// inverses.  The last: substitution is a chain of up to 80 levels each way
+// (23 us per half iteration on 861 rows, 46 us on 256-row blocks of an 80 x 40
+// basin), so where the device has room each block is given to several
+// workgroups; each computes kOwn rows of the block's (LU)^-1 once per solve,
+// keeps them in registers, and applies them to the block's whole right-hand
+// side, which it forms itself (the vectors of all the block's rows are kept
+// by each of its workgroups, the rows applied elsewhere come with the halo).
+// A step of the 41 x 21 basin (861 rows, one block) 1.09 -> 0.65 ms, of an 80
+// x 40 basin 2.38 -> 0.48 ms, FP64, against the substitution.  The rows are
+// computed in 20 to 30 us; what bounds the rest is the exchange.
+enum { kSwept = 0, kSubst = 1, kDense = 2 };
+template <int T>
+struct DenseShape {                      // 512: blocks of up to 256 rows; 1024: of up to 1024
+    static constexpr int kOwn = T == 512 ? 64 : 12;           // rows per workgroup (what LDS holds at set-up)
+    static constexpr int kRows = T == 512 ? 8 : 1;            // per wavefront
+    static constexpr int kLanes = 64 / kRows;                 // lanes per row
+    static constexpr int kCols = (T == 512 ? 256 : 1024) / kLanes;   // columns per lane
+    static constexpr bool kRegs = T == 512;                   // rows in registers, else in LDS
+};
+
 // One row of the solve and its block's halo entries, in registers (1024
 // work-items have half the registers of 256 each: they read the matrix row
 // from cache in every product instead of spilling).  The entries of a row
@@ -1239,23 +1269,30 @@ constexpr int kRowFirst = 8;             // matrix entries always taken
 constexpr int kTriWidth = kFacWidth - 1; // entries of a row on one side of the diagonal
 constexpr int kTriFirst = 6;             // of these always taken
 
-template <typename V, int T, int KH, bool EXACT>
+template <typename V, int T, int KH, int MODE>
 struct ZetaRow {
     using U = typename Slot<V>::U;
     static constexpr bool kHold = T <= 512;
-    static constexpr int kTri = EXACT ? 1 : kTriWidth, kTriWords = (kTri + 1) / 2;
+    static constexpr int kTri = MODE == kSwept ? kTriWidth : 1, kTriWords = (kTri + 1) / 2;
+    using D = DenseShape<T>;
     // matrix row; (sweeps) factor row: L and U entries, inverted pivot
     V a[kHold ? kEllWidth : 1], l[kTri], u[kTri], dinv = 0;
     unsigned lc[kHold ? kEllWidth / 2 : 1], llc[kTriWords], uc[kTriWords];
     const V *ga;
     const unsigned *glc;
     bool more_a = false, more_l = false, more_u = false;   // some row of the wavefront fills the last slots
-    int i, wg, nh, nblk, n, sweeps, send, nsend;
+    int i, wg, nh, nsum, n, sweeps, send, nsend;   // nsum: partial sums of all workgroups
     bool mine;
     int hslot[KH];
     // LDS: operand (rows, then halo), two row buffers; exact: block factors
     V *X, *y, *w;
     SubExact<V, T> sf, sb;
+    // dense: this lane's part of its row of the block inverse, and the rows
+    // of the block that this workgroup applies
+    V pinv[MODE == kDense && D::kRegs ? D::kCols : 1];
+    const V *plds;
+    int own0 = 0, nown = 0;
+    bool own;                                // this work-item's row is one of them (else: every row)
     int rows, group;
     U *xch;
     unsigned long long *pslot;
@@ -1317,7 +1354,31 @@ struct ZetaRow {
     __device__ __attribute__((always_inline)) inline V precond(V t) {
         if (mine) y[threadIdx.x] = t;
         __syncthreads();
-        if constexpr (EXACT) {
+        if constexpr (MODE == kDense) {
+            // row w * kRows + lane / kLanes: the lanes of a row take every
+            // kLanes-th column
+            const int lane = threadIdx.x & 63, part = lane % D::kLanes;
+            V acc = 0;
+            if constexpr (D::kRegs) {
+#pragma unroll
+                for (int j = 0; j < D::kCols; j++) acc = acc + pinv[j] * y[part + D::kLanes * j];
+            } else if ((threadIdx.x >> 6) < D::kOwn) {
+                const V *p = plds + (size_t)(threadIdx.x >> 6) * (D::kLanes * D::kCols) + part;
+#pragma unroll
+                for (int j = 0; j < D::kCols; j++) acc = acc + p[D::kLanes * j] * y[part + D::kLanes * j];
+            }
+            double sum = (double)acc;
+            if constexpr (D::kLanes == 64) {
+                sum = wave_sum(sum);
+            } else {
+                sum = sum + dpp_f64<0xB1>(sum);
+                sum = sum + dpp_f64<0x4E>(sum);
+                sum = sum + dpp_f64<0x141>(sum);
+            }
+            if (part == 0) w[(threadIdx.x >> 6) * D::kRows + lane / D::kLanes] = (V)sum;
+            __syncthreads();
+            return own ? w[threadIdx.x - own0] : (V)0;
+        } else if constexpr (MODE == kSubst) {
             if ((int)threadIdx.x < 64 * group) {
                 sf.template run<false>(y);
                 sb.template run<true>(y);
@@ -1347,10 +1408,11 @@ struct ZetaRow {
         }
     }
     // Exchange of one epoch: the workgroups' partial sums of q (totals
-    // returned to everyone) and, with HALO, the rows' values own (the halo
-    // entries returned in h).  False when a wait ran out.
+    // returned to everyone) and, with HALO, the rows' values v (the halo
+    // entries returned in h; dense: v of the block's other rows too).  False
+    // when a wait ran out.
     template <int NQ, bool HALO>
-    __device__ __attribute__((always_inline)) inline bool exchange(double (&q)[NQ], V own, V (&h)[KH]) {
+    __device__ __attribute__((always_inline)) inline bool exchange(double (&q)[NQ], V &v, V (&h)[KH]) {
         // the wavefronts' sums
         __shared__ double red[NQ][T / 64], tot[NQ][kWaves], hi[NQ][T > kThreads ? kThreads : 1];
 #pragma unroll
@@ -1358,7 +1420,7 @@ struct ZetaRow {
         const int buf = epoch & (kZetaBufs - 1);
         U *vs = xch + (size_t)buf * nsend;
         wait_stores();          // the slots emptied after the last exchange
-        if (HALO && send >= 0) slot_put<V>(vs + send, own);
+        if (HALO && own && send >= 0) slot_put<V>(vs + send, v);
         if ((threadIdx.x & 63) == 0)
 #pragma unroll
             for (int k = 0; k < NQ; k++) red[k][threadIdx.x >> 6] = q[k];
@@ -1366,7 +1428,7 @@ struct ZetaRow {
         // Each block's sum: its wavefronts' in order (a workgroup with more
         // than one block has blocks of whole wavefronts).
         const int bw = group == 1 ? T / 64 : rows / (64 * group);
-        if (nblk == 1) {
+        if (nsum == 1) {
 #pragma unroll
             for (int k = 0; k < NQ; k++) {
                 q[k] = red[k][0];
@@ -1378,12 +1440,13 @@ struct ZetaRow {
             const int copy = e % kPartCopies, g = e / kPartCopies % group, k = e / (kPartCopies * group);
             double t = red[k][g * bw];
             for (int w = 1; w < bw; w++) t += red[k][g * bw + w];
-            if (wg * group + g < nblk) slot_put<double>(part_slot(pslot, buf, copy, k, wg * group + g), t);
+            if (wg * group + g < nsum) slot_put<double>(part_slot(pslot, buf, copy, k, wg * group + g), t);
         }
         const unsigned long long *ps = part_slot(pslot, buf, wg % kPartCopies, 0, threadIdx.x);
         unsigned long long pv[NQ];
-        U hv[KH];
-        const bool hasp = (int)threadIdx.x < nblk;
+        U hv[KH], rv = 0;
+        const bool recv = MODE == kDense && HALO && mine && !own;
+        const bool hasp = (int)threadIdx.x < nsum;
         int spin = 0;
         for (;;) {
             bool ok = true;
@@ -1394,6 +1457,7 @@ struct ZetaRow {
 #pragma unroll
                 for (int k = 0; k < KH; k++)
                     if ((int)threadIdx.x + k * T < nh) hv[k] = slot_get(vs + hslot[k]);
+            if (recv) rv = slot_get(vs + send);
             if (hasp)
 #pragma unroll
                 for (int k = 0; k < NQ; k++) ok = ok && pv[k] != Slot<double>::empty;
@@ -1401,6 +1465,7 @@ struct ZetaRow {
 #pragma unroll
                 for (int k = 0; k < KH; k++)
                     if ((int)threadIdx.x + k * T < nh) ok = ok && hv[k] != Slot<V>::empty;
+            if (recv) ok = ok && rv != Slot<V>::empty;
             if (ok) break;
             if (++spin > kSpinLimit) {
                 *dead = 1;
@@ -1412,7 +1477,8 @@ struct ZetaRow {
         // and i + 256, then the wavefronts' sums, then these in order
 #pragma unroll
         for (int k = 0; k < NQ; k++) q[k] = hasp ? 0. + __builtin_bit_cast(double, pv[k]) : 0.;
-        if (T > kThreads && nblk > kThreads) {
+        if (recv) v = __builtin_bit_cast(V, rv);
+        if (T > kThreads && nsum > kThreads) {
             if (threadIdx.x >= kThreads && threadIdx.x < 2 * kThreads)
 #pragma unroll
                 for (int k = 0; k < NQ; k++) hi[k][threadIdx.x - kThreads] = q[k];
@@ -1446,10 +1512,10 @@ struct ZetaRow {
         // have that done before the next epoch's partials (one barrier later)
         if (epoch >= 1) {
             const int b1 = (epoch - 1) & (kZetaBufs - 1);
-            if (send >= 0) slot_clear(xch + (size_t)b1 * nsend + send, Slot<V>::empty);
+            if (own && send >= 0) slot_clear(xch + (size_t)b1 * nsend + send, Slot<V>::empty);
             for (int e = threadIdx.x; e < kPartSlots * group * kPartCopies; e += T) {
                 const int g = e / kPartCopies % group;
-                if (wg * group + g < nblk)
+                if (wg * group + g < nsum)
                     slot_clear(part_slot(pslot, b1, e % kPartCopies, e / (kPartCopies * group), wg * group + g),
                                Slot<double>::empty);
             }
@@ -1461,10 +1527,11 @@ struct ZetaRow {
 
 // dynamic LDS of k_zeta
 struct ZetaLds {
-    size_t x, y, w, sub[2], total;
+    size_t x, y, w, p, sub[2], total;
 };
 template <typename V>
-__host__ __device__ inline ZetaLds zeta_lds(int rows, int group, int hmax, int chmax, int threads, bool exact) {
+__host__ __device__ inline ZetaLds zeta_lds(int rows, int group, int hmax, int chmax, int threads, int mode, int dmax) {
+    const bool exact = mode == kSubst;
     const size_t sub = (size_t)threads * ((kSubFirst + 1) * sizeof(V) + (kSubFirst / 2 + 2) * sizeof(unsigned)) +
                        (size_t)group * chmax * sizeof(unsigned);
     auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
@@ -1472,11 +1539,84 @@ __host__ __device__ inline ZetaLds zeta_lds(int rows, int group, int hmax, int c
     size_t o = 0;
     // the operand also holds the FP64 residual's (rows and halo)
     l.x = o; o += up((size_t)(rows + hmax) * sizeof(double));
-    l.y = o; o += up((size_t)rows * sizeof(V));
-    l.w = o; o += exact ? 0 : up((size_t)rows * sizeof(V));
+    l.y = o; o += up((size_t)(mode == kDense ? (threads == 512 ? 256 : 1024) : rows) * sizeof(V));
+    l.w = o; o += exact ? 0 : up((size_t)(mode == kDense && rows < 64 ? 64 : rows) * sizeof(V));
+    l.p = o; o += mode == kDense && threads == 1024 ? (size_t)DenseShape<1024>::kOwn * 1024 * sizeof(V) : 0;
     for (int d = 0; d < 2; d++) { l.sub[d] = o; o += exact ? up(sub) : 0; }
     l.total = o;
+    // the inverse's rows are computed before the solve uses its LDS
+    if (mode == kDense) {
+        const size_t setup = up((size_t)rows * (threads == 512 ? DenseShape<512>::kOwn : DenseShape<1024>::kOwn) * sizeof(V)) + up((size_t)dmax * sizeof(V)) +
+                             up((size_t)rows * sizeof(V)) + (size_t)(dmax + 3 * rows + 4) * sizeof(unsigned short);
+        if (setup > l.total) l.total = setup;
+    }
     return l;
+}
+
+// Rows own0 .. own0+nown-1 of the inverse of block blk's factors, this lane's
+// columns of its row into p: e^T U^-1 L^-1 by the transposed factors, a level
+// at a time for all the rows at once (work-items take a level's unknowns
+// times the rows; a level of L is a level of U^T).
+template <typename V, int T, bool BACK>
+__device__ __attribute__((always_inline)) inline void dense_pass(const SolvArgs<V> &a, const ZetaArgs &z, int blk,
+                                                                 int nb, int own0, V *xs, V *tv, const V *dv,
+                                                                 unsigned short *tk, unsigned short *ep,
+                                                                 unsigned short *rows, unsigned short *lp) {
+    constexpr int R = DenseShape<T>::kOwn;
+    const int stride = a.brows + 1;
+    const int *ptr = (BACK ? z.dptr_b : z.dptr_f) + (size_t)blk * stride;
+    const unsigned *ent = (BACK ? z.dent_b : z.dent_f) + (size_t)blk * z.dmax;
+    const int *order = (BACK ? z.rows_b : z.rows_f) + (size_t)blk * a.brows;
+    const int *lptr = (BACK ? a.blptr : a.flptr) + (size_t)blk * stride;
+    const int nlev = (BACK ? a.bnlev : a.fnlev)[blk];
+    const V *lu = a.lu + (size_t)blk * a.mx;
+    for (int e = threadIdx.x; e < ptr[nb]; e += T) {
+        const unsigned w = ent[e];
+        tv[e] = lu[w & 0xffffu];
+        tk[e] = (unsigned short)(w >> 16);
+    }
+    for (int t = threadIdx.x; t <= nb; t += T) {
+        ep[t] = (unsigned short)ptr[t];
+        if (t < nb) rows[t] = (unsigned short)order[t];
+    }
+    for (int l = threadIdx.x; l <= nlev; l += T) lp[l] = (unsigned short)lptr[l];
+    __syncthreads();
+    for (int l = 0; l < nlev; l++) {
+        const int t0 = lp[l], n = (lp[l + 1] - t0) * R;
+        for (int e = threadIdx.x; e < n; e += T) {
+            const int t = t0 + e / R, r = e % R, j = rows[t];
+            V acc = BACK ? xs[(size_t)j * R + r] : (j == own0 + r ? (V)1 : (V)0);
+            for (int q = ep[t]; q < ep[t + 1]; q++) acc = acc - tv[q] * xs[(size_t)tk[q] * R + r];
+            xs[(size_t)j * R + r] = BACK ? acc : acc * dv[j];
+        }
+        __syncthreads();
+    }
+}
+
+template <typename V, int T>
+__device__ __attribute__((always_inline)) inline void dense_rows(const SolvArgs<V> &a, const ZetaArgs &z, int blk,
+                                                                 int nb, int own0, unsigned char *lds,
+                                                                 V (&p)[DenseShape<T>::kCols]) {
+    using D = DenseShape<T>;
+    constexpr int R = D::kOwn;
+    auto up = [](size_t b) { return (b + 15) & ~(size_t)15; };
+    V *xs = reinterpret_cast<V *>(lds);
+    V *tv = reinterpret_cast<V *>(lds + up((size_t)a.brows * R * sizeof(V)));
+    V *dv = reinterpret_cast<V *>(reinterpret_cast<unsigned char *>(tv) + up((size_t)z.dmax * sizeof(V)));
+    unsigned short *tk = reinterpret_cast<unsigned short *>(reinterpret_cast<unsigned char *>(dv) +
+                                                            up((size_t)a.brows * sizeof(V)));
+    unsigned short *ep = tk + z.dmax, *rows = ep + a.brows + 1, *lp = rows + a.brows;
+    for (int t = threadIdx.x; t < nb; t += T)
+        dv[t] = a.lu[(size_t)blk * a.mx + a.pdg[(size_t)blk * a.brows + t]];
+    dense_pass<V, T, false>(a, z, blk, nb, own0, xs, tv, dv, tk, ep, rows, lp);
+    dense_pass<V, T, true>(a, z, blk, nb, own0, xs, tv, dv, tk, ep, rows, lp);
+    const int lane = threadIdx.x & 63, r = (threadIdx.x >> 6) * D::kRows + lane / D::kLanes;
+#pragma unroll
+    for (int j = 0; j < D::kCols; j++) {
+        const int c = lane % D::kLanes + D::kLanes * j;
+        p[j] = c < nb && r < R ? xs[(size_t)c * R + r] : (V)0;
+    }
+    __syncthreads();
 }
 
 // the rows of the workgroup's blocks into LDS, in the order of one substitution
@@ -1528,22 +1668,30 @@ __device__ __attribute__((always_inline)) inline SubExact<V, T> stage_sub(const 
     return s;
 }
 
-template <typename V, int T, int KH, bool EXACT>
+template <typename V, int T, int KH, int MODE>
 __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
     constexpr bool REFINE = sizeof(V) == 4;
     extern __shared__ double smem[];
     __shared__ int dead;
     unsigned char *lds = reinterpret_cast<unsigned char *>(smem);
-    const ZetaLds L = zeta_lds<V>(z.group * a.brows, z.group, z.hmax, z.chmax, T, EXACT);
+    const ZetaLds L = zeta_lds<V>(z.group * a.brows, z.group, z.hmax, z.chmax, T, MODE, z.dmax);
     const int tid = threadIdx.x;
     if (tid == 0) dead = 0;
-    ZetaRow<V, T, KH, EXACT> R;
+    ZetaRow<V, T, KH, MODE> R;
     R.wg = xcd_block(blockIdx.x, gridDim.x);
-    R.nblk = a.nblk; R.n = a.n; R.sweeps = a.sweeps; R.rows = z.group * a.brows; R.group = z.group;
-    const int b0 = R.wg * R.rows, nb = min(a.n, b0 + R.rows) - b0;
+    R.nsum = MODE == kDense ? z.nwg : a.nblk;
+    R.n = a.n; R.sweeps = a.sweeps; R.rows = z.group * a.brows; R.group = z.group;
+    // the workgroup's rows: its blocks, or (dense) its block of several workgroups
+    const int part = MODE == kDense ? R.wg / z.members : R.wg;
+    const int b0 = part * R.rows, nb = min(a.n, b0 + R.rows) - b0;
     R.i = b0 + tid;
     R.mine = tid < nb;
-    R.nh = z.hcnt[R.wg];
+    R.own = R.mine;
+    if (MODE == kDense) {
+        R.own0 = R.wg % z.members * DenseShape<T>::kOwn;
+        R.own = R.mine && tid >= R.own0 && tid < R.own0 + DenseShape<T>::kOwn;
+    }
+    R.nh = z.hcnt[part];
     R.X = reinterpret_cast<V *>(lds + L.x);
     R.y = reinterpret_cast<V *>(lds + L.y);
     R.w = reinterpret_cast<V *>(lds + L.w);
@@ -1559,11 +1707,11 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
 #pragma unroll
     for (int k = 0; k < KH; k++) {
         const bool on = tid + k * T < R.nh;
-        const size_t h = (size_t)R.wg * z.hmax + tid + k * T;
+        const size_t h = (size_t)part * z.hmax + tid + k * T;
         hcol[k] = on ? z.hcol[h] : 0;
         R.hslot[k] = on ? z.hslot[h] : 0;
     }
-    constexpr bool HOLD = ZetaRow<V, T, KH, EXACT>::kHold;
+    constexpr bool HOLD = ZetaRow<V, T, KH, MODE>::kHold;
     R.ga = a.ell_a;
     R.glc = z.lcol;
 #pragma unroll
@@ -1606,7 +1754,23 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
     for (int k = 0; k < R.kTri; k++) R.l[k] = R.u[k] = 0;
 #pragma unroll
     for (int k = 0; k < R.kTriWords; k++) R.llc[k] = R.uc[k] = 0;
-    if constexpr (EXACT) {
+    if constexpr (MODE == kDense) {
+        using D = DenseShape<T>;
+        if constexpr (D::kRegs) {
+            dense_rows<V, T>(a, z, part, nb, R.own0, lds, R.pinv);
+        } else {
+            V p[D::kCols], *pl = reinterpret_cast<V *>(lds + L.p);
+            dense_rows<V, T>(a, z, part, nb, R.own0, lds, p);
+            R.plds = pl;
+            if ((tid >> 6) < D::kOwn)
+#pragma unroll
+                for (int j = 0; j < D::kCols; j++) pl[(size_t)(tid >> 6) * (D::kLanes * D::kCols) + (tid & 63) + D::kLanes * j] = p[j];
+        }
+        // the right-hand side's unused columns: zeros
+        for (int t = tid; t < DenseShape<T>::kLanes * DenseShape<T>::kCols; t += T) R.y[t] = 0;
+        if (tid == 0) dead = 0;
+        __syncthreads();
+    } else if constexpr (MODE == kSubst) {
         R.sf = stage_sub<V, T, false>(a, z, R.wg, lds + L.sub[0]);
         R.sb = stage_sub<V, T, true>(a, z, R.wg, lds + L.sub[1]);
     } else {
@@ -1651,9 +1815,9 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
             for (int k = 0; k < kEllWidth; k++)
                 if (k < len) t = t + (HOLD ? a64[HOLD ? k : 0] : a.aval[q64 + k]) * X64[R.off(cv, k) / sizeof(V)];
             const double r = b64 - t;
-            double rs[2] = {R.mine ? r * r : 0., R.mine ? b64 * b64 : 0.};
-            V none[KH];
-            if (!R.template exchange<2, false>(rs, (V)0, none)) { fail = kWaitExpired; break; }
+            double rs[2] = {R.own ? r * r : 0., R.own ? b64 * b64 : 0.};
+            V none[KH], nov = 0;
+            if (!R.template exchange<2, false>(rs, nov, none)) { fail = kWaitExpired; break; }
             rn = sqrt(rs[0]);
             if (rn <= z.tol * sqrt(rs[1])) { refconv = 1; break; }
             if (nref >= z.maxref) break;
@@ -1674,11 +1838,11 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
 #pragma unroll
         for (int k = 0; k < KH; k++) { hp[k] = hv[k] = hs[k] = ht[k] = 0; hdx[k] = 0; }
         if (!R.mine) r = 0;
-        const V r0 = r;
         dx = 0;
         conv = fail = maxit = 0;
         double q5[5] = {0., 0., 0., 0., 0.}, q1[1] = {(double)r * (double)r};
         if (!R.template exchange<1, true>(q1, r, hr)) { fail = kWaitExpired; break; }
+        const V r0 = r;
         double target = 0., alpha = 0., rho = q1[0], rho_prev = 0., omega = 0.;
         for (int it = 0;; it++) {
             if (it == 0) {
@@ -1718,7 +1882,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
             rho_prev = rho;
             R.operand(p, hp);
             v = R.precond(R.product());
-            q1[0] = R.mine ? (double)r0 * (double)v : 0.;
+            q1[0] = R.own ? (double)r0 * (double)v : 0.;
             if (!R.template exchange<1, true>(q1, v, hv)) { fail = kWaitExpired; break; }
             if (breakdown(q1[0])) { fail = -3; break; }
             alpha = rho / q1[0];
@@ -1728,7 +1892,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
             for (int k = 0; k < KH; k++) hs[k] = hr[k] - va * hv[k];
             R.operand(s, hs);
             t = R.precond(R.product());
-            const double tv = R.mine ? (double)t : 0., sv = R.mine ? (double)s : 0., r0v = (double)r0;
+            const double tv = R.own ? (double)t : 0., sv = R.own ? (double)s : 0., r0v = (double)r0;
             q5[0] = tv * tv;
             q5[1] = tv * sv;
             q5[2] = sv * sv;
@@ -1747,7 +1911,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
         if (tid == 0) a.ctrl[CT_WAIT] = 1;
         return;
     }
-    if (R.mine) {
+    if (R.own) {
         if (REFINE) z.x[i] = x64;
         else a.dx[i] = dx;
     }
@@ -1980,13 +2144,18 @@ static int enqueue_inner(Model &M, SolvArgs<V> &a, int chunk) {
 // work-item and the kind of triangular solve.
 template <typename V>
 using ZetaKernel = void (*)(SolvArgs<V>, ZetaArgs);
+static int zeta_mode(const Model &M) {
+    return M.p.tri_sweeps > 0 ? kSwept : (M.sv.zeta_members > 0 ? kDense : kSubst);
+}
 template <typename V>
 static ZetaKernel<V> zeta_kernel(const Model &M) {
-    const bool exact = M.p.tri_sweeps == 0;
-    if (M.sv.zeta_t == 1024) return k_zeta<V, 1024, 1, true>;
-    if (M.sv.zeta_t == 512) return exact ? k_zeta<V, 512, 1, true> : k_zeta<V, 512, 1, false>;
-    if (M.sv.zeta_hmax <= 256) return exact ? k_zeta<V, 256, 1, true> : k_zeta<V, 256, 1, false>;
-    return exact ? k_zeta<V, 256, 2, true> : k_zeta<V, 256, 2, false>;
+    const int mode = zeta_mode(M);
+    if (M.sv.zeta_t == 1024) return mode == kDense ? k_zeta<V, 1024, 1, kDense> : k_zeta<V, 1024, 1, kSubst>;
+    if (M.sv.zeta_t == 512)
+        return mode == kDense ? k_zeta<V, 512, 1, kDense>
+                              : (mode == kSubst ? k_zeta<V, 512, 1, kSubst> : k_zeta<V, 512, 1, kSwept>);
+    if (M.sv.zeta_hmax <= 256) return mode == kSubst ? k_zeta<V, 256, 1, kSubst> : k_zeta<V, 256, 1, kSwept>;
+    return mode == kSubst ? k_zeta<V, 256, 2, kSubst> : k_zeta<V, 256, 2, kSwept>;
 }
 
 // Workgroups of the one-launch solve wait for each other, so a launch is
@@ -2040,10 +2209,11 @@ static ZetaPlan zeta_plan(Model &M) {
     ZetaPlan p;
     Solver &v = M.sv;
     if (v.zeta_t == 0) return p;
-    const bool exact = M.p.tri_sweeps == 0;
-    // sweeps keep the factor row in registers (and need its slot-major copy)
-    if (!exact && (!v.fs_val || v.brows > kThreads)) return p;
-    p.lds = zeta_lds<V>(v.zeta_group * v.brows, v.zeta_group, v.zeta_hmax, v.zeta_chmax, v.zeta_t, exact).total;
+    const int mode = zeta_mode(M), exact = mode != kSwept;
+    // sweeps keep the factor row in registers (and need its slot-major copy),
+    // and a basin laid out for dense rows has one block's work-items per workgroup
+    if (!exact && (!v.fs_val || v.brows > kThreads || v.zeta_members > 0)) return p;
+    p.lds = zeta_lds<V>(v.zeta_group * v.brows, v.zeta_group, v.zeta_hmax, v.zeta_chmax, v.zeta_t, mode, v.zeta_dmax).total;
     if (v.zeta_occ[exact] == 0) {
         // asked once per model and kind
         int dev = 0, cus = 0, occ = 0, lds_max = 0;
@@ -2081,6 +2251,8 @@ static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::func
     z.lcol = M.m.z_lcol; z.hcol = M.m.z_hcol; z.hslot = M.m.z_hslot; z.hcnt = M.m.z_hcnt;
     z.send = M.m.z_send; z.nsend = M.sv.zeta_nsend;
     z.rows_f = M.m.fwd_rows; z.rows_b = M.m.bwd_rows;
+    z.members = M.sv.zeta_members; z.dmax = M.sv.zeta_dmax;
+    z.dent_f = M.m.z_dentf; z.dent_b = M.m.z_dentb; z.dptr_f = M.m.z_dptrf; z.dptr_b = M.m.z_dptrb;
     z.chunk_f = M.m.z_chf; z.chunk_b = M.m.z_chb; z.nch_f = M.m.z_nchf; z.nch_b = M.m.z_nchb;
     z.xch = M.sv.xch; z.pslot = M.sv.pslot;
     z.rhs = M.s.rhs; z.x = M.s.x; z.tol = M.p.refine_rtol; z.maxref = kMaxRefine;

@@ -24,6 +24,9 @@ CASES = {
     "one_block_small": (lambda: mesh.tidal_basin(nx=5, ny=4), 0, 0),
     "one_block_sweeps": (lambda: mesh.tidal_basin(nx=14, ny=13), 256, 3),
     "exact_256": (lambda: mesh.tidal_basin(nx=41, ny=30), 0, 0),
+    "exact_blocks_of_60": (lambda: mesh.tidal_basin(nx=41, ny=30), 60, 0),
+    "exact_no_dense_rows": (lambda: mesh.lagoon(15000, seed=6, nlv=1, tile=32), 0, 0),
+    "exact_wide_halo": (lambda: mesh.tidal_basin(nx=230, ny=70), 0, 0),
     "exact_blocks_of_300": (lambda: mesh.tidal_basin(nx=41, ny=31), 300, 0),
     "exact_blocks_of_700": (lambda: mesh.tidal_basin(nx=41, ny=40), 700, 0),
     "sweeps_two_blocks_a_group": (lambda: mesh.lagoon(2000, seed=5, lx=6000.0, ly=3000.0, nlv=1, tile=16), 100, 3),
