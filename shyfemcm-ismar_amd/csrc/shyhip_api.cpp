@@ -1200,29 +1200,30 @@ int shyhip_pull(shyhip_model *h, int field, void *host, int dtype, size_t n) {
     const Shape sh = shape_of(M, f.kind);
     if (n != sh.n) return fail(&M, "pull: size mismatch for field " + std::to_string(field));
     if (f.lazy && !*f.ptr) return fail(&M, "pull: field " + std::to_string(field) + " was never pushed");
-    HIPCHK(M, hipStreamSynchronize(M.stream));
     if (f.isint) {
         if (dtype != SHYHIP_I32) return fail(&M, "integer field needs SHYHIP_I32");
         HIPCHK(M, hipMemcpyAsync(host, *f.ptr, n * sizeof(int), hipMemcpyDeviceToHost, M.stream));
         HIPCHK(M, hipStreamSynchronize(M.stream));
         return 0;
     }
-    std::vector<double> t(n);
-    if (f.isdouble_dev || M.prec == SHYHIP_FP64) {
-        HIPCHK(M, hipMemcpyAsync(t.data(), *f.ptr, n * sizeof(double), hipMemcpyDeviceToHost, M.stream));
+    // turned into the host's layout and type on the device, in the element
+    // term scratch of the single-tracer calls (free between calls), as many
+    // columns at a time as it holds
+    const bool dbl = f.isdouble_dev || M.prec == SHYHIP_FP64, out_dbl = dtype == SHYHIP_F64;
+    const size_t vs = out_dbl ? sizeof(double) : sizeof(float), col = (size_t)sh.rows * vs;
+    if (sh.rows == 1 && dbl == out_dbl) {
+        HIPCHK(M, hipMemcpyAsync(host, *f.ptr, n * vs, hipMemcpyDeviceToHost, M.stream));
         HIPCHK(M, hipStreamSynchronize(M.stream));
-    } else {
-        std::vector<float> tf(n);
-        HIPCHK(M, hipMemcpyAsync(tf.data(), *f.ptr, n * sizeof(float), hipMemcpyDeviceToHost, M.stream));
-        HIPCHK(M, hipStreamSynchronize(M.stream));
-        for (size_t i = 0; i < n; i++) t[i] = tf[i];
+        return 0;
     }
-    for (int r = 0; r < sh.rows; r++)
-        for (int c = 0; c < sh.cols; c++) {
-            const size_t hi = (size_t)c * sh.rows + r, di = (size_t)r * sh.cols + c;
-            if (dtype == SHYHIP_F64) ((double *)host)[hi] = t[di];
-            else ((float *)host)[hi] = (float)t[di];
-        }
+    const int step = (int)std::min<size_t>((size_t)sh.cols, conz_hbuf_elems(M, 1) * M.esize() / col);
+    for (int c0 = 0; c0 < sh.cols; c0 += step) {
+        const int nc = std::min(step, sh.cols - c0);
+        if (launch_to_host_layout(M, *f.ptr, dbl, M.s.hbuf, out_dbl, sh.rows, sh.cols, c0, nc)) return 1;
+        HIPCHK(M, hipMemcpyAsync((char *)host + (size_t)c0 * col, M.s.hbuf, (size_t)nc * col, hipMemcpyDeviceToHost,
+                                 M.stream));
+        HIPCHK(M, hipStreamSynchronize(M.stream));
+    }
     return 0;
 }
 
@@ -1264,8 +1265,8 @@ int shyhip_set_members(shyhip_model *h, int nmem, const int *node_start, const i
 // The state a member carries from step to step, copied device to device
 // from member sm of src into member dm of dst (same basin: node, element
 // and layer counts, precision, tracers).  Node arrays [l*nkn + k] and
-// element arrays [l*nel + ie] are copied layer by layer with one strided
-// copy each; 2D arrays are one layer.
+// element arrays [l*nel + ie] are copied layer by layer, 2D arrays are one
+// layer; all arrays in one launch.
 int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int sm) {
     if (!dst || !src) return fail(nullptr, "null handle");
     Model &D = dst->M, &S = src->M;
@@ -1297,6 +1298,7 @@ int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int s
         f.push_back({a.tracer[t], b.tracer[t], es, 0, L});
         f.push_back({a.tracer_bc[t], b.tracer_bc[t], es, 0, L});
     }
+    std::vector<ArrayCopy> list;
     for (const F &x : f) {
         if (!x.d || !x.s) continue;
         const size_t w = (size_t)(x.elem ? ke : kn) * x.sz;
@@ -1304,9 +1306,9 @@ int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int s
         const size_t d0 = (size_t)(x.elem ? D.mem_elem[dm] : D.mem_node[dm]) * x.sz;
         const size_t s0 = (size_t)(x.elem ? S.mem_elem[sm] : S.mem_node[sm]) * x.sz;
         // zenv/zeov are vertex-major [v*nel + ie]: three "layers" of elements
-        HIPCHK(D, hipMemcpy2DAsync((char *)x.d + d0, dp, (const char *)x.s + s0, sp, w, x.nl, hipMemcpyDeviceToDevice,
-                                   D.stream));
+        list.push_back({(char *)x.d + d0, (const char *)x.s + s0, dp, sp, w, (size_t)x.nl});
     }
+    if (launch_copy_arrays(D, list)) return 1;
     HIPCHK(D, hipStreamSynchronize(D.stream));
     return 0;
 }

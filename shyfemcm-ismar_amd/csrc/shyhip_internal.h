@@ -481,6 +481,18 @@ int launch_set_rzv_all(Model &M);
 // (shyhip_forcing.hip); the host has checked that dtime is covered
 int launch_forcing(Model &M, double dtime);
 int launch_mass_flux(Model &M, bool with_rqds);
+// whole state arrays (shyhip_state.hip): strided copies on the model's stream,
+// all in one launch (row lengths and pitches in bytes, multiples of 4); and
+// columns c0 .. c0+nc-1 of a device array [rows][cols] in the host's layout
+// out[(c - c0)*rows + r] and type
+struct ArrayCopy {
+    void *dst;
+    const void *src;
+    size_t dpitch, spitch, width, rows;
+};
+int launch_copy_arrays(Model &M, const std::vector<ArrayCopy> &list);
+int launch_to_host_layout(Model &M, const void *a, bool a_double, void *out, bool out_double, int rows, int cols, int c0,
+                          int nc);
 // rhoset (baroclinic.f90:654-720) niter times: the density anomaly of every
 // node-layer from T, S and the mid-layer pressure (shyhip_hydro.hip)
 int launch_rhoset(Model &M, int niter, hipStream_t st);

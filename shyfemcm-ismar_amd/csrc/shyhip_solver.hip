@@ -81,7 +81,7 @@ struct SolvArgs {
     void *xch;
     unsigned long long *pslot;
     const int *send;
-    int nsend, zmembers;              // (zmembers: partial sums per block)
+    int nsend;
 };
 
 template <typename V>
@@ -116,7 +116,6 @@ static SolvArgs<V> solv_args(Model &M, const V *A, V *b, V *x0) {
         a.pslot = M.sv.pslot;
         a.send = M.m.z_send;
         a.nsend = M.sv.zeta_nsend;
-        a.zmembers = std::max(1, M.sv.zeta_members);
     }
     return a;
 }
@@ -1113,14 +1112,23 @@ __device__ inline void zeta_empty_slots(const SolvArgs<V> &a, int blk, int b0, i
     for (int b = 0; b < kZetaBufs; b++) {
         for (int li = threadIdx.x; li < nb; li += blockDim.x)
             if (const int q = a.send[b0 + li]; q >= 0) slot_clear(xch + (size_t)b * a.nsend + q, Slot<V>::empty);
-        for (int e = threadIdx.x; e < kPartSlots * kPartCopies * a.zmembers; e += blockDim.x)
-            slot_clear(part_slot(a.pslot, b, e % kPartCopies, e / kPartCopies % kPartSlots,
-                                 blk * a.zmembers + e / (kPartCopies * kPartSlots)),
+        if (threadIdx.x < kPartSlots * kPartCopies)
+            slot_clear(part_slot(a.pslot, b, threadIdx.x % kPartCopies, threadIdx.x / kPartCopies, blk),
                        Slot<double>::empty);
     }
     if (blk == 0 && threadIdx.x == 0) {
         a.ctrl[CT_CONV] = 0; a.ctrl[CT_FAIL] = 0; a.ctrl[CT_MAXIT] = 0; a.ctrl[CT_WAIT] = 0;
     }
+}
+
+// the partial-sum slots of all workgroups empty (dense rows: more workgroups
+// than blocks, too many slots for the few workgroups of the factorisation);
+// one buffer's copy and sum per workgroup
+__global__ __launch_bounds__(kThreads) void k_empty_partials(unsigned long long *pslot, int nsum) {
+    const int b = blockIdx.x;
+    unsigned long long *p = part_slot(pslot, b / (kPartCopies * kPartSlots), b / kPartSlots % kPartCopies,
+                                      b % kPartSlots, 0);
+    for (int i = threadIdx.x; i < nsum; i += kThreads) slot_clear(p + i, Slot<double>::empty);
 }
 
 // every store this work-item has issued is complete
@@ -2018,6 +2026,9 @@ static int factor(Model &M, SolvArgs<V> &a) {
     const int stage = vals + lists <= kLdsLimit ? 1 : 0;
     launch_timed(M, T_FACTOR, k_bilu_factor<V>, dim3(M.sv.nblk), dim3(kFactorThreads), stage ? vals + lists : vals,
                  M.stream, a, stage, sweeps);
+    if (M.sv.zeta_members > 0)
+        hipLaunchKernelGGL(k_empty_partials, dim3(kZetaBufs * kPartCopies * kPartSlots), dim3(kThreads), 0, M.stream,
+                           M.sv.pslot, M.sv.zeta_nwg);
     HIPCHK(M, hipGetLastError());
     M.sv.have_lu = true;
     return 0;
