@@ -418,7 +418,7 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.blk_cp_a, (void *)m.blk_cp_b, (void *)m.blk_jd, (void *)m.blk_pcol, (void *)m.blk_prp,
                     (void *)m.blk_pdg, (void *)m.fs_col, (void *)m.fs_meta, (void *)m.blk_fdesc, (void *)m.blk_fpair,
                     (void *)m.blk_elp, (void *)m.blk_elr, (void *)m.blk_enlev, (void *)m.ell_col, (void *)m.ell_len, (void *)m.csr_ell,
-                    (void *)m.z_lcol, (void *)m.z_hcol, (void *)m.z_hslot, (void *)m.z_hcnt, (void *)m.z_send,
+                    (void *)m.z_lcol, (void *)m.z_fcol, (void *)m.z_hcol, (void *)m.z_hslot, (void *)m.z_hcnt, (void *)m.z_send,
                     (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_dentf, (void *)m.z_dentb, (void *)m.z_dptrf,
                     (void *)m.z_dptrb, (void *)m.z_nchf, (void *)m.z_nchb,
                     (void *)m.fwd_rows, (void *)m.fwd_lptr, (void *)m.fwd_nlev, (void *)m.bwd_rows,
@@ -903,11 +903,15 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
             M.sv.zeta_chmax = zt.chmax;
             M.sv.zeta_nsend = zt.nsend;
             M.sv.zeta_occ[0] = M.sv.zeta_occ[1] = 0;
-            if (zt.threads > 0) {
+            if (zt.hmax > 0) {
                 rc |= dalloc(M, &m.z_lcol, zt.lcol.size()) || upload(M, m.z_lcol, zt.lcol.data(), zt.lcol.size());
-                rc |= dalloc(M, &m.z_hcol, zt.hcol.size()) || upload(M, m.z_hcol, zt.hcol.data(), zt.hcol.size());
-                rc |= dalloc(M, &m.z_hslot, zt.hslot.size()) || upload(M, m.z_hslot, zt.hslot.data(), zt.hslot.size());
                 rc |= dalloc(M, &m.z_hcnt, zt.hcnt.size()) || upload(M, m.z_hcnt, zt.hcnt.data(), zt.hcnt.size());
+                rc |= dalloc(M, &m.z_hcol, zt.hcol.size()) || upload(M, m.z_hcol, zt.hcol.data(), zt.hcol.size());
+            }
+            if (zt.hmax > 0 && zt.threads == 0)
+                rc |= dalloc(M, &m.z_fcol, zt.fcol.size()) || upload(M, m.z_fcol, zt.fcol.data(), zt.fcol.size());
+            if (zt.threads > 0) {
+                rc |= dalloc(M, &m.z_hslot, zt.hslot.size()) || upload(M, m.z_hslot, zt.hslot.data(), zt.hslot.size());
                 rc |= dalloc(M, &m.z_send, zt.send.size()) || upload(M, m.z_send, zt.send.data(), zt.send.size());
                 rc |= dalloc(M, &m.z_chf, zt.chf.size()) || upload(M, m.z_chf, zt.chf.data(), zt.chf.size());
                 rc |= dalloc(M, &m.z_chb, zt.chb.size()) || upload(M, m.z_chb, zt.chb.data(), zt.chb.size());

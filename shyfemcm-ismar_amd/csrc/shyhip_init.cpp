@@ -638,6 +638,7 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
 // 0.333 ms, 50k nodes 0.391 / 0.448 against 0.371 / 0.403 ms; the line lies
 // between.  Blocks longer than 512 rows take 1024.
 constexpr int kZetaSmall = 128;
+constexpr int kZetaMost = 224;           // workgroups of a solve (of 512 work-items one to a compute unit)
 constexpr int kZetaDense = 220;          // workgroups of a solve with dense rows (each takes a compute unit)
 
 static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,
@@ -645,7 +646,9 @@ static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector
     // several blocks only of whole wavefronts (their sums are kept apart)
     const int nblk = bs.nblk, group = members == 0 && bs.brows % 64 == 0 ? T / bs.brows : 1, brows = group * bs.brows;
     const int nwg = (nblk + group - 1) / group;
-    if (nblk > T || nblk > 512 || (members > 0 && nblk * members > kZetaDense)) return false;
+    const bool iter = members < 0;         // tables of the two-kernel iteration only
+    if (!iter && (nblk > T || nblk > 512 || nwg > kZetaMost || (members > 0 && nblk * members > kZetaDense)))
+        return false;
     // halos: the columns outside the workgroup's rows, ascending
     std::vector<std::vector<int>> halo(nwg);
     parallel_for(nwg, 16, [&](int b_begin, int b_end) {
@@ -667,6 +670,20 @@ static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector
     zt.hslot.assign((size_t)nwg * hmax, 0);
     zt.send.assign(n, -1);
     zt.lcol.assign((size_t)(kEllWidth / 2) * n, 0u);
+    if (iter) {
+        // factor row: slot 0 the diagonal, then L, then U (as fs_col)
+        zt.fcol.assign((size_t)(kEllWidth / 2) * n, 0u);
+        for (int i = 0; i < n; i++) {
+            const int f0 = bs.rowptr[i], cnt = bs.rowptr[i + 1] - f0, li = i % brows;
+            int nl = 0;
+            for (int p = 0; p < cnt; p++) nl += bs.cols[f0 + p] < li;
+            for (int k = 0; k < kEllWidth; k++) {
+                const int p = k == 0 ? nl : (k <= nl ? k - 1 : k);
+                zt.fcol[(size_t)(k / 2) * n + i] |= (unsigned)((k < cnt ? bs.cols[f0 + p] : li) * esize)
+                                                    << (16 * (k & 1));
+            }
+        }
+    }
     // value slots in row order, each workgroup's first slot on a line of its
     // own (a block of several workgroups: every row)
     if (members > 1) std::fill(zt.send.begin(), zt.send.end(), 0);
@@ -703,6 +720,7 @@ static bool zeta_tables(int n, const std::vector<int> &rowptr, const std::vector
             }
         }
     });
+    if (iter) return true;
     // exact substitution: the rows of each level in chunks of 64; the chunk
     // list ends with three empty chunks (the substitution reads ahead)
     const int stride = bs.brows + 1;
@@ -800,7 +818,9 @@ void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<i
     }
     const int n256 = bs.brows <= 256 ? (bs.brows % 64 == 0 ? (n + 255) / 256 : bs.nblk) : 1 << 30;
     if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, 0, zt)) return;
-    if (bs.brows <= 256) zeta_tables(n, rowptr, cols, bs, esize, 256, 0, zt);
+    if (bs.brows <= 256 && zeta_tables(n, rowptr, cols, bs, esize, 256, 0, zt)) return;
+    zt = ZetaTables();
+    if (bs.brows <= 256 && !zeta_tables(n, rowptr, cols, bs, esize, 256, -1, zt)) zt = ZetaTables();
 }
 
 }  // namespace shy

@@ -94,7 +94,9 @@ struct Mesh {                 // device copies of init-time data
     // workgroup's slots lie together; the exact substitutions' chunks (at most 64 rows of one
     // level: first position | rows << 16, positions in fwd_rows / bwd_rows
     // relative to the block) and chunks per block
-    unsigned *z_lcol = nullptr, *z_chf = nullptr, *z_chb = nullptr;
+    unsigned *z_lcol = nullptr, *z_fcol = nullptr, *z_chf = nullptr, *z_chb = nullptr;
+    // (basins without a one-launch solve: the same of their blocks, and the
+    // byte offsets of the rows' factor columns, for the two-kernel iteration)
     // dense rows (exact solves of small basins): entries of the transposed
     // factors in the order of the two substitutions and their starts
     unsigned *z_dentf = nullptr, *z_dentb = nullptr;
@@ -445,7 +447,7 @@ void host_block_schedule(int n, const std::vector<int> &rowptr, const std::vecto
 // threads: its workgroup size, 0 when the basin's blocks do not fit it
 struct ZetaTables {
     int threads = 0, nwg = 0, group = 1, members = 0, dmax = 0, hmax = 0, chmax = 0, nsend = 0;
-    std::vector<unsigned> lcol, chf, chb, dentf, dentb;
+    std::vector<unsigned> lcol, fcol, chf, chb, dentf, dentb;
     std::vector<int> hcol, hslot, hcnt, send, nchf, nchb, dptrf, dptrb;
 };
 void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<int> &cols, const BlockSchedule &bs,

@@ -82,6 +82,12 @@ struct SolvArgs {
     unsigned long long *pslot;
     const int *send;
     int nsend;
+    // two-kernel iteration with halos (null: not laid out): byte offsets of
+    // the row's columns in its block's operand and of its factor columns in
+    // the block's rows, two per word [k/2][n], each block's halo rows
+    const unsigned *lcol, *fcol;
+    const int *hcol, *hcnt;
+    int hmax;
 };
 
 template <typename V>
@@ -116,6 +122,8 @@ static SolvArgs<V> solv_args(Model &M, const V *A, V *b, V *x0) {
         a.pslot = M.sv.pslot;
         a.send = M.m.z_send;
         a.nsend = M.sv.zeta_nsend;
+    } else if (M.sv.zeta_hmax > 0) {
+        a.lcol = M.m.z_lcol; a.fcol = M.m.z_fcol; a.hcol = M.m.z_hcol; a.hcnt = M.m.z_hcnt; a.hmax = M.sv.zeta_hmax;
     }
     return a;
 }
@@ -613,6 +621,110 @@ struct RowOps {
     }
 };
 
+// A matrix row and its factor row for blocks with halo tables, in registers.
+// The product's operand is formed once per row of the block and once per row
+// of its halo (the neighbour rows in other blocks, some 80 for 256 rows), in
+// LDS, instead of by every row for each of its columns (4 vectors gathered at
+// 10 columns: k_bicg_a on 300k rows in FP64 52 us against 31, k_bicg_b 23
+// against 19; in FP32 on 285k rows 17.4 against 12.3 and 11.9 against 8.2).  Terms
+// are added as in RowOps and FacRow, the padding's as zeros, and slots beyond
+// those that some row of the wavefront fills are left out.
+template <typename V>
+struct HaloRow {
+    V a[kEllWidth], f[kFacWidth];
+    unsigned lc[kEllWidth / 2], fc[kFacWidth / 2];
+    int nl = 0, cnt = 0, len = 0;
+    bool a8, l3, l6, u3, u6;        // some row of the wavefront fills slots 8.., L or U slots 4.. and 7..
+    int h[2], nh;
+    __device__ __attribute__((always_inline)) void load(const SolvArgs<V> &s, int blk, int i, bool valid) {
+#pragma unroll
+        for (int k = 0; k < kEllWidth; k++) a[k] = f[k] = 0;
+#pragma unroll
+        for (int k = 0; k < kEllWidth / 2; k++) lc[k] = fc[k] = 0;
+        nh = s.hcnt[blk];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int e = threadIdx.x + k * kThreads;
+            h[k] = e < s.hmax ? s.hcol[(size_t)blk * s.hmax + e] : 0;
+        }
+        if (valid) {
+            len = s.ell_len[i];
+            const int meta = s.fs_meta[i];
+            nl = meta & 255;
+            cnt = meta >> 8;
+#pragma unroll
+            for (int k = 0; k < kEllWidth; k++) {
+                a[k] = s.ell_a[(size_t)k * s.n + i];
+                f[k] = s.fs_val[(size_t)k * s.n + i];
+            }
+#pragma unroll
+            for (int k = 0; k < kEllWidth / 2; k++) {
+                lc[k] = s.lcol[(size_t)k * s.n + i];
+                fc[k] = s.fcol[(size_t)k * s.n + i];
+            }
+        }
+    }
+    __device__ __attribute__((always_inline)) void bounds() {
+        a8 = __any(len > 8);
+        l3 = __any(nl > 3);
+        l6 = __any(nl > 6);
+        u3 = __any(cnt > 4);
+        u6 = __any(cnt > 7);
+    }
+    __device__ static __attribute__((always_inline)) V at(const V *base, const unsigned *w, int k) {
+        const unsigned o = (k & 1) ? w[k / 2] >> 16 : w[k / 2] & 0xffffu;
+        return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + o);
+    }
+    __device__ __attribute__((always_inline)) V product(const V *X) const {
+        V t = 0, g[kEllWidth];
+#pragma unroll
+        for (int k = 0; k < 8; k++) g[k] = at(X, lc, k);
+#pragma unroll
+        for (int k = 0; k < 8; k++) t = t + a[k] * g[k];
+        if (a8)
+#pragma unroll
+            for (int k = 8; k < kEllWidth; k++) t = t + a[k] * at(X, lc, k);
+        return t;
+    }
+    // t minus the terms of slots K0 .. K0+2 on the wanted side of the diagonal
+    template <int K0, bool UPPER>
+    __device__ __attribute__((always_inline)) V three(V t, const V *src) const {
+        V g[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) g[k] = at(src, fc, K0 + k);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const bool on = UPPER ? K0 + k > nl && K0 + k < cnt : K0 + k <= nl;
+            t = t - (on ? f[K0 + k] : (V)0) * g[k];
+        }
+        return t;
+    }
+    // (LU)^-1 of the block applied to t (in y, visible): this row's result
+    __device__ __attribute__((always_inline)) V lusol(int sweeps, bool mine, V t, V *y, V *w) const {
+        V *src = y, *dst = w, cur = t;
+        for (int sw = 1; sw < sweeps; sw++) {
+            cur = three<1, false>(t, src);
+            if (l3) cur = three<4, false>(cur, src);
+            if (l6) cur = three<7, false>(cur, src);
+            if (mine) dst[threadIdx.x] = cur;
+            __syncthreads();
+            V *x = src; src = dst; dst = x;
+        }
+        const V bl = cur;
+        cur = f[0] * bl;
+        for (int sw = 1; sw < sweeps; sw++) {
+            if (mine) dst[threadIdx.x] = cur;
+            __syncthreads();
+            V *x = src; src = dst; dst = x;
+            cur = three<1, true>(bl, src);
+            if (u3) cur = three<4, true>(cur, src);
+            if (u6) cur = three<7, true>(cur, src);
+            cur = f[0] * cur;
+        }
+        return cur;
+    }
+};
+
 // r0 = M^-1 (b - A x0) (x0 = 0 when zero_x0), dx = 0; (r0,r0) into both
 // slots of region C
 template <typename V, bool STAGE>
@@ -682,15 +794,35 @@ __global__ __launch_bounds__(kThreads) void k_bicg_a(SolvArgs<V> a, int it) {
     const int stop = a.ctrl[CT_STOPIT], fail = a.ctrl[CT_FAIL], refconv = a.ctrl[CT_REFCONV];
     const double alpha_prev = a.scal[SC_ALPHA + pp], target_prev = a.scal[SC_TARGET], rho_prev = a.scal[SC_RHO + pp];
     constexpr bool regs = MODE == 2;       // factor rows in registers, no block staging
+    constexpr bool halo = MODE == 3;       // the same with the block's halo
     BlockStage<V, STAGE> st;
     FacRow<V> fr;
-    if constexpr (regs) fr.load(a, i, mine);
+    HaloRow<V> hr;
+    V hs[2] = {}, ht[2] = {}, hp[2] = {}, hv[2] = {};
+    if constexpr (halo) hr.load(a, blk, i, mine);
+    else if constexpr (regs) fr.load(a, i, mine);
     else st.load(a, blk);
     Partials<5> ps;
     ps.load(a.part, region, a.nparts, a.nblk, nq);
     RowOps<V, 4> ro;
     V r0_i = 0, dx_i = 0;
-    if (pre) {
+    if constexpr (halo) {
+        const V *first = it == 0 ? a.r0 : a.s;
+        if (mine) {
+            r0_i = a.r0[i];
+            ro.own[0] = first[i];
+            if (it > 0) {
+                ro.own[1] = a.t[i]; ro.own[2] = pold[i]; ro.own[3] = vold[i];
+                dx_i = a.dx[i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            if ((int)threadIdx.x + k * kThreads < hr.nh) {
+                hs[k] = first[hr.h[k]];
+                if (it > 0) { ht[k] = a.t[hr.h[k]]; hp[k] = pold[hr.h[k]]; hv[k] = vold[hr.h[k]]; }
+            }
+    } else if (pre) {
         if (it == 0) ro.load(a, i, mine, a.r0, a.r0, a.r0, a.r0);
         else ro.load(a, i, mine, a.s, a.t, pold, vold);
         if (mine) {
@@ -699,7 +831,8 @@ __global__ __launch_bounds__(kThreads) void k_bicg_a(SolvArgs<V> a, int it) {
         }
     }
     if (fail || refconv || (stop != 0 && stop <= it)) return;
-    const BlockView<V> B = regs ? BlockView<V>{} : st.store(a, blk, reinterpret_cast<unsigned char *>(w + a.brows));
+    const BlockView<V> B = regs || halo ? BlockView<V>{}
+                                        : st.store(a, blk, reinterpret_cast<unsigned char *>(w + a.brows));
     double q[5];   // it = 0: (r0,r0) (r0,r0); else (t,t) (t,s) (s,s) (r0,s) (r0,t)
     ps.total(a.part, region, a.nparts, a.nblk, nq, q);
     double rn, rho, omega = 0., alpha = 0.;
@@ -760,7 +893,26 @@ __global__ __launch_bounds__(kThreads) void k_bicg_a(SolvArgs<V> a, int it) {
     }
     if (lead) a.scal[SC_RHO + par] = rho;
     const V vb = (V)beta, vo = (V)omega;
-    if (pre) {
+    V z_i = 0;
+    if constexpr (halo) {
+        V *X = w + a.brows, p = ro.own[0];
+        if (it > 0) p = (ro.own[0] - vo * ro.own[1]) + vb * (ro.own[2] - vo * ro.own[3]);
+        if (mine) {
+            X[threadIdx.x] = p;
+            pnew[i] = p;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            if ((int)threadIdx.x + k * kThreads < hr.nh)
+                X[a.brows + threadIdx.x + k * kThreads] =
+                    it == 0 ? hs[k] : (hs[k] - vo * ht[k]) + vb * (hp[k] - vo * hv[k]);
+        hr.bounds();
+        __syncthreads();
+        const V t = hr.product(X);
+        if (mine) y[threadIdx.x] = t;
+        __syncthreads();
+        z_i = hr.lusol(a.sweeps, mine, t, y, w);
+    } else if (pre) {
         if (mine) {
             V t = 0;
             int q0, q1;
@@ -814,10 +966,18 @@ __global__ __launch_bounds__(kThreads) void k_bicg_a(SolvArgs<V> a, int it) {
             pnew[k] = ri + vb * (pold[k] - vo * vold[k]);
         }
     }
-    __syncthreads();
-    const V *z = regs ? fr.lusol(a.sweeps, mine, threadIdx.x, y, w) : block_lusol(a, B, blk, b0, nb, y, w);
+    const V *z = nullptr;
+    if constexpr (!halo) {
+        __syncthreads();
+        z = regs ? fr.lusol(a.sweeps, mine, threadIdx.x, y, w) : block_lusol(a, B, blk, b0, nb, y, w);
+    }
     double loc[1] = {0.};
-    if (pre) {
+    if constexpr (halo) {
+        if (mine) {
+            vnew[i] = z_i;
+            loc[0] = (double)r0_i * (double)z_i;
+        }
+    } else if (pre) {
         if (mine) {
             vnew[i] = z[threadIdx.x];
             loc[0] = (double)r0_i * (double)z[threadIdx.x];
@@ -851,21 +1011,37 @@ __global__ __launch_bounds__(kThreads) void k_bicg_b(SolvArgs<V> a, int it) {
     const bool mine = pre && (int)threadIdx.x < nb;
     const int stop = a.ctrl[CT_STOPIT], fail = a.ctrl[CT_FAIL], refconv = a.ctrl[CT_REFCONV];
     const double rho = a.scal[SC_RHO + par];
-    constexpr bool regs = MODE == 2;
+    constexpr bool regs = MODE == 2, halo = MODE == 3;
     BlockStage<V, STAGE> st;
     FacRow<V> fr;
-    if constexpr (regs) fr.load(a, i, mine);
+    HaloRow<V> hr;
+    V hs[2] = {}, hv[2] = {};
+    if constexpr (halo) hr.load(a, blk, i, mine);
+    else if constexpr (regs) fr.load(a, i, mine);
     else st.load(a, blk);
     Partials<1> ps;
     ps.load(a.part, PR_A, a.nparts, a.nblk, 1);
     RowOps<V, 2> ro;
     V r0_i = 0;
-    if (pre) {
+    if constexpr (halo) {
+        if (mine) {
+            r0_i = a.r0[i];
+            ro.own[0] = rv[i];
+            ro.own[1] = vnew[i];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            if ((int)threadIdx.x + k * kThreads < hr.nh) {
+                hs[k] = rv[hr.h[k]];
+                hv[k] = vnew[hr.h[k]];
+            }
+    } else if (pre) {
         ro.load(a, i, mine, rv, vnew);
         if (mine) r0_i = a.r0[i];
     }
     if (stop || fail || refconv) return;
-    const BlockView<V> B = regs ? BlockView<V>{} : st.store(a, blk, reinterpret_cast<unsigned char *>(w + a.brows));
+    const BlockView<V> B = regs || halo ? BlockView<V>{}
+                                        : st.store(a, blk, reinterpret_cast<unsigned char *>(w + a.brows));
     double d[1];
     ps.total(a.part, PR_A, a.nparts, a.nblk, 1, d);
     if (breakdown(d[0])) {
@@ -875,8 +1051,24 @@ __global__ __launch_bounds__(kThreads) void k_bicg_b(SolvArgs<V> a, int it) {
     const double alpha = rho / d[0];
     if (lead) a.scal[SC_ALPHA + par] = alpha;
     const V va = (V)alpha;
-    V s_i = 0;
-    if (pre) {
+    V s_i = 0, z_i = 0;
+    if constexpr (halo) {
+        V *X = w + a.brows;
+        s_i = ro.own[0] - va * ro.own[1];
+        if (mine) {
+            X[threadIdx.x] = s_i;
+            a.s[i] = s_i;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            if ((int)threadIdx.x + k * kThreads < hr.nh) X[a.brows + threadIdx.x + k * kThreads] = hs[k] - va * hv[k];
+        hr.bounds();
+        __syncthreads();
+        const V t = hr.product(X);
+        if (mine) y[threadIdx.x] = t;
+        __syncthreads();
+        z_i = hr.lusol(a.sweeps, mine, t, y, w);
+    } else if (pre) {
         if (mine) {
             V t = 0;
             int q0, q1;
@@ -905,13 +1097,17 @@ __global__ __launch_bounds__(kThreads) void k_bicg_b(SolvArgs<V> a, int it) {
             a.s[k] = rv[k] - va * vnew[k];
         }
     }
-    __syncthreads();
-    const V *z = regs ? fr.lusol(a.sweeps, mine, threadIdx.x, y, w) : block_lusol(a, B, blk, b0, nb, y, w);
+    const V *z = nullptr;
+    if constexpr (!halo) {
+        __syncthreads();
+        z = regs ? fr.lusol(a.sweeps, mine, threadIdx.x, y, w) : block_lusol(a, B, blk, b0, nb, y, w);
+        if (pre && mine) z_i = z[threadIdx.x];
+    }
     double loc[5] = {0., 0., 0., 0., 0.};
-    if (pre) {
+    if (halo || pre) {
         if (mine) {
-            const double tv = (double)z[threadIdx.x], sv = (double)s_i, r0 = (double)r0_i;
-            a.t[i] = z[threadIdx.x];
+            const double tv = (double)z_i, sv = (double)s_i, r0 = (double)r0_i;
+            a.t[i] = z_i;
             loc[0] = tv * tv;
             loc[1] = tv * sv;
             loc[2] = sv * sv;
@@ -2001,6 +2197,12 @@ static size_t apply_lds(const Model &M) {
     return stage_fits<V>(M) ? staged_lds<V>(M.sv.brows, M.sv.max_blk_nnz) : 2 * (size_t)M.sv.brows * sizeof(V);
 }
 
+// dynamic LDS of the iteration kernels: with halos y, w and the operand
+template <typename V, int MODE>
+static size_t iter_lds(const Model &M) {
+    return MODE == 3 ? (3 * (size_t)M.sv.brows + M.sv.zeta_hmax) * sizeof(V) : apply_lds<V>(M);
+}
+
 // block factors of the current matrix (exact block ILU(0)), every solve: the
 // wet/dry state changes rows of the zeta matrix from one step to the next
 // (dry-element rows, level boundaries), and factors of an earlier matrix
@@ -2061,12 +2263,13 @@ static int krylov_outcome(Model &M, const int *c, int *iters, int slot) {
 // the work that follows a converged solve, switched on by its flag, before
 // each check.
 // MODE of the iteration kernels: 0 block factors read from global memory,
-// 1 staged in LDS, 2 factor rows in registers (the init kernel stages)
+// 1 staged in LDS, 2 factor rows in registers (the init kernel stages), 3 the
+// same with the blocks' halos in LDS
 template <typename V, int MODE>
 static int bicgstab_t(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x0,
                       const std::function<int()> &tail) {
     const int g = a.nblk;
-    const size_t lds = apply_lds<V>(M);
+    const size_t lds = apply_lds<V>(M), ilds = iter_lds<V, MODE>(M);
     int it = 0, c[CT_WORDS] = {};
     const int maxit = M.p.itermax > 0 ? (M.p.itermax + 1) / 2 + 1 : 100000;
     int chunk = std::max(2, M.sv.last_its[slot] + 1);
@@ -2078,8 +2281,8 @@ static int bicgstab_t(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x
             if (it0 == 0)
                 hipLaunchKernelGGL((k_bicg_init<V, MODE != 0>), dim3(g), dim3(kThreads), lds, M.stream, a, zero_x0);
             for (int q = 0; q < chunk; q++) {
-                launch_timed(M, T_BICG_A, k_bicg_a<V, MODE>, dim3(g), dim3(kThreads), lds, M.stream, a, it0 + q);
-                launch_timed(M, T_BICG_B, k_bicg_b<V, MODE>, dim3(g), dim3(kThreads), lds, M.stream, a, it0 + q);
+                launch_timed(M, T_BICG_A, k_bicg_a<V, MODE>, dim3(g), dim3(kThreads), ilds, M.stream, a, it0 + q);
+                launch_timed(M, T_BICG_B, k_bicg_b<V, MODE>, dim3(g), dim3(kThreads), ilds, M.stream, a, it0 + q);
             }
             HIPCHK(M, hipGetLastError());
             return 0;
@@ -2104,12 +2307,13 @@ static int bicgstab_t(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x
 template <typename V>
 static int iter_mode(const Model &M, const SolvArgs<V> &a) {
     if (!stage_fits<V>(M)) return 0;
-    return (a.fs_val && a.brows <= kThreads) ? 2 : 1;
+    return (a.fs_val && a.brows <= kThreads) ? (a.hcol ? 3 : 2) : 1;
 }
 
 template <typename V>
 static int bicgstab(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x0, const std::function<int()> &tail) {
     switch (iter_mode(M, a)) {
+    case 3: return bicgstab_t<V, 3>(M, a, iters, slot, zero_x0, tail);
     case 2: return bicgstab_t<V, 2>(M, a, iters, slot, zero_x0, tail);
     case 1: return bicgstab_t<V, 1>(M, a, iters, slot, zero_x0, tail);
     default: return bicgstab_t<V, 0>(M, a, iters, slot, zero_x0, tail);
@@ -2122,12 +2326,12 @@ static int bicgstab(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x0,
 template <typename V, int MODE>
 static int enqueue_inner_t(Model &M, SolvArgs<V> &a, int chunk) {
     const int g = a.nblk;
-    const size_t lds = apply_lds<V>(M);
+    const size_t lds = apply_lds<V>(M), ilds = iter_lds<V, MODE>(M);
     auto launches = [&]() -> int {
         hipLaunchKernelGGL((k_bicg_init<V, MODE != 0>), dim3(g), dim3(kThreads), lds, M.stream, a, 1);
         for (int it = 0; it < chunk; it++) {
-            launch_timed(M, T_BICG_A, k_bicg_a<V, MODE>, dim3(g), dim3(kThreads), lds, M.stream, a, it);
-            launch_timed(M, T_BICG_B, k_bicg_b<V, MODE>, dim3(g), dim3(kThreads), lds, M.stream, a, it);
+            launch_timed(M, T_BICG_A, k_bicg_a<V, MODE>, dim3(g), dim3(kThreads), ilds, M.stream, a, it);
+            launch_timed(M, T_BICG_B, k_bicg_b<V, MODE>, dim3(g), dim3(kThreads), ilds, M.stream, a, it);
         }
         HIPCHK(M, hipGetLastError());
         return 0;
@@ -2144,6 +2348,7 @@ static int enqueue_inner_t(Model &M, SolvArgs<V> &a, int chunk) {
 template <typename V>
 static int enqueue_inner(Model &M, SolvArgs<V> &a, int chunk) {
     switch (iter_mode(M, a)) {
+    case 3: return enqueue_inner_t<V, 3>(M, a, chunk);
     case 2: return enqueue_inner_t<V, 2>(M, a, chunk);
     case 1: return enqueue_inner_t<V, 1>(M, a, chunk);
     default: return enqueue_inner_t<V, 0>(M, a, chunk);
