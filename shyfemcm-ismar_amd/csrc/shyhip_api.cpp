@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -411,8 +412,8 @@ int shyhip_destroy(shyhip_model *h) {
     for (void *q : {(void *)m.nen3v, (void *)m.geo, (void *)m.ang, (void *)m.dis, (void *)m.ilhv, (void *)m.ilhkv,
                     m.hm3v, m.hev, m.hlv, m.hldv, m.areakv, (void *)m.ibnd, (void *)m.zbound, (void *)m.iextb,
                     (void *)m.ibtyp, m.fcorv, m.czv, (void *)m.nk_ptr, (void *)m.nk_el, (void *)m.nkc_el,
-                    (void *)m.inc_cnt, (void *)m.inc_el, (void *)m.inc_elc, (void *)m.slot_of, (void *)m.slot_lev,
-                    (void *)m.slot_aj4,
+                    (void *)m.inc_cnt, (void *)m.inc_el, (void *)m.inc_elc, (void *)m.conz_ek, (void *)m.conz_ep,
+                    (void *)m.slot_lev, (void *)m.slot_aj4,
                     (void *)m.rowptr, (void *)m.cols, (void *)m.ijp, (void *)m.bnd_nodes, (void *)m.bnd_id,
                     (void *)m.blk_rowptr, (void *)m.blk_cols, (void *)m.blk_src, (void *)m.blk_diag, (void *)m.blk_cp_ptr,
                     (void *)m.blk_cp_a, (void *)m.blk_cp_b, (void *)m.blk_jd, (void *)m.blk_pcol, (void *)m.blk_prp,
@@ -422,8 +423,9 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.z_chf, (void *)m.z_chb, (void *)m.z_dentf, (void *)m.z_dentb, (void *)m.z_dptrf,
                     (void *)m.z_dptrb, (void *)m.z_nchf, (void *)m.z_nchb,
                     (void *)m.fwd_rows, (void *)m.fwd_lptr, (void *)m.fwd_nlev, (void *)m.bwd_rows,
-                    (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_el, (void *)m.tvd_kn, m.tvd_w,
-                    (void *)m.tvd_lev, (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem,
+                    (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_up, (void *)m.tvd_w,
+                    (void *)m.conz_uoff, (void *)m.conz_uptr, (void *)m.conz_uvert, (void *)m.conz_upair,
+                    (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem,
                     (void *)m.conz_nent, (void *)m.conz_nplace})
         dfree(q);
     Solver &v = M.sv;
@@ -499,6 +501,21 @@ int shyhip_set_params(shyhip_model *h, const shyhip_params *p) {
     if (check_params(&M, p)) return 1;
     M.p = *p;
     return 0;
+}
+
+// conz3d's element-layer list (Mesh::conz_eitem)
+static std::vector<int> elem_layer_items(int nel, const int *ilhv) {
+    std::vector<int> items;
+    items.reserve((size_t)nel * 2);
+    for (int c0 = 0; c0 < nel; c0 += kConzChunk) {
+        const int c1 = std::min(nel, c0 + kConzChunk);
+        int lmax = 0;
+        for (int ie = c0; ie < c1; ie++) lmax = std::max(lmax, ilhv[ie]);
+        for (int l = 1; l <= lmax; l++)
+            for (int ie = c0; ie < c1; ie++)
+                if (ilhv[ie] >= l) items.push_back((ie << 5) | (l - 1));
+    }
+    return items;
 }
 
 int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const float *ygv, const float *hm3v,
@@ -649,7 +666,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
                 el[pos[k]++] = (ie << 2) | ii;
             }
         // colour order: colours ascending, elements ascending within a colour
-        std::vector<int> sof(3 * (size_t)nel), slev(3 * (size_t)nel);
+        std::vector<int> ek(4 * (size_t)nel, 0), ep(4 * (size_t)nel, 0), slev(3 * (size_t)nel);
         std::vector<double> saj4(3 * (size_t)nel);
         for (int c = 1; c <= M.ncolor; c++)
             for (int ie = 0; ie < nel; ie++) {
@@ -658,12 +675,14 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
                     const int k = M.h_nen3v[3 * ie + ii];
                     const int q = pos2[k]++;
                     elc[q] = (ie << 2) | ii;
-                    sof[(size_t)ii * nel + ie] = q;
+                    ek[4 * (size_t)ie + ii] = k;
+                    ep[4 * (size_t)ie + ii] = q;
                     slev[q] = ilhv[ie];
                     saj4[q] = 4. * M.h_ev[19 * (size_t)ie + 9];
                 }
             }
-        rc |= dalloc(M, &m.slot_of, sof.size()) || upload(M, m.slot_of, sof.data(), sof.size());
+        rc |= dalloc(M, &m.conz_ek, ek.size()) || upload(M, m.conz_ek, ek.data(), ek.size());
+        rc |= dalloc(M, &m.conz_ep, ep.size()) || upload(M, m.conz_ep, ep.data(), ep.size());
         rc |= dalloc(M, &m.slot_lev, slev.size()) || upload(M, m.slot_lev, slev.data(), slev.size());
         rc |= dalloc(M, &m.slot_aj4, saj4.size()) || upload(M, m.slot_aj4, saj4.data(), saj4.size());
         rc |= dalloc(M, &m.nk_ptr, nkn + 1) || upload(M, m.nk_ptr, ptr.data(), ptr.size());
@@ -687,16 +706,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
     // elements, layer by layer) and the node tiles (at most node_tile nodes
     // and kNodeItems node-layers each)
     {
-        std::vector<int> items;
-        items.reserve((size_t)nel * 2);
-        for (int c0 = 0; c0 < nel; c0 += kConzChunk) {
-            const int c1 = std::min(nel, c0 + kConzChunk);
-            int lmax = 0;
-            for (int ie = c0; ie < c1; ie++) lmax = std::max(lmax, ilhv[ie]);
-            for (int l = 1; l <= lmax; l++)
-                for (int ie = c0; ie < c1; ie++)
-                    if (ilhv[ie] >= l) items.push_back((ie << 5) | (l - 1));
-        }
+        const std::vector<int> items = elem_layer_items(nel, ilhv);
         if (nel >= (1 << 26)) return fail(&M, "at most 2^26 elements");
         const int tn = M.p.node_tile > 0 ? std::min(M.p.node_tile, kNodeTileMax) : kNodeTileMax;
         std::vector<int> tiles{0};
@@ -1095,13 +1105,80 @@ int shyhip_set_coefficients(shyhip_model *h, const float *fcorv, const float *cz
     return upload_s(M, M.m.czv, t.data(), M.nel);
 }
 
+// The tables of conz3d's element phase over the node-layers of a workgroup's
+// entries (Mesh::conz_uoff ..) from the pairs' upwind nodes and layers;
+// none where some workgroup's list would exceed kConzUniq.
+static int conz_place_tables(Model &M, const std::vector<int> &tup) {
+    Mesh &m = M.m;
+    dfree(m.conz_uoff); dfree(m.conz_uptr); dfree(m.conz_uvert); dfree(m.conz_upair);
+    m.conz_uoff = m.conz_uptr = nullptr;
+    m.conz_uvert = m.conz_upair = nullptr;
+    const std::vector<int> items = elem_layer_items(M.nel, M.h_ilhv.data());
+    const size_t n = items.size(), nel = M.nel;
+    const int nwg = (int)((n + kThreads - 1) / kThreads);
+    if ((size_t)M.nlvdi * M.nkn > 0x7fffffffu) return 0;
+    std::vector<unsigned> vert(n), pair(6 * n, 0);
+    std::vector<std::vector<int>> lists(nwg);
+    std::atomic<bool> fits{true};
+    parallel_for(nwg, 16, [&](int w_begin, int w_end) {
+        // the offsets of a workgroup in an open-addressing table, then sorted
+        constexpr int kSlots = 4 * kConzUniq;
+        std::vector<int> key(kSlots), val(kSlots);
+        for (int w = w_begin; w < w_end && fits; w++) {
+            std::fill(key.begin(), key.end(), -1);
+            std::vector<int> &u = lists[w];
+            auto slot = [&](int off) {
+                unsigned h = ((unsigned)off * 2654435761u) >> 20;
+                static_assert(kSlots == 1 << 12, "hash bits");
+                while (key[h] != off && key[h] != -1) h = (h + 1) & (kSlots - 1);
+                return h;
+            };
+            auto put = [&](int off) {
+                const unsigned h = slot(off);
+                if (key[h] == -1) { key[h] = off; u.push_back(off); }
+            };
+            const size_t i0 = (size_t)w * kThreads, i1 = std::min(n, i0 + kThreads);
+            auto each = [&](size_t i, auto &&vertex, auto &&upwind) {
+                const int ie = (int)((unsigned)items[i] >> 5), l0 = items[i] & 31;
+                for (int q = 0; q < 3; q++) vertex(q, l0 * M.nkn + M.h_nen3v[3 * (size_t)ie + q]);
+                for (int p = 0; p < 6; p++) {
+                    const int *up = &tup[4 * ((size_t)p * nel + ie)];
+                    if (up[3] > l0)
+                        for (int q = 0; q < 3; q++) upwind(p, q, l0 * M.nkn + up[q]);
+                }
+            };
+            for (size_t i = i0; i < i1 && u.size() <= (size_t)kConzUniq; i++)
+                each(i, [&](int, int off) { put(off); }, [&](int, int, int off) { put(off); });
+            if (u.size() > (size_t)kConzUniq) { fits = false; break; }
+            std::sort(u.begin(), u.end());
+            for (size_t j = 0; j < u.size(); j++) val[slot(u[j])] = (int)j;
+            for (size_t i = i0; i < i1; i++)
+                each(
+                    i, [&](int q, int off) { vert[i] |= (unsigned)val[slot(off)] << (10 * q); },
+                    [&](int p, int q, int off) {
+                        pair[(size_t)p * n + i] |= (unsigned)val[slot(off)] << (10 * q) | 1u << 30;
+                    });
+        }
+    });
+    if (!fits) return 0;
+    std::vector<int> ptr(nwg + 1, 0);
+    for (int w = 0; w < nwg; w++) ptr[w + 1] = ptr[w] + (int)lists[w].size();
+    std::vector<int> off(ptr[nwg]);
+    for (int w = 0; w < nwg; w++) std::copy(lists[w].begin(), lists[w].end(), off.begin() + ptr[w]);
+    int rc = dalloc(M, &m.conz_uptr, ptr.size()) || upload(M, m.conz_uptr, ptr.data(), ptr.size());
+    rc |= dalloc(M, &m.conz_uoff, off.size()) || upload(M, m.conz_uoff, off.data(), off.size());
+    rc |= dalloc(M, &m.conz_uvert, vert.size()) || upload(M, m.conz_uvert, vert.data(), vert.size());
+    rc |= dalloc(M, &m.conz_upair, pair.size()) || upload(M, m.conz_upair, pair.data(), pair.size());
+    return rc;
+}
+
 int shyhip_tvd_init(shyhip_model *h) {
     if (!h) return fail(nullptr, "null handle");
     if (pipe_drain(h->M)) return 1;
     Model &M = h->M;
     // upwind tables per member (a member's upwind points lie in its own elements)
     const size_t nel = M.nel;
-    std::vector<int> tel(6 * nel, -1), tkn(18 * nel, 0);
+    std::vector<int> tup(24 * nel, 0);
     std::vector<double> tw(18 * nel, 0.);
     for (size_t m = 0; m + 1 < M.mem_node.size(); m++) {
         const int k0 = M.mem_node[m], e0 = M.mem_elem[m];
@@ -1114,23 +1191,19 @@ int shyhip_tvd_init(shyhip_model *h) {
         for (int p = 0; p < 6; p++)
             for (int ie = 0; ie < ne; ie++) {
                 const int up = ltel[(size_t)p * ne + ie];
-                tel[(size_t)p * nel + e0 + ie] = up < 0 ? -1 : up + e0;
+                const size_t o = (size_t)p * nel + e0 + ie;
                 for (int q = 0; q < 3; q++) {
-                    tkn[((size_t)q * 6 + p) * nel + e0 + ie] = ltkn[((size_t)q * 6 + p) * ne + ie] + k0;
-                    tw[((size_t)q * 6 + p) * nel + e0 + ie] = ltw[((size_t)q * 6 + p) * ne + ie];
+                    tup[4 * o + q] = ltkn[((size_t)q * 6 + p) * ne + ie] + k0;
+                    (q < 2 ? tw[2 * o + q] : tw[12 * nel + o]) = ltw[((size_t)q * 6 + p) * ne + ie];
                 }
+                tup[4 * o + 3] = up >= 0 ? M.h_ilhv[up + e0] : 0;
             }
     }
-    std::vector<int> tlev(6 * nel, 0);
-    for (size_t q = 0; q < tel.size(); q++) tlev[q] = tel[q] >= 0 ? M.h_ilhv[tel[q]] : 0;
-    dfree(M.m.tvd_el); dfree(M.m.tvd_kn); dfree(M.m.tvd_w); dfree(M.m.tvd_lev);
+    dfree(M.m.tvd_up); dfree(M.m.tvd_w);
     int rc = 0;
-    rc |= dalloc(M, &M.m.tvd_el, tel.size()) || upload(M, M.m.tvd_el, tel.data(), tel.size());
-    rc |= dalloc(M, &M.m.tvd_lev, tlev.size()) || upload(M, M.m.tvd_lev, tlev.data(), tlev.size());
-    rc |= dalloc(M, &M.m.tvd_kn, tkn.size()) || upload(M, M.m.tvd_kn, tkn.data(), tkn.size());
-    double *w = nullptr;
-    rc |= dalloc(M, &w, tw.size()) || upload(M, w, tw.data(), tw.size());
-    M.m.tvd_w = w;
+    rc |= dalloc(M, &M.m.tvd_up, tup.size()) || upload(M, M.m.tvd_up, tup.data(), tup.size());
+    rc |= dalloc(M, &M.m.tvd_w, tw.size()) || upload(M, M.m.tvd_w, tw.data(), tw.size());
+    rc |= conz_place_tables(M, tup);
     M.tvd_ready = rc == 0;
     return rc;
 }

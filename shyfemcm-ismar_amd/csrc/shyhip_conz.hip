@@ -1,7 +1,7 @@
 // shyhip_conz.hip -- 3D scalar advection-diffusion (conz3d) on gfx950.
 //
 // Two kernels per substep:
-//   k_conz_elem  one work-item per element-layer of a precomputed work list
+//   k_conz_elem[_lds]  one work-item per element-layer of a precomputed work list
 //                (workgroups of equal work whatever the depth): horizontal
 //                advective fluxes (upwind rule, the itvd=2 TVD scheme with
 //                precomputed upwind interpolation weights, or the itvd=1
@@ -45,16 +45,21 @@ struct ConzArgs {
     const int *nen3v, *ilhv, *ilhkv, *iextb, *ibnd;
     const double *geo, *dis;
     const int *nkc_ptr, *nkc_el;
-    const int *slot_of, *slot_lev;   // colour-order list positions (see Mesh)
+    const int4 *ek, *ep;             // elements' vertices and colour-order list positions (see Mesh)
+    const int *slot_lev;
     const double *slot_aj4;
     int nslot;                       // 3 * nel
-    const int *tvd_el, *tvd_kn, *tvd_lev, *elem_iext;
-    const double *tvd_w;
+    const int *elem_iext;
+    const int4 *tvd_up;              // upwind nodes, layers and weights of the ordered pairs (see Mesh)
+    const double2 *tvd_w;
+    const double *tvd_w2;
+    const int *uoff, *uptr;          // node-layers of a workgroup's entries and places in them (see Mesh)
+    const unsigned *uvert, *upair;
     const S *utn, *vtn, *uto, *vto, *uln, *vln;
     const S *hdkn, *hdko, *hden, *hdeo, *wln, *difv, *mflux;
     S *c[kMaxTracers];               // tracers (in/out)
     const S *cbound[kMaxTracers];    // source concentrations (may be null)
-    S *hbuf;                         // element terms [(l-1)*NT + t][slot_of[ii][ie]]
+    S *hbuf;                         // element terms [l-1][list position][NT]
     int *err;
     // ensembles whose members run different numbers of substeps: member
     // istot (null: all run istot), node/element -> member, this substep and
@@ -69,9 +74,11 @@ struct ConzArgs {
     const int4 *nent;                // node tiles' entries, and the nodes' first places in their tiles
     const int *nplace;
     int clear_below;                 // also write the zeros below the bottom
-    // the step's element-layer records (k_conz_prep): int and double columns
-    int *rec_i;
-    double *rec_d;
+    // the step's element-layer records (k_conz_prep)
+    int *rec_code;
+    uint2 *rec_pair;
+    double *rec_f;
+    S *rec_s;
     // the launch's single tracer's own terms (null: none): nudging factor
     // robs with target cobs and rate rtauv, sinking wsink * wsinkv, loads
     // rload * load (node arrays like the tracer; wsinkv on interfaces)
@@ -105,15 +112,21 @@ __device__ inline double cval(const ConzArgs<S> &a, int t, int l, int k) {
 //
 // Everything of an element-layer that depends on the flow only -- the flux
 // coefficients f, the upwind case, and for TVD the two pairs of the flow
-// direction with their Courant numbers, upwind nodes and interpolation
-// weights -- holds for all the substeps of a step (the transports,
-// velocities and the substep length do not change within it).  k_conz_prep
-// computes it once per step into a record per list entry (ConzRec: columns
-// indexed by the entry, so every load is contiguous); k_conz_elem then
-// reads the record, gathers the tracers at the element's nodes and upwind
-// points, and applies the upwind rule or the limiter.  The arithmetic is
-// that of the element terms computed in one pass (the record holds the
-// values, not approximations of them).
+// direction with their Courant numbers -- holds for all the substeps of a
+// step (the transports, velocities and the substep length do not change
+// within it).  k_conz_prep computes it once per step into a record per list
+// entry (columns indexed by the entry, so every load is contiguous);
+// k_conz_elem then reads the record, gathers the tracers at the element's
+// nodes and upwind points, and applies the upwind rule or the limiter.  The
+// arithmetic is that of the element terms computed in one pass (the record
+// holds the values, not approximations of them).
+//
+// What bounds both: the memory they move.  The record holds what the flow
+// decides, 44 bytes (FP64) or 36 (FP32); an element's vertices, list
+// positions, upwind nodes and weights come from the mesh's tables, which the
+// layers of a chunk share in cache.  With all of it in the record, 144 bytes,
+// it took 119 us a substep for the element terms and 132 us a step for the
+// record on 300k nodes of 20 layers (FP64, T and S); now 92 and 56.
 
 // v[i] for a run-time i in 0..2 without indexing a register array
 template <typename T>
@@ -121,14 +134,34 @@ __device__ inline T sel3(const T (&v)[3], int i) {
     return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
 }
 
-// record columns (int: RI_*, double: RD_*), each n_eitem long
-enum { RI_IE = 0, RI_L, RI_KN, RI_SO = RI_KN + 3, RI_CODE = RI_SO + 3, RI_TKN, RI_N = RI_TKN + 6 };
-enum { RD_F = 0, RD_TW = 3, RD_ALFA = 9, RD_N = 11 };
-// the case word: itot (bits 0-1), isum (2-4), TVD pairs present (5), and per
-// pair k (bits 8 + 8k ..): ic (2 bits), id (2 bits), upwind point present (1)
-__host__ __device__ inline size_t conz_rec_bytes(int n) {
-    return ((size_t)RI_N * n * sizeof(int) + 7) / 8 * 8 + (size_t)RD_N * n * sizeof(double);
-}
+// A record's columns, each n_eitem long: the case word, the flux coefficients
+// (RF_*, double), and in the tracers' precision (RS_*) the Courant numbers of
+// the two pairs and, for itvd = 1 only, the pairs' edge vectors; where the
+// element phase reads the node-layers from LDS, the two pairs' words of
+// Mesh::conz_upair (rec_pair).
+//
+// With one or two vertices taking inflow one vertex, p, stands against the
+// other two, a and b (ascending): the only one with inflow or the only one
+// without.  The pairs are (p, a) and (p, b), upstream to downstream, or with
+// two inflows (a, p) and (b, p); the terms of a and b are the flux
+// coefficient times the pair's face value and p's the negative of their sum.
+// The upwind rule has the same form with the upstream value for the face
+// (except that with one inflow p's term is its own coefficient's), so the
+// whole phase is a straight line.
+// The case word: p - 1 (bits 0-1), two inflows (2), any flux (3), TVD pairs
+// present (4), upwind points present (5, 6).
+enum { RF_A = 0, RF_B, RF_P, RF_N };
+enum { RS_ALFA = 0, RS_EDGE = 2, RS_N = 6 };
+static inline size_t conz_rec_code_bytes(int n) { return ((size_t)n * sizeof(int) + 15) / 16 * 16; }
+
+// the tracers' terms of one list position in hbuf
+template <typename S, int NT>
+struct alignas(NT * sizeof(S)) Terms {
+    S t[NT];
+};
+
+// the place of the ordered pair (ic, id), 1-based, among an element's six
+__device__ inline int tvd_pair(int ic, int id) { return 2 * (ic - 1) + ((id == (ic % 3) + 1) ? 0 : 1); }
 
 template <typename S>
 __global__ __launch_bounds__(kThreads) void k_conz_prep(ConzArgs<S> a) {
@@ -140,12 +173,9 @@ __global__ __launch_bounds__(kThreads) void k_conz_prep(ConzArgs<S> a) {
     const int ie = (int)(w >> 5), l = (int)(w & 31u) + 1;
     const int nel = a.nel;
     const bool use_tvd = a.itvd > 0;
-    int kn[3], so[3];
     double gb[3], gc[3];
 #pragma unroll
     for (int ii = 0; ii < 3; ii++) {
-        kn[ii] = a.nen3v[3 * ie + ii];
-        so[ii] = a.slot_of[(size_t)ii * nel + ie];
         gb[ii] = a.geo[(size_t)ii * nel + ie];
         gc[ii] = a.geo[(size_t)(3 + ii) * nel + ie];
     }
@@ -171,16 +201,17 @@ __global__ __launch_bounds__(kThreads) void k_conz_prep(ConzArgs<S> a) {
         f[ii] = us * gb[ii] + vs * gc[ii];
         if (f[ii] < 0.) { itot++; isum += ii + 1; }
     }
-    int code = itot | (isum << 2);
-    int *ri = a.rec_i;
-    double *rd = a.rec_d;
-    if (use_tvd && iext == 0 && itot >= 1 && itot <= 2) {
+    const bool flux = itot >= 1 && itot <= 2;
+    const int itot2 = itot - 1, itot1 = 2 - itot;
+    const int ip = flux ? itot2 * (6 - isum) + itot1 * isum : 1;
+    int code = (ip - 1) | (itot == 2 ? 4 : 0) | (flux ? 8 : 0);
+    S alfa[2] = {0, 0};
+    unsigned up[2] = {0, 0};
+    if (use_tvd && iext == 0 && flux) {
         // TVD fluxes (tvd_fluxes, tvd_admin.f90:673-823): the two pairs
         // (ic, id) of the flow direction -- the vertices other than ip,
         // ascending -- and their Courant numbers and upwind points
-        code |= 1 << 5;
-        const int itot2 = itot - 1, itot1 = 2 - itot;
-        const int ip = itot2 * (6 - isum) + itot1 * isum;
+        code |= 1 << 4;
         const R ajr = (R)(24. * ajr0);
         const double dte = a.mem_istot ? a.dtp / (double)a.mem_istot[a.elem_mem[ie]] : a.dt;
 #pragma unroll
@@ -188,7 +219,6 @@ __global__ __launch_bounds__(kThreads) void k_conz_prep(ConzArgs<S> a) {
             const int ii = k == 0 ? (ip == 1 ? 2 : 1) : (ip == 3 ? 2 : 3);
             const int ic = itot2 * ii + itot1 * ip;
             const int id = itot2 * ip + itot1 * ii;
-            const int pidx = 2 * (ic - 1) + ((id == (ic % 3) + 1) ? 0 : 1);
             const int iop = 6 - (id + ic);
             const int tet1 = 1 + iop % 3;
             R dx = (R)((double)ajr * sel3(gc, iop - 1));
@@ -197,34 +227,27 @@ __global__ __launch_bounds__(kThreads) void k_conz_prep(ConzArgs<S> a) {
             dy = (R)(-2 * (tet1 == ic ? 1 : 0)) * dy + dy;
             const R dis = (R)sel3(dis3, iop - 1);
             const R vel = (R)fabs((double)(ul * dx + vl * dy)) / dis;
-            const R alfa = (R)((dte * (double)vel) / (double)dis);
+            alfa[k] = (R)((dte * (double)vel) / (double)dis);
             if (a.itvd == 2) {
-                const size_t po = (size_t)pidx * nel + ie;
-                const bool pup = a.tvd_el[po] >= 0 && a.tvd_lev[po] >= l;
-                code |= (ic | (id << 2) | ((pup ? 1 : 0) << 4)) << (8 + 8 * k);
-#pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    ri[(size_t)(RI_TKN + 3 * k + q) * n + i] = a.tvd_kn[((size_t)q * 6 + pidx) * nel + ie];
-                    rd[(size_t)(RD_TW + 3 * k + q) * n + i] = a.tvd_w[((size_t)q * 6 + pidx) * nel + ie];
-                }
+                const int pr = tvd_pair(ic, id);
+                if (a.upair) up[k] = a.upair[(size_t)pr * n + i];
+                else if (a.tvd_up[(size_t)pr * nel + ie].w >= l) code |= 1 << (5 + k);
             } else {
                 // itvd = 1: the edge vector, for the gradient's projection
-                code |= (ic | (id << 2)) << (8 + 8 * k);
-                rd[(size_t)(RD_TW + 3 * k) * n + i] = (double)dx;
-                rd[(size_t)(RD_TW + 3 * k + 1) * n + i] = (double)dy;
+                a.rec_s[(size_t)(RS_EDGE + 2 * k) * n + i] = dx;
+                a.rec_s[(size_t)(RS_EDGE + 2 * k + 1) * n + i] = dy;
             }
-            rd[(size_t)(RD_ALFA + k) * n + i] = (double)alfa;
         }
     }
-    ri[(size_t)RI_IE * n + i] = ie;
-    ri[(size_t)RI_L * n + i] = l;
+    a.rec_code[i] = code;
+    if (a.upair) a.rec_pair[i] = make_uint2(up[0], up[1]);
+    a.rec_f[(size_t)RF_A * n + i] = sel3(f, ip == 1 ? 1 : 0);
+    a.rec_f[(size_t)RF_B * n + i] = sel3(f, ip == 3 ? 1 : 2);
+    if (!(code & (4 | 16))) a.rec_f[(size_t)RF_P * n + i] = sel3(f, ip - 1);
+    if (use_tvd) {
 #pragma unroll
-    for (int ii = 0; ii < 3; ii++) {
-        ri[(size_t)(RI_KN + ii) * n + i] = kn[ii];
-        ri[(size_t)(RI_SO + ii) * n + i] = so[ii];
-        rd[(size_t)(RD_F + ii) * n + i] = f[ii];
+        for (int k = 0; k < 2; k++) a.rec_s[(size_t)(RS_ALFA + k) * n + i] = alfa[k];
     }
-    ri[(size_t)RI_CODE * n + i] = code;
 }
 
 // ------------------------------------------------------------------ gradient TVD
@@ -346,6 +369,18 @@ __global__ __launch_bounds__(kThreads) void k_tvd_grad_node(ConzArgs<S> a) {
     }
 }
 
+// A pair's flux with the limited face value (tvd_fluxes): upstream conc,
+// downstream cond, grad the limiter's upwind difference, flux coefficient f.
+template <typename R>
+__device__ inline double tvd_term(R conc, R cond, R grad, R alfa, double f) {
+    const R rq = grad / (cond - conc) - (R)1;
+    const R rf = (R)fabs((double)(conc - cond)) < (R)1.e-8 ? (R)-1 : rq;
+    const double rfd = (double)rf;
+    const R psi = (R)fmax(0., fmax(fmin(1., 2. * rfd), fmin(2., rfd)));
+    const R conf = conc + (R)0.5 * psi * (cond - conc) * ((R)1 - alfa);
+    return (double)(R)((double)conf * f);
+}
+
 // GRAD: itvd = 1 (the upstream node's gradient in place of the upwind point)
 // HDIF: horizontal diffusion (rkpar > 0): the element's term
 // rk3 hmed wdiff (concentration_omp.f90:560-570,727-735) is taken off the
@@ -355,124 +390,94 @@ __global__ __launch_bounds__(kThreads) void k_conz_elem(ConzArgs<S> a) {
     using R = S;
     const int i = xcd_block() * kThreads + threadIdx.x;
     if (i >= a.n_eitem) return;
-    const int n = a.n_eitem, nkn = a.nkn;
-    const int *ri = a.rec_i;
-    const double *rd = a.rec_d;
-    if (a.mem_istot && a.isact > a.mem_istot[a.elem_mem[ri[(size_t)RI_IE * n + i]]]) return;
-    const int l = ri[(size_t)RI_L * n + i], code = ri[(size_t)RI_CODE * n + i];
-    int kn[3], so[3];
-    double f[3];
+    const int n = a.n_eitem, nkn = a.nkn, nel = a.nel;
+    const bool use_tvd = a.itvd > 0;
+    const unsigned w = (unsigned)a.eitem[i];
+    const int code = a.rec_code[i];
+    const double f[2] = {a.rec_f[(size_t)RF_A * n + i], a.rec_f[(size_t)RF_B * n + i]};
+    R alfa[2] = {0, 0};
+    if (use_tvd)
 #pragma unroll
-    for (int ii = 0; ii < 3; ii++) {
-        kn[ii] = ri[(size_t)(RI_KN + ii) * n + i];
-        so[ii] = ri[(size_t)(RI_SO + ii) * n + i];
-        f[ii] = rd[(size_t)(RD_F + ii) * n + i];
-    }
-    const int itot = code & 3, isum = (code >> 2) & 7;
-    const bool tvd = (code >> 5) & 1;
+        for (int k = 0; k < 2; k++) alfa[k] = a.rec_s[(size_t)(RS_ALFA + k) * n + i];
+    const int ie = (int)(w >> 5), l = (int)(w & 31u) + 1;
+    if (a.mem_istot && a.isact > a.mem_istot[a.elem_mem[ie]]) return;
+    const int p = code & 3;
+    const bool two = code & 4, flux = code & 8, tvd = code & 16;
+    const int4 kp = a.ek[ie], ep = a.ep[ie];
+    // vertices and list positions of p, a and b
+    const int kn[3] = {p == 0 ? kp.x : (p == 1 ? kp.y : kp.z), p == 0 ? kp.y : kp.x, p == 2 ? kp.y : kp.z};
+    const int so[3] = {p == 0 ? ep.x : (p == 1 ? ep.y : ep.z), p == 0 ? ep.y : ep.x, p == 2 ? ep.y : ep.z};
+    const size_t lo = (size_t)(l - 1) * nkn;
     S cr[NT][3];
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int ii = 0; ii < 3; ii++) cr[t][ii] = a.c[t][(size_t)(l - 1) * nkn + kn[ii]];
+        for (int q = 0; q < 3; q++) cr[t][q] = a.c[t][lo + kn[q]];
+    // a pair's upwind point (nodes, weights; also where there is none or the
+    // element takes the upwind rule: valid addresses, not used) or gradient
+    S cu[2][NT][3] = {};
+    double tw[2][3] = {};
+    if (use_tvd) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if (GRAD) {
+                const int kc = two ? kn[k + 1] : kn[0];
+                if (tvd)
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        tw[k][q] = (double)a.rec_s[(size_t)(RS_EDGE + 2 * k + q) * n + i];
+#pragma unroll
+                        for (int t = 0; t < NT; t++) cu[k][t][q] = a.grad[ngrad_at(nkn, NT, t, q, l, kc)];
+                    }
+            } else {
+                const int v = k == 0 ? (p == 0 ? 1 : 0) : (p == 2 ? 1 : 2);
+                const size_t po = (size_t)(two ? tvd_pair(v + 1, p + 1) : tvd_pair(p + 1, v + 1)) * nel + ie;
+                const int4 up = a.tvd_up[po];
+                const double2 w01 = a.tvd_w[po];
+                tw[k][0] = w01.x; tw[k][1] = w01.y; tw[k][2] = a.tvd_w2[po];
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    cu[k][t][0] = a.c[t][lo + up.x];
+                    cu[k][t][1] = a.c[t][lo + up.y];
+                    cu[k][t][2] = a.c[t][lo + up.z];
+                }
+            }
+        }
+    }
+    double fp = 0.;
+    if (!two && !tvd) fp = a.rec_f[(size_t)RF_P * n + i];
     auto clip = [&](int t, S v) -> S { return (a.clip[t] && v < (S)1.e-15) ? (S)0 : v; };
     double fl[NT][3];
 #pragma unroll
-    for (int t = 0; t < NT; t++) fl[t][0] = fl[t][1] = fl[t][2] = 0.;
-    if (!tvd) {
-        // upwind rule (also the elements of a TVD run at an external
-        // boundary); no flux when no vertex or all take inflow
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            double cl[3];
-            for (int ii = 0; ii < 3; ii++) cl[ii] = (double)clip(t, cr[t][ii]);
-            if (itot == 1) {
-                const double cu1 = sel3(cl, isum - 1);
-                for (int ii = 0; ii < 3; ii++) fl[t][ii] = f[ii] * cu1;
-            } else if (itot == 2) {
-                const int is2 = 6 - isum;
-                for (int ii = 0; ii < 3; ii++) fl[t][ii] = (ii == is2 - 1) ? 0. : f[ii] * cl[ii];
-                const double sum = fl[t][0] + fl[t][1] + fl[t][2];
-                for (int ii = 0; ii < 3; ii++)
-                    if (ii == is2 - 1) fl[t][ii] = -sum;
-            }
-        }
-    } else {
-        // the two pairs' upwind values, then each tracer's limiter
-        const int itot2 = itot - 1, itot1 = 2 - itot;
-        const int ip = itot2 * (6 - isum) + itot1 * isum;
-        const R fact = (R)(-itot2 + itot1);
-        // itvd = 2: upwind nodes and weights; itvd = 1: the edge vector
-        // (tw[k][0..1])
-        int tkn[2][3] = {};
-        double tw[2][3] = {};
-        R alfa[2];
+    for (int t = 0; t < NT; t++) {
+        const R cp = clip(t, cr[t][0]);
+        double u[2];
 #pragma unroll
         for (int k = 0; k < 2; k++) {
-#pragma unroll
-            for (int q = 0; q < (GRAD ? 2 : 3); q++) {
-                if (!GRAD) tkn[k][q] = ri[(size_t)(RI_TKN + 3 * k + q) * n + i];
-                tw[k][q] = rd[(size_t)(RD_TW + 3 * k + q) * n + i];
-            }
-            alfa[k] = (R)rd[(size_t)(RD_ALFA + k) * n + i];
-        }
-        S cu[2][NT][3];
-        if (!GRAD) {
-#pragma unroll
-            for (int k = 0; k < 2; k++)
-                if ((code >> (12 + 8 * k)) & 1)
-#pragma unroll
-                    for (int t = 0; t < NT; t++)
-#pragma unroll
-                        for (int q = 0; q < 3; q++) cu[k][t][q] = a.c[t][(size_t)(l - 1) * nkn + tkn[k][q]];
-        } else {
-            // the gradient (x, y) of each tracer at each pair's upstream node
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                const int kc = sel3(kn, ((code >> (8 + 8 * k)) & 3) - 1);
-#pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    cu[k][t][0] = a.grad[ngrad_at(nkn, NT, t, 0, l, kc)];
-                    cu[k][t][1] = a.grad[ngrad_at(nkn, NT, t, 1, l, kc)];
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int ck = code >> (8 + 8 * k);
-            const int ic = ck & 3, id = (ck >> 2) & 3;
-            const bool pup = (ck >> 4) & 1;
-            const int ii = k == 0 ? (ip == 1 ? 2 : 1) : (ip == 3 ? 2 : 3);
-            const double fii = sel3(f, ii - 1);
-#pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const R conc = clip(t, sel3(cr[t], ic - 1)), cond = clip(t, sel3(cr[t], id - 1));
+            const R ci = clip(t, cr[t][k + 1]);
+            const R conc = two ? ci : cp, cond = two ? cp : ci;
+            u[k] = f[k] * (double)conc;
+            if (use_tvd) {
                 R grad;
                 if (GRAD) {
-                    // itvd = 1: grad = 2 (g(kc) . edge), the edge vector in tw[k][0..1]
-                    grad = (R)2. * ((R)cu[k][t][0] * (R)tw[k][0] + (R)cu[k][t][1] * (R)tw[k][1]);
+                    // itvd = 1: grad = 2 (g(kc) . edge)
+                    grad = (R)2. * (cu[k][t][0] * (R)tw[k][0] + cu[k][t][1] * (R)tw[k][1]);
                 } else {
-                    R conu = cond;
-                    if (pup) {
-                        double zh = 0.;
-                        for (int q = 0; q < 3; q++) zh = zh + (double)clip(t, cu[k][t][q]) * tw[k][q];
-                        conu = (R)zh;
-                    }
-                    grad = cond - conu;
+                    double zh = 0.;
+#pragma unroll
+                    for (int q = 0; q < 3; q++) zh = zh + (double)clip(t, cu[k][t][q]) * tw[k][q];
+                    grad = cond - (((code >> (5 + k)) & 1) ? (R)zh : cond);
                 }
-                R rf;
-                if ((R)fabs((double)(conc - cond)) < (R)1.e-8) rf = -1;
-                else rf = grad / (cond - conc) - (R)1;
-                const double rfd = (double)rf;
-                const R psi = (R)fmax(0., fmax(fmin(1., 2. * rfd), fmin(2., rfd)));
-                const R conf = conc + (R)0.5 * psi * (cond - conc) * ((R)1 - alfa[k]);
-                const R term = (R)((double)(fact * conf) * fii);
-                for (int q = 0; q < 3; q++) {
-                    if (q == ic - 1) fl[t][q] = fl[t][q] - (double)term;
-                    if (q == id - 1) fl[t][q] = fl[t][q] + (double)term;
-                }
+                const double term = tvd_term(conc, cond, grad, alfa[k], f[k]);
+                if (tvd) u[k] = term;
             }
         }
+        fl[t][0] = two || tvd ? -(u[0] + u[1]) : fp * (double)cp;
+        fl[t][1] = u[0];
+        fl[t][2] = u[1];
+        // no flux when no vertex or all take inflow
+#pragma unroll
+        for (int q = 0; q < 3; q++) fl[t][q] = flux ? fl[t][q] : 0.;
     }
     double hd[NT][3];
 #pragma unroll
@@ -480,8 +485,7 @@ __global__ __launch_bounds__(kThreads) void k_conz_elem(ConzArgs<S> a) {
     if (HDIF) {
         // rk3 = 3 rkpar difhv in the tracers' precision, hmed the element
         // layer's thickness at this substep, wdiff(ii) = sum over iii of
-        // wdifhv(iii, ii) c(iii)
-        const int ie = ri[(size_t)RI_IE * n + i], nel = a.nel;
+        // wdifhv(iii, ii) c(iii), in the element's own order of the vertices
         const size_t o = (size_t)(l - 1) * nel + ie;
         double rso = a.rso;
         if (a.mem_istot) rso = (a.isact - 1) / (double)a.mem_istot[a.elem_mem[ie]];
@@ -494,24 +498,138 @@ __global__ __launch_bounds__(kThreads) void k_conz_elem(ConzArgs<S> a) {
             for (int q = 0; q < 3; q++) wv[ii][q] = (double)a.wdif[(size_t)(3 * ii + q) * nel + ie];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            double cl[3];
-#pragma unroll
-            for (int q = 0; q < 3; q++) cl[q] = (double)clip(t, cr[t][q]);
+            const double cv[3] = {(double)clip(t, cr[t][0]), (double)clip(t, cr[t][1]), (double)clip(t, cr[t][2])};
+            const double cl[3] = {p == 0 ? cv[0] : cv[1], p == 0 ? cv[1] : (p == 1 ? cv[0] : cv[2]),
+                                  p == 2 ? cv[0] : cv[2]};
+            double h[3];
 #pragma unroll
             for (int ii = 0; ii < 3; ii++) {
                 double waux = 0.;
 #pragma unroll
                 for (int q = 0; q < 3; q++) waux = waux + wv[ii][q] * cl[q];
-                hd[t][ii] = rk3 * hmed * waux;
+                h[ii] = rk3 * hmed * waux;
             }
+            hd[t][0] = sel3(h, p);
+            hd[t][1] = sel3(h, p == 0 ? 1 : 0);
+            hd[t][2] = sel3(h, p == 2 ? 1 : 2);
         }
     }
+    Terms<S, NT> *const hb = (Terms<S, NT> *)a.hbuf + (size_t)(l - 1) * a.nslot;
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+    for (int q = 0; q < 3; q++) {
+        Terms<S, NT> v;
 #pragma unroll
-        for (int ii = 0; ii < 3; ii++)
-            a.hbuf[((size_t)(l - 1) * NT + t) * a.nslot + so[ii]] = (S)(HDIF ? 3. * fl[t][ii] - hd[t][ii]
-                                                                               : 3. * fl[t][ii]);
+        for (int t = 0; t < NT; t++) v.t[t] = (S)(HDIF ? 3. * fl[t][q] - hd[t][q] : 3. * fl[t][q]);
+        hb[so[q]] = v;
+    }
+}
+
+// The same for itvd = 2 without horizontal diffusion, over the node-layers of
+// the workgroup's entries (Mesh::conz_uoff): each is read once into LDS, both
+// tracers side by side, and an entry gathers there by 10-bit places.
+//
+// What bounds it: memory, at 3.7 TB/s of the 4.8 of a copy.  Gathering the
+// tracers at three vertices and six upwind nodes from memory, 18 gathers of
+// 8 bytes, kept the address path busy instead (1,250 cache accesses a
+// wavefront against 670): 107 us a launch on 300k nodes of 20 layers (FP64, T
+// and S) against 92, 15.1 against 12.4 on the 50k-node lagoon, FP32 on 285k
+// nodes 42.6 against 33.  The lists hold 620 node-layers on average where
+// the elements are numbered with locality; beyond kConzUniq the copies into
+// LDS outgrow the gathers they save and k_conz_elem runs.
+template <typename S, int NT>
+__global__ __launch_bounds__(kThreads) void k_conz_elem_lds(ConzArgs<S> a) {
+    using R = S;
+    __shared__ Terms<S, NT> val[kConzUniq];
+    const int wg = xcd_block();
+    const int n = a.n_eitem, nel = a.nel;
+    const int i0 = wg * kThreads + threadIdx.x;
+    const int i = min(i0, n - 1);             // (the last workgroup's spare work-items read its last entry)
+    // the workgroup's node-layers; kConzUniq of them at most
+    const int u0 = a.uptr[wg], nu = a.uptr[wg + 1] - u0;
+    constexpr int kPer = kConzUniq / kThreads;
+    int uo[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+        const int j = q * kThreads + threadIdx.x;
+        uo[q] = j < nu ? a.uoff[u0 + j] : -1;
+    }
+    const unsigned w = (unsigned)a.eitem[i];
+    const int code = a.rec_code[i];
+    const unsigned uv = a.uvert[i];
+    const uint2 rp = a.rec_pair[i];
+    const unsigned up[2] = {rp.x, rp.y};
+    const double f[2] = {a.rec_f[(size_t)RF_A * n + i], a.rec_f[(size_t)RF_B * n + i]};
+    const R alfa[2] = {a.rec_s[(size_t)(RS_ALFA + 0) * n + i], a.rec_s[(size_t)(RS_ALFA + 1) * n + i]};
+    Terms<S, NT> uc[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; q++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) uc[q].t[t] = uo[q] >= 0 ? a.c[t][uo[q]] : (S)0;
+    const int ie = (int)(w >> 5), l = (int)(w & 31u) + 1;
+    const int p = code & 3;
+    const bool two = code & 4, flux = code & 8, tvd = code & 16;
+    const int4 ep = a.ep[ie];
+    double tw[2][3];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int v = k == 0 ? (p == 0 ? 1 : 0) : (p == 2 ? 1 : 2);
+        const size_t po = (size_t)(two ? tvd_pair(v + 1, p + 1) : tvd_pair(p + 1, v + 1)) * nel + ie;
+        const double2 w01 = a.tvd_w[po];
+        tw[k][0] = w01.x; tw[k][1] = w01.y; tw[k][2] = a.tvd_w2[po];
+    }
+    double fp = 0.;
+    if (!two && !tvd) fp = a.rec_f[(size_t)RF_P * n + i];
+    bool on = i0 < n;
+    if (a.mem_istot && a.isact > a.mem_istot[a.elem_mem[ie]]) on = false;
+    auto clip = [&](int t, S v) -> S { return (a.clip[t] && v < (S)1.e-15) ? (S)0 : v; };
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+        if (uo[q] < 0) continue;
+        Terms<S, NT> v;
+#pragma unroll
+        for (int t = 0; t < NT; t++) v.t[t] = clip(t, uc[q].t[t]);
+        val[q * kThreads + threadIdx.x] = v;
+    }
+    __syncthreads();
+    if (!on) return;
+    // list positions and values of p, a and b
+    const int so[3] = {p == 0 ? ep.x : (p == 1 ? ep.y : ep.z), p == 0 ? ep.y : ep.x, p == 2 ? ep.y : ep.z};
+    const int vp[3] = {10 * p, p == 0 ? 10 : 0, p == 2 ? 10 : 20};
+    Terms<S, NT> cr[3], cu[2][3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        cr[q] = val[(uv >> vp[q]) & (kConzUniq - 1)];
+#pragma unroll
+        for (int k = 0; k < 2; k++) cu[k][q] = val[(up[k] >> (10 * q)) & (kConzUniq - 1)];
+    }
+    double fl[NT][3];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const R cp = cr[0].t[t];
+        double u[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const R ci = cr[k + 1].t[t];
+            const R conc = two ? ci : cp, cond = two ? cp : ci;
+            double zh = 0.;
+#pragma unroll
+            for (int q = 0; q < 3; q++) zh = zh + (double)cu[k][q].t[t] * tw[k][q];
+            const R grad = cond - ((up[k] >> 30) ? (R)zh : cond);
+            const double term = tvd_term(conc, cond, grad, alfa[k], f[k]);
+            u[k] = tvd ? term : f[k] * (double)conc;
+        }
+        fl[t][0] = two || tvd ? -(u[0] + u[1]) : fp * (double)cp;
+        fl[t][1] = u[0];
+        fl[t][2] = u[1];
+    }
+    Terms<S, NT> *const hb = (Terms<S, NT> *)a.hbuf + (size_t)(l - 1) * a.nslot;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        Terms<S, NT> v;
+#pragma unroll
+        for (int t = 0; t < NT; t++) v.t[t] = (S)(3. * (flux ? fl[t][q] : 0.));
+        hb[so[q]] = v;
+    }
 }
 
 // ------------------------------------------------------------------ node phase
@@ -519,9 +637,8 @@ __global__ __launch_bounds__(kThreads) void k_conz_elem(ConzArgs<S> a) {
 // tvd_admin.f90:930-1016): centre conc, downstream cond, upstream conu,
 // Courant number alfa.
 __device__ inline double tvd_face(double conc, double cond, double conu, double alfa) {
-    double rf;
-    if (fabs(conc - cond) < (double)1.e-8f) rf = -1.;
-    else rf = (cond - conu) / (cond - conc) - 1.;
+    const double rq = (cond - conu) / (cond - conc) - 1.;
+    const double rf = fabs(conc - cond) < (double)1.e-8f ? -1. : rq;
     const double psi = fmax(0., fmax(fmin(1., 2. * rf), fmin(2., rf)));
     return conc + 0.5 * psi * (cond - conc) * (1. - alfa);
 }
@@ -545,7 +662,8 @@ __device__ inline double tvd_face(double conc, double cond, double conu, double 
 // barriers), reading the list start and the elements' layers as data, and
 // evaluating a limited face per sign of the vertical velocity took 26.5 us a
 // launch on the 50k-node lagoon and 159 us on 300k nodes of 20 layers (T and
-// S, FP64), against 21.5 and 115 us.
+// S, FP64), against 21.5 and 115 us; 20.4 and 105 with an incident element's
+// terms of both tracers in one load and selects in place of branches.
 template <typename S, int NT, bool EXT>
 __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
     using R = S;
@@ -583,17 +701,17 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
         // The first kIncWidth positions are read unconditionally (clamped to
         // the list), contiguous for the node; the last two pairs only by
         // wavefronts that hold such a node; the rest one by one.
-        double saj[kIncWidth], shf0[kIncWidth], shf1[kIncWidth];
-        const size_t hl = (size_t)(l - 1) * NT * a.nslot;
+        double saj[kIncWidth];
+        Terms<S, NT> shf[kIncWidth];
+        const Terms<S, NT> *const hb = (const Terms<S, NT> *)a.hbuf + (size_t)(l - 1) * a.nslot;
         const bool any6 = __any(cnt > 6), any8 = __any(cnt > 8);
 #pragma unroll
         for (int s = 0; s < kIncWidth; s++) {
-            saj[s] = 0.; shf0[s] = 0.; shf1[s] = 0.;
+            saj[s] = 0.; shf[s] = {};
             if (s < 6 || (s < 8 ? any6 : any8)) {
                 const int q = min(q0 + s, a.nslot - 1);
                 saj[s] = a.slot_aj4[q];
-                shf0[s] = (double)a.hbuf[hl + q];
-                if (NT > 1) shf1[s] = (double)a.hbuf[hl + (size_t)a.nslot + q];
+                shf[s] = hb[q];
             }
         }
         // node column around l (zero outside 1..lmaxk)
@@ -688,14 +806,14 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
             // without a layer below l, [1] with one.  They differ only for a
             // rising flow, whose upstream value [0] is the downstream one: the
             // limiter is zero there and the face takes the centre's value.
-            double vt[2] = {0., 0.};
-            if (l >= 2) {
+            double vt[2];
+            {
                 const double w = wtop;
                 const bool up = w > 0.;
                 double face = up ? c2 : c1;
                 if (btvdv) face = tvd_face(face, up ? c1 : c2, up ? c3 : (l - 2 >= 1 ? c0 : c2), alfa_t);
-                vt[1] = w * face;
-                vt[0] = up ? w * c2 : vt[1];
+                vt[1] = l >= 2 ? w * face : 0.;
+                vt[0] = l >= 2 && up ? w * c2 : vt[1];
             }
             // flux across the bottom interface (none for v = 0): [0] for
             // v = 1, [1] for v = 2, differing in the same way
@@ -717,37 +835,34 @@ __global__ __launch_bounds__(kThreads) void k_conz_node(ConzArgs<S> a) {
 #pragma unroll
         for (int t = 0; t < NT; t++) cn[t] = 0.;
         // One element's terms (whether it has layer l, the next one, the one
-        // after; 4 * area aj4, horizontal terms hf0 and hf1 of tracers 0 and
-        // 1).  A macro rather than a lambda: the lambda's captures stayed in
-        // scratch memory.
-        static_assert(NT <= 2, "two tracers per launch");
-#define CONZ_ADD(has_, deep_, deeper_, aj4_, hf0_, hf1_)                                             \
+        // after; 4 * area, horizontal terms of the tracers).  A position
+        // without the layer (or beyond the list) adds zeros, to sums that are
+        // never -0.: straight line instead of a branch per position.
+        // (A macro rather than a lambda: the lambda's captures stayed in scratch
+        // memory.)
+#define CONZ_ADD(has_, deep_, deeper_, aj4_, hf_)                                                   \
     do {                                                                                           \
-        if (has_) {                                                                                \
-            const double aj4 = (aj4_), hfv[2] = {(hf0_), (hf1_)};                                  \
-            const bool deep = (deep_), deeper = (deeper_); /* v >= 1, v == 2 */                    \
-            _Pragma("unroll") for (int t = 0; t < NT; t++) {                                       \
-                const double fw = deeper ? fw2[t] : (deep ? fw1[t] : fw0[t]);                      \
-                const double fd = deep ? fd1[t] : fd0[t];                                          \
-                const double cexpl = aj4 * (hoc * ckw[t][2] + dt * (hfn + hfv[t] - fw - fd));      \
-                cn[t] += cexpl;                                                                    \
-            }                                                                                      \
-            clo += aj4 * dt * clm;                                                                 \
-            chi += aj4 * dt * (deep ? clpv[1] : clpv[0]);                                          \
-            cd += aj4 * dt * (deep ? clcv[1] : clcv[0]) + aj4 * (1. + dt * 0.) * hnc;              \
+        const bool has = (has_), deep = (deep_), deeper = (deeper_); /* layer, v >= 1, v == 2 */    \
+        const double aj4 = has ? (aj4_) : 0.;                                                       \
+        const Terms<S, NT> hf = (hf_);                                                              \
+        _Pragma("unroll") for (int t = 0; t < NT; t++) {                                           \
+            const double fw = deeper ? fw2[t] : (deep ? fw1[t] : fw0[t]);                          \
+            const double fd = deep ? fd1[t] : fd0[t];                                              \
+            cn[t] += aj4 * (hoc * ckw[t][2] + dt * (hfn + (has ? (double)hf.t[t] : 0.) - fw - fd)); \
         }                                                                                          \
+        clo += aj4 * dt * clm;                                                                     \
+        chi += aj4 * dt * (deep ? clpv[1] : clpv[0]);                                              \
+        cd += aj4 * dt * (deep ? clcv[1] : clcv[0]) + aj4 * (1. + dt * 0.) * hnc;                  \
     } while (0)
-        // (a position beyond the list has no layer)
         const unsigned reach = (unsigned)ent.z;
 #pragma unroll
         for (int s = 0; s < kIncWidth; s++)
             if (s < 6 || (s < 8 ? any6 : any8))
                 CONZ_ADD((reach >> s) & 1u, (reach >> (kIncWidth + s)) & 1u, (reach >> (2 * kIncWidth + s)) & 1u, saj[s],
-                         shf0[s], shf1[s]);
+                         shf[s]);
         for (int q = q0 + kIncWidth; q < q0 + cnt; q++) {
             const int ilev = a.slot_lev[q];
-            CONZ_ADD(ilev >= l, ilev > l, ilev > l + 1, a.slot_aj4[q], (double)a.hbuf[hl + q],
-                     NT > 1 ? (double)a.hbuf[hl + (size_t)a.nslot + q] : 0.);
+            if (ilev >= l) CONZ_ADD(true, ilev > l, ilev > l + 1, a.slot_aj4[q], hb[q]);
         }
 #undef CONZ_ADD
         // conz3d_nodes: boundary mass flux
@@ -875,6 +990,8 @@ static int conz_t(Model &M, const TracerSet &ts, int istot, int isact, hipStream
         HIPCHK(M, hipGetLastError());
         if (a.wdif) launch_timed(M, T_CONZ_ELEM, k_conz_elem<S, NT, true, true>, dim3(ge), dim3(kThreads), 0, st, a);
         else launch_timed(M, T_CONZ_ELEM, k_conz_elem<S, NT, true, false>, dim3(ge), dim3(kThreads), 0, st, a);
+    } else if (a.uoff) {
+        launch_timed(M, T_CONZ_ELEM, k_conz_elem_lds<S, NT>, dim3(ge), dim3(kThreads), 0, st, a);
     } else {
         if (a.wdif) launch_timed(M, T_CONZ_ELEM, k_conz_elem<S, NT, false, true>, dim3(ge), dim3(kThreads), 0, st, a);
         else launch_timed(M, T_CONZ_ELEM, k_conz_elem<S, NT, false, false>, dim3(ge), dim3(kThreads), 0, st, a);
@@ -906,9 +1023,14 @@ static ConzArgs<S> conz_args(Model &M, const TracerSet &ts, int istot, int isact
     a.nen3v = M.m.nen3v; a.ilhv = M.m.ilhv; a.ilhkv = M.m.ilhkv; a.iextb = M.m.iextb; a.ibnd = M.m.ibnd;
     a.geo = M.m.geo; a.dis = M.m.dis;
     a.nkc_ptr = M.m.nk_ptr; a.nkc_el = M.m.nkc_el;
-    a.slot_of = M.m.slot_of; a.slot_lev = M.m.slot_lev; a.slot_aj4 = M.m.slot_aj4; a.nslot = 3 * M.nel;
-    a.tvd_el = M.m.tvd_el; a.tvd_kn = M.m.tvd_kn; a.tvd_w = (const double *)M.m.tvd_w;
-    a.tvd_lev = M.m.tvd_lev; a.elem_iext = M.m.elem_iext;
+    a.ek = (const int4 *)M.m.conz_ek; a.ep = (const int4 *)M.m.conz_ep;
+    a.slot_lev = M.m.slot_lev; a.slot_aj4 = M.m.slot_aj4; a.nslot = 3 * M.nel;
+    a.tvd_up = (const int4 *)M.m.tvd_up; a.tvd_w = (const double2 *)M.m.tvd_w;
+    a.tvd_w2 = M.m.tvd_w ? M.m.tvd_w + 12 * (size_t)M.nel : nullptr;
+    a.elem_iext = M.m.elem_iext;
+    if (M.p.itvd == 2 && !(M.p.rkpar > 0.f) && M.m.conz_uoff) {
+        a.uoff = M.m.conz_uoff; a.uptr = M.m.conz_uptr; a.uvert = M.m.conz_uvert; a.upair = M.m.conz_upair;
+    }
     a.utn = (const S *)M.s.utn; a.vtn = (const S *)M.s.vtn; a.uto = (const S *)M.s.uto; a.vto = (const S *)M.s.vto;
     a.uln = (const S *)M.s.uln; a.vln = (const S *)M.s.vln;
     a.hdkn = (const S *)M.s.hdkn; a.hdko = (const S *)M.s.hdko; a.hden = (const S *)M.s.hden;
@@ -953,14 +1075,19 @@ static ConzArgs<S> conz_args(Model &M, const TracerSet &ts, int istot, int isact
     a.inc_cnt = M.m.inc_cnt; a.inc_el = M.m.inc_el; a.nk_el = M.m.nk_el;
     // the node gradients follow the element terms in the same buffer
     a.grad = (M.p.itvd == 1 && hbuf) ? (S *)hbuf + conz_hbuf_terms(M, ts.n) : nullptr;
-    a.rec_i = (int *)rec;
-    a.rec_d = rec ? (double *)((char *)rec + conz_rec_bytes(M.m.n_eitem) -
-                               (size_t)RD_N * M.m.n_eitem * sizeof(double))
-                  : nullptr;
+    if (rec) {
+        a.rec_code = (int *)rec;
+        a.rec_pair = (uint2 *)((char *)rec + conz_rec_code_bytes(M.m.n_eitem));
+        a.rec_f = (double *)(a.rec_pair + M.m.n_eitem);
+        a.rec_s = (S *)(a.rec_f + 3 * (size_t)M.m.n_eitem);
+    }
     return a;
 }
 
-size_t conz_record_bytes(const Model &M) { return conz_rec_bytes(M.m.n_eitem); }
+size_t conz_record_bytes(const Model &M) {
+    const size_t n = M.m.n_eitem;
+    return conz_rec_code_bytes(M.m.n_eitem) + n * sizeof(uint2) + RF_N * n * sizeof(double) + (size_t)RS_N * n * M.esize();
+}
 
 size_t conz_hbuf_terms(const Model &M, int ntr) { return (size_t)ntr * 3 * M.nlvdi * M.nel; }
 size_t conz_hbuf_elems(const Model &M, int ntr) {

@@ -32,6 +32,7 @@ constexpr int kIncWidth = 10;                        // incident elements per no
 // nodes (one work-item each) and kNodeItems node-layers (one pass of a
 // workgroup)
 constexpr int kConzChunk = 64;
+constexpr int kConzUniq = 1024;
 constexpr int kNodeTileMax = kThreads;
 constexpr int kNodeItems = kThreads;
 constexpr int kNodeCntMax = 63;                      // list lengths from here on are read from the list
@@ -57,11 +58,12 @@ struct Mesh {                 // device copies of init-time data
     // 0, a valid element), and the list lengths, so that a node's element
     // loads can all be issued at once
     int *inc_cnt = nullptr, *inc_el = nullptr, *inc_elc = nullptr;
-    // positions of the colour-order lists (nk_ptr / nkc_el): the position of
-    // vertex ii of element ie ([ii][ie]), and each position's element bottom
-    // layer and 4 * area (the conz3d element terms are stored by position, so
-    // a node reads its incident elements' terms contiguously)
-    int *slot_of = nullptr, *slot_lev = nullptr;
+    // positions of the colour-order lists (nk_ptr / nkc_el): per element its
+    // vertices and their positions (int4 each, three used), and each
+    // position's element bottom layer and 4 * area (the conz3d element terms
+    // are stored by position, so a node reads its incident elements' terms
+    // contiguously)
+    int *conz_ek = nullptr, *conz_ep = nullptr, *slot_lev = nullptr;
     double *slot_aj4 = nullptr;
     int *rowptr = nullptr, *cols = nullptr, *ijp = nullptr;   // zeta CSR; ijp[ie*9+i*3+j]
     int *bnd_nodes = nullptr; int *bnd_id = nullptr; int nbnd_nodes = 0;
@@ -106,10 +108,16 @@ struct Mesh {                 // device copies of init-time data
     int *fwd_rows = nullptr, *fwd_lptr = nullptr, *fwd_nlev = nullptr;
     int *bwd_rows = nullptr, *bwd_lptr = nullptr, *bwd_nlev = nullptr;
     // TVD upwind tables: per element 6 ordered pairs (ic,id); [p*nel + ie]
-    int *tvd_el = nullptr;    // upwind element or -1
-    int *tvd_kn = nullptr;    // [3][6][nel] its nodes
-    void *tvd_w = nullptr;    // double [3][6][nel] interpolation weights (adjusted xi)
-    int *tvd_lev = nullptr;   // [6][nel] bottom layer of the upwind element (0 if none)
+    int *tvd_up = nullptr;    // int4: the upwind element's nodes and bottom layer (0 if there is none)
+    double *tvd_w = nullptr;  // its interpolation weights (adjusted xi): double2 [6][nel], then double [6][nel]
+    // the node-layers that each kThreads entries of conz_eitem read, as
+    // offsets (l-1)*nkn + k in ascending order, with the starts of the lists;
+    // and per entry its vertices' places in its list (10 bits each) and, per
+    // ordered pair ([6][n_eitem]), the upwind nodes' places (bit 30: there is
+    // an upwind point in the layer).  Null where a list would exceed
+    // kConzUniq (elements numbered without locality).
+    int *conz_uoff = nullptr, *conz_uptr = nullptr;
+    unsigned *conz_uvert = nullptr, *conz_upair = nullptr;
     int *elem_iext = nullptr; // [nel] vertices of the element flagged external (iextb)
     // conz3d work division (set_basin): the element-layer list, ie << 5 |
     // (l - 1), in chunks of kConzChunk elements taken layer by layer; node
