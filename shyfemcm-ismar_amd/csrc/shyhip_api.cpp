@@ -426,7 +426,7 @@ int shyhip_destroy(shyhip_model *h) {
                     (void *)m.bwd_lptr, (void *)m.bwd_nlev, (void *)m.tvd_up, (void *)m.tvd_w,
                     (void *)m.conz_uoff, (void *)m.conz_uptr, (void *)m.conz_uvert, (void *)m.conz_upair,
                     (void *)m.elem_iext, (void *)m.conz_eitem, (void *)m.conz_ntile, (void *)m.conz_nitem,
-                    (void *)m.conz_nent, (void *)m.conz_nplace})
+                    (void *)m.conz_nent, (void *)m.conz_nplace, (void *)m.h_tile, (void *)m.h_ent, (void *)m.h_place})
         dfree(q);
     Solver &v = M.sv;
     for (void *q : {v.lu, v.ell_a, v.fs_val, v.r0, v.r, v.p0, v.p1, v.v0, v.v1, v.s, v.t, v.dx, v.b, v.x0, (void *)v.part,
@@ -769,6 +769,39 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         });
         rc |= dalloc(M, &m.conz_nent, ent.size()) || upload(M, m.conz_nent, ent.data(), ent.size());
         rc |= dalloc(M, &m.conz_nplace, place.size()) || upload(M, m.conz_nplace, place.data(), place.size());
+    }
+    if (M.nlv > 1) {
+        std::vector<int> tiles{0}, place(nel);
+        int cnt = 0, next = 0;
+        for (int ie = 0; ie < nel; ie++) {
+            if (cnt == kThreads || next + ilhv[ie] > kThreads) {
+                tiles.push_back(ie);
+                cnt = next = 0;
+            }
+            place[ie] = next;
+            cnt++;
+            next += ilhv[ie];
+        }
+        tiles.push_back(nel);
+        m.n_htile = (int)tiles.size() - 1;
+        std::vector<int> ent((size_t)m.n_htile * kThreads * 2, -1);
+        parallel_for(m.n_htile, 64, [&](int t_begin, int t_end) {
+            for (int t = t_begin; t < t_end; t++) {
+                int lmax = 0;
+                for (int ie = tiles[t]; ie < tiles[t + 1]; ie++) lmax = std::max(lmax, ilhv[ie]);
+                int *e = &ent[(size_t)t * kThreads * 2];
+                for (int l = 1; l <= lmax; l++)
+                    for (int ie = tiles[t]; ie < tiles[t + 1]; ie++) {
+                        if (ilhv[ie] < l) continue;
+                        e[0] = (l - 1) | (ilhv[ie] - 1) << 5 | (place[ie] + l - 1) << 10;
+                        e[1] = ie;
+                        e += 2;
+                    }
+            }
+        });
+        rc |= dalloc(M, &m.h_tile, tiles.size()) || upload(M, m.h_tile, tiles.data(), tiles.size());
+        rc |= dalloc(M, &m.h_ent, ent.size()) || upload(M, m.h_ent, ent.data(), ent.size());
+        rc |= dalloc(M, &m.h_place, place.size()) || upload(M, m.h_place, place.data(), place.size());
     }
     // CSR pattern
     rc |= dalloc(M, &m.rowptr, nkn + 1) || upload(M, m.rowptr, M.h_rowptr.data(), nkn + 1);

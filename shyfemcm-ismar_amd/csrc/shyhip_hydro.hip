@@ -59,6 +59,9 @@ struct HydroArgs {
     int sv_have_prev;
     int *sv_ctrl;
     int *err;
+    // hydro_intern's element tiles (see Mesh)
+    const int *h_tile, *h_place;
+    const int2 *h_ent;
 };
 
 template <typename S>
@@ -94,6 +97,7 @@ static HydroArgs<S> make_args(Model &M) {
     a.utfix = (const S *)M.s.utfix; a.vtfix = (const S *)M.s.vtfix;
     a.zel = M.s.zel; a.aval = M.s.aval; a.rhs = M.s.rhs; a.x = M.s.x;
     a.err = M.d_err;
+    a.h_tile = M.m.h_tile; a.h_place = M.m.h_place; a.h_ent = (const int2 *)M.m.h_ent;
     return a;
 }
 
@@ -141,6 +145,86 @@ __device__ inline S friction(const HydroArgs<S> &a, int ie, int lmax) {
 }
 
 // ------------------------------------------------------------------ hydro_intern
+// what a column's elimination takes from the element
+template <typename S>
+struct InternElem {
+    using R = S;
+    R dt, at, grav, rowass, gammat, rfric;
+    int ilevel, kn[3];
+    double b[3], c[3];
+    double bz, cz, zmm, taux, tauy, bpres, cpres;
+
+    // (the wind stress only where top, the friction where bottom)
+    __device__ void load(const HydroArgs<S> &a, int ie, int lmax, bool top, bool bottom) {
+        const int nel = a.nel;
+        dt = (R)a.dt; at = (R)a.at; grav = (R)a.grav; rowass = (R)a.rowass;
+        ilevel = lmax;
+        bz = cz = zmm = taux = tauy = bpres = cpres = 0.;
+        for (int ii = 0; ii < 3; ii++) kn[ii] = a.nen3v[3 * ie + ii];
+        for (int ii = 0; ii < 3; ii++) {
+            b[ii] = a.geo[(size_t)ii * nel + ie];
+            c[ii] = a.geo[(size_t)(3 + ii) * nel + ie];
+            const R ze = a.zeo[(size_t)ii * nel + ie];
+            // the level relative to the equilibrium tide, and the atmospheric
+            // pressure gradient (hydrodynamic.f90:1025-1033)
+            const double zz = (double)(a.zeqv ? (R)(ze - a.zeqv[kn[ii]]) : ze);
+            zmm += (double)ze;
+            bz += zz * b[ii];
+            cz += zz * c[ii];
+            if (a.ppv) {
+                bpres += (double)a.ppv[kn[ii]] * b[ii];
+                cpres += (double)a.ppv[kn[ii]] * c[ii];
+            }
+            if (top) {
+                taux += (double)a.taux[kn[ii]];
+                tauy += (double)a.tauy[kn[ii]];
+            }
+        }
+        zmm = zmm * kDrittl;
+        taux = taux * kDrittl;
+        tauy = tauy * kDrittl;
+        gammat = a.fcorv[ie];
+        rfric = bottom ? friction(a, ie, ilevel) : (R)0;
+    }
+
+    // layer l of the decoupled columns: diagonal d, off-diagonals lo (above)
+    // and up (below), right-hand sides ppx and ppy, from the transports u, v
+    // and thicknesses h of the layers above (m), at (i) and below (p), the
+    // inverse thicknesses rh and the interface viscosities al (below) and
+    // alm (above); the right-hand sides without the wind stress and the
+    // explicit terms, which rhs() adds
+    __device__ void row(bool first, bool last, R uui, R uuip, R uuim, R vvi, R vvip, R vvim, R hhi, R hhip, R hhim,
+                        R rhi, R rhip, R rhim, R al, R alm, double &d, double &lo, double &up, R &ppx, R &ppy) const {
+        R rhp = 0, rhm = 0;
+        if (hhi > (R)0) {
+            if (hhip > (R)0) rhp = (R)2.0 * al / (hhi + hhip);
+            if (hhim > (R)0) rhm = (R)2.0 * alm / (hhi + hhim);
+        }
+        const R aux = dt * at;
+        R aa = aux * rhi * (rhm + rhp);
+        R aat = (R)1 * rhi * (rhm + rhp);
+        const R bb = aux * rhip * rhp;
+        const R bbt = (R)1 * rhip * rhp;
+        const R cc = aux * rhim * rhm;
+        const R cct = (R)1 * rhim * rhm;
+        if (last) { aa = aa + dt * rfric; aat = aat + rfric; }
+        const R gravx = (R)(1.0 * grav * hhi * bz);
+        const R gravy = (R)(1.0 * grav * hhi * cz);
+        const R presx = (R)bpres, presy = (R)cpres;
+        ppx = aat * uui - bbt * uuip - cct * uuim - gammat * vvi + gravx + (hhi / rowass) * presx;
+        ppy = aat * vvi - bbt * vvip - cct * vvim + gammat * uui + gravy + (hhi / rowass) * presy;
+        d = (double)((R)1 + aa);
+        up = last ? 0.0 : (double)(-bb);
+        lo = first ? 0.0 : (double)(-cc);
+    }
+
+    __device__ static double rhs(bool first, double tau, R pp, R expl) {
+        double p = 0.;
+        if (first) p = p - tau;
+        return p + (double)(R)(pp + expl);
+    }
+};
+
 // hydro_transports / hydro_intern, hydrodynamic.f90:758-1416.  One work-item
 // per element column.  Without Coriolis (gamma = 0) the 2L x 2L pentadiagonal
 // system decouples into two identical tridiagonal systems in u and v; the
@@ -153,35 +237,13 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
     const int ie = blockIdx.x * blockDim.x + threadIdx.x;
     if (ie >= a.nel) return;
     const int nel = a.nel, nkn = a.nkn;
-    const R dt = (R)a.dt, af = (R)a.af, at = (R)a.at, grav = (R)a.grav, rowass = (R)a.rowass;
-    const int ilevel = a.ilhv[ie];
-    const int k1 = a.nen3v[3 * ie], k2 = a.nen3v[3 * ie + 1], k3 = a.nen3v[3 * ie + 2];
-    const int kn[3] = {k1, k2, k3};
-    double b[3], c[3];
-    double bz = 0., cz = 0., zmm = 0., taux = 0., tauy = 0., bpres = 0., cpres = 0.;
-    for (int ii = 0; ii < 3; ii++) {
-        b[ii] = a.geo[(size_t)ii * nel + ie];
-        c[ii] = a.geo[(size_t)(3 + ii) * nel + ie];
-        const R ze = a.zeo[(size_t)ii * nel + ie];
-        // the level relative to the equilibrium tide, and the atmospheric
-        // pressure gradient (hydrodynamic.f90:1025-1033)
-        const double zz = (double)(a.zeqv ? (R)(ze - a.zeqv[kn[ii]]) : ze);
-        zmm += (double)ze;
-        bz += zz * b[ii];
-        cz += zz * c[ii];
-        if (a.ppv) {
-            bpres += (double)a.ppv[kn[ii]] * b[ii];
-            cpres += (double)a.ppv[kn[ii]] * c[ii];
-        }
-        taux += (double)a.taux[kn[ii]];
-        tauy += (double)a.tauy[kn[ii]];
-    }
-    zmm = zmm * kDrittl;
-    taux = taux * kDrittl;
-    tauy = tauy * kDrittl;
-    const R gammat = a.fcorv[ie];
+    InternElem<S> e;
+    e.load(a, ie, a.ilhv[ie], true, true);
+    const R dt = e.dt, af = (R)a.af, at = e.at, grav = e.grav, rowass = e.rowass, gammat = e.gammat, rfric = e.rfric;
+    const int ilevel = e.ilevel, k1 = e.kn[0], k2 = e.kn[1], k3 = e.kn[2];
+    const double(&b)[3] = e.b, (&c)[3] = e.c;
+    const double bz = e.bz, cz = e.cz, zmm = e.zmm, taux = e.taux, tauy = e.tauy, bpres = e.bpres, cpres = e.cpres;
     const R gamma = af * dt * gammat;
-    const R rfric = friction(a, ie, ilevel);
     a.rfric[ie] = rfric;
 
     // layer thickness, inverse thickness, element viscosity
@@ -274,32 +336,12 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
             const R uuim = l > 1 ? uoc[l > 1 ? l - 2 : 0] : uoc[0];
             const R vvi = voc[l - 1], vvip = below ? voc[l < NL ? l : l - 1] : voc[l - 1];
             const R vvim = l > 1 ? voc[l > 1 ? l - 2 : 0] : voc[0];
-            const R hhi = hact[l], hhip = hact[l + 1], hhim = hact[l - 1];
-            R rhp = 0, rhm = 0;
-            if (hhi > (R)0) {
-                if (hhip > (R)0) rhp = (R)2.0 * alev[l] / (hhi + hhip);
-                if (hhim > (R)0) rhm = (R)2.0 * alev[l - 1] / (hhi + hhim);
-            }
-            const R aux = dt * at;
-            R aa = aux * rhact[l] * (rhm + rhp);
-            R aat = (R)1 * rhact[l] * (rhm + rhp);
-            const R bb = aux * rhact[l + 1] * rhp;
-            const R bbt = (R)1 * rhact[l + 1] * rhp;
-            const R cc = aux * rhact[l - 1] * rhm;
-            const R cct = (R)1 * rhact[l - 1] * rhm;
-            double ppx = 0., ppy = 0.;
-            if (bfirst) { ppx = ppx - taux; ppy = ppy - tauy; }
-            if (blast) { aa = aa + dt * rfric; aat = aat + rfric; }
-            const R gravx = (R)(1.0 * grav * hhi * bz);
-            const R gravy = (R)(1.0 * grav * hhi * cz);
-            const R presx = (R)bpres, presy = (R)cpres, xexpl = xex[l - 1], yexpl = yex[l - 1];
-            const R ppx_aux = aat * uui - bbt * uuip - cct * uuim - gammat * vvi + gravx + (hhi / rowass) * presx + xexpl;
-            const R ppy_aux = aat * vvi - bbt * vvip - cct * vvim + gammat * uui + gravy + (hhi / rowass) * presy + yexpl;
-            ppx = ppx + (double)ppx_aux;
-            ppy = ppy + (double)ppy_aux;
-            const double d = (double)((R)1 + aa);
-            up[l - 1] = blast ? 0.0 : (double)(-bb);
-            const double lo = bfirst ? 0.0 : (double)(-cc);
+            double d, lo;
+            R rx, ry;
+            e.row(bfirst, blast, uui, uuip, uuim, vvi, vvip, vvim, hact[l], hact[l + 1], hact[l - 1], rhact[l],
+                  rhact[l + 1], rhact[l - 1], alev[l], alev[l - 1], d, lo, up[l - 1], rx, ry);
+            const double ppx = e.rhs(bfirst, taux, rx, xex[l - 1]), ppy = e.rhs(bfirst, tauy, ry, yex[l - 1]);
+            const R hhi = hact[l];
             if (l == 1) {
                 xd[0] = d;
                 gx[0] = ppx;
@@ -465,6 +507,165 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
     const double az = (double)a.az;
     a.zel[(size_t)4 * nel + ie] = az * uhat + (1. - az) * uold;
     a.zel[(size_t)5 * nel + ie] = az * vhat + (1. - az) * vold;
+}
+
+// The same without Coriolis for columns of several layers.  One workgroup per
+// tile of consecutive elements (Mesh::h_tile; at most kThreads elements and
+// element-layers).  Phase 1, one work-item per element-layer: the layer's row
+// of the tridiagonal system, into LDS.  Phase 2, one work-item per element:
+// the elimination and the column's sums.  Phase 3, one work-item per
+// element-layer: the results.
+//
+// What bounds it: the loads of the layers' rows (about 35 a work-item).  One
+// work-item per column, its layers unrolled in registers, walked every
+// wavefront down to the deepest layer of the basin, one wavefront to a SIMD
+// from 16 layers on: 489 us on 300k nodes of 20 layers, 14.6 on 3k nodes of
+// 10 (FP64) against 184 and 8.8; equal (28 to 30 us) on 50k nodes of 12.
+// The rows in scratch memory with rolled loops took 337 us, the columns split
+// by depth between two kernels 331.
+template <typename S>
+__global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) {
+    using R = S;
+    // by place in the tile (element after element, top down): the row's
+    // diagonals, right-hand sides and thickness, which the elimination
+    // replaces by the solutions; old transports (then new ones); density
+    // gradients; and per element the wind stress
+    __shared__ double dL[kThreads], loL[kThreads], upL[kThreads], pxL[kThreads], pyL[kThreads], hL[kThreads];
+    __shared__ double brL[kThreads], crL[kThreads], txL[kThreads], tyL[kThreads];
+    __shared__ R uL[kThreads], vL[kThreads];
+    const int nel = a.nel, nkn = a.nkn;
+    const int tile = xcd_block();
+    const int2 ent = a.h_ent[(size_t)tile * kThreads + threadIdx.x];
+    const int e0 = a.h_tile[tile], tn = a.h_tile[tile + 1] - e0;
+    const bool on = ent.x >= 0;
+    const int ie = on ? ent.y : 0, l = (ent.x & 31) + 1, ilevel = ((ent.x >> 5) & 31) + 1, it = (ent.x >> 10) & 255;
+    const size_t o = (size_t)(l - 1) * nel + ie;
+    if (on) {
+        const bool first = l == 1, last = l == ilevel;
+        // the layer above and below (its own at the column's ends)
+        const size_t om = first ? o : o - nel, op = last ? o : o + nel;
+        R h = a.hdeo[o], hm = a.hdeo[om], hp = a.hdeo[op];
+        const R u = a.uto[o], um = a.uto[om], up = a.uto[op], v = a.vto[o], vm = a.vto[om], vp = a.vto[op];
+        InternElem<S> e;
+        e.load(a, ie, ilevel, first, last);
+        const size_t ob = (size_t)l * nkn, ot = ob - nkn;
+        const R vb = a.visv[ob + e.kn[0]] + a.visv[ob + e.kn[1]] + a.visv[ob + e.kn[2]];
+        const R vt = a.visv[ot + e.kn[0]] + a.visv[ot + e.kn[1]] + a.visv[ot + e.kn[2]];
+        if (last) a.rfric[ie] = e.rfric;
+        hm = first ? (R)0 : hm;
+        hp = last ? (R)0 : hp;
+        if (a.iclin) {
+            if (first) h = (R)(h - e.zmm);
+            if (l == 2) hm = (R)(hm - e.zmm);
+        }
+        auto inverse = [](R x) { return (x <= (R)0) ? (R)0 : (R)1 / x; };
+        auto viscosity = [&](R sum) { return (R)((double)a.vismol + (double)(sum / (R)3)); };
+        double d, lo, upp;
+        R rx, ry;
+        e.row(first, last, u, up, um, v, vp, vm, h, hp, hm, inverse(h), inverse(hp), inverse(hm), viscosity(vb),
+              viscosity(vt), d, lo, upp, rx, ry);
+        dL[it] = d; loL[it] = lo; upL[it] = upp; hL[it] = (double)h;
+        uL[it] = u; vL[it] = v;
+        if (a.rhov) {
+            // the density gradient; the pressure gradient is its integral
+            // down the column
+            double br = 0., cr = 0.;
+#pragma unroll
+            for (int ii = 0; ii < 3; ii++) {
+                const double r = (double)a.rhov[ot + e.kn[ii]];
+                br = br + e.b[ii] * r;
+                cr = cr + e.c[ii] * r;
+            }
+            brL[it] = br; crL[it] = cr;
+            pxL[it] = (double)rx; pyL[it] = (double)ry;
+            if (first) { txL[ie - e0] = e.taux; tyL[ie - e0] = e.tauy; }
+        } else {
+            pxL[it] = e.rhs(first, e.taux, rx, (R)0);
+            pyL[it] = e.rhs(first, e.tauy, ry, (R)0);
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < tn) {
+        const int ec = e0 + threadIdx.x, n = a.ilhv[ec], p0 = a.h_place[ec];
+        // the baroclinic pressure gradient integrated down (see k_hydro_intern)
+        const double raux = (double)((R)a.grav / (R)a.rowass);
+        double px = 0., py = 0., brup = 0., crup = 0., hhup = 0.;
+        double xp = 0., upp = 0., gxp = 0., gyp = 0., ghp = 0.;
+        for (int m = 0; m < n; m++) {
+            const int i = p0 + m;
+            double x = dL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
+            const double lo = loL[i], up = upL[i];
+            if (a.rhov) {
+                const double hlayer = (double)a.hldv[m];
+                const double hh = 0.5 * hlayer;
+                const double hint = hh + hhup;
+                const double br = brL[i], cr = crL[i];
+                const double brint = m == 0 ? br : 0.5 * (br + brup);
+                const double crint = m == 0 ? cr : 0.5 * (cr + crup);
+                brup = br;
+                crup = cr;
+                hhup = hh;
+                px = px + hint * brint;
+                py = py + hint * crint;
+                gx = InternElem<S>::rhs(m == 0, txL[threadIdx.x], (R)gx, (R)(0.0 + raux * hlayer * px));
+                gy = InternElem<S>::rhs(m == 0, tyL[threadIdx.x], (R)gy, (R)(0.0 + raux * hlayer * py));
+            }
+            if (m > 0) {
+                const double w = lo / xp;
+                x = x - w * upp;
+                gx = gx - w * gxp;
+                gy = gy - w * gyp;
+                gh = gh - w * ghp;
+            }
+            dL[i] = x; pxL[i] = gx; pyL[i] = gy; hL[i] = gh;
+            xp = x; upp = up; gxp = gx; gyp = gy; ghp = gh;
+        }
+        double su = 0., sv = 0., sh = 0.;
+        for (int m = n - 1; m >= 0; m--) {
+            const int i = p0 + m;
+            const double x = dL[i], up = upL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
+            const bool last = m == n - 1;
+            su = (last ? gx : gx - up * su) / x;
+            sv = (last ? gy : gy - up * sv) / x;
+            sh = (last ? gh : gh - up * sh) / x;
+            pxL[i] = su; pyL[i] = sv; hL[i] = sh;
+        }
+        // u^hat = u_old - dt * A^-1 F (or the fixed transports) and the sums
+        const int afix = a.iuvfix ? 1 - a.iuvfix[ec] : 1;
+        const R dtafix = (R)a.dt * (R)afix;
+        double uold = 0., vold = 0., uhat = 0., vhat = 0., dsum = 0.;
+        for (int m = 0; m < n; m++) {
+            const int i = p0 + m;
+            const size_t oc = (size_t)m * nel + ec;
+            const R uo = uL[i], vo = vL[i];
+            S unew, vnew;
+            if (afix != 0) {
+                unew = (S)((double)uo - (double)dtafix * pxL[i]);
+                vnew = (S)((double)vo - (double)dtafix * pyL[i]);
+            } else {
+                unew = a.utfix ? a.utfix[oc] : uo;
+                vnew = a.vtfix ? a.vtfix[oc] : vo;
+            }
+            uL[i] = unew; vL[i] = vnew;
+            uold += (double)uo; vold += (double)vo;
+            uhat += (double)unew; vhat += (double)vnew;
+            dsum += hL[i];
+        }
+        a.zel[(size_t)0 * nel + ec] = dsum;
+        a.zel[(size_t)1 * nel + ec] = 0.;
+        a.zel[(size_t)2 * nel + ec] = 0.;
+        a.zel[(size_t)3 * nel + ec] = dsum;
+        const double az = (double)a.az;
+        a.zel[(size_t)4 * nel + ec] = az * uhat + (1. - az) * uold;
+        a.zel[(size_t)5 * nel + ec] = az * vhat + (1. - az) * vold;
+    }
+    __syncthreads();
+    if (!on) return;
+    // the cross terms ddx(jv), ddy(ju) stay zero (never written on this path)
+    a.utn[o] = uL[it];
+    a.vtn[o] = vL[it];
+    a.ddx[(size_t)(2 * l - 2) * nel + ie] = (S)hL[it];
+    a.ddy[(size_t)(2 * l - 1) * nel + ie] = (S)hL[it];
 }
 
 // ------------------------------------------------------------------ hydro_zeta
@@ -1053,15 +1254,9 @@ __global__ __launch_bounds__(kThreads) void k_setdepth_node(HydroArgs<S> a, cons
 // workgroup per tile of consecutive nodes: one work-item per node-layer
 // gathers the incident elements (element order, the reference's scatter
 // order) into LDS, then one work-item per node integrates its column.
-template <int NL>
-struct VertTile {
-    static constexpr int TN = NL <= 16 ? 64 : 32;
-};
-
-template <typename S, int NL>
+template <typename S, int NL, int TN>
 __global__ __launch_bounds__(kThreads) void k_hydro_vertical(HydroArgs<S> a) {
     using R = S;
-    constexpr int TN = VertTile<NL>::TN;
     __shared__ R vfL[NL][TN], vaL[NL][TN], dvL[NL][TN];
     const int nel = a.nel, nkn = a.nkn, nlvdi = a.nlvdi;
     const int k0 = xcd_block() * TN;
@@ -1382,7 +1577,8 @@ template <typename S, int NL>
 static int hydro_intern_nl(Model &M) {
     auto a = make_args<S>(M);
     if (M.has_coriolis) LAUNCH(M, (k_hydro_intern<S, NL, true>), nblocks(M.nel), a);
-    else LAUNCH(M, (k_hydro_intern<S, NL, false>), nblocks(M.nel), a);
+    else if constexpr (NL == 1) LAUNCH(M, (k_hydro_intern<S, NL, false>), nblocks(M.nel), a);
+    else LAUNCH(M, k_hydro_intern_tile<S>, M.m.n_htile, a);
     return 0;
 }
 template <typename S>
@@ -1491,7 +1687,14 @@ int launch_elem_after_solve(Model &M) {
 template <typename S, int NL>
 static int vertical_nl(Model &M) {
     auto a = make_args<S>(M);
-    LAUNCH(M, (k_hydro_vertical<S, NL>), (M.nkn + VertTile<NL>::TN - 1) / VertTile<NL>::TN, a);
+    // wide tiles where every compute unit gets one: the layers of a shallow
+    // column keep fewer of a tile's work-items busy the narrower it is (300k
+    // nodes of 20 layers, FP64: 171 us with 32 nodes, 122 with 64, 108 with
+    // 128; 50k nodes of 12: 27.9, 21.9, 20.7); 64 is what LDS holds of more
+    // than 20 layers in FP64
+    constexpr int kWide = sizeof(S) * NL <= 160 ? 128 : 64, kNarrow = NL <= 16 ? 64 : 32;
+    if (M.nkn >= 256 * kWide) LAUNCH(M, (k_hydro_vertical<S, NL, kWide>), (M.nkn + kWide - 1) / kWide, a);
+    else LAUNCH(M, (k_hydro_vertical<S, NL, kNarrow>), (M.nkn + kNarrow - 1) / kNarrow, a);
     return 0;
 }
 template <typename S>

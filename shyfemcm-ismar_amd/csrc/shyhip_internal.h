@@ -131,6 +131,13 @@ struct Mesh {                 // device copies of init-time data
     // each, kIncWidth apart), node}, -1 in the first word of unused entries;
     // and each node's first place in its tile (its layers follow one another)
     int *conz_nent = nullptr, *conz_nplace = nullptr;
+    // hydro_intern's element tiles (basins of several layers): first elements
+    // [n_htile + 1], the tiles' element-layers, layer by layer with the
+    // elements ascending in each, [tile*kThreads + i] as int2: {(l-1) |
+    // (lmax-1) << 5 | place << 10, element}, -1 in the first word of unused
+    // entries; and each element's first place in its tile
+    int *h_tile = nullptr, *h_ent = nullptr, *h_place = nullptr;
+    int n_htile = 0;
     // the node-layer list, k << 5 | (l - 1), in chunks of kConzChunk nodes
     // taken layer by layer (scalar_stability)
     int *conz_nitem = nullptr;
