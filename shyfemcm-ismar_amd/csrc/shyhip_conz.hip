@@ -1346,7 +1346,15 @@ __device__ inline void max_into(unsigned long long *p, unsigned long long v) {
 // kStabBatch at a time: each batch's loads are issued together (the list
 // entries, then every element's data and its vertices, then the vertices'
 // vertical velocities), and the batch is then added in order.
-constexpr int kStabBatch = 3;
+//
+// What bounds it: the gathers, so only what a term uses is read: the vertices
+// before this one (the node's own velocities are loaded once), and the layer
+// thicknesses only where the diffusion has an explicit part.  With all of
+// them, three elements at a time and two wavefronts to a SIMD: 191 us on 300k
+// nodes of 20 layers, 36.5 on 50k of 12 (FP64), 134 in FP32 on 285k of 10,
+// against 137, 27 and 93.  Batches of one (141, 26.5, 93; 15.8 on 3k nodes
+// against 13.5) and three (160, 31, 105) lose.
+constexpr int kStabBatch = 2;
 
 template <typename S>
 __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, int nlv, const int *ilhv,
@@ -1368,11 +1376,18 @@ __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, 
     const double dbot = l < nlv ? (double)difv[(size_t)l * nkn + k] : 0.;
     const double hn = (double)hdkn[(size_t)(l - 1) * nkn + k], ho = (double)hdko[(size_t)(l - 1) * nkn + k];
     const double rtau = rtauv ? (double)rtauv[(size_t)(l - 1) * nkn + k] : 0.;
+    // the vertical velocity at the top (at = l - 1) and bottom (at = l) of
+    // node kk's layer, less the tracer's sinking in the tracers' precision
+    auto wvel = [&](int at, int kk) {
+        const size_t o = (size_t)at * nkn + kk;
+        return wsinkv ? (double)(S)(wln[o] - (S)wsink * wsinkv[o]) : (double)wln[o];
+    };
+    const double wtk = l > 1 ? wvel(l - 1, k) : 0., wbk = l < nlv ? wvel(l, k) : 0.;
     const int p0 = nk_ptr[k], p1 = nk_ptr[k + 1];
     for (int pb = p0; pb < p1; pb += kStabBatch) {
-        int ie[kStabBatch], iv[kStabBatch], ilev[kStabBatch], kj[kStabBatch][3];
+        int ie[kStabBatch], iv[kStabBatch], ilev[kStabBatch], kj[kStabBatch][2];
         double aj4[kStabBatch], us[kStabBatch], vs[kStabBatch], hdv[kStabBatch], hdt[kStabBatch], hdb[kStabBatch];
-        double gb[kStabBatch][3], gc[kStabBatch][3], wt[kStabBatch][3], wb[kStabBatch][3];
+        double gb[kStabBatch][3], gc[kStabBatch][3], wt[kStabBatch][2], wb[kStabBatch][2];
         double rk3[kStabBatch], wd[kStabBatch];
 #pragma unroll
         for (int b = 0; b < kStabBatch; b++) {
@@ -1388,9 +1403,12 @@ __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, 
             aj4[b] = 4. * geo[(size_t)6 * nel + el];
             us[b] = az * (double)utn[le] + azt * (double)uto[le];
             vs[b] = az * (double)vtn[le] + azt * (double)vto[le];
-            hdv[b] = (double)hdeo[le];
-            hdt[b] = l > 1 ? (double)hdeo[le - nel] : 0.;
-            hdb[b] = l < nlv ? (double)hdeo[le + nel] : 0.;
+            hdv[b] = hdt[b] = hdb[b] = 1.;
+            if (adt != 0.) {
+                hdv[b] = (double)hdeo[le];
+                hdt[b] = l > 1 ? (double)hdeo[le - nel] : 0.;
+                hdb[b] = l < nlv ? (double)hdeo[le + nel] : 0.;
+            }
             rk3[b] = 0.;
             wd[b] = 0.;
             if (wdif) {
@@ -1401,25 +1419,27 @@ __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, 
             }
 #pragma unroll
             for (int jj = 0; jj < 3; jj++) {
-                kj[b][jj] = nen3v[3 * el + jj];
-                gb[b][jj] = geo[(size_t)jj * nel + el];
-                gc[b][jj] = geo[(size_t)(3 + jj) * nel + el];
+                gb[b][jj] = gc[b][jj] = 0.;
+                if (jj <= iv[b]) {
+                    gb[b][jj] = geo[(size_t)jj * nel + el];
+                    gc[b][jj] = geo[(size_t)(3 + jj) * nel + el];
+                }
+                if (jj < 2) {
+                    kj[b][jj] = k;
+                    if (jj < iv[b]) kj[b][jj] = nen3v[3 * el + jj];
+                }
             }
         }
+        // (the vertices before this one; the node itself has its own)
 #pragma unroll
         for (int b = 0; b < kStabBatch; b++)
 #pragma unroll
-            for (int jj = 0; jj < 3; jj++) {
-                wt[b][jj] = l > 1 ? (double)wln[(size_t)(l - 1) * nkn + kj[b][jj]] : 0.;
-                wb[b][jj] = l < nlv ? (double)wln[(size_t)l * nkn + kj[b][jj]] : 0.;
-                if (wsinkv) {
-                    // less the tracer's sinking, in the tracers' precision
-                    if (l > 1)
-                        wt[b][jj] = (double)(S)(wln[(size_t)(l - 1) * nkn + kj[b][jj]] -
-                                                (S)wsink * wsinkv[(size_t)(l - 1) * nkn + kj[b][jj]]);
-                    if (l < nlv)
-                        wb[b][jj] = (double)(S)(wln[(size_t)l * nkn + kj[b][jj]] -
-                                                (S)wsink * wsinkv[(size_t)l * nkn + kj[b][jj]]);
+            for (int jj = 0; jj < 2; jj++) {
+                wt[b][jj] = wtk;
+                wb[b][jj] = wbk;
+                if (jj < iv[b]) {
+                    if (l > 1) wt[b][jj] = wvel(l - 1, kj[b][jj]);
+                    if (l < nlv) wb[b][jj] = wvel(l, kj[b][jj]);
                 }
             }
 #pragma unroll
@@ -1432,8 +1452,8 @@ __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, 
                 if (jj > iv[b]) break;
                 const double f = us[b] * gb[b][jj] + vs[b] * gc[b][jj];
                 double fwin = 0., fwout = 0.;
-                const double w_t = wt[b][jj];
-                const double w_b = below ? wb[b][jj] : 0.;
+                const double w_t = jj < 2 ? wt[b][jj < 2 ? jj : 0] : wtk;
+                const double w_b = below ? (jj < 2 ? wb[b][jj < 2 ? jj : 0] : wbk) : 0.;
                 if (w_t > 0.) fwout = fwout + aat * w_t;
                 else fwin = fwin - aat * w_t;
                 if (w_b > 0.) fwin = fwin + aat * w_b;
@@ -1445,10 +1465,12 @@ __device__ inline unsigned long long stab_ratio(int l, int k, int nkn, int nel, 
                 cadv = coadv > ciadv ? coadv : ciadv;
             }
             chigh = chigh + cadv;
-            double hmtop = 0., hmbot = 0.;
-            if (l > 1) hmtop = 2. * dtop / (hdt[b] + hdv[b]);
-            if (below) hmbot = 2. * dbot / (hdv[b] + hdb[b]);
-            cn = cn + aj4[b] * (adt * (hmtop + hmbot));
+            if (adt != 0.) {
+                double hmtop = 0., hmbot = 0.;
+                if (l > 1) hmtop = 2. * dtop / (hdt[b] + hdv[b]);
+                if (below) hmbot = 2. * dbot / (hdv[b] + hdb[b]);
+                cn = cn + aj4[b] * (adt * (hmtop + hmbot));
+            }
             clow = clow + aj4[b] * rk3[b] * ho * wd[b];
             if (rtauv) co = co + aj4[b] * ho * (double)robs * rtau;      // nudging
             cdiag = cdiag + aj4[b] * (ho < hn ? ho : hn);
