@@ -1767,6 +1767,26 @@ static int check_dev_err(Model &M, const char *where) {
 static int hydro_impl(Model &M, double dtime, bool final_check) {
     M.dtime = dtime;
     int iloop = 0, changed = 0, its_total = 0;
+    // one element kernel: transports_final, setzev + setuvd + baro2l, the
+    // element depths of make_new_depth, compute_velocities (ulnv/vlnv,
+    // unv/vnv) -- then the node depths (+ check_volume) and hydro_vertical.
+    // Enqueued behind a one-launch solve's report, so that the device does
+    // not wait for the host to read that the loop has settled (20 us a step);
+    // the kernels return when it has not.
+    const std::function<int(const int *)> after = [&](const int *go) {
+        M.after_go = go;
+        timer_begin(M, T_FINAL);
+        int rc = launch_elem_after_solve(M);
+        timer_end(M);
+        timer_begin(M, T_DEPTH);
+        rc = rc || launch_setdepth_node(M);
+        timer_end(M);
+        timer_begin(M, T_VERT);
+        rc = rc || launch_hydro_vertical(M);
+        timer_end(M);
+        M.after_go = nullptr;
+        return rc;
+    };
     timer_begin(M, T_INTERN);
     if (launch_hydro_intern(M)) return 1;          // hydro_transports (invariant over the wet/dry loop)
     timer_end(M);
@@ -1786,7 +1806,8 @@ static int hydro_impl(Model &M, double dtime, bool final_check) {
         const int bnew = M.dtime != M.dtime_old;
         timer_begin(M, T_SOLVE);
         int ref = 0;
-        const int rc = solver_solve(M, &its, &ref, bnew);
+        M.h_pinned[HP_GO] = 0;
+        const int rc = solver_solve(M, &its, &ref, bnew, M.timing ? nullptr : &after);
         M.last_refine = ref;
         timer_end(M);
         its_total += its;
@@ -1798,18 +1819,7 @@ static int hydro_impl(Model &M, double dtime, bool final_check) {
     M.last_nloop = iloop;
     M.last_iters = its_total;
     if (report_dev_err(M, M.h_pinned[0], "hydro loop")) return 3;   // read with the setweg counter
-    // one element kernel: transports_final, setzev + setuvd + baro2l, the
-    // element depths of make_new_depth, compute_velocities (ulnv/vlnv,
-    // unv/vnv) -- then the node depths (+ check_volume) and hydro_vertical
-    timer_begin(M, T_FINAL);
-    if (launch_elem_after_solve(M)) return 1;
-    timer_end(M);
-    timer_begin(M, T_DEPTH);
-    if (launch_setdepth_node(M)) return 1;
-    timer_end(M);
-    timer_begin(M, T_VERT);
-    if (launch_hydro_vertical(M)) return 1;
-    timer_end(M);
+    if (!M.h_pinned[HP_GO] && after(nullptr)) return 1;
     return final_check ? check_dev_err(M, "hydro") : 0;
 }
 

@@ -59,6 +59,7 @@ struct HydroArgs {
     int sv_have_prev;
     int *sv_ctrl;
     int *err;
+    const int *go;          // do nothing unless *go (null: always; see solver_solve)
     // hydro_intern's element tiles (see Mesh)
     const int *h_tile, *h_place;
     const int2 *h_ent;
@@ -97,6 +98,7 @@ static HydroArgs<S> make_args(Model &M) {
     a.utfix = (const S *)M.s.utfix; a.vtfix = (const S *)M.s.vtfix;
     a.zel = M.s.zel; a.aval = M.s.aval; a.rhs = M.s.rhs; a.x = M.s.x;
     a.err = M.d_err;
+    a.go = M.after_go;
     a.h_tile = M.m.h_tile; a.h_place = M.m.h_place; a.h_ent = (const int2 *)M.m.h_ent;
     return a;
 }
@@ -1180,6 +1182,7 @@ __global__ __launch_bounds__(kThreads) void k_setdepth_elem(HydroArgs<S> a, cons
 template <typename S, int NL>
 __global__ __launch_bounds__(kThreads) void k_setdepth_node(HydroArgs<S> a, const S *zen, S *hdkn) {
     using R = S;
+    if (a.go && !*a.go) return;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= a.nkn) return;
     const int nel = a.nel, nkn = a.nkn;
@@ -1257,6 +1260,7 @@ __global__ __launch_bounds__(kThreads) void k_setdepth_node(HydroArgs<S> a, cons
 template <typename S, int NL, int TN>
 __global__ __launch_bounds__(kThreads) void k_hydro_vertical(HydroArgs<S> a) {
     using R = S;
+    if (a.go && !*a.go) return;
     __shared__ R vfL[NL][TN], vaL[NL][TN], dvL[NL][TN];
     const int nel = a.nel, nkn = a.nkn, nlvdi = a.nlvdi;
     const int k0 = xcd_block() * TN;
@@ -1389,6 +1393,7 @@ __global__ __launch_bounds__(kThreads) void k_ttov_uvint(HydroArgs<S> a) {
 // node levels and its own element's data only, in the reference's order.
 template <typename S, bool CORI>
 __global__ __launch_bounds__(kThreads) void k_elem_after_solve(HydroArgs<S> a) {
+    if (a.go && !*a.go) return;
     const int ie = blockIdx.x * blockDim.x + threadIdx.x;
     if (ie >= a.nel) return;
     transports_final_el<S, CORI>(a, ie);

@@ -37,6 +37,8 @@ constexpr int kNodeTileMax = kThreads;
 constexpr int kNodeItems = kThreads;
 constexpr int kNodeCntMax = 63;                      // list lengths from here on are read from the list
 
+// d_err word: the state after a solve has settled (k_report)
+constexpr int kErrGo = 14;
 // error codes written by kernels into Model::d_err[0]
 enum DevErr { ERR_NONE = 0, ERR_SETNOD = 1, ERR_SETUVD = 3, ERR_SETDEPTH = 4, ERR_VOLUME = 5,
               ERR_CONZ = 7, ERR_PENTA = 8, ERR_WIND = 9, ERR_MFLUX = 10 };
@@ -203,7 +205,7 @@ enum { CT_STOPIT = 0, CT_CONV = 1, CT_FAIL = 2, CT_NMV = 3, CT_ITS = 4, CT_REFCO
 
 // words of Model::h_pinned: device error words, scalar-stability results (one
 // model), solver control words, and the numbers of the last reports
-enum { HP_ERR = 0, HP_STAB = 8, HP_CTRL = 16, HP_SEQ = 40, HP_SEQ_STAB = 41 };
+enum { HP_ERR = 0, HP_STAB = 8, HP_CTRL = 16, HP_SEQ = 40, HP_SEQ_STAB = 41, HP_GO = 42 };
 
 struct Solver {               // Krylov work space (value type V = S of the model)
     int nblk = 0, brows = 0, max_blk_nnz = 0, max_blk_pairs = 0, nparts = 0, max_elev = 0;
@@ -295,6 +297,7 @@ struct Model {
     State s;
     Solver sv;
     int nnz = 0, ncolor = 0, nbnd = 0;
+    const int *after_go = nullptr;   // gate of the kernels being enqueued behind a solve (solver_solve)
     int *d_err = nullptr;     // [16] device error words + counters; [8..13] the
                               // scalar-stability maximum and result (64-bit words)
     int *h_pinned = nullptr;  // pinned host mirror for small readbacks (HP_*), written by kernels
@@ -525,7 +528,11 @@ int solver_setup(Model &M);
 // convergence flag, before each host read of the solver flags, so one
 // read-back returns the solver state, d_err[0] and the changed-element
 // count (in h_pinned[0..1]).
-int solver_solve(Model &M, int *iters, int *refinements, int wetdry_bnew = -1);
+// after (may be null): enqueues what follows a solve whose wet/dry state has
+// settled, before the host knows; its kernels return unless *go.  They ran
+// when h_pinned[HP_GO] is set afterwards (cleared by the caller).
+int solver_solve(Model &M, int *iters, int *refinements, int wetdry_bnew = -1,
+                 const std::function<int(const int *go)> *after = nullptr);
 // the tracers one conz3d launch transports together (1 or 2): slots, whether
 // small values are clipped (not temperature), source concentrations (device,
 // may be null)

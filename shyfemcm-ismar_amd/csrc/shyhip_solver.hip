@@ -2160,8 +2160,17 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
 // The solver's control words and the device error words into the host's
 // pinned memory, then the number of this report: the host waits for it
 // (wait_report) instead of two copies and a stream synchronisation.
-__global__ __launch_bounds__(64) void k_report(const int *ctrl, const int *err, int *host, int seq) {
+// go (may be null): whether the solve converged (word `conv`), no error is
+// set and no element changed its wet/dry state, for the kernels enqueued
+// behind the report.
+__global__ __launch_bounds__(64) void k_report(const int *ctrl, const int *err, int *host, int seq, int conv, int *go) {
     const int t = threadIdx.x;
+    if (t == 0 && go) {
+        const bool ok = ctrl[conv] && !ctrl[CT_FACTOR] && !err[0] && !err[1] &&
+                        (conv == CT_REFCONV || !(ctrl[CT_FAIL] || ctrl[CT_MAXIT]));
+        *go = ok;
+        host[HP_GO] = ok;
+    }
     if (t < CT_WORDS) host[HP_CTRL + t] = ctrl[t];
     else if (t < CT_WORDS + 2) host[HP_ERR + t - CT_WORDS] = err[t - CT_WORDS];
     __threadfence_system();
@@ -2171,11 +2180,14 @@ __global__ __launch_bounds__(64) void k_report(const int *ctrl, const int *err, 
 
 // one read-back: the solver's control words and the device error word and
 // counter d_err[0..1] (into h_pinned[HP_ERR..])
-static int read_ctrl(Model &M, int *out, int n) {
+static int read_ctrl(Model &M, int *out, int n, const std::function<int(const int *)> *after = nullptr,
+                     int conv = CT_CONV) {
     const int seq = ++M.report_seq;
+    int *go = after ? M.d_err + kErrGo : nullptr;
     hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, M.stream, (const int *)M.sv.ctrl, (const int *)M.d_err,
-                       M.h_pinned, seq);
+                       M.h_pinned, seq, conv, go);
     HIPCHK(M, hipGetLastError());
+    if (after && (*after)(go)) return 1;
     if (wait_report(M, HP_SEQ, seq)) return 1;
     for (int i = 0; i < n; i++) out[i] = M.h_pinned[HP_CTRL + i];
     return 0;
@@ -2459,7 +2471,8 @@ static ZetaPlan zeta_plan(Model &M) {
 // the launch, `tail` and the read-back of the control words; *done false
 // when a wait expired
 template <typename V>
-static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::function<int()> &tail, int *c, bool *done) {
+static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::function<int()> &tail,
+                    const std::function<int(const int *)> *after, int *c, bool *done) {
     ZetaArgs z;
     std::memset(&z, 0, sizeof z);
     z.nwg = M.sv.zeta_nwg; z.group = M.sv.zeta_group;
@@ -2477,7 +2490,7 @@ static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::func
     hipLaunchKernelGGL(zeta_kernel<V>(M), dim3(M.sv.zeta_nwg), dim3(M.sv.zeta_t), p.lds, M.stream, a, z);
     HIPCHK(M, hipGetLastError());
     if (tail && tail()) return 1;
-    if (read_ctrl(M, c, CT_WORDS)) return 1;
+    if (read_ctrl(M, c, CT_WORDS, after, std::is_same<V, double>::value ? CT_CONV : CT_REFCONV)) return 1;
     *done = c[CT_CONV] || c[CT_REFCONV] || !c[CT_WAIT];
     return 0;
 }
@@ -2493,7 +2506,8 @@ __global__ void k_ctrl_restart(int *ctrl) {
 
 // one zeta solve; fed: the row assembly already wrote its inputs (or a
 // first attempt did)
-static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, bool fed) {
+static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, bool fed,
+                      const std::function<int(const int *)> *after) {
     const int n = M.nkn;
     const int g1 = (n + kThreads - 1) / kThreads;
     int it_total = 0, nref = 0;
@@ -2531,7 +2545,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         const ZetaPlan plan = zeta_plan<double>(M);
         if (plan.cost >= 0.) {
             int c[CT_WORDS] = {};
-            if (zeta_run<double>(M, plan, a, tail, c, &done)) return 1;
+            if (zeta_run<double>(M, plan, a, tail, after, c, &done)) return 1;
             if (done) rc = krylov_outcome(M, c, &its, 0);
             else M.solver_retries++;
         }
@@ -2587,7 +2601,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         bool done = false;
         if (zp.cost >= 0.) {
             auto tail = [&]() -> int { return wetdry(M.sv.ctrl + CT_REFCONV, nullptr); };
-            if (zeta_run<float>(M, zp, a, tail, c, &done)) return 1;
+            if (zeta_run<float>(M, zp, a, tail, after, c, &done)) return 1;
             if (done) enq = maxref;       // all its rounds are behind it
             else M.solver_retries++;
         }
@@ -2643,19 +2657,20 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
 // the sweeps: rows switched by wetting and drying) is done again with exact
 // factors from where it stopped, so the warm start can cost iterations but
 // never a solve.
-int solver_solve(Model &M, int *iters, int *refinements, int wetdry_bnew) {
+int solver_solve(Model &M, int *iters, int *refinements, int wetdry_bnew,
+                 const std::function<int(const int *)> *after) {
     // inputs already written by the row assembly of this step's system?
     const bool fed = M.sv.fed;
     M.sv.fed = false;
     if (++M.sv.solves_since_exact >= kWarmRefresh) M.sv.have_lu = false;
-    const int rc = solve_once(M, iters, refinements, wetdry_bnew, fed);
+    const int rc = solve_once(M, iters, refinements, wetdry_bnew, fed, after);
     if (rc != 2 || !M.sv.last_warm) return rc;
     M.solver_retries++;
     M.sv.have_lu = false;
     hipLaunchKernelGGL(k_ctrl_restart, dim3(1), dim3(64), 0, M.stream, M.sv.ctrl);
     HIPCHK(M, hipGetLastError());
     M.err.clear();
-    return solve_once(M, iters, refinements, wetdry_bnew, true);
+    return solve_once(M, iters, refinements, wetdry_bnew, true, after);
 }
 
 }  // namespace shy
