@@ -1426,8 +1426,7 @@ int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int s
 int shyhip_set_wind_uniform(shyhip_model *h, float taux, float tauy) {
     if (!h) return fail(nullptr, "null handle");
     Model &M = h->M;
-    if (launch_fill(M, M.s.taux, taux, M.nkn)) return 1;
-    return launch_fill(M, M.s.tauy, tauy, M.nkn);
+    return launch_fill2(M, M.s.taux, taux, M.s.tauy, tauy, M.nkn);
 }
 
 int shyhip_set_member_wind(shyhip_model *h, int m, float taux, float tauy) {
@@ -1435,8 +1434,7 @@ int shyhip_set_member_wind(shyhip_model *h, int m, float taux, float tauy) {
     Model &M = h->M;
     if (m < 0 || m + 1 >= (int)M.mem_node.size()) return fail(&M, "set_member_wind: member out of range");
     const size_t k0 = (size_t)M.mem_node[m], n = (size_t)(M.mem_node[m + 1] - M.mem_node[m]);
-    if (launch_fill(M, (char *)M.s.taux + k0 * M.esize(), taux, n)) return 1;
-    return launch_fill(M, (char *)M.s.tauy + k0 * M.esize(), tauy, n);
+    return launch_fill2(M, (char *)M.s.taux + k0 * M.esize(), taux, (char *)M.s.tauy + k0 * M.esize(), tauy, n);
 }
 
 // ------------------------------------------------------------ forcing series

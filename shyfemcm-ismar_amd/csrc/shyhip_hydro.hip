@@ -751,6 +751,9 @@ __global__ __launch_bounds__(kThreads) void k_zeta_elem(HydroArgs<S> a) {
 // registers by position in the row (all element loads issued first); rows
 // longer than kEllWidth or nodes with more than kIncWidth elements
 // accumulate in place.
+// What bounds it: the gathers (70 loads of a row at most); the solve's copies
+// are written from the same registers (reading the row back for them: 127 us
+// on 300k nodes against 61, 22 on 50k against 15, 13.9 on 3k against 11.3).
 template <typename S>
 __global__ __launch_bounds__(kThreads) void k_zeta_rows(HydroArgs<S> a) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -791,7 +794,13 @@ __global__ __launch_bounds__(kThreads) void k_zeta_rows(HydroArgs<S> a) {
         }
 #pragma unroll
         for (int t = 0; t < kEllWidth; t++)
-            if (t < len) a.aval[r0 + t] = acc[t];
+            if (t < len) {
+                a.aval[r0 + t] = acc[t];
+                if (a.sv_ell) {
+                    a.sv_ell[(size_t)t * a.nkn + k] = (S)acc[t];
+                    if (a.sv_a32) a.sv_a32[r0 + t] = (float)acc[t];
+                }
+            }
     } else {
         for (int q = r0; q < r0 + len; q++) a.aval[q] = 0.;
         for (int q = a.nk_ptr[k]; q < a.nk_ptr[k + 1]; q++) {
@@ -803,17 +812,18 @@ __global__ __launch_bounds__(kThreads) void k_zeta_rows(HydroArgs<S> a) {
             }
             rhs = rhs + (double)a.zrow[(9 + i) * nel + ie];
         }
+        if (a.sv_ell)
+            for (int q = r0; q < r0 + len; q++) {
+                const double v = a.aval[q];
+                if (q - r0 < kEllWidth) a.sv_ell[(size_t)(q - r0) * a.nkn + k] = (S)v;
+                if (a.sv_a32) a.sv_a32[q] = (float)v;
+            }
     }
     rhs = rhs + (double)(dt * rq);
     a.rhs[k] = rhs;
     if (a.sv_ell) {
-        // the solve's inputs: the row in the ELL slots (and in FP32), the
-        // initial guess (FP32 path: extrapolated in time), cleared words
-        for (int q = r0; q < r0 + len; q++) {
-            const double v = a.aval[q];
-            if (q - r0 < kEllWidth) a.sv_ell[(size_t)(q - r0) * a.nkn + k] = (S)v;
-            if (a.sv_a32) a.sv_a32[q] = (float)v;
-        }
+        // the solve's inputs besides the row in the ELL slots (and in FP32):
+        // the initial guess (FP32 path: extrapolated in time), cleared words
         const double z = (double)a.zn[k];
         if (a.sv_zprev) {
             a.x[k] = a.sv_have_prev ? 2. * z - (double)a.sv_zprev[k] : z;
@@ -1436,6 +1446,14 @@ __global__ void k_fill(S *p, S v, size_t n) {
 }
 
 template <typename S>
+__global__ void k_fill2(S *p, S v, S *q, S w, size_t n) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    p[i] = v;
+    q[i] = w;
+}
+
+template <typename S>
 __global__ void k_copy(S *dst, const S *src, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
@@ -1804,6 +1822,13 @@ int launch_set_rzv_all(Model &M) {
     else
         LAUNCH(M, k_set_rzv_all<float>, nblocks(n), (float *)M.s.rzv, M.m.bnd_nodes, M.m.bnd_id, M.m.ibtyp, n,
                (const float *)M.d_levels);
+    return 0;
+}
+
+int launch_fill2(Model &M, void *p, double v, void *q, double w, size_t n) {
+    const int g = (int)((n + kThreads - 1) / kThreads);
+    if (M.prec == SHYHIP_FP64) LAUNCH(M, k_fill2<double>, g, (double *)p, v, (double *)q, w, n);
+    else LAUNCH(M, k_fill2<float>, g, (float *)p, (float)v, (float *)q, (float)w, n);
     return 0;
 }
 

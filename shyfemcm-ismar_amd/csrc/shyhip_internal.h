@@ -517,6 +517,7 @@ int launch_to_host_layout(Model &M, const void *a, bool a_double, void *out, boo
 // node-layer from T, S and the mid-layer pressure (shyhip_hydro.hip)
 int launch_rhoset(Model &M, int niter, hipStream_t st);
 int launch_fill(Model &M, void *ptr, double value, size_t n);
+int launch_fill2(Model &M, void *p, double v, void *q, double w, size_t n);   // two arrays, one launch
 int launch_volume(Model &M, int mode, double *vol);
 // the allocation-free volume / tracer mass of caller device arrays
 int noalloc_masscont(int dtype, int nkn, const int *ilhkv, const void *hdk, const void *areakv, const void *conc,
