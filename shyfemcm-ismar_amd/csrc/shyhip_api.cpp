@@ -770,7 +770,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         rc |= dalloc(M, &m.conz_nent, ent.size()) || upload(M, m.conz_nent, ent.data(), ent.size());
         rc |= dalloc(M, &m.conz_nplace, place.size()) || upload(M, m.conz_nplace, place.data(), place.size());
     }
-    if (M.nlv > 1) {
+    {
         std::vector<int> tiles{0}, place(nel);
         int cnt = 0, next = 0;
         for (int ie = 0; ie < nel; ie++) {

@@ -227,296 +227,18 @@ struct InternElem {
     }
 };
 
-// hydro_transports / hydro_intern, hydrodynamic.f90:758-1416.  One work-item
-// per element column.  Without Coriolis (gamma = 0) the 2L x 2L pentadiagonal
-// system decouples into two identical tridiagonal systems in u and v; the
-// tridiagonal elimination below performs exactly the operations that
-// penta_fact/penta_solve (penta.f90:104-321) perform on the decoupled bands.
-// The coupled case runs the pentadiagonal elimination itself.
-template <typename S, int NL, bool CORI>
-__global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
-    using R = S;
-    const int ie = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ie >= a.nel) return;
-    const int nel = a.nel, nkn = a.nkn;
-    InternElem<S> e;
-    e.load(a, ie, a.ilhv[ie], true, true);
-    const R dt = e.dt, af = (R)a.af, at = e.at, grav = e.grav, rowass = e.rowass, gammat = e.gammat, rfric = e.rfric;
-    const int ilevel = e.ilevel, k1 = e.kn[0], k2 = e.kn[1], k3 = e.kn[2];
-    const double(&b)[3] = e.b, (&c)[3] = e.c;
-    const double bz = e.bz, cz = e.cz, zmm = e.zmm, taux = e.taux, tauy = e.tauy, bpres = e.bpres, cpres = e.cpres;
-    const R gamma = af * dt * gammat;
-    a.rfric[ie] = rfric;
-
-    // layer thickness, inverse thickness, element viscosity
-    // The column's loads are issued at once, unconditionally: rows below the
-    // bottom layer read the bottom layer again (a valid address) and are
-    // replaced by zeros or not used.
-    R hact[NL + 2], rhact[NL + 2], alev[NL + 1];
-    R vsum[NL + 1];
-    R uoc[NL], voc[NL];
-#pragma unroll
-    for (int l = 1; l <= NL; l++) {
-        const size_t o = (size_t)(min(l, ilevel) - 1) * nel + ie;
-        hact[l] = a.hdeo[o];
-        uoc[l - 1] = a.uto[o];
-        voc[l - 1] = a.vto[o];
-    }
-#pragma unroll
-    for (int l = 0; l <= NL; l++) {
-        const size_t o = (size_t)min(l, ilevel) * nkn;
-        vsum[l] = a.visv[o + k1] + a.visv[o + k2] + a.visv[o + k3];
-    }
-    hact[0] = 0;
-    hact[NL + 1] = 0;
-#pragma unroll
-    for (int l = 1; l <= NL; l++)
-        if (l > ilevel) hact[l] = 0;
-    if (a.iclin) hact[1] = (R)(hact[1] - zmm);
-#pragma unroll
-    for (int l = 0; l <= NL + 1; l++) rhact[l] = (hact[l] <= (R)0) ? (R)0 : (R)1 / hact[l];
-#pragma unroll
-    for (int l = 0; l <= NL; l++) {
-        if (l <= ilevel) {
-            double vis = (double)a.vismol;
-            vis = vis + (double)(vsum[l] / (R)3);
-            alev[l] = (R)vis;
-        } else {
-            alev[l] = 0;
-        }
-    }
-
-    // explicit terms: the baroclinic pressure gradient (set_explicit ->
-    // set_barocl_new_interface, explicit.f90:193,1226-1530, z-layers) when
-    // the density anomaly is carried, else zero.  Per layer the anomaly
-    // gradient from the element's P1 gradients, averaged onto the interface
-    // above (the first layer uses its own), integrated down over the
-    // interface thicknesses, times g/rho0 and the nominal layer thickness;
-    // rounded to the reference's real as fxv/fyv are.
-    R xex[NL], yex[NL];
-    if (a.rhov) {
-        const double raux = (double)(grav / rowass);
-        double px = 0., py = 0., brup = 0., crup = 0., hhup = 0.;
-#pragma unroll
-        for (int l = 1; l <= NL; l++) {
-            const size_t o = (size_t)(min(l, ilevel) - 1) * nkn;
-            const R r[3] = {a.rhov[o + k1], a.rhov[o + k2], a.rhov[o + k3]};
-            const double hlayer = (double)a.hldv[l - 1];
-            const double hh = 0.5 * hlayer;
-            const double hint = hh + hhup;
-            double br = 0., cr = 0.;
-#pragma unroll
-            for (int ii = 0; ii < 3; ii++) {
-                br = br + b[ii] * (double)r[ii];
-                cr = cr + c[ii] * (double)r[ii];
-            }
-            const double brint = l == 1 ? br : 0.5 * (br + brup);
-            const double crint = l == 1 ? cr : 0.5 * (cr + crup);
-            brup = br;
-            crup = cr;
-            hhup = hh;
-            px = px + hint * brint;
-            py = py + hint * crint;
-            xex[l - 1] = (R)(0.0 + raux * hlayer * px);
-            yex[l - 1] = (R)(0.0 + raux * hlayer * py);
-        }
-    } else {
-#pragma unroll
-        for (int l = 0; l < NL; l++) xex[l] = yex[l] = 0;
-    }
-
-    double sxu[NL], sxv[NL], sh[NL];      // solutions: -F^x, -F^y and H rows
-    if constexpr (!CORI) {
-        double xd[NL], up[NL], gx[NL], gy[NL], gh[NL];
-#pragma unroll
-        for (int l = 1; l <= NL; l++) {
-            if (l > ilevel) continue;
-            const bool bfirst = (l == 1), blast = (l == ilevel);
-            // layers min(l+1, ilevel) and max(l-1, 1), from registers
-            const bool below = l < NL && l + 1 <= ilevel;
-            const R uui = uoc[l - 1], uuip = below ? uoc[l < NL ? l : l - 1] : uoc[l - 1];
-            const R uuim = l > 1 ? uoc[l > 1 ? l - 2 : 0] : uoc[0];
-            const R vvi = voc[l - 1], vvip = below ? voc[l < NL ? l : l - 1] : voc[l - 1];
-            const R vvim = l > 1 ? voc[l > 1 ? l - 2 : 0] : voc[0];
-            double d, lo;
-            R rx, ry;
-            e.row(bfirst, blast, uui, uuip, uuim, vvi, vvip, vvim, hact[l], hact[l + 1], hact[l - 1], rhact[l],
-                  rhact[l + 1], rhact[l - 1], alev[l], alev[l - 1], d, lo, up[l - 1], rx, ry);
-            const double ppx = e.rhs(bfirst, taux, rx, xex[l - 1]), ppy = e.rhs(bfirst, tauy, ry, yex[l - 1]);
-            const R hhi = hact[l];
-            if (l == 1) {
-                xd[0] = d;
-                gx[0] = ppx;
-                gy[0] = ppy;
-                gh[0] = (double)hhi;
-            } else {
-                const double w = lo / xd[l - 2];
-                xd[l - 1] = d - w * up[l - 2];
-                gx[l - 1] = ppx - w * gx[l - 2];
-                gy[l - 1] = ppy - w * gy[l - 2];
-                gh[l - 1] = (double)hhi - w * gh[l - 2];
-            }
-        }
-        double su = 0., sv = 0., shh = 0.;
-#pragma unroll
-        for (int l = NL; l >= 1; l--) {
-            if (l > ilevel) continue;
-            if (l == ilevel) {
-                su = gx[l - 1] / xd[l - 1];
-                sv = gy[l - 1] / xd[l - 1];
-                shh = gh[l - 1] / xd[l - 1];
-            } else {
-                su = (gx[l - 1] - up[l - 1] * su) / xd[l - 1];
-                sv = (gy[l - 1] - up[l - 1] * sv) / xd[l - 1];
-                shh = (gh[l - 1] - up[l - 1] * shh) / xd[l - 1];
-            }
-            sxu[l - 1] = su;
-            sxv[l - 1] = sv;
-            sh[l - 1] = shh;
-        }
-    } else {
-        // coupled u/v columns: pentadiagonal elimination of penta.f90
-        constexpr int N2 = 2 * NL;
-        double vm2[N2], vm1[N2], v0[N2], vp1[N2], vp2[N2], r0[N2], r1[N2], r2[N2];
-#pragma unroll
-        for (int i = 0; i < N2; i++) { vm2[i] = vm1[i] = v0[i] = vp1[i] = vp2[i] = 0.; r0[i] = r1[i] = r2[i] = 0.; }
-        const int n = 2 * ilevel;
-        for (int l = 1; l <= ilevel; l++) {
-            const bool bfirst = (l == 1), blast = (l == ilevel);
-            const int lp = (l + 1 < ilevel) ? l + 1 : ilevel;
-            const int lm = (l - 1 > 1) ? l - 1 : 1;
-            const R uui = a.uto[(size_t)(l - 1) * nel + ie], uuip = a.uto[(size_t)(lp - 1) * nel + ie];
-            const R uuim = a.uto[(size_t)(lm - 1) * nel + ie];
-            const R vvi = a.vto[(size_t)(l - 1) * nel + ie], vvip = a.vto[(size_t)(lp - 1) * nel + ie];
-            const R vvim = a.vto[(size_t)(lm - 1) * nel + ie];
-            const R hhi = hact[l], hhip = hact[l + 1], hhim = hact[l - 1];
-            R rhp = 0, rhm = 0;
-            if (hhi > (R)0) {
-                if (hhip > (R)0) rhp = (R)2.0 * alev[l] / (hhi + hhip);
-                if (hhim > (R)0) rhm = (R)2.0 * alev[l - 1] / (hhi + hhim);
-            }
-            const R aux = dt * at;
-            R aa = aux * rhact[l] * (rhm + rhp);
-            R aat = (R)1 * rhact[l] * (rhm + rhp);
-            const R bb = aux * rhact[l + 1] * rhp;
-            const R bbt = (R)1 * rhact[l + 1] * rhp;
-            const R cc = aux * rhact[l - 1] * rhm;
-            const R cct = (R)1 * rhact[l - 1] * rhm;
-            double ppx = 0., ppy = 0.;
-            if (bfirst) { ppx = ppx - taux; ppy = ppy - tauy; }
-            if (blast) { aa = aa + dt * rfric; aat = aat + rfric; }
-            const R gravx = (R)(1.0 * grav * hhi * bz);
-            const R gravy = (R)(1.0 * grav * hhi * cz);
-            const R presx = (R)bpres, presy = (R)cpres, xexpl = xex[l - 1], yexpl = yex[l - 1];
-            const R ppx_aux = aat * uui - bbt * uuip - cct * uuim - gammat * vvi + gravx + (hhi / rowass) * presx + xexpl;
-            const R ppy_aux = aat * vvi - bbt * vvip - cct * vvim + gammat * uui + gravy + (hhi / rowass) * presy + yexpl;
-            ppx = ppx + (double)ppx_aux;
-            ppy = ppy + (double)ppy_aux;
-            const int ju = 2 * l - 2, jv = 2 * l - 1;
-            v0[ju] = (double)((R)1 + aa);
-            v0[jv] = (double)((R)1 + aa);
-            vm1[jv] = (double)gamma;
-            vp1[ju] = (double)(-gamma);
-            if (!blast) { vp2[ju] = -bb; vp2[jv] = -bb; }
-            if (!bfirst) { vm2[ju] = -cc; vm2[jv] = -cc; }
-            r0[ju] = ppx; r0[jv] = ppy;
-            r1[ju] = (double)hhi; r2[jv] = (double)hhi;
-        }
-        double xx[N2], yy[N2], zz[N2 + 1];
-        int bad = 0;
-        zz[0] = 0.;
-        for (int i = 0; i < n; i++) {
-            double t = v0[i];
-            if (i >= 1) t = t - yy[i - 1] * zz[i];
-            if (i >= 2) t = t - vm2[i] * vp2[i - 2];
-            if (t == 0.) bad = 1;
-            xx[i] = t;
-            yy[i] = (i < n - 1) ? vp1[i] - ((i >= 1) ? zz[i] * vp2[i - 1] : 0.) : 0.;
-            if (i == 0) yy[0] = vp1[0];
-            if (i + 1 < n) zz[i + 1] = (vm1[i + 1] - ((i >= 1) ? vm2[i + 1] * yy[i - 1] : 0.)) / t;
-            if (i + 2 < n) vm2[i + 2] = vm2[i + 2] / t;
-        }
-        if (bad) atomicCAS(a.err, 0, ERR_PENTA);
-        double g0[N2], g1[N2], g2[N2];
-        for (int i = 0; i < n; i++) {
-            g0[i] = r0[i]; g1[i] = r1[i]; g2[i] = r2[i];
-            if (i >= 1) { g0[i] -= zz[i] * g0[i - 1]; g1[i] -= zz[i] * g1[i - 1]; g2[i] -= zz[i] * g2[i - 1]; }
-            if (i >= 2) { g0[i] -= vm2[i] * g0[i - 2]; g1[i] -= vm2[i] * g1[i - 2]; g2[i] -= vm2[i] * g2[i - 2]; }
-        }
-        double s0[N2], s1[N2], s2[N2];
-        for (int i = n - 1; i >= 0; i--) {
-            double t0 = g0[i], t1 = g1[i], t2 = g2[i];
-            if (i + 1 < n) { t0 -= yy[i] * s0[i + 1]; t1 -= yy[i] * s1[i + 1]; t2 -= yy[i] * s2[i + 1]; }
-            if (i + 2 < n) { t0 -= vp2[i] * s0[i + 2]; t1 -= vp2[i] * s1[i + 2]; t2 -= vp2[i] * s2[i + 2]; }
-            s0[i] = t0 / xx[i]; s1[i] = t1 / xx[i]; s2[i] = t2 / xx[i];
-        }
-        // store the coupled result into the same per-layer slots
-        double dbb = 0., dbc = 0., dcb = 0., dcc = 0.;
-        for (int l = 1; l <= ilevel; l++) {
-            const int ju = 2 * l - 2, jv = 2 * l - 1;
-            sxu[l - 1] = s0[ju];
-            sxv[l - 1] = s0[jv];
-            a.ddx[(size_t)ju * nel + ie] = (S)s1[ju];
-            a.ddx[(size_t)jv * nel + ie] = (S)s1[jv];
-            a.ddy[(size_t)ju * nel + ie] = (S)s2[ju];
-            a.ddy[(size_t)jv * nel + ie] = (S)s2[jv];
-            dbb += s1[ju]; dbc += s2[ju]; dcb += s1[jv]; dcc += s2[jv];
-        }
-        a.zel[(size_t)0 * nel + ie] = dbb;
-        a.zel[(size_t)1 * nel + ie] = dbc;
-        a.zel[(size_t)2 * nel + ie] = dcb;
-        a.zel[(size_t)3 * nel + ie] = dcc;
-    }
-    // u^hat = u_old - dt * A^-1 F ; store A^-1 H.  Elements with fixed
-    // transports (afix = 0, hydrodynamic.f90:1383-1392) keep the ones they
-    // hold: the prescribed transports, or those of the previous step.
-    const int afix = a.iuvfix ? 1 - a.iuvfix[ie] : 1;
-    const R dtafix = dt * (R)afix;
-    double uold = 0., vold = 0., uhat = 0., vhat = 0.;
-    double dsum = 0.;
-#pragma unroll
-    for (int l = 1; l <= NL; l++) {
-        if (l > ilevel) continue;
-        const size_t ol = (size_t)(l - 1) * nel + ie;
-        const R uo = a.uto[ol], vo = a.vto[ol];
-        S unew, vnew;
-        if (afix != 0) {
-            unew = (S)((double)uo - (double)dtafix * sxu[l - 1]);
-            vnew = (S)((double)vo - (double)dtafix * sxv[l - 1]);
-        } else {
-            unew = a.utfix ? a.utfix[ol] : uo;
-            vnew = a.vtfix ? a.vtfix[ol] : vo;
-        }
-        a.utn[(size_t)(l - 1) * nel + ie] = unew;
-        a.vtn[(size_t)(l - 1) * nel + ie] = vnew;
-        uold += (double)uo; vold += (double)vo;
-        uhat += (double)unew; vhat += (double)vnew;
-        if constexpr (!CORI) {
-            // decoupled columns: the cross terms ddx(jv), ddy(ju) are zero and
-            // stay zero in the arrays (never written on this path)
-            const int ju = 2 * l - 2, jv = 2 * l - 1;
-            a.ddx[(size_t)ju * nel + ie] = (S)sh[l - 1];
-            a.ddy[(size_t)jv * nel + ie] = (S)sh[l - 1];
-            dsum += sh[l - 1];
-        }
-    }
-    if constexpr (!CORI) {
-        a.zel[(size_t)0 * nel + ie] = dsum;
-        a.zel[(size_t)1 * nel + ie] = 0.;
-        a.zel[(size_t)2 * nel + ie] = 0.;
-        a.zel[(size_t)3 * nel + ie] = dsum;
-    }
-    const double az = (double)a.az;
-    a.zel[(size_t)4 * nel + ie] = az * uhat + (1. - az) * uold;
-    a.zel[(size_t)5 * nel + ie] = az * vhat + (1. - az) * vold;
-}
-
-// The same without Coriolis for columns of several layers.  One workgroup per
-// tile of consecutive elements (Mesh::h_tile; at most kThreads elements and
-// element-layers).  Phase 1, one work-item per element-layer: the layer's row
-// of the tridiagonal system, into LDS.  Phase 2, one work-item per element:
+// hydro_transports / hydro_intern, hydrodynamic.f90:758-1416.  One workgroup
+// per tile of consecutive elements (Mesh::h_tile; at most kThreads elements
+// and element-layers).  Phase 1, one work-item per element-layer: the layer's
+// rows of the column's system, into LDS.  Phase 2, one work-item per element:
 // the elimination and the column's sums.  Phase 3, one work-item per
 // element-layer: the results.
+// Without Coriolis (gamma = 0) the 2L x 2L pentadiagonal system decouples
+// into two identical tridiagonal systems in u and v; the tridiagonal
+// elimination performs exactly the operations that penta_fact/penta_solve
+// (penta.f90:104-321) perform on the decoupled bands.  The coupled case (CORI)
+// runs the pentadiagonal elimination itself, row 2l of layer l for u and
+// 2l + 1 for v.
 //
 // What bounds it: the loads of the layers' rows (about 35 a work-item).  One
 // work-item per column, its layers unrolled in registers, walked every
@@ -524,9 +246,10 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
 // from 16 layers on: 489 us on 300k nodes of 20 layers, 14.6 on 3k nodes of
 // 10 (FP64) against 184 and 8.8; equal (28 to 30 us) on 50k nodes of 12.
 // The rows in scratch memory with rolled loops took 337 us, the columns split
-// by depth between two kernels 331.
-template <typename S>
-__global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) {
+// by depth between two kernels 331.  Coupled columns in scratch memory took
+// 95 us on 9k nodes of 12 layers against 16.6.
+template <typename S, bool CORI>
+__global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
     using R = S;
     // by place in the tile (element after element, top down): the row's
     // diagonals, right-hand sides and thickness, which the elimination
@@ -535,6 +258,10 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) 
     __shared__ double dL[kThreads], loL[kThreads], upL[kThreads], pxL[kThreads], pyL[kThreads], hL[kThreads];
     __shared__ double brL[kThreads], crL[kThreads], txL[kThreads], tyL[kThreads];
     __shared__ R uL[kThreads], vL[kThreads];
+    // coupled columns: the second upper diagonal of both rows, the right-hand
+    // sides of the v row for H in x and of both rows for H in y
+    constexpr int kCori = CORI ? kThreads : 1;
+    __shared__ double yuL[kCori], yvL[kCori], hxvL[kCori], hyuL[kCori], hyvL[kCori];
     const int nel = a.nel, nkn = a.nkn;
     const int tile = xcd_block();
     const int2 ent = a.h_ent[(size_t)tile * kThreads + threadIdx.x];
@@ -570,7 +297,7 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) 
         uL[it] = u; vL[it] = v;
         if (a.rhov) {
             // the density gradient; the pressure gradient is its integral
-            // down the column
+            // down the column (below)
             double br = 0., cr = 0.;
 #pragma unroll
             for (int ii = 0; ii < 3; ii++) {
@@ -589,53 +316,136 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) 
     __syncthreads();
     if ((int)threadIdx.x < tn) {
         const int ec = e0 + threadIdx.x, n = a.ilhv[ec], p0 = a.h_place[ec];
-        // the baroclinic pressure gradient integrated down (see k_hydro_intern)
+        // the baroclinic pressure gradient, when the density anomaly is carried
+        // (set_explicit -> set_barocl_new_interface, explicit.f90:193,
+        // 1226-1530, z-layers): the anomaly gradient of each layer averaged
+        // onto the interface above (the first layer uses its own), integrated
+        // down over the interface thicknesses, times g/rho0 and the nominal
+        // layer thickness; rounded to the reference's real as fxv/fyv are
         const double raux = (double)((R)a.grav / (R)a.rowass);
         double px = 0., py = 0., brup = 0., crup = 0., hhup = 0.;
-        double xp = 0., upp = 0., gxp = 0., gyp = 0., ghp = 0.;
-        for (int m = 0; m < n; m++) {
-            const int i = p0 + m;
-            double x = dL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
-            const double lo = loL[i], up = upL[i];
-            if (a.rhov) {
-                const double hlayer = (double)a.hldv[m];
-                const double hh = 0.5 * hlayer;
-                const double hint = hh + hhup;
-                const double br = brL[i], cr = crL[i];
-                const double brint = m == 0 ? br : 0.5 * (br + brup);
-                const double crint = m == 0 ? cr : 0.5 * (cr + crup);
-                brup = br;
-                crup = cr;
-                hhup = hh;
-                px = px + hint * brint;
-                py = py + hint * crint;
-                gx = InternElem<S>::rhs(m == 0, txL[threadIdx.x], (R)gx, (R)(0.0 + raux * hlayer * px));
-                gy = InternElem<S>::rhs(m == 0, tyL[threadIdx.x], (R)gy, (R)(0.0 + raux * hlayer * py));
+        auto pressure = [&](int m, int i, double &gx, double &gy) {
+            const double hlayer = (double)a.hldv[m];
+            const double hh = 0.5 * hlayer;
+            const double hint = hh + hhup;
+            const double br = brL[i], cr = crL[i];
+            const double brint = m == 0 ? br : 0.5 * (br + brup);
+            const double crint = m == 0 ? cr : 0.5 * (cr + crup);
+            brup = br;
+            crup = cr;
+            hhup = hh;
+            px = px + hint * brint;
+            py = py + hint * crint;
+            gx = InternElem<S>::rhs(m == 0, txL[threadIdx.x], (R)gx, (R)(0.0 + raux * hlayer * px));
+            gy = InternElem<S>::rhs(m == 0, tyL[threadIdx.x], (R)gy, (R)(0.0 + raux * hlayer * py));
+        };
+        if constexpr (!CORI) {
+            double xp = 0., upp = 0., gxp = 0., gyp = 0., ghp = 0.;
+            for (int m = 0; m < n; m++) {
+                const int i = p0 + m;
+                double x = dL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
+                const double lo = loL[i], up = upL[i];
+                if (a.rhov) pressure(m, i, gx, gy);
+                if (m > 0) {
+                    const double w = lo / xp;
+                    x = x - w * upp;
+                    gx = gx - w * gxp;
+                    gy = gy - w * gyp;
+                    gh = gh - w * ghp;
+                }
+                dL[i] = x; pxL[i] = gx; pyL[i] = gy; hL[i] = gh;
+                xp = x; upp = up; gxp = gx; gyp = gy; ghp = gh;
             }
-            if (m > 0) {
-                const double w = lo / xp;
-                x = x - w * upp;
-                gx = gx - w * gxp;
-                gy = gy - w * gyp;
-                gh = gh - w * ghp;
+            double su = 0., sv = 0., sh = 0.;
+            for (int m = n - 1; m >= 0; m--) {
+                const int i = p0 + m;
+                const double x = dL[i], up = upL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
+                const bool last = m == n - 1;
+                su = (last ? gx : gx - up * su) / x;
+                sv = (last ? gy : gy - up * sv) / x;
+                sh = (last ? gh : gh - up * sh) / x;
+                pxL[i] = su; pyL[i] = sv; hL[i] = sh;
             }
-            dL[i] = x; pxL[i] = gx; pyL[i] = gy; hL[i] = gh;
-            xp = x; upp = up; gxp = gx; gyp = gy; ghp = gh;
-        }
-        double su = 0., sv = 0., sh = 0.;
-        for (int m = n - 1; m >= 0; m--) {
-            const int i = p0 + m;
-            const double x = dL[i], up = upL[i], gx = pxL[i], gy = pyL[i], gh = hL[i];
-            const bool last = m == n - 1;
-            su = (last ? gx : gx - up * su) / x;
-            sv = (last ? gy : gy - up * sv) / x;
-            sh = (last ? gh : gh - up * sh) / x;
-            pxL[i] = su; pyL[i] = sv; hL[i] = sh;
+        } else {
+            const double gamma = (double)((R)a.af * (R)a.dt * (R)a.fcorv[ec]);
+            // of the layer above: pivots x, first upper diagonals y, second
+            // upper diagonal up, right-hand sides (0: -F, 1: H in x, 2: H in y)
+            double xu = 1., xv = 1., yu = 0., yv = 0., upp = 0., gu[3] = {0., 0., 0.}, gv[3] = {0., 0., 0.};
+            bool bad = false;
+            for (int m = 0; m < n; m++) {
+                const int i = p0 + m;
+                const bool below = m > 0, last = m == n - 1;
+                const double d = dL[i], lo = loL[i], up = upL[i], h = hL[i];
+                double ru[3] = {pxL[i], h, 0.}, rv[3] = {pyL[i], 0., h};
+                if (a.rhov) pressure(m, i, ru[0], rv[0]);
+                // row u: second lower diagonal w, first lower diagonal z
+                double w = 0., z = 0., t = d, y = -gamma;
+                if (below) {
+                    w = lo / xu;
+                    z = (0. - w * yu) / xv;
+                    t = t - yv * z;
+                    t = t - w * upp;
+                    y = y - z * upp;
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        ru[q] = ru[q] - z * gv[q];
+                        ru[q] = ru[q] - w * gu[q];
+                    }
+                }
+                bad = bad || t == 0.;
+                const double xuc = t, yuc = y;
+                // row v
+                w = 0.;
+                z = gamma;
+                if (below) {
+                    w = lo / xv;
+                    z = z - w * yv;
+                }
+                z = z / xuc;
+                t = d - yuc * z;
+                if (below) t = t - w * upp;
+                y = last ? 0. : 0. - z * up;
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    rv[q] = rv[q] - z * ru[q];
+                    if (below) rv[q] = rv[q] - w * gv[q];
+                }
+                bad = bad || t == 0.;
+                xu = xuc; yu = yuc; xv = t; yv = y; upp = up;
+#pragma unroll
+                for (int q = 0; q < 3; q++) { gu[q] = ru[q]; gv[q] = rv[q]; }
+                dL[i] = xu; loL[i] = xv; yuL[i] = yu; yvL[i] = yv;
+                pxL[i] = gu[0]; hL[i] = gu[1]; hyuL[i] = gu[2];
+                pyL[i] = gv[0]; hxvL[i] = gv[1]; hyvL[i] = gv[2];
+            }
+            if (bad) atomicCAS(a.err, 0, ERR_PENTA);
+            double su[3] = {0., 0., 0.}, sv[3] = {0., 0., 0.};
+            for (int m = n - 1; m >= 0; m--) {
+                const int i = p0 + m;
+                const bool above = m < n - 1;
+                const double up = upL[i], xuc = dL[i], xvc = loL[i], yuc = yuL[i], yvc = yvL[i];
+                double tu[3] = {pxL[i], hL[i], hyuL[i]}, tv[3] = {pyL[i], hxvL[i], hyvL[i]};
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    if (above) {
+                        tv[q] = tv[q] - yvc * su[q];
+                        tv[q] = tv[q] - up * sv[q];
+                    }
+                    tv[q] = tv[q] / xvc;
+                    tu[q] = tu[q] - yuc * tv[q];
+                    if (above) tu[q] = tu[q] - up * su[q];
+                    tu[q] = tu[q] / xuc;
+                    su[q] = tu[q]; sv[q] = tv[q];
+                }
+                pxL[i] = su[0]; hL[i] = su[1]; hyuL[i] = su[2];
+                pyL[i] = sv[0]; hxvL[i] = sv[1]; hyvL[i] = sv[2];
+            }
         }
         // u^hat = u_old - dt * A^-1 F (or the fixed transports) and the sums
         const int afix = a.iuvfix ? 1 - a.iuvfix[ec] : 1;
         const R dtafix = (R)a.dt * (R)afix;
-        double uold = 0., vold = 0., uhat = 0., vhat = 0., dsum = 0.;
+        // (column sums of A^-1 H: x and y parts of the u rows, then of the v rows)
+        double uold = 0., vold = 0., uhat = 0., vhat = 0., dsum[4] = {0., 0., 0., 0.};
         for (int m = 0; m < n; m++) {
             const int i = p0 + m;
             const size_t oc = (size_t)m * nel + ec;
@@ -651,23 +461,34 @@ __global__ __launch_bounds__(kThreads) void k_hydro_intern_tile(HydroArgs<S> a) 
             uL[i] = unew; vL[i] = vnew;
             uold += (double)uo; vold += (double)vo;
             uhat += (double)unew; vhat += (double)vnew;
-            dsum += hL[i];
+            dsum[0] += hL[i];
+            if constexpr (CORI) {
+                dsum[1] += hyuL[i];
+                dsum[2] += hxvL[i];
+                dsum[3] += hyvL[i];
+            }
         }
-        a.zel[(size_t)0 * nel + ec] = dsum;
-        a.zel[(size_t)1 * nel + ec] = 0.;
-        a.zel[(size_t)2 * nel + ec] = 0.;
-        a.zel[(size_t)3 * nel + ec] = dsum;
+        if constexpr (!CORI) dsum[3] = dsum[0];
+#pragma unroll
+        for (int q = 0; q < 4; q++) a.zel[(size_t)q * nel + ec] = dsum[q];
         const double az = (double)a.az;
         a.zel[(size_t)4 * nel + ec] = az * uhat + (1. - az) * uold;
         a.zel[(size_t)5 * nel + ec] = az * vhat + (1. - az) * vold;
     }
     __syncthreads();
     if (!on) return;
-    // the cross terms ddx(jv), ddy(ju) stay zero (never written on this path)
     a.utn[o] = uL[it];
     a.vtn[o] = vL[it];
-    a.ddx[(size_t)(2 * l - 2) * nel + ie] = (S)hL[it];
-    a.ddy[(size_t)(2 * l - 1) * nel + ie] = (S)hL[it];
+    const size_t ou = (size_t)(2 * l - 2) * nel + ie, ov = ou + nel;
+    a.ddx[ou] = (S)hL[it];
+    if constexpr (CORI) {
+        a.ddx[ov] = (S)hxvL[it];
+        a.ddy[ou] = (S)hyuL[it];
+        a.ddy[ov] = (S)hyvL[it];
+    } else {
+        // (the cross terms stay zero: never written on this path)
+        a.ddy[ov] = (S)hL[it];
+    }
 }
 
 // ------------------------------------------------------------------ hydro_zeta
@@ -1596,27 +1417,12 @@ static int setnod_t(Model &M) {
 }
 int launch_setnod(Model &M) { return M.prec == SHYHIP_FP64 ? setnod_t<double>(M) : setnod_t<float>(M); }
 
-template <typename S, int NL>
-static int hydro_intern_nl(Model &M) {
-    auto a = make_args<S>(M);
-    if (M.has_coriolis) LAUNCH(M, (k_hydro_intern<S, NL, true>), nblocks(M.nel), a);
-    else if constexpr (NL == 1) LAUNCH(M, (k_hydro_intern<S, NL, false>), nblocks(M.nel), a);
-    else LAUNCH(M, k_hydro_intern_tile<S>, M.m.n_htile, a);
-    return 0;
-}
 template <typename S>
 static int hydro_intern_t(Model &M) {
-    switch (M.nl_tmpl) {
-    case 1: return hydro_intern_nl<S, 1>(M);
-    case 2: return hydro_intern_nl<S, 2>(M);
-    case 4: return hydro_intern_nl<S, 4>(M);
-    case 8: return hydro_intern_nl<S, 8>(M);
-    case 12: return hydro_intern_nl<S, 12>(M);
-    case 16: return hydro_intern_nl<S, 16>(M);
-    case 20: return hydro_intern_nl<S, 20>(M);
-    case 24: return hydro_intern_nl<S, 24>(M);
-    default: return hydro_intern_nl<S, 32>(M);
-    }
+    auto a = make_args<S>(M);
+    if (M.has_coriolis) LAUNCH(M, (k_hydro_intern<S, true>), M.m.n_htile, a);
+    else LAUNCH(M, (k_hydro_intern<S, false>), M.m.n_htile, a);
+    return 0;
 }
 int launch_hydro_intern(Model &M) { return M.prec == SHYHIP_FP64 ? hydro_intern_t<double>(M) : hydro_intern_t<float>(M); }
 

@@ -133,7 +133,7 @@ struct Mesh {                 // device copies of init-time data
     // each, kIncWidth apart), node}, -1 in the first word of unused entries;
     // and each node's first place in its tile (its layers follow one another)
     int *conz_nent = nullptr, *conz_nplace = nullptr;
-    // hydro_intern's element tiles (basins of several layers): first elements
+    // hydro_intern's element tiles: first elements
     // [n_htile + 1], the tiles' element-layers, layer by layer with the
     // elements ascending in each, [tile*kThreads + i] as int2: {(l-1) |
     // (lmax-1) << 5 | place << 10, element}, -1 in the first word of unused
