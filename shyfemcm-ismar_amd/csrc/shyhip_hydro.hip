@@ -1,8 +1,8 @@
 // shyhip_hydro.hip -- gfx950 kernels of the semi-implicit hydro step.
 //
-// Every kernel is one work-item per element column or per node column, with
-// layer-major arrays so that a wavefront reads 64 consecutive elements of one
-// layer.  Element -> node accumulations are gathers over the node's incident
+// A kernel's work-items are element or node columns, or the layers of a tile of
+// them (hydro_intern, hydro_vertical), with layer-major arrays so that a
+// wavefront reads consecutive elements of one layer.  Element -> node accumulations are gathers over the node's incident
 // elements in ascending element order: atomic-free, deterministic, and the
 // same summation order as the reference's sequential element loops.
 // Arithmetic order and operand types follow the reference (`real` locals are

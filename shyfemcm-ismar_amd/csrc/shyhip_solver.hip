@@ -2378,12 +2378,17 @@ static int zeta_mode(const Model &M) {
 template <typename V>
 static ZetaKernel<V> zeta_kernel(const Model &M) {
     const int mode = zeta_mode(M);
-    if (M.sv.zeta_t == 1024) return mode == kDense ? k_zeta<V, 1024, 1, kDense> : k_zeta<V, 1024, 1, kSubst>;
-    if (M.sv.zeta_t == 512)
-        return mode == kDense ? k_zeta<V, 512, 1, kDense>
-                              : (mode == kSubst ? k_zeta<V, 512, 1, kSubst> : k_zeta<V, 512, 1, kSwept>);
-    if (M.sv.zeta_hmax <= 256) return mode == kSubst ? k_zeta<V, 256, 1, kSubst> : k_zeta<V, 256, 1, kSwept>;
-    return mode == kSubst ? k_zeta<V, 256, 2, kSubst> : k_zeta<V, 256, 2, kSwept>;
+    // (exact substitution in FP64 only, see host_zeta_tables)
+    if constexpr (std::is_same<V, double>::value) {
+        if (mode == kDense) return M.sv.zeta_t == 1024 ? k_zeta<V, 1024, 1, kDense> : k_zeta<V, 512, 1, kDense>;
+        if (mode == kSubst)
+            return M.sv.zeta_t == 1024 ? k_zeta<V, 1024, 1, kSubst>
+                                       : (M.sv.zeta_t == 512 ? k_zeta<V, 512, 1, kSubst>
+                                                             : (M.sv.zeta_hmax <= 256 ? k_zeta<V, 256, 1, kSubst>
+                                                                                      : k_zeta<V, 256, 2, kSubst>));
+    }
+    if (M.sv.zeta_t == 512) return k_zeta<V, 512, 1, kSwept>;
+    return M.sv.zeta_hmax <= 256 ? k_zeta<V, 256, 1, kSwept> : k_zeta<V, 256, 2, kSwept>;
 }
 
 // Workgroups of the one-launch solve wait for each other, so a launch is
@@ -2438,6 +2443,7 @@ static ZetaPlan zeta_plan(Model &M) {
     Solver &v = M.sv;
     if (v.zeta_t == 0) return p;
     const int mode = zeta_mode(M), exact = mode != kSwept;
+    if (exact && sizeof(V) == 4) return p;        // FP64 only (see host_zeta_tables)
     // sweeps keep the factor row in registers (and need its slot-major copy),
     // and a basin laid out for dense rows has one block's work-items per workgroup
     if (!exact && (!v.fs_val || v.brows > kThreads || v.zeta_members > 0)) return p;
