@@ -79,21 +79,21 @@ def _kernel_bytes(b, p, brows, ntr=2):
     spmv = nnz * (p + 4) + N * 4                # values, columns, row pointers
     return {
         # utlov vtlov hdeov read, utlnv vtlnv written, ddxv ddyv (2 planes) written,
-        # visv at the interfaces, per element geometry/levels/summaries
-        "hydro_intern": 9 * EL * p + (NL + N) * p + E * (12 + 56 + 6 * p + 4 + 48),
-        # once per step: utlnv vtlnv utlov vtlov ulnv vlnv read, per element
-        # nodes, list positions, geometry (7 doubles), distances (3), levels,
-        # external flags and the TVD upwind tables (6 points: element, level,
-        # 3 nodes, 3 weights) read; the element-layer record written (15
-        # ints, 11 doubles)
-        "conz3d_prep": 6 * EL * p + E * (12 + 12 + 56 + 24 + 4 + 4 + 264) + EL * 148,
-        # per substep: the record read, 3 horizontal terms per tracer
-        # written, each tracer gathered
-        "conz3d_elem": 3 * ntr * EL * p + ntr * NL * p + EL * 148,
-        # horizontal terms read; hdknv hdkov wlnv difv read, each tracer read
-        # and written; per list position its bottom layer and 4 * area, per
-        # node its list start and bottom layer
-        "conz3d_node": 3 * ntr * EL * p + (4 + 2 * ntr) * NL * p + 2 * N * p + 3 * E * 12 + 2 * N * 4,
+        # visv at the interfaces, the tiles' entries, per element
+        # geometry/levels/summaries
+        "hydro_intern": 9 * EL * p + (NL + N) * p + 8 * EL + E * (12 + 56 + 6 * p + 4 + 48),
+        # once per step: utlnv vtlnv utlov vtlov ulnv vlnv, the list entry and
+        # two pairs' places read, per element geometry (7 doubles), distances
+        # (3) and the external flag; the record written (case word, 2 places,
+        # 2 flux coefficients, 2 Courant numbers)
+        "conz3d_prep": 6 * EL * p + 12 * EL + E * (56 + 24 + 4) + EL * (28 + 2 * p),
+        # per substep: the record, the list entry and the vertices' places
+        # read, per element its list positions and two pairs' weights; 3
+        # horizontal terms per tracer written, each tracer read
+        "conz3d_elem": 3 * ntr * EL * p + ntr * NL * p + EL * (36 + 2 * p) + E * (16 + 48),
+        # horizontal terms and 4 * area per list position read; the tile's
+        # entry, hdknv hdkov wlnv difv read, each tracer read and written
+        "conz3d_node": 3 * ntr * EL * p + (4 + 2 * ntr) * NL * p + 2 * N * p + 3 * E * 8 + 16 * NL + 2 * N * 4,
         "transports_final": 8 * EL * p + E * (12 + 56 + 3 * p + 2 * p),
         "hydro_vertical": 4 * EL * p + 4 * NL * p + N * p,
         "setdepth": EL * p + NL * p + E * 3 * p,
@@ -109,11 +109,10 @@ def _kernel_bytes(b, p, brows, ntr=2):
 # kernel names of the timed groups as rocprofv3 prints them (value type V)
 # kernel-name prefixes (template arguments after the value type vary with
 # the iteration-kernel variant) of each timed group's kernel
-KERNEL_NAMES = {"bicg_a": "k_bicg_a<{v},", "bicg_b": "k_bicg_b<{v},",
-                "bilu_factor": "k_bilu_factor<{v}>", "conz3d_elem": "k_conz_elem<{v}, 2, false, false>",
+KERNEL_NAMES = {"bilu_factor": "k_bilu_factor<{v}>", "conz3d_elem": "k_conz_elem_lds<{v}, 2>",
                 "conz3d_prep": "k_conz_prep<{v}>",
-                "conz3d_node": "k_conz_node<{v}, 12, 2, false>", "hydro_vertical": "k_hydro_vertical<{v}, 12>",
-                "hydro_intern": "k_hydro_intern<{v}, 12, false>"}
+                "conz3d_node": "k_conz_node<{v}, 2, false>", "hydro_vertical": "k_hydro_vertical<{v}, 12,",
+                "hydro_intern": "k_hydro_intern<{v}, false>"}
 
 
 def _measured_traffic(path, group, vtype):
