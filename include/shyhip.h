@@ -55,7 +55,7 @@ typedef struct {
     int iclin;
     /* zeta solver */
     double rtol, atol;                          /* BiCGStab tolerances (1e-8)   */
-    int itermax;                                /* max matvecs (1000)           */
+    int itermax;  /* max matvecs (1000); <= 0: 100000 iterations, FP32 500 a round */
     double refine_rtol;                         /* FP32 path: FP64 refinement residual target */
     int block_rows;                             /* block-ILU(0) block size (<= 1024), 0 = auto */
     int tri_sweeps;                             /* 0: exact level-scheduled triangular solves;

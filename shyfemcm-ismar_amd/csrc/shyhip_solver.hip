@@ -1357,6 +1357,7 @@ struct ZetaArgs {
     double *x;
     double tol;
     int maxref;
+    int maxit;                           // iterations of a Krylov solve (krylov_cap)
 };
 
 // Exact substitution with one triangular factor of a block by one wavefront
@@ -2072,6 +2073,9 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
             nmv = 1 + 2 * it;
             if (!(rn > target)) { conv = 1; break; }
             if (it > 0 && a.itermax > 0 && 1 + 2 * it >= a.itermax) { maxit = 1; break; }
+            // without an itermax nothing else ends a recurrence that
+            // stagnates above its target (no convergence: the host's errors)
+            if (it >= z.maxit) break;
             if (it == 0) {
                 p = r;
 #pragma unroll
@@ -2267,6 +2271,13 @@ static int krylov_outcome(Model &M, const int *c, int *iters, int slot) {
     return 0;
 }
 
+// Iterations of one Krylov solve at most (FP32: of one refinement round),
+// also without an itermax.
+static int krylov_cap(const Model &M) {
+    if (M.prec == SHYHIP_FP64) return M.p.itermax > 0 ? (M.p.itermax + 1) / 2 + 1 : 100000;
+    return M.p.itermax > 0 ? (M.p.itermax + 1) / 2 : 500;
+}
+
 // One iteration is two kernels (k_bicg_a, k_bicg_b).  Iterations are
 // enqueued in chunks between host checks of the device flags;
 // the first chunk is the iteration count of the previous solve of the same
@@ -2283,7 +2294,7 @@ static int bicgstab_t(Model &M, SolvArgs<V> &a, int *iters, int slot, int zero_x
     const int g = a.nblk;
     const size_t lds = apply_lds<V>(M), ilds = iter_lds<V, MODE>(M);
     int it = 0, c[CT_WORDS] = {};
-    const int maxit = M.p.itermax > 0 ? (M.p.itermax + 1) / 2 + 1 : 100000;
+    const int maxit = krylov_cap(M);
     int chunk = std::max(2, M.sv.last_its[slot] + 1);
     for (;;) {
         // the chunk's iterations (after the initialisation, for the first)
@@ -2490,7 +2501,7 @@ static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::func
     z.dent_f = M.m.z_dentf; z.dent_b = M.m.z_dentb; z.dptr_f = M.m.z_dptrf; z.dptr_b = M.m.z_dptrb;
     z.chunk_f = M.m.z_chf; z.chunk_b = M.m.z_chb; z.nch_f = M.m.z_nchf; z.nch_b = M.m.z_nchb;
     z.xch = M.sv.xch; z.pslot = M.sv.pslot;
-    z.rhs = M.s.rhs; z.x = M.s.x; z.tol = M.p.refine_rtol; z.maxref = kMaxRefine;
+    z.rhs = M.s.rhs; z.x = M.s.x; z.tol = M.p.refine_rtol; z.maxref = kMaxRefine; z.maxit = krylov_cap(M);
     ZetaHold hold(p.dev, p.cost, p.cap);
     static_assert(kZetaSlotWords == (size_t)kZetaBufs * kPartCopies * kPartStride, "partial slots");
     hipLaunchKernelGGL(zeta_kernel<V>(M), dim3(M.sv.zeta_nwg), dim3(M.sv.zeta_t), p.lds, M.stream, a, z);
@@ -2580,7 +2591,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         a.rtol = M.p.inner_rtol;
         a.atol = 0.0;
         const int maxref = kMaxRefine;
-        const int itmax_inner = M.p.itermax > 0 ? (M.p.itermax + 1) / 2 : 500;
+        const int itmax_inner = krylov_cap(M);
         // iterations enqueued for round r: that round's count in the previous
         // solve plus one (kernels beyond convergence return at once but
         // still cost a launch); a round cut short by its chunk leaves a
