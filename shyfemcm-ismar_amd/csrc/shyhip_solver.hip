@@ -35,10 +35,9 @@
 
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <functional>
-#include <mutex>
 
+#include "shyhip_budget.h"
 #include "shyhip_internal.h"
 
 namespace shy {
@@ -2410,32 +2409,15 @@ static ZetaKernel<V> zeta_kernel(const Model &M) {
 // them for some hundred microseconds).  Launches that need no other
 // workgroup to proceed (everything else) end by themselves and only delay it.
 namespace {
-struct ZetaUnits {
-    std::mutex mu;
-    std::condition_variable cv;
-    std::unordered_map<int, double> used;     // per device
-};
-ZetaUnits &zeta_units() {
-    static ZetaUnits u;
+UnitBudget &zeta_units() {
+    static UnitBudget u;
     return u;
 }
 struct ZetaHold {
     int dev;
-    double cost;
-    ZetaHold(int d, double c, double cap) : dev(d), cost(c) {
-        ZetaUnits &u = zeta_units();
-        std::unique_lock<std::mutex> lk(u.mu);
-        u.cv.wait(lk, [&] { return u.used[dev] + cost <= cap; });
-        u.used[dev] += cost;
-    }
-    ~ZetaHold() {
-        ZetaUnits &u = zeta_units();
-        {
-            std::lock_guard<std::mutex> lk(u.mu);
-            u.used[dev] -= cost;
-        }
-        u.cv.notify_all();
-    }
+    long parts;
+    ZetaHold(int d, long n, long budget) : dev(d), parts(n) { zeta_units().take(dev, parts, budget); }
+    ~ZetaHold() { zeta_units().give(dev, parts); }
     ZetaHold(const ZetaHold &) = delete;
     ZetaHold &operator=(const ZetaHold &) = delete;
 };
@@ -2446,7 +2428,7 @@ struct ZetaHold {
 struct ZetaPlan {
     size_t lds = 0;
     int dev = 0;
-    double cost = -1., cap = 0.;
+    long cost = -1, cap = 0;
 };
 template <typename V>
 static ZetaPlan zeta_plan(Model &M) {
@@ -2479,8 +2461,8 @@ static ZetaPlan zeta_plan(Model &M) {
     }
     if (v.zeta_occ[exact] < 1) return p;
     p.dev = v.zeta_dev;
-    p.cap = 0.875 * v.zeta_cus;      // some units left to the rest of the step
-    const double cost = (double)v.zeta_nwg / v.zeta_occ[exact];
+    p.cap = unit_budget(v.zeta_cus);
+    const long cost = unit_parts(v.zeta_nwg, v.zeta_occ[exact]);
     if (cost <= p.cap) p.cost = cost;
     return p;
 }
@@ -2560,7 +2542,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         int rc = 0;
         bool done = false;
         const ZetaPlan plan = zeta_plan<double>(M);
-        if (plan.cost >= 0.) {
+        if (plan.cost >= 0) {
             int c[CT_WORDS] = {};
             if (zeta_run<double>(M, plan, a, tail, after, c, &done)) return 1;
             if (done) rc = krylov_outcome(M, c, &its, 0);
@@ -2616,7 +2598,7 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
         int plan = std::min((int)CT_NRITS, std::max(1, M.sv.last_nref)), enq = 0, c[CT_WORDS] = {}, boost = 1;
         const ZetaPlan zp = zeta_plan<float>(M);
         bool done = false;
-        if (zp.cost >= 0.) {
+        if (zp.cost >= 0) {
             auto tail = [&]() -> int { return wetdry(M.sv.ctrl + CT_REFCONV, nullptr); };
             if (zeta_run<float>(M, zp, a, tail, after, c, &done)) return 1;
             if (done) enq = maxref;       // all its rounds are behind it
