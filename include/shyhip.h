@@ -371,6 +371,14 @@ int  shyhip_set_deferred_checks(shyhip_model *h, int on);
  * shyhip_graph_stats: graphs instantiated and replays since create. */
 int  shyhip_set_graphs(shyhip_model *h, int on);
 int  shyhip_graph_stats(shyhip_model *h, long *builds, long *replays);
+/* The zeta solve in one launch (no counterpart in the reference): its
+ * workgroups wait for each other, at most `polls` polls each time (negative:
+ * the default, about 0.1 s).  A wait that runs out ends the launch, the solve
+ * is made with two kernels per iteration instead, and so are the next 16
+ * (twice as many after each further expiry, at most 1024); it counts as a
+ * solver retry.  With 0 polls nearly every wait runs out.  A call also
+ * forgets earlier expiries. */
+int  shyhip_set_wait_polls(shyhip_model *h, int polls);
 /* kernel-group timing with HIP events on the handle's stream (off by
  * default; enabling it adds a synchronisation at the end of every step).
  * id = 0 .. 19: set_dry, copy_uvz, hydro_intern, setnod, zeta_assemble,

@@ -2206,6 +2206,14 @@ int shyhip_set_graphs(shyhip_model *h, int on) {
     return 0;
 }
 
+int shyhip_set_wait_polls(shyhip_model *h, int polls) {
+    if (!h) return fail(nullptr, "null handle");
+    Solver &v = h->M.sv;
+    v.zeta_spins = polls;
+    v.zeta_rest = v.zeta_back = 0;
+    return 0;
+}
+
 int shyhip_graph_stats(shyhip_model *h, long *builds, long *replays) {
     if (!h || !builds || !replays) return fail(h ? &h->M : nullptr, "null argument");
     *builds = h->M.graph_builds;

@@ -238,6 +238,10 @@ struct Solver {               // Krylov work space (value type V = S of the mode
     void *xch = nullptr;
     unsigned long long *pslot = nullptr;
     int zeta_occ[2] = {0, 0}, zeta_dev = 0, zeta_cus = 0;
+    // polls of one of its waits (< 0: the default); after an expired wait the
+    // solves still to be made without it, and the number the next expiry
+    // doubles
+    int zeta_spins = -1, zeta_rest = 0, zeta_back = 0;
 };
 
 constexpr size_t kZetaSlotWords = (size_t)4 * 16 * 512 * 5;   // partial-sum slots of the one-launch solve

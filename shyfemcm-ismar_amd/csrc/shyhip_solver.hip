@@ -1253,12 +1253,13 @@ __global__ __launch_bounds__(kThreads) void k_resid_check(const double *part, in
 // The waits are bounded: the launch is made only when all its workgroups
 // can be resident together (zeta_slots), and a wait that still runs out sets
 // CT_WAIT and ends the workgroup.  Every other workgroup then runs out of
-// its own wait, and the host makes the solve with the two-kernel iteration.
+// its own wait, and the host makes the solve with the two-kernel iteration,
+// and the next ones too (zeta_expired).
 // The result counts only once every workgroup has written its part of it:
 // each puts one more partial after its stores, and the workgroup that sets
 // the convergence flags collects them first.
 constexpr int kWaitExpired = -9;
-constexpr int kSpinLimit = 1 << 17;      // polls of one wait (about 0.1 s)
+constexpr int kSpinLimit = 1 << 17;      // polls of one wait (about 0.1 s), unless the model sets its own
 constexpr int kZetaBufs = 4;
 // Partial sums per diagonal block and buffer, and their copies: every
 // workgroup reads all of them, so one copy makes all workgroups wait for the
@@ -1357,6 +1358,7 @@ struct ZetaArgs {
     double tol;
     int maxref;
     int maxit;                           // iterations of a Krylov solve (krylov_cap)
+    int spins;                           // polls of one wait
 };
 
 // Exact substitution with one triangular factor of a block by one wavefront
@@ -1500,7 +1502,7 @@ struct ZetaRow {
     int rows, group;
     U *xch;
     unsigned long long *pslot;
-    int epoch = 0;
+    int epoch = 0, spins;
     int *dead;
 
     // byte offset k of the offsets packed two per word
@@ -1671,7 +1673,7 @@ struct ZetaRow {
                     if ((int)threadIdx.x + k * T < nh) ok = ok && hv[k] != Slot<V>::empty;
             if (recv) ok = ok && rv != Slot<V>::empty;
             if (ok) break;
-            if (++spin > kSpinLimit) {
+            if (++spin > spins) {
                 *dead = 1;
                 break;
             }
@@ -1902,6 +1904,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
     R.xch = (typename Slot<V>::U *)z.xch;
     R.pslot = z.pslot;
     R.dead = &dead;
+    R.spins = z.spins;
     R.send = -1;
     R.nsend = z.nsend;
     int hcol[KH];
@@ -2133,7 +2136,7 @@ __global__ __launch_bounds__(T) void k_zeta(SolvArgs<V> a, ZetaArgs z) {
         if (tid < z.nwg) {
             int spin = 0;
             while (slot_get(ps + tid) == Slot<double>::empty) {
-                if (++spin > kSpinLimit) {
+                if (++spin > z.spins) {
                     dead = 1;
                     break;
                 }
@@ -2423,8 +2426,8 @@ struct ZetaHold {
 };
 }  // namespace
 
-// LDS, device share and capacity of this model's one-launch solve under its
-// current parameters; cost < 0: it cannot run (the two-kernel iteration does)
+// LDS, device share and capacity of this model's next one-launch solve under
+// its current parameters; cost < 0: it cannot run (the two-kernel iteration does)
 struct ZetaPlan {
     size_t lds = 0;
     int dev = 0;
@@ -2435,6 +2438,10 @@ static ZetaPlan zeta_plan(Model &M) {
     ZetaPlan p;
     Solver &v = M.sv;
     if (v.zeta_t == 0) return p;
+    if (v.zeta_rest > 0) {                        // see zeta_expired
+        v.zeta_rest--;
+        return p;
+    }
     const int mode = zeta_mode(M), exact = mode != kSwept;
     if (exact && sizeof(V) == 4) return p;        // FP64 only (see host_zeta_tables)
     // sweeps keep the factor row in registers (and need its slot-major copy),
@@ -2467,6 +2474,17 @@ static ZetaPlan zeta_plan(Model &M) {
     return p;
 }
 
+// A wait that expired costs the solve about 0.1 s, and what kept its
+// workgroups apart (another process's work on the device) may last: the next
+// solves are made with the two-kernel iteration, twice as many after each
+// further expiry.
+constexpr int kZetaBackFirst = 16, kZetaBackMost = 1024;
+static void zeta_expired(Model &M) {
+    M.solver_retries++;
+    M.sv.zeta_back = std::min(kZetaBackMost, std::max(kZetaBackFirst, 2 * M.sv.zeta_back));
+    M.sv.zeta_rest = M.sv.zeta_back;
+}
+
 // the launch, `tail` and the read-back of the control words; *done false
 // when a wait expired
 template <typename V>
@@ -2484,6 +2502,7 @@ static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::func
     z.chunk_f = M.m.z_chf; z.chunk_b = M.m.z_chb; z.nch_f = M.m.z_nchf; z.nch_b = M.m.z_nchb;
     z.xch = M.sv.xch; z.pslot = M.sv.pslot;
     z.rhs = M.s.rhs; z.x = M.s.x; z.tol = M.p.refine_rtol; z.maxref = kMaxRefine; z.maxit = krylov_cap(M);
+    z.spins = M.sv.zeta_spins >= 0 ? M.sv.zeta_spins : kSpinLimit;
     ZetaHold hold(p.dev, p.cost, p.cap);
     static_assert(kZetaSlotWords == (size_t)kZetaBufs * kPartCopies * kPartStride, "partial slots");
     hipLaunchKernelGGL(zeta_kernel<V>(M), dim3(M.sv.zeta_nwg), dim3(M.sv.zeta_t), p.lds, M.stream, a, z);
@@ -2491,6 +2510,8 @@ static int zeta_run(Model &M, const ZetaPlan &p, SolvArgs<V> &a, const std::func
     if (tail && tail()) return 1;
     if (read_ctrl(M, c, CT_WORDS, after, std::is_same<V, double>::value ? CT_CONV : CT_REFCONV)) return 1;
     *done = c[CT_CONV] || c[CT_REFCONV] || !c[CT_WAIT];
+    if (*done) M.sv.zeta_back /= 2;
+    else zeta_expired(M);
     return 0;
 }
 
@@ -2546,7 +2567,6 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
             int c[CT_WORDS] = {};
             if (zeta_run<double>(M, plan, a, tail, after, c, &done)) return 1;
             if (done) rc = krylov_outcome(M, c, &its, 0);
-            else M.solver_retries++;
         }
         if (!done) rc = bicgstab<double>(M, a, &its, 0, 0, tail);
         it_total = its;
@@ -2602,7 +2622,6 @@ static int solve_once(Model &M, int *iters, int *refinements, int wetdry_bnew, b
             auto tail = [&]() -> int { return wetdry(M.sv.ctrl + CT_REFCONV, nullptr); };
             if (zeta_run<float>(M, zp, a, tail, after, c, &done)) return 1;
             if (done) enq = maxref;       // all its rounds are behind it
-            else M.solver_retries++;
         }
         for (;;) {
             if (!done) {

@@ -403,6 +403,12 @@ class Model:
         graphs (on by default); off launches every kernel directly."""
         self._chk(self.lib.shyhip_set_graphs(self.h, 1 if on else 0), "set_graphs")
 
+    def set_wait_polls(self, polls):
+        """Polls of one wait between the workgroups of a one-launch zeta solve
+        (negative: the default); a wait that runs out sends the solve, and the
+        next ones, to the two-kernel iteration."""
+        self._chk(self.lib.shyhip_set_wait_polls(self.h, int(polls)), "set_wait_polls")
+
     def graph_stats(self):
         """(graphs instantiated, graph replays) since create."""
         b, r = C.c_long(), C.c_long()

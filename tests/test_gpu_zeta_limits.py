@@ -60,3 +60,83 @@ def test_no_iteration_limit(gpu, nx, ny, brows, sweeps, prec):
     rc, z = _solve(m, b)
     assert rc == 0 and np.isfinite(z).all()
     m.close()
+
+
+# basins solved in one launch of several workgroups: swept, exact by dense
+# rows and by substitution
+SHAPES = {
+    "swept_256": (lambda: mesh.lagoon(6000, seed=5, lx=9000.0, ly=4500.0, nlv=1, tile=16), 256, 3),
+    "swept_512": (lambda: mesh.lagoon(33500, seed=6, nlv=1, tile=32), 256, 3),
+    "dense": (lambda: mesh.tidal_basin(nx=41, ny=30), 0, 0),
+    "substitution": (lambda: mesh.lagoon(15000, seed=6, nlv=1, tile=32), 256, 0),
+}
+
+
+# (exact substitution in FP32 takes two kernels per iteration anyway)
+@pytest.mark.parametrize("shape, prec", [(s, p) for s in SHAPES for p in ("fp64", "fp32")
+                                         if p == "fp64" or SHAPES[s][2] > 0])
+def test_expired_waits(gpu, shape, prec):
+    make, brows, sweeps = SHAPES[shape]
+    b = make()
+    m = gpu.Model(b, prec, params=dict(dt=300.0, ireib=5, block_rows=brows, tri_sweeps=sweeps, rtol=1e-11, atol=0.0,
+                                       refine_rtol=1e-12))
+    hia, hik = _element_systems(b, 3)
+    _assemble(m, b, hia, hik)
+    rc, want = _solve(m, b)
+    assert rc == 0 and m.stats()["solver_retries"] == 0
+    scale = np.abs(want).max()
+
+    def solves(n):
+        for _ in range(n):
+            rc, z = _solve(m, b)
+            assert rc == 0
+            # both residuals are at most 1e-11 (1e-12) of the load, times a
+            # condition of a few thousand, and rounded to 32 bits
+            assert np.abs(z - want).max() < 1e-6 * scale
+        return m.stats()["solver_retries"]
+
+    m.set_wait_polls(0)
+    assert solves(1) == 1              # expired, solved all the same
+    assert solves(16) == 1             # without the one-launch solve
+    assert solves(1) == 2              # tried again
+    assert solves(32) == 2             # twice as many without
+    assert solves(1) == 3
+    m.set_wait_polls(-1)               # forgets the expiries
+    assert solves(3) == 3
+    m.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_steps_through_expired_waits(gpu, prec):
+    """Hydro steps whose solves all expire, with elements that fall dry and
+    wet: in FP64 the same bits as the one-launch solves (the two iterations
+    add in the same order)."""
+    b = mesh.lagoon(3000, seed=7, lx=8000.0, ly=4000.0, nlv=1, tile=16, hmin=0.05)
+    params = dict(dt=60.0, ireib=5, block_rows=256, tri_sweeps=3)
+    names = ("znv", "utlnv", "vtlnv", "wlnv", "hdknv", "iwegv")
+
+    def run(expire):
+        m = gpu.Model(b, prec, params=params)
+        nloop = []
+        for n in range(1, 61):
+            if expire:
+                m.set_wait_polls(0)
+            m.step(-0.6 * min(1.0, n / 20.0) + 0.3 * np.sin(n / 8.0))
+            nloop.append(m.stats()["nloop"])
+        out = {k: m.pull(k) for k in names}
+        retries = m.stats()["solver_retries"]
+        m.close()
+        return out, nloop, retries
+
+    a, la, ra = run(False)
+    e, le, re = run(True)
+    assert ra == 0 and re == 60        # (a step's further solves follow an expiry)
+    assert max(la) > 1                 # the wet/dry loop repeated a solve
+    if prec == "fp64":
+        assert la == le
+        for k in names:
+            assert np.array_equal(a[k], e[k]), k
+    else:
+        # two solves to the same residual target differ in the last bits of
+        # 32-bit levels of about 1 m (6e-8), which 60 steps carry along
+        assert np.abs(a["znv"] - e["znv"]).max() < 2e-5
