@@ -2426,6 +2426,8 @@ struct ZetaHold {
 };
 }  // namespace
 
+constexpr size_t kZetaStatic = 20480;         // at least the kernels' static LDS
+
 // LDS, device share and capacity of this model's next one-launch solve under
 // its current parameters; cost < 0: it cannot run (the two-kernel iteration does)
 struct ZetaPlan {
@@ -2451,18 +2453,22 @@ static ZetaPlan zeta_plan(Model &M) {
     if (v.zeta_occ[exact] == 0) {
         // asked once per model and kind
         int dev = 0, cus = 0, occ = 0, lds_max = 0;
-        v.zeta_occ[exact] = -1;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-            p.lds + 20480 > (size_t)lds_max)
-            return p;
         const void *fn = (const void *)zeta_kernel<V>(M);
-        if (p.lds > kLdsLimit &&
-            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
+        // (the limit belongs to the kernel, which models of several sizes
+        // share: always the most that any of them may ask for)
+        const bool ok =
+            hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+            hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+            p.lds + kZetaStatic <= (size_t)lds_max &&
+            (p.lds <= kLdsLimit || hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       lds_max - (int)kZetaStatic) == hipSuccess) &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, v.zeta_t, p.lds) == hipSuccess && occ >= 1;
+        v.zeta_occ[exact] = ok ? occ : -1;
+        if (!ok) {
+            (void)hipGetLastError();     // (a refusal is no error of the launches that follow)
             return p;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, v.zeta_t, p.lds) != hipSuccess || occ < 1) return p;
-        v.zeta_occ[exact] = occ;
+        }
         v.zeta_dev = dev;
         v.zeta_cus = cus;
     }

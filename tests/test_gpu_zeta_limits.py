@@ -140,3 +140,23 @@ def test_steps_through_expired_waits(gpu, prec):
         # two solves to the same residual target differ in the last bits of
         # 32-bit levels of about 1 m (6e-8), which 60 steps carry along
         assert np.abs(a["znv"] - e["znv"]).max() < 2e-5
+
+
+def test_models_of_one_kernel(gpu):
+    """Two models whose solves run the same kernel with different amounts of
+    LDS above 64 KB (dense rows of blocks of 256 and of 150 rows), in turn."""
+    b = mesh.tidal_basin(nx=41, ny=30)
+    hia, hik = _element_systems(b, 3)
+    ms = [gpu.Model(b, "fp64", params=dict(dt=300.0, ireib=5, block_rows=r, tri_sweeps=0, rtol=1e-11, atol=0.0))
+          for r in (256, 150)]
+    got = []
+    for m in (ms[0], ms[1], ms[0], ms[1]):
+        _assemble(m, b, hia, hik)
+        rc, z = _solve(m, b)
+        assert rc == 0, m.lib.shyhip_last_error(m.h)
+        got.append(z)
+    for z in got[1:]:
+        assert np.abs(z - got[0]).max() < 1e-6 * np.abs(got[0]).max()
+    assert [m.stats()["solver_retries"] for m in ms] == [0, 0]
+    for m in ms:
+        m.close()
