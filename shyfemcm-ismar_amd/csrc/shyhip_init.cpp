@@ -811,10 +811,9 @@ void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<i
     // the residual target, which shows in the small components of a flow
     // (1e-4 of the cross-channel transports of a tidal channel; 1e-6 of the
     // levels)
-    if (exact && esize == 4) {
-        if (bs.brows <= 256 && !zeta_tables(n, rowptr, cols, bs, esize, 256, -1, zt)) zt = ZetaTables();
-        return;
-    }
+    if (exact && esize == 4) return;
+    // sweeps take one row per work-item of 256, as the two-kernel iteration does
+    if (!exact && bs.brows > kThreads) return;
     if (exact) {
         // dense rows of the blocks' inverses: 64 rows of a block of at most
         // 256, or 12 of a larger one, per workgroup (DenseShape)
@@ -829,8 +828,10 @@ void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<i
     const int n256 = bs.brows <= 256 ? (bs.brows % 64 == 0 ? (n + 255) / 256 : bs.nblk) : 1 << 30;
     if (n256 > kZetaSmall && zeta_tables(n, rowptr, cols, bs, esize, 512, 0, zt)) return;
     if (bs.brows <= 256 && zeta_tables(n, rowptr, cols, bs, esize, 256, 0, zt)) return;
+    // the halos of the two-kernel iteration, for sweeps (with exact
+    // substitution it stages its blocks instead)
     zt = ZetaTables();
-    if (bs.brows <= 256 && !zeta_tables(n, rowptr, cols, bs, esize, 256, -1, zt)) zt = ZetaTables();
+    if (!exact && !zeta_tables(n, rowptr, cols, bs, esize, 256, -1, zt)) zt = ZetaTables();
 }
 
 }  // namespace shy
