@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -668,18 +669,19 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
         // colour order: colours ascending, elements ascending within a colour
         std::vector<int> ek(4 * (size_t)nel, 0), ep(4 * (size_t)nel, 0), slev(3 * (size_t)nel);
         std::vector<double> saj4(3 * (size_t)nel);
-        for (int c = 1; c <= M.ncolor; c++)
-            for (int ie = 0; ie < nel; ie++) {
-                if (M.h_color[ie] != c) continue;
-                for (int ii = 0; ii < 3; ii++) {
-                    const int k = M.h_nen3v[3 * ie + ii];
-                    const int q = pos2[k]++;
-                    elc[q] = (ie << 2) | ii;
-                    ek[4 * (size_t)ie + ii] = k;
-                    ep[4 * (size_t)ie + ii] = q;
-                    slev[q] = ilhv[ie];
-                    saj4[q] = 4. * M.h_ev[19 * (size_t)ie + 9];
-                }
+        std::vector<int> cstart(M.ncolor + 2, 0), bycol(nel);
+        for (int ie = 0; ie < nel; ie++) cstart[M.h_color[ie] + 1]++;
+        for (int c = 0; c <= M.ncolor; c++) cstart[c + 1] += cstart[c];
+        for (int ie = 0; ie < nel; ie++) bycol[cstart[M.h_color[ie]]++] = ie;
+        for (int ie : bycol)
+            for (int ii = 0; ii < 3; ii++) {
+                const int k = M.h_nen3v[3 * ie + ii];
+                const int q = pos2[k]++;
+                elc[q] = (ie << 2) | ii;
+                ek[4 * (size_t)ie + ii] = k;
+                ep[4 * (size_t)ie + ii] = q;
+                slev[q] = ilhv[ie];
+                saj4[q] = 4. * M.h_ev[19 * (size_t)ie + 9];
             }
         rc |= dalloc(M, &m.conz_ek, ek.size()) || upload(M, m.conz_ek, ek.data(), ek.size());
         rc |= dalloc(M, &m.conz_ep, ep.size()) || upload(M, m.conz_ep, ep.data(), ep.size());
@@ -706,7 +708,7 @@ int shyhip_set_basin(shyhip_model *h, const int *nen3v, const float *xgv, const 
     // elements, layer by layer) and the node tiles (at most node_tile nodes
     // and kNodeItems node-layers each)
     {
-        const std::vector<int> items = elem_layer_items(nel, ilhv);
+        const std::vector<int> &items = M.h_eitem = elem_layer_items(nel, ilhv);
         if (nel >= (1 << 26)) return fail(&M, "at most 2^26 elements");
         const int tn = M.p.node_tile > 0 ? std::min(M.p.node_tile, kNodeTileMax) : kNodeTileMax;
         std::vector<int> tiles{0};
@@ -1146,51 +1148,56 @@ static int conz_place_tables(Model &M, const std::vector<int> &tup) {
     dfree(m.conz_uoff); dfree(m.conz_uptr); dfree(m.conz_uvert); dfree(m.conz_upair);
     m.conz_uoff = m.conz_uptr = nullptr;
     m.conz_uvert = m.conz_upair = nullptr;
-    const std::vector<int> items = elem_layer_items(M.nel, M.h_ilhv.data());
+    const std::vector<int> &items = M.h_eitem;
     const size_t n = items.size(), nel = M.nel;
     const int nwg = (int)((n + kThreads - 1) / kThreads);
     if ((size_t)M.nlvdi * M.nkn > 0x7fffffffu) return 0;
-    std::vector<unsigned> vert(n), pair(6 * n, 0);
+    // (not cleared: the threads that fill them touch them first)
+    std::unique_ptr<unsigned[]> vert(new unsigned[n]), pair(new unsigned[6 * n]);
     std::vector<std::vector<int>> lists(nwg);
     std::atomic<bool> fits{true};
     parallel_for(nwg, 16, [&](int w_begin, int w_end) {
-        // the offsets of a workgroup in an open-addressing table, then sorted
-        constexpr int kSlots = 4 * kConzUniq;
-        std::vector<int> key(kSlots), val(kSlots);
+        // the offsets of a workgroup in an open-addressing table, then sorted;
+        // at[]: the table's slot of each of an entry's offsets, three vertices
+        // and three nodes of each pair's upwind element (-1: none)
+        constexpr int kSlots = 4 * kConzUniq, kOffs = 21;
+        std::vector<int> key(kSlots), val(kSlots), at(kOffs * kThreads);
         for (int w = w_begin; w < w_end && fits; w++) {
             std::fill(key.begin(), key.end(), -1);
             std::vector<int> &u = lists[w];
-            auto slot = [&](int off) {
+            auto put = [&](int off) -> int {
                 unsigned h = ((unsigned)off * 2654435761u) >> 20;
                 static_assert(kSlots == 1 << 12, "hash bits");
                 while (key[h] != off && key[h] != -1) h = (h + 1) & (kSlots - 1);
-                return h;
-            };
-            auto put = [&](int off) {
-                const unsigned h = slot(off);
                 if (key[h] == -1) { key[h] = off; u.push_back(off); }
+                return (int)h;
             };
             const size_t i0 = (size_t)w * kThreads, i1 = std::min(n, i0 + kThreads);
-            auto each = [&](size_t i, auto &&vertex, auto &&upwind) {
+            for (size_t i = i0; i < i1 && u.size() <= (size_t)kConzUniq; i++) {
                 const int ie = (int)((unsigned)items[i] >> 5), l0 = items[i] & 31;
-                for (int q = 0; q < 3; q++) vertex(q, l0 * M.nkn + M.h_nen3v[3 * (size_t)ie + q]);
+                int *a = &at[kOffs * (i - i0)];
+                for (int q = 0; q < 3; q++) *a++ = put(l0 * M.nkn + M.h_nen3v[3 * (size_t)ie + q]);
                 for (int p = 0; p < 6; p++) {
                     const int *up = &tup[4 * ((size_t)p * nel + ie)];
-                    if (up[3] > l0)
-                        for (int q = 0; q < 3; q++) upwind(p, q, l0 * M.nkn + up[q]);
+                    for (int q = 0; q < 3; q++) *a++ = up[3] > l0 ? put(l0 * M.nkn + up[q]) : -1;
                 }
-            };
-            for (size_t i = i0; i < i1 && u.size() <= (size_t)kConzUniq; i++)
-                each(i, [&](int, int off) { put(off); }, [&](int, int, int off) { put(off); });
+            }
             if (u.size() > (size_t)kConzUniq) { fits = false; break; }
             std::sort(u.begin(), u.end());
-            for (size_t j = 0; j < u.size(); j++) val[slot(u[j])] = (int)j;
-            for (size_t i = i0; i < i1; i++)
-                each(
-                    i, [&](int q, int off) { vert[i] |= (unsigned)val[slot(off)] << (10 * q); },
-                    [&](int p, int q, int off) {
-                        pair[(size_t)p * n + i] |= (unsigned)val[slot(off)] << (10 * q) | 1u << 30;
-                    });
+            for (size_t j = 0; j < u.size(); j++) {
+                unsigned h = ((unsigned)u[j] * 2654435761u) >> 20;
+                while (key[h] != u[j]) h = (h + 1) & (kSlots - 1);
+                val[h] = (int)j;
+            }
+            for (size_t i = i0; i < i1; i++) {
+                const int *a = &at[kOffs * (i - i0)];
+                auto places = [&](const int *b) { return (unsigned)(val[b[0]] | val[b[1]] << 10 | val[b[2]] << 20); };
+                vert[i] = places(a);
+                for (int p = 0; p < 6; p++) {
+                    const int *b = a + 3 + 3 * p;
+                    pair[(size_t)p * n + i] = b[0] < 0 ? 0u : places(b) | 1u << 30;
+                }
+            }
         }
     });
     if (!fits) return 0;
@@ -1200,8 +1207,8 @@ static int conz_place_tables(Model &M, const std::vector<int> &tup) {
     for (int w = 0; w < nwg; w++) std::copy(lists[w].begin(), lists[w].end(), off.begin() + ptr[w]);
     int rc = dalloc(M, &m.conz_uptr, ptr.size()) || upload(M, m.conz_uptr, ptr.data(), ptr.size());
     rc |= dalloc(M, &m.conz_uoff, off.size()) || upload(M, m.conz_uoff, off.data(), off.size());
-    rc |= dalloc(M, &m.conz_uvert, vert.size()) || upload(M, m.conz_uvert, vert.data(), vert.size());
-    rc |= dalloc(M, &m.conz_upair, pair.size()) || upload(M, m.conz_upair, pair.data(), pair.size());
+    rc |= dalloc(M, &m.conz_uvert, n) || upload(M, m.conz_uvert, vert.get(), n);
+    rc |= dalloc(M, &m.conz_upair, 6 * n) || upload(M, m.conz_upair, pair.get(), 6 * n);
     return rc;
 }
 

@@ -351,6 +351,7 @@ struct Model {
     std::string err;
     // host-side copies needed for init / plugin / checks
     std::vector<int> h_nen3v, h_rowptr, h_cols, h_ijp, h_color, h_ilhv, h_ilhkv, h_ibnd, h_ibtyp, h_iextb;
+    std::vector<int> h_eitem; // Mesh::conz_eitem
     std::vector<float> h_x, h_y;
     std::vector<double> h_ev;             // [19*nel] reference ev layout
     std::vector<double> h_coo, h_rvec;    // plugin accumulation (c2coo, rvec2d)
