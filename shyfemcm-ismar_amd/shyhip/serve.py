@@ -54,16 +54,24 @@ class Request:
 
 
 def footprint_bytes(basin, precision: str, ntracer: int = 0) -> int:
-    """Estimated device memory of one resident run: about 30 element-layer
-    and 20 node-layer state arrays, the zeta matrix with its block factors
-    (CSR and fixed-stride copies), its ELL slices and 12 Krylov vectors, plus
-    the connectivity and geometry tables."""
+    """Estimated device memory of one resident run: the state, geometry and
+    column tables by their extents (all element-layers and node-layers for
+    the fields, the existing ones for the work lists), the zeta matrix with its
+    block factors, ELL slices and Krylov vectors per node, the transport's
+    scratch, records, TVD tables and spare fields with tracers, and 15 % for
+    the granularity of allocations."""
     p = 8 if precision == "fp64" else 4
-    EL = basin.nel * basin.nlv
-    NL = basin.nkn * (basin.nlv + 1)
-    nnz = 7 * basin.nkn
-    return int(30 * EL * p + (20 + 2 * ntracer) * NL * p + nnz * (8 + 4 + 3 * p + 24) + 12 * basin.nkn * 8
-               + 10 * basin.nkn * (8 + p) + basin.nel * (12 + 56 + 6 * 12 + 18 * 12))
+    L, E, N = basin.nlv, basin.nel, basin.nkn
+    elems, nodes = int(np.asarray(basin.ilhv).sum()), int(np.asarray(basin.ilhkv).sum())
+    nnz = N + 2 * (N + E)
+    n = p * (E * (13 * L + 38) + N * (8 * L + 10) + (3 * E + 2 * N) * L) + 300 * E + 130 * N
+    n += 12.5 * elems + 21 * nodes
+    n += N * (1100 + 40 * p) + 12 * nnz
+    if ntracer:
+        n += ntracer * p * (2 * L * N + (3 * E + 2 * N) * L)
+        n += (ntracer + 1) // 2 * elems * (36 + 6 * p) + p * (5 * E + 2 * N) * L
+        n += 38 * elems + 240 * E
+    return int(1.15 * n)
 
 
 def forcing(req: Request, n: int, dt: float):
