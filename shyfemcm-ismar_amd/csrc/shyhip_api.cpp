@@ -30,7 +30,7 @@ int hip_check(Model &M, hipError_t e, const char *what) {
 }
 
 int wait_report(Model &M, int word, int seq) {
-    const auto there = [&] { return __atomic_load_n(M.h_pinned + word, __ATOMIC_ACQUIRE) == seq; };
+    const auto there = [&] { return (int)((unsigned)__atomic_load_n(M.h_pinned + word, __ATOMIC_ACQUIRE) - (unsigned)seq) >= 0; };
     const auto t0 = std::chrono::steady_clock::now();
     for (int i = 1;; i++) {
         if (there()) return 0;

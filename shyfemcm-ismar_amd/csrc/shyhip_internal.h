@@ -205,7 +205,7 @@ enum { CT_STOPIT = 0, CT_CONV = 1, CT_FAIL = 2, CT_NMV = 3, CT_ITS = 4, CT_REFCO
 
 // words of Model::h_pinned: device error words, scalar-stability results (one
 // model), solver control words, and the numbers of the last reports
-enum { HP_ERR = 0, HP_STAB = 8, HP_CTRL = 16, HP_SEQ = 40, HP_SEQ_STAB = 41, HP_GO = 42 };
+enum { HP_ERR = 0, HP_STAB = 8, HP_CTRL = 16, HP_SEQ = 40, HP_SEQ_STAB = 41, HP_GO = 42, HP_PIECE = 43 };
 
 struct Solver {               // Krylov work space (value type V = S of the model)
     int nblk = 0, brows = 0, max_blk_nnz = 0, max_blk_pairs = 0, nparts = 0, max_elev = 0;
@@ -578,8 +578,8 @@ int launch_bndo(Model &M, const TracerSet &ts, hipStream_t st, int isact, void *
 int launch_scalar_stability(Model &M, float rstol, int *istot, double *rindex);
 
 // helpers
-// Waits until word `word` of h_pinned holds seq, which a kernel on the
-// model's stream writes after its results: polled for a few milliseconds (a
+// Waits until word `word` of h_pinned holds seq or a later number, which a
+// kernel on the model's stream writes after its results: polled for a few milliseconds (a
 // stream synchronisation returns 10 us later, and a copy before it is one
 // more kernel), then by synchronising.
 int wait_report(Model &M, int word, int seq);

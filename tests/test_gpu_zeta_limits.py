@@ -160,3 +160,29 @@ def test_models_of_one_kernel(gpu):
     assert [m.stats()["solver_retries"] for m in ms] == [0, 0]
     for m in ms:
         m.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_iterations_in_pieces(gpu, prec):
+    """A basin beyond the one-launch solve whose iterations are enqueued in
+    several pieces (of 28 iterations at 140k rows): replayed from graphs or
+    launched one by one, the same bits."""
+    b = mesh.lagoon(140000, seed=7, nlv=1, tile=32)
+    hia, hik = _element_systems(b, 3)
+    out, its = [], C.c_int()
+    for graphs in (True, False):
+        m = gpu.Model(b, prec, params=dict(dt=300.0, ireib=5, block_rows=256, tri_sweeps=3, rtol=1e-13, atol=0.0,
+                                           inner_rtol=1e-7, refine_rtol=1e-12))
+        m.set_graphs(graphs)
+        _assemble(m, b, hia, hik)
+        for _ in range(2):                      # the second enqueues the iterations of the first
+            rc, z = _solve(m, b)
+            assert rc == 0
+        assert m.lib.shyhip_system_solve_device(m.h, C.byref(its)) == 0
+        out.append((z, its.value))
+        builds = m.graph_stats()[0]
+        assert builds > 2 if graphs else builds == 0
+        m.close()
+    print(prec, "iterations", out[0][1])
+    assert out[0][1] == out[1][1] > (42 if prec == "fp64" else 0)
+    assert np.array_equal(out[0][0], out[1][0])
