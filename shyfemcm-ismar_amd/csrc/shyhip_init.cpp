@@ -805,12 +805,14 @@ void host_zeta_tables(int n, const std::vector<int> &rowptr, const std::vector<i
     if (bs.brows > 1024) return;
     for (int i = 0; i < n; i++)
         if (rowptr[i + 1] - rowptr[i] > kEllWidth) return;
-    // FP32 with exact substitution keeps the two-kernel iteration, whose
-    // rounds of the refinement end at the iterations enqueued for them: run to
-    // their inner tolerance in one launch they leave another remainder below
-    // the residual target, which shows in the small components of a flow
-    // (1e-4 of the cross-channel transports of a tidal channel; 1e-6 of the
-    // levels)
+    // FP32 with exact substitution keeps the two-kernel iteration and its
+    // results.  In one launch a refinement round runs to its inner tolerance,
+    // on two kernels to the iterations enqueued for it, and each leaves
+    // another remainder below the residual target.  Rounded into a 32-bit
+    // state that moves the small components of a flow by as much as they are
+    // off anyway: with sweeps the cross-channel transports of tidal channels
+    // differ by up to 4e-4 of their norm between the two, and both are 3e-4
+    // from the FP64 model's (levels 9e-7 and 7e-7).
     if (exact && esize == 4) return;
     // sweeps take one row per work-item of 256, as the two-kernel iteration does
     if (!exact && bs.brows > kThreads) return;

@@ -186,3 +186,35 @@ def test_iterations_in_pieces(gpu, prec):
     print(prec, "iterations", out[0][1])
     assert out[0][1] == out[1][1] > (42 if prec == "fp64" else 0)
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("nx, ny", [(41, 21), (80, 9), (120, 60)])
+def test_fp32_steps_in_one_launch(gpu, nx, ny):
+    """A tidal channel in FP32 with swept solves at the default tolerances, by
+    one launch and by two kernels per iteration: no component, the weak
+    cross-channel transports included, is further from the FP64 model in the
+    one launch.  Both errors are those of a 32-bit state that rounds another
+    remainder of the solve every step, sums of many independent roundings:
+    of one size, not of one value."""
+    b = mesh.tidal_basin(nx=nx, ny=ny)
+    names = ("znv", "utlnv", "vtlnv")
+
+    def run(prec, polls, **kw):
+        m = gpu.Model(b, prec, params=dict(dt=300.0, ireib=5, block_rows=256, tri_sweeps=3, **kw))
+        m.set_wind(*mesh.wind_stress(3.0, 0.4))
+        for n in range(1, 25):
+            m.set_wait_polls(polls)
+            m.step(min(1.0, n / 12) * mesh.tide_level(n * 300.0))
+        out = {k: m.pull(k).astype(np.float64) for k in names}
+        retries = m.stats()["solver_retries"]
+        m.close()
+        return out, retries
+
+    ref, _ = run("fp64", -1, rtol=1e-13, atol=0.0)
+    one, r1 = run("fp32", -1)
+    two, r2 = run("fp32", 0)
+    assert r1 == 0 and r2 == 24
+    for k in names:
+        e1, e2 = (np.linalg.norm(o[k] - ref[k]) / np.linalg.norm(ref[k]) for o in (one, two))
+        print(nx, ny, k, "one launch %.2e two kernels %.2e" % (e1, e2))
+        assert e1 < 1.5 * e2
