@@ -55,8 +55,12 @@ int graph_run(Model &M, hipStream_t st, const std::string &key, const std::funct
     if (it == M.graphs.end()) {
         std::lock_guard<std::recursive_mutex> lock(device_lock());
         // a bounded cache: the argument sets of a run are few (rotating
-        // buffers, substep counts); start over if a run keeps making new ones
+        // buffers, substep counts); start over if a run keeps making new ones,
+        // once the replays enqueued on any of the model's streams have ended
         if (M.graphs.size() >= 256) {
+            HIPCHK(M, hipStreamSynchronize(M.stream));
+            if (M.tr0_stream) HIPCHK(M, hipStreamSynchronize(M.tr0_stream));
+            for (hipStream_t s : M.tr_stream) HIPCHK(M, hipStreamSynchronize(s));
             for (auto &g : M.graphs) (void)hipGraphExecDestroy(g.second);
             M.graphs.clear();
         }
