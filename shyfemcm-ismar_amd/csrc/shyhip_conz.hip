@@ -19,8 +19,8 @@
 //                the boundary mass flux of conz3d_nodes; the column
 //                coefficients go to LDS.  Phase 2, one work-item per node:
 //                the implicit vertical solve (:757-886) and the write-back.
-// Nudging, settling velocity and loads are not part of the supported
-// configurations; horizontal diffusion (rkpar) must be zero.
+// Horizontal diffusion (rkpar > 0) is part of the element term; nudging,
+// sinking and loads belong to launches of a single tracer (k_conz_node's EXT).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -1352,8 +1352,9 @@ __device__ inline void max_into(unsigned long long *p, unsigned long long v) {
 // thicknesses only where the diffusion has an explicit part.  With all of
 // them, three elements at a time and two wavefronts to a SIMD: 191 us on 300k
 // nodes of 20 layers, 36.5 on 50k of 12 (FP64), 134 in FP32 on 285k of 10,
-// against 137, 27 and 93.  Batches of one (141, 26.5, 93; 15.8 on 3k nodes
-// against 13.5) and three (160, 31, 105) lose.
+// against 137, 27 and 93.  Batches of one gain a little on 50k nodes and lose
+// more on 300k and 3k of 6 layers (141, 26.5, 93; 15.8 against 13.5), batches
+// of three lose everywhere (160, 31, 105; 13.7).
 constexpr int kStabBatch = 2;
 
 template <typename S>

@@ -244,10 +244,10 @@ struct InternElem {
 // work-item per column, its layers unrolled in registers, walked every
 // wavefront down to the deepest layer of the basin, one wavefront to a SIMD
 // from 16 layers on: 489 us on 300k nodes of 20 layers, 14.6 on 3k nodes of
-// 10 (FP64) against 184 and 8.8; equal (28 to 30 us) on 50k nodes of 12.
+// 6 (FP64) against 184 and 8.8; equal (28 to 30 us) on 50k nodes of 12.
 // The rows in scratch memory with rolled loops took 337 us, the columns split
 // by depth between two kernels 331.  Coupled columns in scratch memory took
-// 95 us on 9k nodes of 12 layers against 16.6.
+// 95 us on 9k nodes of 10 layers against 16.6.
 template <typename S, bool CORI>
 __global__ __launch_bounds__(kThreads) void k_hydro_intern(HydroArgs<S> a) {
     using R = S;

@@ -1225,9 +1225,11 @@ __global__ __launch_bounds__(kThreads) void k_resid_check(const double *part, in
 // rounds of loads of the matrix, factors and vectors every time: 16.4 us per
 // FP64 iteration on the 50k-node lagoon (196 blocks), 9.7 us as one launch;
 // a hydro step there 0.60 -> 0.37 ms, on 3k nodes 0.35 -> 0.21 ms, FP32 on
-// 60k nodes 0.61 -> 0.40 ms.  A load that sees another XCD's store takes
-// 0.9 us (12 workgroups) to 1.5 us (98), the two sums 0.4 us, the product
-// and 3 sweeps 1.6 us (256 work-items) or 2.0 us (512).
+// 60k nodes 0.61 -> 0.40 ms.  Of the clocks of a half iteration (4.9 us) on
+// 50k rows, 98 workgroups of 512, in all 11,400: 3,400 waiting for the slots,
+// 4,100 in the rest of the exchange (sums, puts, barriers), 2,900 in the
+// product and 3 sweeps; on 20k rows, 79 of 256, 9,600: 3,000, 3,200 and
+// 2,200; on 3k rows, 12 of 256, 8,400: 2,000, 3,100 and 2,200.
 //
 // Exchange.  Each half iteration has an epoch.  A workgroup puts its partial
 // sums into its own slots, and the elements of v (or t) that rows of other
@@ -1450,9 +1452,11 @@ struct SubExact {
 // keeps them in registers, and applies them to the block's whole right-hand
 // side, which it forms itself (the vectors of all the block's rows are kept
 // by each of its workgroups, the rows applied elsewhere come with the halo).
-// A step of the 41 x 21 basin (861 rows, one block) 1.09 -> 0.65 ms, of an 80
+// A step of the 41 x 21 basin (861 rows, one block) 1.09 -> 0.56 ms, of an 80
 // x 40 basin 2.38 -> 0.48 ms, FP64, against the substitution.  The rows are
-// computed in 20 to 30 us; what bounds the rest is the exchange.
+// computed in 20 to 30 us; of the 18,200 clocks of a half iteration on 861
+// rows 7,800 are the product (the matrix row read from cache) and the dense
+// rows, 6,200 the exchange outside its wait, 2,300 the wait.
 enum { kSwept = 0, kSubst = 1, kDense = 2 };
 template <int T>
 struct DenseShape {                      // 512: blocks of up to 256 rows; 1024: of up to 1024
