@@ -1387,7 +1387,7 @@ int shyhip_set_members(shyhip_model *h, int nmem, const int *node_start, const i
 // from member sm of src into member dm of dst (same basin: node, element
 // and layer counts, precision, tracers).  Node arrays [l*nkn + k] and
 // element arrays [l*nel + ie] are copied layer by layer, 2D arrays are one
-// layer; all arrays in one launch.
+// layer; all arrays in one launch (one strided copy each between devices).
 int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int sm) {
     if (!dst || !src) return fail(nullptr, "null handle");
     Model &D = dst->M, &S = src->M;
@@ -1429,7 +1429,18 @@ int shyhip_copy_member_state(shyhip_model *dst, int dm, shyhip_model *src, int s
         // zenv/zeov are vertex-major [v*nel + ie]: three "layers" of elements
         list.push_back({(char *)x.d + d0, (const char *)x.s + s0, dp, sp, w, (size_t)x.nl});
     }
-    if (launch_copy_arrays(D, list)) return 1;
+    // (models of two devices: a kernel of one cannot be relied on to read the
+    // other's memory)
+    hipDevice_t dd = 0, ds = 0;
+    HIPCHK(D, hipStreamGetDevice(D.stream, &dd));
+    HIPCHK(D, hipStreamGetDevice(S.stream, &ds));
+    if (dd == ds) {
+        if (launch_copy_arrays(D, list)) return 1;
+    } else {
+        for (const ArrayCopy &c : list)
+            HIPCHK(D, hipMemcpy2DAsync(c.dst, c.dpitch, c.src, c.spitch, c.width, c.rows, hipMemcpyDeviceToDevice,
+                                       D.stream));
+    }
     HIPCHK(D, hipStreamSynchronize(D.stream));
     return 0;
 }
